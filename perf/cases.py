@@ -288,3 +288,185 @@ def tolerance(case):
     if kind in ("block", "block_jvp"):
         return {"rel": 2e-2, "max": 0.2}
     return {"rel": 1.5e-3, "max": 0.0125} if case["dtype"] == "fp16" else {"rel": 1e-2, "max": 0.1}
+
+
+# ---------------------------------------------------------------------------------------------------------- in 64 bits
+ROWS = 4096                  # query rows worked on at once
+EXACT_FLOPS = 4e13           # beyond that a pass in 64 bits takes too long
+
+
+def _attend(q, k, v, tq=None, tk=None, tv=None, lens=None):
+    """softmax(q k^T / sqrt(d)) v of [B, H, L, d] tensors in 64 bits, its tangent (None without tq) and the log-sum-exp."""
+    scale = q.shape[-1] ** -0.5
+    o, lse = torch.empty_like(q), torch.empty(q.shape[:-1], device=q.device, dtype=q.dtype)
+    to = None if tq is None else torch.empty_like(q)
+    for b in range(q.shape[0]):
+        n = k.shape[2] if lens is None else int(lens[b])
+        for h in range(q.shape[1]):
+            kk, vv = k[b, h, :n], v[b, h, :n]
+            for r in range(0, q.shape[2], ROWS):
+                i = (b, h, slice(r, r + ROWS))
+                p = (q[i] @ kk.T).mul_(scale)
+                lse[i] = torch.logsumexp(p, dim=-1)
+                p.sub_(lse[i][:, None]).exp_()
+                o[i] = p @ vv
+                if tq is not None:
+                    s = tq[i] @ kk.T
+                    if tk is not None:
+                        s.addmm_(q[i], tk[b, h, :n].T)
+                    s.mul_(scale).mul_(p)
+                    to[i] = s @ vv - s.sum(dim=-1, keepdim=True) * o[i]
+                    if tv is not None:
+                        to[i] += p @ tv[b, h, :n]
+    return o, to, lse
+
+
+def _attend_grads(q, k, v, o, lse, dout):
+    scale = q.shape[-1] ** -0.5
+    dq, dk, dv = torch.empty_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    delta = (o * dout).sum(dim=-1, keepdim=True)
+    for b in range(q.shape[0]):
+        for h in range(q.shape[1]):
+            for r in range(0, q.shape[2], ROWS):
+                i = (b, h, slice(r, r + ROWS))
+                p = (q[i] @ k[b, h].T).mul_(scale).sub_(lse[i][:, None]).exp_()
+                dv[b, h] += p.T @ dout[i]
+                p.mul_((dout[i] @ v[b, h].T).sub_(delta[i])).mul_(scale)
+                dq[i] = p @ k[b, h]
+                dk[b, h] += p.T @ q[i]
+    return dq, dk, dv
+
+
+class _Attend(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, k, v):
+        o, _, lse = _attend(q, k, v)
+        ctx.save_for_backward(q, k, v, o, lse)
+        return o
+
+    @staticmethod
+    def backward(ctx, dout):
+        return _attend_grads(*ctx.saved_tensors, dout)
+
+
+def _norm_rope(x, weight, angles):
+    """x [B, S, H, D]; angles [S, D] or None."""
+    n = x * torch.rsqrt(x.pow(2).mean(dim=-1, keepdim=True) + 1e-6) * weight
+    if angles is None:
+        return n
+    a = angles[:, None, :]
+    return n * torch.cos(a) + torch.cat([-n[..., D // 2:], n[..., : D // 2]], dim=-1) * torch.sin(a)
+
+
+def _both(f, primals, tangents):
+    """f(*primals) as a tuple, and its tangents: Nones where `tangents` is None."""
+    if tangents is None:
+        y = f(*primals)
+        return y, (None,) * len(y)
+    return torch.func.jvp(f, primals, tuple(torch.zeros_like(p) if t is None else t for p, t in zip(primals, tangents)))
+
+
+def _block(w, heads, x, emb, lora, text, angles, tx=None, temb=None, tlora=None):
+    """A transformer block in 64 bits: x [B, T, H, W, K] -> its output and the output's tangent (None without tx)."""
+    F = torch.nn.functional
+    K, moves = x.shape[-1], tx is not None
+    attend = _Attend.apply if torch.is_grad_enabled() else lambda q, k, v: _attend(q, k, v)[0]
+    for name in ("self_attn", "cross_attn", "mlp"):
+        mod = "adaln_modulation_%s." % name
+
+        def modulated(x, emb, lora):
+            m = F.linear(F.linear(F.silu(emb), w[mod + "1.weight"]), w[mod + "2.weight"]) + lora
+            shift, scale, gate = (c[:, :, None, None, :] for c in m.chunk(3, dim=-1))
+            return F.layer_norm(x, (K,), eps=1e-6) * (1 + scale) + shift, gate
+
+        (n, gate), (tn, tgate) = _both(modulated, (x, emb, lora), (tx, temb, tlora) if moves else None)
+        if name == "mlp":
+            (r,), (tr,) = _both(lambda n: (F.linear(F.gelu(F.linear(n, w["mlp.layer1.weight"])), w["mlp.layer2.weight"]),),
+                                (n,), (tn,) if moves else None)
+        else:
+            own, g = name == "self_attn", lambda part: w["%s.%s.weight" % (name, part)]
+            split = lambda t: t.reshape(t.shape[0], -1, heads, D)
+            query = lambda n: (_norm_rope(split(F.linear(n, g("q_proj"))), g("q_norm"), angles if own else None).transpose(1, 2),)
+            keys = lambda c: (_norm_rope(split(F.linear(c, g("k_proj"))), g("k_norm"), angles if own else None).transpose(1, 2),
+                              split(F.linear(c, g("v_proj"))).transpose(1, 2))
+            (q,), (tq,) = _both(query, (n,), (tn,) if moves else None)
+            (k, v), (tk, tv) = _both(keys, (n if own else text,), (tn,) if moves and own else None)
+            merge = lambda o: F.linear(o.transpose(1, 2).flatten(-2), g("output_proj")).reshape(x.shape)
+            if moves:
+                o, to, _ = _attend(q, k, v, tq, tk, tv)
+                r, tr = merge(o), merge(to)
+            else:
+                r, tr = merge(attend(q, k, v)), None
+        (x,), (tx,) = _both(lambda x, r, gate: (x + gate * r,), (x, r, gate), (tx, tr, tgate) if moves else None)
+    return x, tx
+
+
+def _network(s, case):
+    F = torch.nn.functional
+    net, f = s["net"], lambda t: t.double()
+    w = {n: f(p) for n, p in net.named_parameters()}
+    B, T, Hh, W, K = case["B"], case["T"], case["Hh"], case["W"], case["H"] * D
+    pos = net.pos_embedder
+    rates = [10000.0 ** -f(r) for r in (pos.dim_temporal_range, pos.dim_spatial_range, pos.dim_spatial_range)]
+    steps = [torch.arange(n, device="cuda", dtype=torch.float64) for n in (T, Hh, W)]
+    steps[0] = steps[0] / f(s["fps"][0]) * pos.base_fps
+    e = [torch.outer(p, r) for p, r in zip(steps, rates)]
+    half = torch.cat([e[0][:, None, None].expand(T, Hh, W, -1), e[1][None, :, None].expand(T, Hh, W, -1),
+                      e[2][None, None].expand(T, Hh, W, -1)], dim=-1).reshape(T * Hh * W, -1)
+    angles = torch.cat([half, half], dim=-1)
+    x = torch.cat([f(s["x"]), f(s["mask"])[:, :, None].expand(B, 1, T, 2 * Hh, 2 * W)], dim=1)
+    x = x.reshape(B, -1, T, Hh, 2, W, 2).permute(0, 2, 3, 5, 1, 4, 6).flatten(-3)
+    x = F.linear(x, w["x_embedder.proj.1.weight"])
+    turn = f(s["time"])[..., None] * torch.exp(-math.log(10000.0) * torch.arange(K // 2, device="cuda", dtype=torch.float64) / (K // 2))
+    wave = torch.cat([torch.cos(turn), torch.sin(turn)], dim=-1)
+    lora = F.linear(F.silu(F.linear(wave, w["t_embedder.1.linear_1.weight"])), w["t_embedder.1.linear_2.weight"])
+    emb = wave * torch.rsqrt(wave.pow(2).mean(dim=-1, keepdim=True) + 1e-6) * w["t_embedding_norm.weight"]
+    for i in range(case["blocks"]):
+        own = "blocks.%d." % i
+        x, _ = _block({n[len(own):]: p for n, p in w.items() if n.startswith(own)}, case["H"], x, emb, lora, f(s["text"]), angles)
+    m = F.linear(F.linear(F.silu(emb), w["final_layer.adaln_modulation.1.weight"]), w["final_layer.adaln_modulation.2.weight"])
+    shift, scale = (c[:, :, None, None, :] for c in (m + lora[..., : 2 * K]).chunk(2, dim=-1))
+    y = F.linear(F.layer_norm(x, (K,), eps=1e-6) * (1 + scale) + shift, w["final_layer.linear.weight"])
+    y = y.reshape(B, T, Hh, W, 2, 2, 16)
+    return y.permute(0, 6, 1, 2, 4, 3, 5).reshape(B, 16, T, 2 * Hh, 2 * W)
+
+
+def exact(case, seed):
+    """What `run` returns, in 64-bit torch arithmetic on the same inputs; None for the largest cases."""
+    if _flops(case) > EXACT_FLOPS:
+        return None
+    s, kind = prepare(case, seed), case["kind"]
+    f = lambda t: t.detach().double()
+    if kind in ("attention_jvp", "cross_jvp"):
+        o, to, lse = _attend(*(f(t) for t in s["in"][:4]), *(f(t) for t in s["in"][4:]), lens=s.get("lens"))
+        return (o, to) if kind == "attention_jvp" else (o, to, lse)
+    if kind in ("attention", "attention_train", "cross_train"):
+        q, k, v = (f(t).transpose(1, 2).contiguous() for t in s["in"])
+        o, _, lse = _attend(q, k, v)
+        if kind == "attention":
+            return o.transpose(1, 2).contiguous()
+        grads = _attend_grads(q, k, v, o, lse, f(s["dout"]).transpose(1, 2).contiguous())
+        return tuple(t.transpose(1, 2).contiguous() for t in (o, *grads))
+    if kind.startswith("norm_rope"):
+        x, weight, angles, other = f(s["x"]), f(s["weight"]), f(s["angles"]).reshape(-1, D), f(s["other"])
+        if kind == "norm_rope_jvp":
+            return torch.func.jvp(lambda x: _norm_rope(x, weight, angles), (x,), (other,))
+        x.requires_grad_(True)
+        weight.requires_grad_(True)
+        y = _norm_rope(x, weight, angles)
+        return (y.detach(), *torch.autograd.grad(y, (x, weight), other))
+    if kind == "network":
+        with torch.no_grad():
+            return _network(s, case)
+    train = kind == "block_train"
+    w = {n: f(p).requires_grad_(train) for n, p in s["block"].named_parameters()}
+    x, angles = f(s["x"]).requires_grad_(train), f(s["angles"]).reshape(-1, D)
+    args = (w, case["H"], x, f(s["emb"]), f(s["lora"]), f(s["text"]), angles)
+    if not train:
+        with torch.no_grad():
+            if kind == "block":
+                return _block(*args)[0]
+            return _block(*args, f(s["tx"]), f(s["temb"]), f(s["tlora"]))
+    y, _ = _block(*args)
+    y.backward(f(s["dout"]))
+    return {"y": y.detach(), "dx": x.grad, **{n: p.grad for n, p in w.items()}}
