@@ -944,11 +944,11 @@ struct BwdGeom {
             k_tile_bytes = (size_t)(2 * ndb) * kFragBytes;            // the key stream holds K^T alone
             k_img_bytes = bh * n_k_tiles * k_tile_bytes;
         }
-        dkdv = plan(n_kblk, spill ? group : (int)bh, n_q_tiles, d->causal != 0);
-        dq = plan((d->Lq + kBlock - 1) / kBlock, (int)bh, n_k_tiles, d->causal != 0);
+        dkdv = plan(n_kblk, spill ? group : (int)bh, n_q_tiles, d->causal != 0, d->d, true);
+        dq = plan((d->Lq + kBlock - 1) / kBlock, (int)bh, n_k_tiles, d->causal != 0, d->d, false);
         size_t p1 = (size_t)dkdv.n_rem * dkdv.splits * kBlock * 2 * d->d * sizeof(float);
         if (spill && bh % group) {   // the last, smaller group has a plan of its own
-            const Plan last = plan(n_kblk, (int)(bh % group), n_q_tiles, d->causal != 0);
+            const Plan last = plan(n_kblk, (int)(bh % group), n_q_tiles, d->causal != 0, d->d, true);
             const size_t p3 = (size_t)last.n_rem * last.splits * kBlock * 2 * d->d * sizeof(float);
             p1 = p1 > p3 ? p1 : p3;
         }
@@ -963,11 +963,12 @@ struct BwdGeom {
     // How the (block of stationary rows, head) pairs of a kernel are dealt out (see choose_splits): the pairs of a partly
     // filled last round of workgroups are cut along the stream and bwd_combine_kernel adds the ranges up.
     struct Plan { int n_blk, n_pairs, n_full, n_rem, splits; };
-    static Plan plan(int n_blk, int bh, int n_stream_tiles, bool causal) {
+    static Plan plan(int n_blk, int bh, int n_stream_tiles, bool causal, int d, bool dkdv) {
         Plan s;
         s.n_blk = n_blk; s.n_pairs = n_blk * bh; s.n_full = s.n_pairs; s.n_rem = 0; s.splits = 1;
         const int rem = s.n_pairs % kNumCUs;
-        const int splits = causal ? 1 : choose_splits(rem, n_stream_tiles);
+        const double part = 0.3 + 0.7 * d / 128.0;
+        const int splits = causal ? 1 : choose_splits(rem, n_stream_tiles, StepCost{1.08 * part, 8.0}, (double)kBlock * (dkdv ? 2 : 1) * d * sizeof(float));
         if (splits < 2) return s;
         s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = splits;
         return s;
@@ -1105,7 +1106,7 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
         qp.n_blk = (g.n_q_tiles + kDqWaves - 1) / kDqWaves; qp.causal = d->causal; qp.sm_scale = d->sm_scale;
         for (int bh0 = 0; bh0 < BH; bh0 += g.group) {
             const int heads = BH - bh0 < g.group ? BH - bh0 : g.group;
-            const BwdGeom::Plan pl = heads == g.group ? g.dkdv : BwdGeom::plan(g.dkdv.n_blk, heads, g.n_q_tiles, d->causal != 0);
+            const BwdGeom::Plan pl = heads == g.group ? g.dkdv : BwdGeom::plan(g.dkdv.n_blk, heads, g.n_q_tiles, d->causal != 0, d->d, true);
             bp.bh0 = bh0;
             if (!launch(k_spill, lds_dkdv, pl, bp, true)) return COSMOS_ATTN_LAUNCH_FAILED;
             qp.bh0 = bh0;

@@ -110,21 +110,37 @@ inline bool allow_lds(const void* fn, size_t bytes) {
 
 // One workgroup of the attention kernels fits on a compute unit, so a launch of n_pairs equal workgroups runs in rounds
 // of kNumCUs and a partly filled last round costs a whole one.  The `rem` workgroups of that round may instead be cut
-// into S ranges of their stream (keys or queries) each: rem * S shorter workgroups that take ceil(rem S / kNumCUs) / S
-// of a round, plus a merge kernel.  Returns the smallest S (1 = leave it) that minimises that cost, among the S that
-// leave every range at least kMinStepsPerSplit barrier steps, if it saves at least a tenth of a round.
+// into S ranges of their stream (keys or queries) each: rem * S shorter workgroups, plus a merge kernel.  Returns the S
+// (1 = leave it) of the least cost in microseconds, where
+//   * a round of workgroups takes `steps` barrier steps of step_us each and range_us to start and end;
+//   * the step of a round that fills only a part of the chip is faster, as the part then clocks higher under its power limit:
+//     0.7 of the full chip's time for a few workgroups, growing with the square of the filled part (forward only, one round,
+//     384-row steps: 1.86 us at 112 of 256 workgroups, 1.95 at 160, 2.34 at 224, 2.66 in full rounds);
+//   * every range leaves slot_bytes of partial results, written once and read once by the merge kernel: 3.8 MB of them cost a
+//     microsecond, the merge kernel's launch three.
+// The constants are fits to B*H = 16 .. 80, 255 .. 17600 positions and S = 1 .. 16, every S measured.  What the rule that
+// counted rounds alone chose, and this one (us, forward + tangents unless said, head dim 128, with the re-tiling):
+//   1 x 16 x 1560: S = 11 243, S = 1 77;   1 x 40 x 512: S = 3 64, S = 1 40;   1 x 16 x 7040: S = 16 1093, S = 2 1012;
+//   forward only 1 x 16 x 3520: S = 8 222, S = 1 133;   1 x 16 x 5000: S = 8 388, S = 1 217;
+//   backward 1 x 16 x 1560: S = 11 267, S = 1 113.
+// The cost of a split has to come out at least a twentieth lower: the fits are no better than that.
 constexpr int kNumCUs = 256;          // MI355X
 constexpr int kMaxSplits = 16;
 constexpr int kMinStepsPerSplit = 4;
-inline int choose_splits(int rem, int n_steps) {
+struct StepCost { double step_us, range_us; };   // a barrier step in full rounds, and what a workgroup costs besides its steps
+inline int choose_splits(int rem, int n_steps, StepCost c, double slot_bytes) {
     if (rem <= 0) return 1;
     int best = 1;
-    double best_cost = 1.0;
-    for (int S = 2; S <= kMaxSplits && S * kMinStepsPerSplit <= n_steps; ++S) {
-        const double cost = (double)((rem * S + kNumCUs - 1) / kNumCUs) / S;
-        if (cost < best_cost - 1e-9) { best_cost = cost; best = S; }
+    double best_cost = 0.0;
+    for (int S = 1; S <= kMaxSplits && (S == 1 || S * kMinStepsPerSplit <= n_steps); ++S) {
+        const int rounds = (rem * S + kNumCUs - 1) / kNumCUs;
+        const double filled = (double)(rem * S) / (rounds * kNumCUs);
+        double cost = rounds * ((double)n_steps / S * c.step_us * (0.7 + 0.3 * filled * filled) + c.range_us);
+        if (S > 1) cost += 3.0 + (double)rem * S * slot_bytes / 3.8e6;
+        if (S == 1) best_cost = 0.95 * cost;
+        else if (cost < best_cost) { best_cost = cost; best = S; }
     }
-    return best_cost <= 0.9 ? best : 1;
+    return best;
 }
 
 // The workgroup-to-XCD maps and the rounds-of-kNumCUs arithmetic of the attention kernels assume a whole MI355X (256 compute

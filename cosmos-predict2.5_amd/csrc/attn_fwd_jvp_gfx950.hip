@@ -1533,7 +1533,10 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
     if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
     const int rem = s.n_pairs % kNumCUs;
     const int n_steps = fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d);   // barrier steps: 64 keys forward only, 32 with tangents
-    const int splits = choose_splits(rem, n_steps);
+    // (smaller head dims: fewer matrix instructions per step, the same exponentials)
+    const double part = 0.3 + 0.7 * (d->d_qk + d->d_v) / 256.0;
+    const StepCost c = fwd ? StepCost{2.66 * part, 13.0} : StepCost{1.21 * part, 8.0};
+    const int splits = choose_splits(rem, n_steps, c, (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4)));
     if (splits < 2) return s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = splits;
     return s;

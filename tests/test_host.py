@@ -88,6 +88,27 @@ def test_status_codes_for_bad_descriptors(pkg):
     assert L.status_string(0) == "ok"
 
 
+@pytest.mark.parametrize("H,L,tangents,ranges", [
+    (16, 1560, True, 1),      # 208 pairs in one round: a cut would only add partial results
+    (16, 2600, True, 3),      # 336 pairs: 80 of a second round, 3 ranges each
+    (16, 7040, True, 2),      # 880 pairs: 112 of a fourth round, 2 ranges each
+    (2, 2048, True, 6),       # 32 pairs, 64 steps: six ranges are as fast as the eight that fill the chip, with less to merge
+    (16, 3520, False, 1),     # forward only, 384 rows per pair: 160 pairs in one round
+    (16, 2000, False, 2),     # 96 pairs
+    (16, 37440, False, 8),    # 1568 pairs: 32 of a seventh round, 8 ranges each
+    (1, 100, False, 1),       # 2 steps: too short to cut
+])
+def test_key_range_plan(pkg, H, L, tangents, ranges):
+    """How many key ranges the pairs of a partly filled last round are cut into, read off the workspace for their partial results."""
+    lib = pkg._lib.load_library()
+    t = 0x8000000 if tangents else None
+    D = good_desc(pkg, B=1, H=H, Lq=L, Lkv=L, d_v=128, tq=t, tk=t, tv=t, to=t)
+    block = 128 if tangents else 384
+    rem = (L + block - 1) // block * H % 256
+    extra = lib.cosmos_attn_workspace_bytes(ctypes.byref(D)) - lib.cosmos_attn_packed_bytes(ctypes.byref(D))
+    assert extra == (0 if ranges == 1 else rem * ranges * block * (128 * (2 if tangents else 1) * 4 + 16))
+
+
 def good_bwd_desc(pkg, **over):
     D = pkg._lib.AttnBwdDesc()
     D.abi_version, D.dtype = pkg._lib.ABI_VERSION, pkg._lib.DTYPE_BF16
