@@ -172,6 +172,31 @@ class GeluDesc(ctypes.Structure):
     ]
 
 
+class LnModulateBwdDesc(ctypes.Structure):
+    """Mirror of ``struct cosmos_ln_modulate_bwd_desc``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("D", ctypes.c_int32), ("rows_per_group", ctypes.c_int32),
+        ("eps", ctypes.c_float), ("reserved", ctypes.c_int32),
+        ("rows", ctypes.c_int64),
+        ("x", ctypes.c_void_p), ("scale", ctypes.c_void_p), ("dy", ctypes.c_void_p), ("dskip", ctypes.c_void_p),
+        ("dx", ctypes.c_void_p), ("dshift", ctypes.c_void_p), ("dscale", ctypes.c_void_p),
+    ]
+
+
+class GatedResidualBwdDesc(ctypes.Structure):
+    """Mirror of ``struct cosmos_gated_residual_bwd_desc``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("D", ctypes.c_int32), ("rows_per_group", ctypes.c_int32),
+        ("rows", ctypes.c_int64),
+        ("dy", ctypes.c_void_p), ("res", ctypes.c_void_p), ("gate", ctypes.c_void_p),
+        ("dres", ctypes.c_void_p), ("dgate", ctypes.c_void_p),
+    ]
+
+
 EXPORTS = {
     "cosmos_attn_abi_version": (ctypes.c_int, []),
     "cosmos_attn_status_string": (ctypes.c_char_p, [ctypes.c_int]),
@@ -190,6 +215,10 @@ EXPORTS = {
     "cosmos_norm_rope_bwd": (ctypes.c_int, [ctypes.POINTER(NormRopeBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_ln_modulate": (ctypes.c_int, [ctypes.POINTER(LnModulateDesc), ctypes.c_void_p]),
     "cosmos_gated_residual": (ctypes.c_int, [ctypes.POINTER(GatedResidualDesc), ctypes.c_void_p]),
+    "cosmos_ln_modulate_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(LnModulateBwdDesc)]),
+    "cosmos_ln_modulate_bwd": (ctypes.c_int, [ctypes.POINTER(LnModulateBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "cosmos_gated_residual_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(GatedResidualBwdDesc)]),
+    "cosmos_gated_residual_bwd": (ctypes.c_int, [ctypes.POINTER(GatedResidualBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_gelu": (ctypes.c_int, [ctypes.POINTER(GeluDesc), ctypes.c_void_p]),
 }
 

@@ -28,26 +28,26 @@ from .dit_attention import Attention, I2VCrossAttention
 
 
 class _LnModulateFn(torch.autograd.Function):
-    """``LayerNorm(x) * (1 + scale) + shift`` as the fused pass, differentiable: the backward pass recomputes the
-    expression in fp32 with tensor-library ops and takes their gradients (x ``[B, T, H, W, D]``, shift / scale
-    ``[B, T, 1, 1, D]``)."""
+    """``LayerNorm(x) * (1 + scale) + shift`` as the fused pass, differentiable (x ``[B, T, H, W, D]``, shift / scale
+    ``[B, T, 1, 1, D]``).  Returns x as well, for the residual connection around what follows: both gradients of x then meet in
+    the fused backward pass."""
 
     @staticmethod
     def forward(ctx, x, shift, scale, eps):
         D = x.shape[-1]
         y, _ = ops.ln_modulate(x, shift.reshape(-1, D), scale.reshape(-1, D), eps=eps)
-        ctx.save_for_backward(x, shift, scale)
+        ctx.save_for_backward(x, scale)
         ctx.eps = eps
-        return y
+        ctx.set_materialize_grads(False)
+        return y, x
 
     @staticmethod
-    def backward(ctx, dy):
-        x, shift, scale = ctx.saved_tensors
-        with torch.enable_grad():
-            xf, sh, sc = (t.detach().float().requires_grad_(True) for t in (x, shift, scale))
-            y = F.layer_norm(xf, (x.shape[-1],), eps=ctx.eps) * (1 + sc) + sh
-        dx, dsh, dsc = torch.autograd.grad(y, (xf, sh, sc), dy.float())
-        return dx.to(x.dtype), dsh.to(shift.dtype), dsc.to(scale.dtype), None
+    def backward(ctx, dy, dskip):
+        x, scale = ctx.saved_tensors
+        if dy is None:
+            return dskip, None, None, None
+        dx, dshift, dscale = ops.ln_modulate_bwd(x, scale, dy, dskip, eps=ctx.eps)
+        return dx, dshift.reshape(scale.shape), dscale.reshape(scale.shape), None
 
 
 class _GatedResidualFn(torch.autograd.Function):
@@ -62,8 +62,8 @@ class _GatedResidualFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         res, gate = ctx.saved_tensors
-        dgate = (dy.float() * res.float()).sum(dim=(2, 3), keepdim=True).to(gate.dtype)
-        return dy, dy * gate, dgate
+        dres, dgate = ops.gated_residual_bwd(res, gate, dy)
+        return dy, dres, dgate.reshape(gate.shape)
 
 
 class _GeluFn(torch.autograd.Function):
@@ -241,14 +241,14 @@ class Block(nn.Module):
 
     def _forward_autograd(self, x, emb, crossattn_emb, rope, lora):
         """The differentiable path: the same kernels as the inference path (so both give the same bits), each behind an
-        autograd rule -- attention and RMSNorm + RoPE through their HIP backward kernels, the elementwise passes through
-        fp32 tensor-library arithmetic."""
+        autograd rule: attention, RMSNorm + RoPE, LayerNorm + modulation and the gated residuals through their HIP backward
+        kernels."""
         B, T, H, W, D = x.shape
         for name, norm, sub in (("self_attn", self.layer_norm_self_attn, self.self_attn),
                                 ("cross_attn", self.layer_norm_cross_attn, self.cross_attn),
                                 ("mlp", self.layer_norm_mlp, self.mlp)):
             shift, scale, gate = self._modulation(getattr(self, "adaln_modulation_" + name), emb, lora, x)
-            n = _LnModulateFn.apply(x, shift, scale, norm.eps)
+            n, x = _LnModulateFn.apply(x, shift, scale, norm.eps)
             if name == "mlp":
                 r = sub(n)
             else:

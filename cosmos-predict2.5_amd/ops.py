@@ -527,6 +527,54 @@ def gated_residual(x, res, gate, tx=None, tres=None, tgate=None, inplace: bool =
     return out, tout
 
 
+def _launch_with_workspace(fn_name: str, desc, device) -> None:
+    lib = _lib.load_library()
+    with torch.cuda.device(device):
+        n = getattr(lib, fn_name + "_workspace_bytes")(ctypes.byref(desc))
+        workspace = torch.empty(n, device=device, dtype=torch.uint8) if n else None
+        status = getattr(lib, fn_name)(ctypes.byref(desc), _ptr(workspace), n, torch.cuda.current_stream(device).cuda_stream)
+    _lib.raise_for_status(status)
+
+
+def ln_modulate_bwd(x, scale, dy, dskip=None, eps: float = 1e-6):
+    """Reverse mode of :func:`ln_modulate` (what autograd derives for
+    cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:1166-1167): ``(dx, dshift, dscale)`` for the gradient ``dy`` of its
+    output; ``dskip``: a gradient that reaches ``x`` on another way, added to ``dx``.  ``dshift`` / ``dscale``: ``[G, D]``."""
+    _check_elementwise(x)
+    D = x.shape[-1]
+    assert dy.shape == x.shape and dy.dtype == x.dtype and (dskip is None or (dskip.shape == x.shape and dskip.dtype == x.dtype))
+    xs, dy, dskip = _dense16(x), _dense16(dy), (None if dskip is None else _dense16(dskip))
+    scale = _dense16(scale.to(x.dtype)).reshape(-1, D)
+    rows = xs.numel() // D
+    assert rows % scale.shape[0] == 0
+    dx, dshift, dscale = torch.empty_like(xs), torch.empty_like(scale), torch.empty_like(scale)
+    d = _lib.LnModulateBwdDesc()
+    d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[x.dtype]
+    d.D, d.rows_per_group, d.eps, d.reserved, d.rows = D, rows // scale.shape[0], float(eps), 0, rows
+    d.x, d.scale, d.dy, d.dskip = _ptr(xs), _ptr(scale), _ptr(dy), _ptr(dskip)
+    d.dx, d.dshift, d.dscale = _ptr(dx), _ptr(dshift), _ptr(dscale)
+    _launch_with_workspace("cosmos_ln_modulate_bwd", d, x.device)
+    return dx, dshift, dscale
+
+
+def gated_residual_bwd(res, gate, dy):
+    """Reverse mode of :func:`gated_residual` for ``res`` and ``gate``: ``(dres, dgate)``, ``dgate`` ``[G, D]``; the gradient of
+    ``x`` is ``dy`` itself."""
+    _check_elementwise(res)
+    D = res.shape[-1]
+    assert dy.shape == res.shape and dy.dtype == res.dtype
+    res, dy, gate = _dense16(res), _dense16(dy), _dense16(gate.to(res.dtype)).reshape(-1, D)
+    rows = res.numel() // D
+    assert rows % gate.shape[0] == 0
+    dres, dgate = torch.empty_like(res), torch.empty_like(gate)
+    d = _lib.GatedResidualBwdDesc()
+    d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[res.dtype]
+    d.D, d.rows_per_group, d.rows = D, rows // gate.shape[0], rows
+    d.dy, d.res, d.gate, d.dres, d.dgate = _ptr(dy), _ptr(res), _ptr(gate), _ptr(dres), _ptr(dgate)
+    _launch_with_workspace("cosmos_gated_residual_bwd", d, res.device)
+    return dres, dgate
+
+
 def gelu(h, th=None, inplace: bool = False):
     """Exact (erf) GELU and its tangent ``th * gelu'(h)`` in one pass (``nn.GELU()`` of
     cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:225).  Returns ``(a, ta)``."""

@@ -274,6 +274,39 @@ COSMOS_ATTN_API int cosmos_ln_modulate(const cosmos_ln_modulate_desc *desc, void
 COSMOS_ATTN_API int cosmos_gated_residual(const cosmos_gated_residual_desc *desc, void *stream);
 COSMOS_ATTN_API int cosmos_gelu(const cosmos_gelu_desc *desc, void *stream);
 
+/*
+ * Reverse mode of cosmos_ln_modulate and cosmos_gated_residual (what autograd derives for networks/minimal_v4_dit.py:1166-1167
+ * and :1199), one pass over the tensors plus a small one for the modulation vectors; sums in fp32, in a fixed order.
+ *
+ * cosmos_ln_modulate_bwd:     dx = [dskip +] r (dn - mean(dn) - n mean(dn n)),  dn = dy (1 + scale),  n = LayerNorm(x)
+ *                             dscale = sum over the group's rows of dy n,  dshift = sum of dy
+ *                             (dskip: a gradient that reaches x on another way, added before the one rounding; may be NULL)
+ * cosmos_gated_residual_bwd:  dres = dy gate,  dgate = sum over the group's rows of dy res       (dx is dy itself)
+ * The workspace (bytes from the function beside each; may be 0) holds partial sums.
+ */
+typedef struct cosmos_ln_modulate_bwd_desc {
+    int32_t abi_version, dtype;
+    int32_t D, rows_per_group;         /* D % 8 == 0, D <= 8192; rows % rows_per_group == 0 */
+    float eps;
+    int32_t reserved;
+    int64_t rows;
+    const void *x, *scale, *dy, *dskip;   /* [rows, D], [rows / rows_per_group, D], [rows, D], [rows, D] or NULL */
+    void *dx, *dshift, *dscale;           /* [rows, D], [rows / rows_per_group, D] twice */
+} cosmos_ln_modulate_bwd_desc;
+
+typedef struct cosmos_gated_residual_bwd_desc {
+    int32_t abi_version, dtype;
+    int32_t D, rows_per_group;
+    int64_t rows;
+    const void *dy, *res, *gate;       /* [rows, D], [rows, D], [rows / rows_per_group, D] */
+    void *dres, *dgate;                /* [rows, D], [rows / rows_per_group, D] */
+} cosmos_gated_residual_bwd_desc;
+
+COSMOS_ATTN_API size_t cosmos_ln_modulate_bwd_workspace_bytes(const cosmos_ln_modulate_bwd_desc *desc);
+COSMOS_ATTN_API int cosmos_ln_modulate_bwd(const cosmos_ln_modulate_bwd_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
+COSMOS_ATTN_API size_t cosmos_gated_residual_bwd_workspace_bytes(const cosmos_gated_residual_bwd_desc *desc);
+COSMOS_ATTN_API int cosmos_gated_residual_bwd(const cosmos_gated_residual_bwd_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -101,6 +101,32 @@ def test_gated_residual(pkg, block_oracle, gpu, dtype, rows, D, rpg):
     check("tout (fixed gate, in place)", t3, twant3, dtype)
 
 
+@pytest.mark.parametrize("rows,rpg,D", [(24, 4, 8), (17, 17, 264), (66, 33, 2048), (8, 1, 2056), (90, 45, 4104), (40, 40, 5120), (21, 21, 8192),
+                                        (9000, 4500, 64)])      # (the last: rows enough for runs longer than the shortest)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_reverse_mode(pkg, gpu, rows, rpg, D, dtype):
+    """Groups of one run and of several, ragged ones among them; columns that fill the 256 threads' chunks of 8 once to four
+    times, with and without a remainder; against torch's own reverse mode in 64 bits.  Bounds: one rounding of each result, as
+    above; a sum over n rows of products of size one is off by sqrt(n) 2^-24 more."""
+    g = torch.Generator().manual_seed(rows + D)
+    x, res, dy, dskip = rnd(g, dtype, rows, D, std=2.0, mean=0.5), *(rnd(g, dtype, rows, D) for _ in range(3))
+    sc, gate = rnd(g, dtype, rows // rpg, D, std=0.3), rnd(g, dtype, rows // rpg, D)
+    rep = lambda m: m.repeat_interleave(rpg, dim=0)
+    xr, scr, shr, rr, gr = (t.double().requires_grad_(True) for t in (x, sc, torch.zeros_like(sc), res, gate))
+    y = torch.nn.functional.layer_norm(xr, (D,), eps=1e-6) * (1 + rep(scr)) + rep(shr)
+    dx, dsc, dsh = torch.autograd.grad(y, (xr, scr, shr), dy.double())
+    d = lambda t: t.to(gpu)
+    for skip in (None, dskip):
+        got = pkg.ops.ln_modulate_bwd(d(x), d(sc), d(dy), None if skip is None else d(skip))
+        check("dx", got[0], dx if skip is None else dx + skip.double(), dtype)
+        check("dshift", got[1], dsh, dtype)
+        check("dscale", got[2], dsc, dtype)
+    dres, dgate = torch.autograd.grad(rep(gr) * rr, (rr, gr), dy.double())
+    got = pkg.ops.gated_residual_bwd(d(res), d(gate), d(dy))
+    check("dres", got[0], dres, dtype)
+    check("dgate", got[1], dgate, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n", [8, 1000, 1 << 20])
 def test_gelu(pkg, block_oracle, gpu, dtype, n):

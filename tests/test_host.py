@@ -319,6 +319,32 @@ def test_block_elementwise_desc_layouts_and_status_codes(pkg):
         pkg.gelu(torch.zeros(8, dtype=torch.bfloat16))
 
 
+def test_block_reverse_mode_desc_layouts_and_status_codes(pkg):
+    L, lib = pkg._lib, pkg._lib.load_library()
+    assert ctypes.sizeof(L.LnModulateBwdDesc) == 24 + 8 + 7 * 8 and L.LnModulateBwdDesc.x.offset == 32
+    assert ctypes.sizeof(L.GatedResidualBwdDesc) == 16 + 8 + 5 * 8 and L.GatedResidualBwdDesc.dy.offset == 24
+    P = 0x7F0000000000   # never dereferenced: every case below is rejected on the host
+
+    def desc(cls, names, **over):
+        D = cls()
+        D.abi_version, D.dtype, D.D, D.rows_per_group, D.rows = L.ABI_VERSION, L.DTYPE_BF16, 256, 40, 80
+        for i, n in enumerate(names):
+            setattr(D, n, P + 0x10000 * i)
+        for k, v in over.items():
+            setattr(D, k, v)
+        return D
+
+    for fn, cls, names, vectors in (("cosmos_ln_modulate_bwd", L.LnModulateBwdDesc, ("x", "scale", "dy", "dskip", "dx", "dshift", "dscale"), 2),
+                                    ("cosmos_gated_residual_bwd", L.GatedResidualBwdDesc, ("dy", "res", "gate", "dres", "dgate"), 1)):
+        for over, want in [(dict(abi_version=1), L.ST_BAD_ARG), (dict(rows=0), L.ST_BAD_ARG), (dict(dy=None), L.ST_BAD_ARG),
+                           (dict(dtype=7), L.ST_UNSUPPORTED), (dict(D=252), L.ST_BAD_SHAPE), (dict(rows_per_group=33), L.ST_BAD_SHAPE),
+                           (dict(dy=P + 2), L.ST_BAD_STRIDE), ({}, L.ST_WORKSPACE)]:
+            assert getattr(lib, fn)(ctypes.byref(desc(cls, names, **over)), None, 0, None) == want, (fn, over)
+        need = getattr(lib, fn + "_workspace_bytes")
+        assert need(ctypes.byref(desc(cls, names))) == 2 * 5 * vectors * 256 * 4            # two groups of five runs of eight rows
+        assert need(ctypes.byref(desc(cls, names, rows_per_group=16))) == 0                # short groups are one run
+
+
 def test_dit_block_mirrors_reference_surface(pkg):
     m = pkg.Block(64, 48, 2, mlp_ratio=4.0, use_adaln_lora=True, adaln_lora_dim=8)
     names = sorted(m.state_dict())
