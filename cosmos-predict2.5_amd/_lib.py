@@ -197,6 +197,18 @@ class GatedResidualBwdDesc(ctypes.Structure):
     ]
 
 
+class ModulationDesc(ctypes.Structure):
+    """Mirror of ``struct cosmos_ln_modulation_desc``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("rows", ctypes.c_int32), ("K", ctypes.c_int32), ("hidden", ctypes.c_int32), ("D", ctypes.c_int32),
+        ("emb", ctypes.c_void_p), ("temb", ctypes.c_void_p), ("lora", ctypes.c_void_p), ("tlora", ctypes.c_void_p),
+        ("w1", ctypes.c_void_p * 3), ("w2", ctypes.c_void_p * 3),
+        ("out", ctypes.c_void_p), ("tout", ctypes.c_void_p),
+    ]
+
+
 EXPORTS = {
     "cosmos_attn_abi_version": (ctypes.c_int, []),
     "cosmos_attn_status_string": (ctypes.c_char_p, [ctypes.c_int]),
@@ -219,6 +231,8 @@ EXPORTS = {
     "cosmos_ln_modulate_bwd": (ctypes.c_int, [ctypes.POINTER(LnModulateBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_gated_residual_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(GatedResidualBwdDesc)]),
     "cosmos_gated_residual_bwd": (ctypes.c_int, [ctypes.POINTER(GatedResidualBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "cosmos_ln_modulation_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(ModulationDesc)]),
+    "cosmos_ln_modulation": (ctypes.c_int, [ctypes.POINTER(ModulationDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_gelu": (ctypes.c_int, [ctypes.POINTER(GeluDesc), ctypes.c_void_p]),
 }
 

@@ -80,6 +80,17 @@ class _GeluFn(torch.autograd.Function):
         return torch.ops.aten.gelu_backward(dy, h, approximate="none")
 
 
+# A call of up to this many rows (twice as many with tangents) forms the modulation vectors in two launches of its own kernels;
+# those read the weights again for every 16 rows, so that many rows are the library's (5120 channels, us: 64 rows 45 against 100,
+# 128 rows 76 against 112; with tangents 64 rows 76 against 344).
+_FUSED_MODULATION_ROWS = 64
+
+
+def _bare(m: nn.Module) -> bool:
+    """Is calling m the same as computing its forward?"""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__)
+
+
 class GPT2FeedForward(nn.Module):
     def __init__(self, d_model: int, d_ff: int):
         super().__init__()
@@ -204,6 +215,33 @@ class Block(nn.Module):
         cut = lambda z: tuple(c[:, :, None, None, :].type_as(like) for c in z.chunk(3, dim=-1))
         return cut(m), cut(tm)
 
+    def _fused_modulations(self, emb, lora, like, temb=None, tlora=None, tangent=False):
+        """All three sub-layers' modulation vectors in two launches: ``[3, 3, rows, D]`` (sub-layer; shift, scale, gate) and its
+        tangent, or None where the modules compute something else than the plain MLPs of one 16-bit type, or for many rows."""
+        if not self.use_adaln_lora or self.use_wan_fp32_strategy or lora is None or torch.is_autocast_enabled("cuda"):
+            return None
+        mods = (self.adaln_modulation_self_attn, self.adaln_modulation_cross_attn, self.adaln_modulation_mlp)
+        w1, w2 = [], []
+        for m in mods:
+            if type(m) is not nn.Sequential or len(m) != 3 or not _bare(m) or not all(_bare(c) for c in m):
+                return None
+            if type(m[0]) is not nn.SiLU or any(type(c) is not nn.Linear or c.bias is not None or type(c.weight) is not nn.Parameter for c in m[1:]):
+                return None
+            w1.append(m[1].weight)
+            w2.append(m[2].weight)
+        K, D = emb.shape[-1], like.shape[-1]
+        rows = emb.numel() // K
+        given = [t for t in (emb, lora, temb, tlora) if t is not None]
+        if rows > _FUSED_MODULATION_ROWS or K % 32 or D % 16 or w1[0].shape[0] % 32 or like.dtype not in (torch.bfloat16, torch.float16):
+            return None
+        if any(t.dtype != like.dtype or t.device != like.device or not t.is_cuda for t in (*given, *w1, *w2)):
+            return None
+        if any(t.shape[:-1] != emb.shape[:-1] for t in given) or lora.shape[-1] != 3 * D or (tlora is not None and tlora.shape != lora.shape):
+            return None
+        if any(w.shape != (w1[0].shape[0], K) for w in w1) or any(w.shape != (3 * D, w1[0].shape[0]) for w in w2):
+            return None
+        return ops.modulation(emb, lora, w1, w2, temb, tlora, tangent)
+
     def _fp32_region(self, t: torch.Tensor):
         return torch.autocast(t.device.type, enabled=self.use_wan_fp32_strategy, dtype=torch.float32)
 
@@ -261,10 +299,14 @@ class Block(nn.Module):
         one fused HIP pass instead of a chain of tensor-library ops."""
         B, T, H, W, D = x.shape
         flat2 = lambda m: m.reshape(-1, D)
-        for name, norm, sub in (("self_attn", self.layer_norm_self_attn, self.self_attn),
-                                ("cross_attn", self.layer_norm_cross_attn, self.cross_attn),
-                                ("mlp", self.layer_norm_mlp, self.mlp)):
-            shift, scale, gate = self._modulation(getattr(self, "adaln_modulation_" + name), emb, lora, x)
+        fused = self._fused_modulations(emb, lora, x)
+        for i, (name, norm, sub) in enumerate((("self_attn", self.layer_norm_self_attn, self.self_attn),
+                                               ("cross_attn", self.layer_norm_cross_attn, self.cross_attn),
+                                               ("mlp", self.layer_norm_mlp, self.mlp))):
+            if fused is not None:
+                shift, scale, gate = fused[0][i].unbind(0)
+            else:
+                shift, scale, gate = self._modulation(getattr(self, "adaln_modulation_" + name), emb, lora, x)
             n, _ = ops.ln_modulate(x, flat2(shift), flat2(scale), eps=norm.eps)
             if name == "mlp":
                 r = sub(n)
@@ -296,19 +338,24 @@ class Block(nn.Module):
         B, T, H, W, D = x.shape
         flat = lambda z: z.reshape(B, T * H * W, D)
         vid = lambda z: z.reshape(B, T, H, W, D)
-        args = (emb_B_T_D, temb_B_T_D, adaln_lora_B_T_3D, tadaln_lora_B_T_3D, x)
+        fused = self._fused_modulations(emb_B_T_D, adaln_lora_B_T_3D, x, temb_B_T_D, tadaln_lora_B_T_3D, tangent=True)
 
-        mod, tmod = self._modulation_jvp(self.adaln_modulation_self_attn, *args)
+        def modulation(i, layers):
+            if fused is not None:
+                return fused[0][i].unbind(0), fused[1][i].unbind(0)
+            return self._modulation_jvp(layers, emb_B_T_D, temb_B_T_D, adaln_lora_B_T_3D, tadaln_lora_B_T_3D, x)
+
+        mod, tmod = modulation(0, self.adaln_modulation_self_attn)
         n, tn = self._modulate_jvp(self.layer_norm_self_attn, x, tx, mod, tmod)
         r, tr = self.self_attn.forward_jvp(flat(n), flat(tn), rope_emb=rope_emb_L_1_1_D)
         x, tx = self._gated_residual_jvp(x, tx, vid(r), vid(tr), mod, tmod)
 
-        mod, tmod = self._modulation_jvp(self.adaln_modulation_cross_attn, *args)
+        mod, tmod = modulation(1, self.adaln_modulation_cross_attn)
         n, tn = self._modulate_jvp(self.layer_norm_cross_attn, x, tx, mod, tmod)
         r, tr = self.cross_attn.forward_jvp(flat(n), flat(tn), crossattn_emb, None, rope_emb=rope_emb_L_1_1_D)
         x, tx = self._gated_residual_jvp(x, tx, vid(r), vid(tr), mod, tmod)
 
-        mod, tmod = self._modulation_jvp(self.adaln_modulation_mlp, *args)
+        mod, tmod = modulation(2, self.adaln_modulation_mlp)
         n, tn = self._modulate_jvp(self.layer_norm_mlp, x, tx, mod, tmod)
         r, tr = self.mlp.forward_jvp(n, tn)
         x, tx = self._gated_residual_jvp(x, tx, r, tr, mod, tmod)

@@ -575,6 +575,33 @@ def gated_residual_bwd(res, gate, dy):
     return dres, dgate
 
 
+def modulation(emb, lora, w1, w2, temb=None, tlora=None, tangent: bool = False):
+    """The modulation vectors of a block's three sub-layers (cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:1131-1162):
+    ``w2[i] (w1[i] silu(emb)) + lora`` for i = 0, 1, 2, as ``[3, 3, rows, D]`` (sub-layer; shift, scale, gate), and with
+    ``tangent`` its derivative along (``temb``, ``tlora``; None = it does not move), else None.  ``emb``: ``[..., K]``;
+    ``lora``: ``[..., 3 D]`` of as many rows; ``w1``: three ``[hidden, K]``; ``w2``: three ``[3 D, hidden]``; one 16-bit type."""
+    _check_elementwise(emb)
+    K, D = emb.shape[-1], lora.shape[-1] // 3
+    rows, hidden = emb.numel() // K, w1[0].shape[0]
+    assert lora.shape[-1] == 3 * D and lora.numel() == rows * 3 * D
+    assert all(w.shape == (hidden, K) for w in w1) and all(w.shape == (3 * D, hidden) for w in w2)
+    assert (temb is None or temb.shape == emb.shape) and (tlora is None or tlora.shape == lora.shape)
+    ins = [None if t is None else _dense16(t) for t in (emb, temb, lora, tlora, *w1, *w2)]
+    assert all(t is None or (t.dtype == emb.dtype and t.device == emb.device) for t in ins)
+    assert tangent or (temb is None and tlora is None)
+    out = torch.empty((3, 3, rows, D), device=emb.device, dtype=emb.dtype)
+    tout = torch.empty_like(out) if tangent else None
+    d = _lib.ModulationDesc()
+    d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[emb.dtype]
+    d.rows, d.K, d.hidden, d.D = rows, K, hidden, D
+    d.emb, d.temb, d.lora, d.tlora = (_ptr(t) for t in ins[:4])
+    for i in range(3):
+        d.w1[i], d.w2[i] = _ptr(ins[4 + i]), _ptr(ins[7 + i])
+    d.out, d.tout = _ptr(out), _ptr(tout)
+    _launch_with_workspace("cosmos_ln_modulation", d, emb.device)
+    return out, tout
+
+
 def gelu(h, th=None, inplace: bool = False):
     """Exact (erf) GELU and its tangent ``th * gelu'(h)`` in one pass (``nn.GELU()`` of
     cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:225).  Returns ``(a, ta)``."""

@@ -307,6 +307,24 @@ COSMOS_ATTN_API int cosmos_ln_modulate_bwd(const cosmos_ln_modulate_bwd_desc *de
 COSMOS_ATTN_API size_t cosmos_gated_residual_bwd_workspace_bytes(const cosmos_gated_residual_bwd_desc *desc);
 COSMOS_ATTN_API int cosmos_gated_residual_bwd(const cosmos_gated_residual_bwd_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * The modulation vectors of a block (networks/minimal_v4_dit.py:1131-1162, with the LoRA term): for each of three MLPs i
+ *     out[i][v] = the v-th third of  W2_i (W1_i silu(emb)) + lora,      v = shift, scale, gate
+ *     tout[i][v]: its derivative along (temb, tlora); tout NULL = values only, temb / tlora NULL = they do not move
+ * silu(emb) and W1 silu(emb) are rounded to the element type, sums are fp32.  Meant for few rows (one per batch row and frame).
+ */
+typedef struct cosmos_ln_modulation_desc {
+    int32_t abi_version, dtype;
+    int32_t rows, K, hidden, D;        /* K % 32 == 0, hidden % 32 == 0, D % 16 == 0; rows <= 65536 */
+    const void *emb, *temb;            /* [rows, K] */
+    const void *lora, *tlora;          /* [rows, 3 D] */
+    const void *w1[3], *w2[3];         /* [hidden, K], [3 D, hidden] */
+    void *out, *tout;                  /* [3, 3, rows, D] */
+} cosmos_ln_modulation_desc;
+
+COSMOS_ATTN_API size_t cosmos_ln_modulation_workspace_bytes(const cosmos_ln_modulation_desc *desc);
+COSMOS_ATTN_API int cosmos_ln_modulation(const cosmos_ln_modulation_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -345,6 +345,30 @@ def test_block_reverse_mode_desc_layouts_and_status_codes(pkg):
         assert need(ctypes.byref(desc(cls, names, rows_per_group=16))) == 0                # short groups are one run
 
 
+def test_modulation_desc_layout_and_status_codes(pkg):
+    L, lib = pkg._lib, pkg._lib.load_library()
+    assert ctypes.sizeof(L.ModulationDesc) == 24 + 12 * 8 and L.ModulationDesc.emb.offset == 24 and L.ModulationDesc.out.offset == 24 + 10 * 8
+    P = 0x7F0000000000   # never dereferenced: every case below is rejected on the host
+
+    def desc(**over):
+        D = L.ModulationDesc()
+        D.abi_version, D.dtype, D.rows, D.K, D.hidden, D.D = L.ABI_VERSION, L.DTYPE_BF16, 5, 256, 64, 256
+        D.emb, D.lora, D.out = P, P + 0x10000, P + 0x20000
+        for i in range(3):
+            D.w1[i], D.w2[i] = P + 0x30000, P + 0x40000
+        for k, v in over.items():
+            setattr(D, k, v)
+        return D
+
+    none3 = (ctypes.c_void_p * 3)(P, None, P)
+    for over, want in [(dict(abi_version=1), L.ST_BAD_ARG), (dict(rows=0), L.ST_BAD_ARG), (dict(lora=None), L.ST_BAD_ARG), (dict(temb=P), L.ST_BAD_ARG),
+                       (dict(w1=none3), L.ST_BAD_ARG), (dict(dtype=7), L.ST_UNSUPPORTED), (dict(K=40), L.ST_BAD_SHAPE), (dict(hidden=48), L.ST_BAD_SHAPE),
+                       (dict(D=24), L.ST_BAD_SHAPE), (dict(emb=P + 2), L.ST_BAD_STRIDE), ({}, L.ST_WORKSPACE)]:
+        assert lib.cosmos_ln_modulation(ctypes.byref(desc(**over)), None, 0, None) == want, over
+    assert lib.cosmos_ln_modulation_workspace_bytes(ctypes.byref(desc())) == 3 * 5 * 64 * 2
+    assert lib.cosmos_ln_modulation_workspace_bytes(ctypes.byref(desc(tout=P))) == 2 * 3 * 5 * 64 * 2
+
+
 def test_dit_block_mirrors_reference_surface(pkg):
     m = pkg.Block(64, 48, 2, mlp_ratio=4.0, use_adaln_lora=True, adaln_lora_dim=8)
     names = sorted(m.state_dict())
