@@ -128,17 +128,23 @@ constexpr int kNumCUs = 256;          // MI355X
 constexpr int kMaxSplits = 16;
 constexpr int kMinStepsPerSplit = 4;
 struct StepCost { double step_us, range_us; };   // a barrier step in full rounds, and what a workgroup costs besides its steps
+// `pairs` workgroups of n_steps / S steps each, in rounds
+inline double rounds_cost(int64_t pairs, double n_steps, StepCost c) {
+    if (pairs <= 0) return 0.0;
+    const int64_t rounds = (pairs + kNumCUs - 1) / kNumCUs;
+    const double filled = (double)pairs / (double)(rounds * kNumCUs);
+    return (double)rounds * (n_steps * c.step_us * (0.7 + 0.3 * filled * filled) + c.range_us);
+}
+inline double split_cost(int rem, int n_steps, int S, StepCost c, double slot_bytes) {
+    return rounds_cost((int64_t)rem * S, (double)n_steps / S, c) + (S > 1 ? 3.0 + (double)rem * S * slot_bytes / 3.8e6 : 0.0);
+}
 inline int choose_splits(int rem, int n_steps, StepCost c, double slot_bytes) {
     if (rem <= 0) return 1;
     int best = 1;
-    double best_cost = 0.0;
-    for (int S = 1; S <= kMaxSplits && (S == 1 || S * kMinStepsPerSplit <= n_steps); ++S) {
-        const int rounds = (rem * S + kNumCUs - 1) / kNumCUs;
-        const double filled = (double)(rem * S) / (rounds * kNumCUs);
-        double cost = rounds * ((double)n_steps / S * c.step_us * (0.7 + 0.3 * filled * filled) + c.range_us);
-        if (S > 1) cost += 3.0 + (double)rem * S * slot_bytes / 3.8e6;
-        if (S == 1) best_cost = 0.95 * cost;
-        else if (cost < best_cost) { best_cost = cost; best = S; }
+    double best_cost = 0.95 * split_cost(rem, n_steps, 1, c, slot_bytes);
+    for (int S = 2; S <= kMaxSplits && S * kMinStepsPerSplit <= n_steps; ++S) {
+        const double cost = split_cost(rem, n_steps, S, c, slot_bytes);
+        if (cost < best_cost) { best_cost = cost; best = S; }
     }
     return best;
 }

@@ -1522,32 +1522,41 @@ size_t tiles_bytes_of(const cosmos_attn_desc* d) { return (size_t)d->B * d->H * 
 // workgroups are cut along the keys, and a small second kernel merges the ranges.
 // a head dim of 256 goes to attn_wide_kernel
 bool is_wide(const cosmos_attn_desc* d) { return d->d_qk == 256 || d->d_v == 256; }
-struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; };
+struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // us: estimated time of the launches
 SplitPlan plan_split(const cosmos_attn_desc* d) {
     SplitPlan s;
     const bool fwd = mode_of(d) == MODE_FWD;
+    // (smaller head dims: fewer matrix instructions per step, the same exponentials; tangent on q only: two thirds of them)
+    const double part = 0.3 + 0.7 * (d->d_qk + d->d_v) / 256.0;
+    const StepCost c = fwd ? StepCost{2.66 * part, 13.0} : StepCost{(mode_of(d) == MODE_JVP_Q ? 0.86 : 1.21) * part, 8.0};
+    const int n_steps = fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d);   // barrier steps: 64 keys forward only, 32 with tangents
     s.block_m = fwd ? kSymBlockM : kBlockM;
     s.n_qt = (d->Lq + s.block_m - 1) / s.block_m;
     s.n_pairs = s.n_qt * d->B * d->H;
     s.n_rem = 0; s.splits = 1; s.n_full = s.n_pairs;
-    if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
     const int rem = s.n_pairs % kNumCUs;
-    const int n_steps = fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d);   // barrier steps: 64 keys forward only, 32 with tangents
-    // (smaller head dims: fewer matrix instructions per step, the same exponentials)
-    const double part = 0.3 + 0.7 * (d->d_qk + d->d_v) / 256.0;
-    const StepCost c = fwd ? StepCost{2.66 * part, 13.0} : StepCost{1.21 * part, 8.0};
-    const int splits = choose_splits(rem, n_steps, c, (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4)));
+    const StepCost alone = StepCost{c.step_us, 13.0};                    // (a workgroup that is a whole pair also starts and ends it)
+    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
+    if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
+    const double slot_bytes = (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4));
+    const int splits = choose_splits(rem, n_steps, c, slot_bytes);
     if (splits < 2) return s;
+    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + split_cost(rem, n_steps, splits, c, slot_bytes);
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = splits;
     return s;
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
-// of compute units (every unit gets the same number of equal pieces); it pays from a few blocks per workgroup on.
+// of compute units (every unit gets the same number of equal pieces).  It is chosen where the units' share of query blocks, at
+// block_us + tile_us per key tile each, comes out faster than the other kernels' rounds: a finished block costs it little, a key
+// tile costs it more than the forward-only kernel (which has three wavefronts per SIMD).  Measured (us, stream / other kernel,
+// 16 heads; B*H = 40 and the lengths between alike): tangent on q 3520 x 512 keys 45 / 62, 7040 x 512 78 / 109, 37440 x 2048
+// 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  With all tangents the
+// two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
 // cosmos_attn_set_stream_override() replaces the choice (tuning and tests); nothing in the per-call path reads the environment.
 constexpr int kStreamMaxTiles = 64;       // up to 2048 keys
 constexpr int kStreamGroupsPerCU = 1;       // one workgroup fills a compute unit (8 wavefronts, 2 per SIMD at 256 registers): a single round
-constexpr int kStreamMinPairs = 1024;     // four blocks per workgroup: from there on the stream is faster than one workgroup per block (measured)
+constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
 std::atomic<int> g_stream_groups{0};      // number of workgroups, 0 = the library's own choice
 int stream_groups_of(const cosmos_attn_desc* d) {
@@ -1562,7 +1571,14 @@ int stream_groups_of(const cosmos_attn_desc* d) {
         return groups > (1 << 30) ? 0 : (int)groups;
     }
     if (const int groups = g_stream_groups.load(std::memory_order_relaxed)) return (groups + 7) / 8 * 8;
-    return pairs >= kStreamMinPairs ? kNumCUs * kStreamGroupsPerCU : 0;
+    if (pairs < kStreamMinPairs) return 0;
+    const int groups = kNumCUs * kStreamGroupsPerCU;
+    const int mode = mode_of(d);
+    const double part = 0.3 + 0.7 * d->d_qk / 128.0;
+    if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
+    const double tile_us = (mode == MODE_FWD ? 0.575 : 0.79) * part, block_us = mode == MODE_FWD ? 2.4 : 6.0;
+    const double stream_us = (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
+    return stream_us <= 1.03 * plan_split(d).us ? groups : 0;     // (40 heads, 7040 x 512 keys, forward only: 109 us against 117)
 }
 // LDS of attn_qstream_kernel: the layout of attn_fwd_jvp_kernel (AttnCfg::LDS_BYTES) + the per-block statistics slots
 size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {

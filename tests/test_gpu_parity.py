@@ -351,6 +351,31 @@ def test_streaming_kernels_match_the_block_kernels_bitwise_free(pkg, oracle, gpu
     assert (got[0].float() - ref[0].float()).abs().max().item() <= 1e-2
 
 
+@pytest.mark.parametrize("H,Lq,Lkv,tangents,padded", [
+    (10, 1560, 512, "none", False), (10, 1560, 2000, "none", False),      # 130 query blocks, half a round: streamed, and not
+    (2, 8064, 300, "q", False), (2, 8130, 300, "q", True),                # 126 blocks (too few) and 128; ragged last ones
+    (9, 7300, 130, "q", True), (9, 7300, 1100, "none", False),            # 522: two and three blocks a workgroup
+])
+def test_streaming_choice_agrees_with_the_block_kernels(pkg, oracle, gpu, stream_override, H, Lq, Lkv, tangents, padded):
+    """Both sides of the rule that sends short key sequences to the streaming kernels: the library's choice against one workgroup
+    per query block, from [B, S, H, d] views; two correct kernels differ by the roundings of the 16-bit probabilities and results."""
+    shape = (1, H, Lq, 128)
+    q, k, v, tq, _, _ = oracle.make_inputs(shape, (1, H, Lkv, 128), seed=Lq + Lkv)
+    view = lambda x: x.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+    args = [view(x) for x in (q, k, v)] + ([view(tq)] if tangents == "q" else [])
+    lens = torch.tensor([Lkv - 37], dtype=torch.int32, device=gpu) if padded else None
+    got = pkg.fwd_jvp(*args, key_lens=lens)
+    packed = pkg.run_packed(args[0], pkg.pack_kv(args[1], args[2]), *args[3:], key_lens=lens)
+    stream_override(chunk=1)
+    want = pkg.fwd_jvp(*args, key_lens=lens)
+    for a, p, w in zip(got, packed, want):
+        if w is None:
+            continue
+        for x in (a, p):
+            rel = float((x.float() - w.float()).norm() / w.float().norm())
+            assert rel <= 5e-3 and bool(torch.isfinite(x).all()), rel
+
+
 def test_streaming_kernel_reproducible(pkg, oracle, gpu, stream_override):
     stream_override(chunk=5)
     q, k, v, tq, _, _ = oracle.make_inputs((1, 4, 2000, 128), (1, 4, 200, 128), seed=8)
