@@ -98,7 +98,7 @@ class NormRopeDesc(ctypes.Structure):
         ("H", ctypes.c_int32),
         ("D", ctypes.c_int32),
         ("eps", ctypes.c_float),
-        ("reserved", ctypes.c_int32),
+        ("weight_type", ctypes.c_int32),
         ("x", ctypes.c_void_p),
         ("tx", ctypes.c_void_p),
         ("weight", ctypes.c_void_p),
@@ -121,7 +121,7 @@ class NormRopeBwdDesc(ctypes.Structure):
         ("H", ctypes.c_int32),
         ("D", ctypes.c_int32),
         ("eps", ctypes.c_float),
-        ("reserved", ctypes.c_int32),
+        ("weight_type", ctypes.c_int32),
         ("x", ctypes.c_void_p),
         ("dy", ctypes.c_void_p),
         ("weight", ctypes.c_void_p),

@@ -43,10 +43,11 @@ constexpr int kThreads = 256;
 struct NormRopeParams {
     const uint16_t *x, *tx;      // tx may be null
     uint16_t *y, *ty;
-    const float* weight;         // [D] or null (ones)
+    const void* weight;          // [D] or null (ones): float, or the element type (weight16)
     const float* angles;         // [S, D] or null (no rotation)
     int64_t x_sb, x_ss, x_sh, y_sb, y_ss, y_sh;
     int B, S, H, D;
+    int weight16;
     float eps;
     int heads_per_unit;          // heads served by one thread group: a multiple of kHeadsPerStep
     int head_groups;             // ceil(H / heads_per_unit)
@@ -85,6 +86,24 @@ template <bool BF16>
 __device__ __forceinline__ void round4(float* f) {
     const uint2 r = pack4<BF16>(f);
     unpack4<BF16>(r, f);
+}
+
+// the eight weights of thread `part` of a row.  A module in 16 bits holds its weight in 16 bits: converted here, not by a launch
+// of its own on every call (3 us each, three per transformer block).
+template <bool BF16>
+__device__ __forceinline__ void load_weight(const void* weight, int weight16, int part, int D, float* g) {
+    if (!weight) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) g[i] = 1.0f;
+    } else if (weight16) {
+        const uint16_t* w = (const uint16_t*)weight + 4 * part;
+        unpack4<BF16>(*reinterpret_cast<const uint2*>(w), g);
+        unpack4<BF16>(*reinterpret_cast<const uint2*>(w + D / 2), g + 4);
+    } else {
+        const float* w = (const float*)weight + 4 * part;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { g[i] = w[i]; g[4 + i] = w[D / 2 + i]; }
+    }
 }
 
 // Sum over the TPR (2, 4, 8, 16 or 32) adjacent lanes of a thread group, result in every lane, by data-parallel-primitive
@@ -137,11 +156,7 @@ __global__ void __launch_bounds__(kThreads) norm_rope_kernel(const NormRopeParam
     uint16_t* typ = TANGENT ? p.ty + yo : nullptr;
 
     float g[8], sn[8], cs[8];   // [0, 4): the lower-half elements, [4, 8): their partners in the upper half
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g[i] = p.weight ? p.weight[4 * part + i] : 1.0f;
-        g[4 + i] = p.weight ? p.weight[D / 2 + 4 * part + i] : 1.0f;
-    }
+    load_weight<BF16>(p.weight, p.weight16, part, D, g);
     if (p.angles) {
         const float4 a0 = *reinterpret_cast<const float4*>(p.angles + (int64_t)s * D + 4 * part);
         const float4 a1 = *reinterpret_cast<const float4*>(p.angles + (int64_t)s * D + D / 2 + 4 * part);
@@ -247,11 +262,12 @@ norm_rope_kernel_t pick(int d) {
 struct NormRopeBwdParams {
     const uint16_t *x, *dy;
     uint16_t* dx;
-    const float* weight;         // [D] or null (ones)
+    const void* weight;          // [D] or null (ones): float, or the element type (weight16)
     const float* angles;         // [S, D] or null (no rotation)
     float* partials;             // [blocks, D] or null (no dweight wanted)
     int64_t x_sb, x_ss, x_sh, g_sb, g_ss, g_sh, o_sb, o_ss, o_sh;   // strides of x, dy, dx
     int B, S, H, D;
+    int weight16;
     float eps;
     int heads_per_unit, head_groups;
     int64_t units;
@@ -277,11 +293,7 @@ __global__ void __launch_bounds__(kThreads) norm_rope_bwd_kernel(const NormRopeB
     uint16_t* op = p.dx + (int64_t)b * p.o_sb + (int64_t)s * p.o_ss + (int64_t)h0 * p.o_sh + 4 * part;
 
     float g[8], sn[8], cs[8], wacc[8];   // [0, 4): the lower-half elements, [4, 8): their partners in the upper half
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g[i] = p.weight ? p.weight[4 * part + i] : 1.0f;
-        g[4 + i] = p.weight ? p.weight[D / 2 + 4 * part + i] : 1.0f;
-    }
+    load_weight<BF16>(p.weight, p.weight16, part, D, g);
 #pragma unroll
     for (int i = 0; i < 8; ++i) wacc[i] = 0.f;
     if (p.angles) {
@@ -423,10 +435,12 @@ COSMOS_ATTN_API int cosmos_norm_rope(const cosmos_norm_rope_desc* d, void* strea
     if (d->D != 16 && d->D != 32 && d->D != 64 && d->D != 128 && d->D != 256) return COSMOS_ATTN_BAD_SHAPE;
     if (!aligned16(d->x) || !aligned16(d->y) || (d->tx && (!aligned16(d->tx) || !aligned16(d->ty)))) return COSMOS_ATTN_BAD_STRIDE;
     if (d->angles && !aligned16(d->angles)) return COSMOS_ATTN_BAD_STRIDE;
+    if (d->weight_type != 0 && d->weight_type != 1) return COSMOS_ATTN_BAD_ARG;
+    if (d->weight && d->weight_type && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
     if (!strides_ok(d->x_stride) || !strides_ok(d->y_stride)) return COSMOS_ATTN_BAD_STRIDE;
     NormRopeParams p;
     p.x = (const uint16_t*)d->x; p.tx = (const uint16_t*)d->tx; p.y = (uint16_t*)d->y; p.ty = (uint16_t*)d->ty;
-    p.weight = d->weight; p.angles = d->angles;
+    p.weight = d->weight; p.weight16 = d->weight_type; p.angles = d->angles;
     p.x_sb = d->x_stride[0]; p.x_ss = d->x_stride[1]; p.x_sh = d->x_stride[2];
     p.y_sb = d->y_stride[0]; p.y_ss = d->y_stride[1]; p.y_sh = d->y_stride[2];
     p.B = d->B; p.S = d->S; p.H = d->H; p.D = d->D;
@@ -450,6 +464,8 @@ static int validate_norm_rope_bwd(const cosmos_norm_rope_bwd_desc* d) {
     if (d->dtype != COSMOS_ATTN_BF16 && d->dtype != COSMOS_ATTN_FP16) return COSMOS_ATTN_UNSUPPORTED;
     if (d->D != 16 && d->D != 32 && d->D != 64 && d->D != 128 && d->D != 256) return COSMOS_ATTN_BAD_SHAPE;
     if (!aligned16(d->x) || !aligned16(d->dy) || !aligned16(d->dx)) return COSMOS_ATTN_BAD_STRIDE;
+    if (d->weight_type != 0 && d->weight_type != 1) return COSMOS_ATTN_BAD_ARG;
+    if (d->weight && d->weight_type && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
     if (d->angles && !aligned16(d->angles)) return COSMOS_ATTN_BAD_STRIDE;
     if (!strides_ok(d->x_stride) || !strides_ok(d->dy_stride) || !strides_ok(d->dx_stride)) return COSMOS_ATTN_BAD_STRIDE;
     if (plan_units(d->B, d->S, d->H, d->D).blocks > 0x7FFFFFFF) return COSMOS_ATTN_BAD_SHAPE;
@@ -470,7 +486,7 @@ COSMOS_ATTN_API int cosmos_norm_rope_bwd(const cosmos_norm_rope_bwd_desc* d, voi
     if (need && !aligned16(workspace)) return COSMOS_ATTN_BAD_STRIDE;
     NormRopeBwdParams p;
     p.x = (const uint16_t*)d->x; p.dy = (const uint16_t*)d->dy; p.dx = (uint16_t*)d->dx;
-    p.weight = d->weight; p.angles = d->angles;
+    p.weight = d->weight; p.weight16 = d->weight_type; p.angles = d->angles;
     p.partials = d->dweight ? (float*)workspace : nullptr;
     p.x_sb = d->x_stride[0]; p.x_ss = d->x_stride[1]; p.x_sh = d->x_stride[2];
     p.g_sb = d->dy_stride[0]; p.g_ss = d->dy_stride[1]; p.g_sh = d->dy_stride[2];

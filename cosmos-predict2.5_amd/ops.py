@@ -314,6 +314,15 @@ def bwd(
     return dq, dk, dv
 
 
+def _norm_weight(weight: Optional[torch.Tensor], x: torch.Tensor) -> Optional[torch.Tensor]:
+    """RMSNorm's weight as the kernels take it: of the element type as it is, anything else as fp32."""
+    if weight is None:
+        return None
+    if weight.dtype == x.dtype and weight.device == x.device and weight.is_contiguous() and weight.data_ptr() % 16 == 0:
+        return weight
+    return weight.to(device=x.device, dtype=torch.float32).contiguous()
+
+
 def norm_rope(
     x: torch.Tensor,
     weight: Optional[torch.Tensor] = None,
@@ -344,8 +353,7 @@ def norm_rope(
     if not x.is_cuda:
         raise RuntimeError("cosmos attention (HIP) needs tensors on a GPU; there is no CPU path")
     x, tx = _prep_pair(x, tx)
-    if weight is not None:
-        weight = weight.to(device=x.device, dtype=torch.float32).contiguous()
+    weight = _norm_weight(weight, x)
     if rope_emb is not None:
         rope_emb = rope_emb.to(device=x.device, dtype=torch.float32).reshape(S, D).contiguous()
     if out_layout == "bshd":
@@ -361,7 +369,7 @@ def norm_rope(
     desc.dtype = _DTYPES[x.dtype]
     desc.B, desc.S, desc.H, desc.D = B, S, H, D
     desc.eps = float(eps)
-    desc.reserved = 0
+    desc.weight_type = int(weight is not None and weight.dtype != torch.float32)
     desc.x, desc.tx = x.data_ptr(), (tx.data_ptr() if tx is not None else None)
     desc.weight = weight.data_ptr() if weight is not None else None
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None
@@ -399,8 +407,7 @@ def norm_rope_bwd(
         raise RuntimeError("cosmos attention (HIP) needs tensors on a GPU; there is no CPU path")
     x = x if _kernel_ready(x) else x.contiguous()
     dy = dy if _kernel_ready(dy) else dy.contiguous()
-    if weight is not None:
-        weight = weight.to(device=x.device, dtype=torch.float32).contiguous()
+    weight = _norm_weight(weight, x)
     if rope_emb is not None:
         rope_emb = rope_emb.to(device=x.device, dtype=torch.float32).reshape(S, D).contiguous()
     dx = torch.empty((B, S, H, D), device=x.device, dtype=x.dtype)
@@ -411,7 +418,7 @@ def norm_rope_bwd(
     desc.dtype = _DTYPES[x.dtype]
     desc.B, desc.S, desc.H, desc.D = B, S, H, D
     desc.eps = float(eps)
-    desc.reserved = 0
+    desc.weight_type = int(weight is not None and weight.dtype != torch.float32)
     desc.x, desc.dy, desc.dx = x.data_ptr(), dy.data_ptr(), dx.data_ptr()
     desc.weight = weight.data_ptr() if weight is not None else None
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None

@@ -189,9 +189,9 @@ typedef struct cosmos_norm_rope_desc {
     int32_t dtype;           /* enum cosmos_attn_dtype: element type of x, tx, y, ty */
     int32_t B, S, H, D;      /* D in {16,32,64,128,256} */
     float eps;               /* 1e-6 in the DiT */
-    int32_t reserved;        /* 0 */
+    int32_t weight_type;     /* 0: weight is fp32; 1: weight has the element type */
     const void *x, *tx;      /* device; tx may be NULL (then ty must be NULL) */
-    const float *weight;     /* [D] fp32 (RMSNorm's gamma), device; NULL = ones */
+    const void *weight;      /* [D] (RMSNorm's gamma), device; NULL = ones */
     const float *angles;     /* [S, D] fp32 contiguous, device; NULL = no rotation (cross-attention keys, :409) */
     void *y, *ty;            /* outputs, device */
     int64_t x_stride[3];     /* (batch, sequence, head) element strides of x and tx */
@@ -215,9 +215,9 @@ typedef struct cosmos_norm_rope_bwd_desc {
     int32_t dtype;           /* element type of x, dy, dx */
     int32_t B, S, H, D;
     float eps;
-    int32_t reserved;        /* 0 */
+    int32_t weight_type;     /* 0: weight is fp32; 1: weight has the element type */
     const void *x, *dy;      /* device */
-    const float *weight;     /* [D] fp32 or NULL = ones */
+    const void *weight;      /* [D] or NULL = ones */
     const float *angles;     /* [S, D] fp32 or NULL = no rotation */
     void *dx;                /* device */
     float *dweight;          /* [D] fp32, device; NULL = not wanted */

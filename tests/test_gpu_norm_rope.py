@@ -313,3 +313,19 @@ def test_more_than_2_31_elements(pkg, nr_oracle, gpu):
     want_dx, _ = nr_oracle.norm_rope_grads_closed_form(xs, w.cpu().numpy(), as_, xs)
     check_grad("dx[sample]", dx[:, idx], want_dx)
     assert torch.isfinite(dw).all()
+
+
+@pytest.mark.parametrize("D", [16, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weight_of_the_element_type(pkg, gpu, D, dtype):
+    """A 16-bit weight is read as it is: the same bits as its fp32 copy gives, forward, tangent and reverse mode; a weight of the
+    other 16-bit type, or one that does not start at 16 bytes, takes the way through fp32."""
+    g = torch.Generator().manual_seed(D)
+    x, tx, dy = ((torch.randn(2, 37, 5, D, generator=g)).to(dtype).to(gpu) for _ in range(3))
+    a = torch.randn(37, D, generator=g).to(gpu)
+    w = (1.0 + 0.2 * torch.randn(D + 1, generator=g)).to(dtype).to(gpu)
+    other = torch.float16 if dtype == torch.bfloat16 else torch.bfloat16
+    for wt in (w[:D], w[1:], w[:D].to(other)):
+        for got, want in zip((*pkg.norm_rope(x, wt, a, tx), *pkg.norm_rope(x, wt, a)[:1], *pkg.norm_rope_bwd(x, wt, a, dy)),
+                             (*pkg.norm_rope(x, wt.float(), a, tx), *pkg.norm_rope(x, wt.float(), a)[:1], *pkg.norm_rope_bwd(x, wt.float(), a, dy))):
+            assert torch.equal(got, want)
