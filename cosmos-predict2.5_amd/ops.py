@@ -22,11 +22,13 @@ REFERENCE_HEAD_DIMS = (16, 32, 64, 128, 256)  # what the reference accepts (…j
 
 def _kernel_ready(x: torch.Tensor) -> bool:
     """True if the view can be handed to the kernel as is: d stride 1, 16-byte rows and base."""
-    return (
-        x.stride(-1) == 1
-        and x.data_ptr() % 16 == 0
-        and all(s % 8 == 0 for s in x.stride()[:-1])
-    )
+    *outer, last = x.stride()
+    if last != 1 or x.data_ptr() % 16:
+        return False
+    for s in outer:
+        if s % 8:
+            return False
+    return True
 
 
 def _prep_pair(x: torch.Tensor, tx: Optional[torch.Tensor]):
@@ -38,8 +40,20 @@ def _prep_pair(x: torch.Tensor, tx: Optional[torch.Tensor]):
     return x.contiguous(), tx.contiguous()
 
 
+_Int64x3 = ctypes.c_int64 * 3
+
+
 def _strides3(x: torch.Tensor):
-    return (ctypes.c_int64 * 3)(x.stride(0), x.stride(1), x.stride(2))
+    return _Int64x3(*x.stride()[:3])
+
+
+def _on_device(device: torch.device, launch):
+    """``launch(stream)`` with ``device`` current, ``stream`` its current stream's handle.  The usual case, that it is current
+    already, goes without torch's device guard and stream object: they cost 5 us a call."""
+    if torch.cuda.current_device() == device.index:
+        return launch(torch._C._cuda_getCurrentRawStream(device.index))
+    with torch.cuda.device(device):
+        return launch(torch.cuda.current_stream(device).cuda_stream)
 
 
 def _alloc_outputs(B, H, Lq, d_v, q, have_tangent, out_layout, need_lse):
@@ -134,15 +148,12 @@ def fwd_jvp(
     desc.key_lens = key_lens.data_ptr() if key_lens is not None else None
 
     lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.cosmos_attn_workspace_bytes(ctypes.byref(desc))
-        if ws_bytes == 0:
-            # invalid descriptor: let the launch entry produce the precise status
-            _lib.raise_for_status(lib.cosmos_attn_fwd_jvp(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
-        workspace = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        status = lib.cosmos_attn_fwd_jvp(ctypes.byref(desc), workspace.data_ptr(), ws_bytes, stream)
-    _lib.raise_for_status(status)
+    ws_bytes = lib.cosmos_attn_workspace_bytes(ctypes.byref(desc))
+    if ws_bytes == 0:
+        # invalid descriptor: let the launch entry produce the precise status
+        _lib.raise_for_status(lib.cosmos_attn_fwd_jvp(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
+    workspace = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+    _lib.raise_for_status(_on_device(q.device, lambda stream: lib.cosmos_attn_fwd_jvp(ctypes.byref(desc), workspace.data_ptr(), ws_bytes, stream)))
     # workspace / converted inputs are freed to torch's caching allocator here; it is stream-ordered on
     # the launch stream, so reuse by later work on this stream is safe.
     return o, to, lse
@@ -191,13 +202,11 @@ def pack_kv(k: torch.Tensor, v: torch.Tensor) -> PackedKV:
     desc.q, desc.o, desc.tq, desc.to, desc.lse, desc.key_lens = k.data_ptr(), k.data_ptr(), None, None, None, None
     desc.q_stride, desc.o_stride = _strides3(k), _strides3(k)
     lib = _lib.load_library()
-    with torch.cuda.device(k.device):
-        nbytes = lib.cosmos_attn_packed_bytes(ctypes.byref(desc))
-        if nbytes == 0:
-            _lib.raise_for_status(lib.cosmos_attn_pack_kv(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
-        image = torch.empty(nbytes, device=k.device, dtype=torch.uint8)
-        status = lib.cosmos_attn_pack_kv(ctypes.byref(desc), image.data_ptr(), nbytes, torch.cuda.current_stream(k.device).cuda_stream)
-    _lib.raise_for_status(status)
+    nbytes = lib.cosmos_attn_packed_bytes(ctypes.byref(desc))
+    if nbytes == 0:
+        _lib.raise_for_status(lib.cosmos_attn_pack_kv(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
+    image = torch.empty(nbytes, device=k.device, dtype=torch.uint8)
+    _lib.raise_for_status(_on_device(k.device, lambda stream: lib.cosmos_attn_pack_kv(ctypes.byref(desc), image.data_ptr(), nbytes, stream)))
     return PackedKV(image, B, H, Lkv, d_qk, d_v, k.dtype, k.device)
 
 
@@ -235,10 +244,8 @@ def run_packed(
     desc.lse = lse.data_ptr() if lse is not None else None
     desc.key_lens = key_lens.data_ptr() if key_lens is not None else None
     lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        status = lib.cosmos_attn_run(ctypes.byref(desc), packed.image.data_ptr(), packed.image.numel(),
-                                     torch.cuda.current_stream(q.device).cuda_stream)
-    _lib.raise_for_status(status)
+    _lib.raise_for_status(_on_device(q.device, lambda stream: lib.cosmos_attn_run(
+        ctypes.byref(desc), packed.image.data_ptr(), packed.image.numel(), stream)))
     return o, to, lse
 
 
@@ -303,14 +310,11 @@ def bwd(
     desc.dq_stride, desc.dk_stride, desc.dv_stride = _strides3(dq), _strides3(dk), _strides3(dv)
 
     lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.cosmos_attn_bwd_workspace_bytes(ctypes.byref(desc))
-        if ws_bytes == 0:
-            _lib.raise_for_status(lib.cosmos_attn_bwd(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
-        workspace = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        status = lib.cosmos_attn_bwd(ctypes.byref(desc), workspace.data_ptr(), ws_bytes, stream)
-    _lib.raise_for_status(status)
+    ws_bytes = lib.cosmos_attn_bwd_workspace_bytes(ctypes.byref(desc))
+    if ws_bytes == 0:
+        _lib.raise_for_status(lib.cosmos_attn_bwd(ctypes.byref(desc), None, 0, None) or _lib.ST_BAD_ARG)
+    workspace = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8)
+    _lib.raise_for_status(_on_device(q.device, lambda stream: lib.cosmos_attn_bwd(ctypes.byref(desc), workspace.data_ptr(), ws_bytes, stream)))
     return dq, dk, dv
 
 
@@ -375,10 +379,7 @@ def norm_rope(
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None
     desc.y, desc.ty = y.data_ptr(), (ty.data_ptr() if ty is not None else None)
     desc.x_stride, desc.y_stride = _strides3(x), _strides3(y)
-    lib = _lib.load_library()
-    with torch.cuda.device(x.device):
-        status = lib.cosmos_norm_rope(ctypes.byref(desc), torch.cuda.current_stream(x.device).cuda_stream)
-    _lib.raise_for_status(status)
+    _launch("cosmos_norm_rope", desc, x.device)
     return y, ty
 
 
@@ -424,13 +425,7 @@ def norm_rope_bwd(
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None
     desc.dweight = dweight.data_ptr() if dweight is not None else None
     desc.x_stride, desc.dy_stride, desc.dx_stride = _strides3(x), _strides3(dy), _strides3(dx)
-    lib = _lib.load_library()
-    with torch.cuda.device(x.device):
-        ws_bytes = lib.cosmos_norm_rope_bwd_workspace_bytes(ctypes.byref(desc))
-        workspace = torch.empty(max(ws_bytes, 16), device=x.device, dtype=torch.uint8)
-        status = lib.cosmos_norm_rope_bwd(ctypes.byref(desc), workspace.data_ptr(), ws_bytes,
-                                          torch.cuda.current_stream(x.device).cuda_stream)
-    _lib.raise_for_status(status)
+    _launch_with_workspace("cosmos_norm_rope_bwd", desc, x.device)
     return dx, dweight
 
 
@@ -465,10 +460,8 @@ def _check_elementwise(x: torch.Tensor) -> None:
 
 
 def _launch(fn_name: str, desc, device) -> None:
-    lib = _lib.load_library()
-    with torch.cuda.device(device):
-        status = getattr(lib, fn_name)(ctypes.byref(desc), torch.cuda.current_stream(device).cuda_stream)
-    _lib.raise_for_status(status)
+    fn = getattr(_lib.load_library(), fn_name)
+    _lib.raise_for_status(_on_device(device, lambda stream: fn(ctypes.byref(desc), stream)))
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -536,11 +529,9 @@ def gated_residual(x, res, gate, tx=None, tres=None, tgate=None, inplace: bool =
 
 def _launch_with_workspace(fn_name: str, desc, device) -> None:
     lib = _lib.load_library()
-    with torch.cuda.device(device):
-        n = getattr(lib, fn_name + "_workspace_bytes")(ctypes.byref(desc))
-        workspace = torch.empty(n, device=device, dtype=torch.uint8) if n else None
-        status = getattr(lib, fn_name)(ctypes.byref(desc), _ptr(workspace), n, torch.cuda.current_stream(device).cuda_stream)
-    _lib.raise_for_status(status)
+    fn, n = getattr(lib, fn_name), getattr(lib, fn_name + "_workspace_bytes")(ctypes.byref(desc))
+    workspace = torch.empty(n, device=device, dtype=torch.uint8) if n else None
+    _lib.raise_for_status(_on_device(device, lambda stream: fn(ctypes.byref(desc), _ptr(workspace), n, stream)))
 
 
 def ln_modulate_bwd(x, scale, dy, dskip=None, eps: float = 1e-6):

@@ -95,8 +95,8 @@ class VideoRopePosition3DEmb(nn.Module):
         )
         t_pos = self.seq[:T]
         if self.enable_fps_modulation:
-            uniform_fps = (fps is None) or (fps.min() == fps.max())
-            assert uniform_fps or B == 1 or T == 1, (
+            # (the frame rates are looked at last: that waits for the GPU)
+            assert fps is None or B == 1 or T == 1 or (fps.min() == fps.max()), (
                 "For video batch, batch size should be 1 for non-uniform fps. For image batch, T should be 1"
             )
             if fps is None:
