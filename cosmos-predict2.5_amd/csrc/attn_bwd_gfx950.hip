@@ -124,12 +124,11 @@ __host__ __device__ constexpr int quad_unit_slot(int q, int cK, int hK) {
 
 struct PackSrc { const uint16_t* ptr; int64_t sb, sh, sl; };
 struct PackBwdParams {
-    PackSrc a1, a2, c1, c2;      // the K-type sections and the V^T-type sections (n_vt of them: 0, 1 or 2)
+    PackSrc a1, a2, c1, c2;      // the K-type sections and the V^T-type sections (n_vt of them: 1 or 2)
     const float2* stats;         // null: no statistics fragment
     uint4* out;
     int H, L, d, n_tiles, nc, ndb, tile_frags;
     int n_vt;                    // number of V^T-type sections
-    int swz;                     // K-type sections in the unit order of attn_dkdv_quad_kernel (quad_unit_slot) instead of fragment by fragment
 };
 
 // grid (n_tiles, B*H); every 16-byte unit of a tile image is produced by one thread.
@@ -142,7 +141,6 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
         int frag = u >> 6;
         const int l = u & 63, i = l & 31, hh = l >> 5;
         uint4 val = make_uint4(0u, 0u, 0u, 0u);
-        int where = u;           // 16-byte unit of the tile image this value goes to
         if (frag < ktype_frags) {
             const int sec = frag < p.nc ? 0 : 1;
             const PackSrc& s = sec ? p.a2 : p.a1;
@@ -150,7 +148,6 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
             const int row = t * kRows + i;
             if (row < p.L)
                 val = *reinterpret_cast<const uint4*>(s.ptr + (int64_t)b * s.sb + (int64_t)h * s.sh + (int64_t)row * s.sl + 16 * frag + 8 * hh);
-            if (p.swz) where = sec * p.nc * 64 + quad_unit_slot(i, frag, hh);
         } else if (frag < ktype_frags + vt_frags * p.n_vt) {
             frag -= ktype_frags;
             const PackSrc& s = frag < vt_frags ? p.c1 : p.c2;
@@ -181,8 +178,64 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
             val = make_uint4(__builtin_bit_cast(uint32_t, f[0]), __builtin_bit_cast(uint32_t, f[1]),
                              __builtin_bit_cast(uint32_t, f[2]), __builtin_bit_cast(uint32_t, f[3]));
         }
-        dst[where] = val;
+        dst[u] = val;
     }
+}
+
+// The query stream of attn_dkdv_quad_kernel in one pass over q, dout and o (head dim 128): both K-type sections in its unit order
+// and the statistics fragment, whose row sums dout . o come from the rows just read.  HBM-bound; as bwd_stats_kernel followed by
+// pack_stream_kernel, dout was read twice and a row's 256 bytes by 16 threads that were not neighbours.  Eight threads per row,
+// two 16-byte units of each tensor per thread, rows read whole.  grid (n_tiles, B*H).
+// Measured at 16 heads x 37440 rows (bf16): 79 + 114 -> 145 us = 5.4 TB/s; x 24640 rows 52 + 87 -> 93 us.
+struct PackQuadParams {
+    PackSrc q, g, o;             // q, dout, o
+    const float* lse;            // [B,H,L]
+    float2* stats;               // [B*H][L] : (LSE log2 e, D)
+    char* out;
+    int H, L, n_tiles;
+};
+template <bool BF16>
+__global__ void __launch_bounds__(kPackThreads) pack_quad_stream_kernel(const PackQuadParams p) {
+    static_assert(kPackThreads == 8 * kRows, "eight threads per row of a tile");
+    constexpr int NC = 8;        // 16-channel chunks of a row
+    const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H, t = blockIdx.x;
+    const int r = threadIdx.x >> 3, part = threadIdx.x & 7, row = t * kRows + r;
+    const bool live = row < p.L;
+    uint4* dst = reinterpret_cast<uint4*>(p.out) + ((size_t)bh * p.n_tiles + t) * (size_t)((2 * NC + 1) * (kFragBytes / 16));
+    uint4 q[2], g[2], o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int c = 8 * (part + 8 * i);
+        auto unit = [&](const PackSrc& s) {
+            return live ? *reinterpret_cast<const uint4*>(s.ptr + (int64_t)b * s.sb + (int64_t)h * s.sh + (int64_t)row * s.sl + c) : make_uint4(0u, 0u, 0u, 0u);
+        };
+        q[i] = unit(p.q); g[i] = unit(p.g); o[i] = unit(p.o);
+    }
+    float lse = INFINITY;        // rows past the end: LSE = +inf (so P = 0) and D = 0
+    if (live) lse = p.lse[(int64_t)bh * p.L + row] * 1.4426950408889634f;
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t ow[4] = {o[i].x, o[i].y, o[i].z, o[i].w}, gw[4] = {g[i].x, g[i].y, g[i].z, g[i].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            acc += half_bits_to_float((uint16_t)(ow[k] & 0xFFFF), BF16) * half_bits_to_float((uint16_t)(gw[k] & 0xFFFF), BF16);
+            acc += half_bits_to_float((uint16_t)(ow[k] >> 16), BF16) * half_bits_to_float((uint16_t)(gw[k] >> 16), BF16);
+        }
+        const int C = part + 8 * i, slot = quad_unit_slot(r, C >> 1, C & 1);
+        dst[slot] = q[i];
+        dst[NC * 64 + slot] = g[i];
+    }
+    acc += __shfl_xor(acc, 1); acc += __shfl_xor(acc, 2); acc += __shfl_xor(acc, 4);
+    float* st = reinterpret_cast<float*>(dst + 2 * NC * 64);
+    if (part == 0) {
+        if (live) p.stats[(int64_t)bh * p.L + row] = make_float2(lse, acc);
+        // statistics fragment: 32 LSE values, then 32 D values, each half wavefront's 16 streamed rows together
+        const int idx = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
+        st[idx] = lse;
+        st[32 + idx] = acc;
+    }
+    if (threadIdx.x >= 16 && threadIdx.x < 64) dst[2 * NC * 64 + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);   // the fragment's unused rest
 }
 
 // ---------------------------------------------------------------------------------------------- main kernels
@@ -1049,29 +1102,36 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
         return true;
     };
 
-    {   // per-query statistics
-        StatsParams sp;
-        sp.o = (const uint16_t*)d->o; sp.dout = (const uint16_t*)d->dout;
-        sp.o_sb = d->o_stride[0]; sp.o_sh = d->o_stride[1]; sp.o_sl = d->o_stride[2];
-        sp.g_sb = d->dout_stride[0]; sp.g_sh = d->dout_stride[1]; sp.g_sl = d->dout_stride[2];
-        sp.lse = d->lse; sp.stats = stats; sp.H = d->H; sp.Lq = d->Lq; sp.d = d->d; sp.bf16 = bf16 ? 1 : 0;
-        hipLaunchKernelGGL(bwd_stats_kernel, dim3((d->Lq + kPackThreads / 8 - 1) / (kPackThreads / 8), BH), dim3(kPackThreads), 0, stream, sp);
-    }
-    {   // query stream: Q, dO, dO^T, Q^T, statistics
-        PackBwdParams pp;
-        pp.a1 = src_of(d->q, d->q_stride); pp.a2 = src_of(d->dout, d->dout_stride);
-        pp.c1 = src_of(d->dout, d->dout_stride); pp.c2 = src_of(d->q, d->q_stride);
-        pp.n_vt = g.quad ? 0 : 2; pp.swz = g.quad ? 1 : 0;
-        pp.stats = stats; pp.out = (uint4*)q_img;
-        pp.H = d->H; pp.L = d->Lq; pp.d = d->d; pp.n_tiles = g.n_q_tiles; pp.nc = g.nc; pp.ndb = g.ndb;
-        pp.tile_frags = (int)(g.q_tile_bytes / kFragBytes);
-        hipLaunchKernelGGL(pack_stream_kernel, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
+    if (g.quad) {   // query stream of attn_dkdv_quad_kernel: Q, dO, statistics
+        PackQuadParams pp;
+        pp.q = src_of(d->q, d->q_stride); pp.g = src_of(d->dout, d->dout_stride); pp.o = src_of(d->o, d->o_stride);
+        pp.lse = d->lse; pp.stats = stats; pp.out = q_img; pp.H = d->H; pp.L = d->Lq; pp.n_tiles = g.n_q_tiles;
+        hipLaunchKernelGGL(bf16 ? pack_quad_stream_kernel<true> : pack_quad_stream_kernel<false>, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
+    } else {
+        {   // per-query statistics
+            StatsParams sp;
+            sp.o = (const uint16_t*)d->o; sp.dout = (const uint16_t*)d->dout;
+            sp.o_sb = d->o_stride[0]; sp.o_sh = d->o_stride[1]; sp.o_sl = d->o_stride[2];
+            sp.g_sb = d->dout_stride[0]; sp.g_sh = d->dout_stride[1]; sp.g_sl = d->dout_stride[2];
+            sp.lse = d->lse; sp.stats = stats; sp.H = d->H; sp.Lq = d->Lq; sp.d = d->d; sp.bf16 = bf16 ? 1 : 0;
+            hipLaunchKernelGGL(bwd_stats_kernel, dim3((d->Lq + kPackThreads / 8 - 1) / (kPackThreads / 8), BH), dim3(kPackThreads), 0, stream, sp);
+        }
+        {   // query stream: Q, dO, dO^T, Q^T, statistics
+            PackBwdParams pp;
+            pp.a1 = src_of(d->q, d->q_stride); pp.a2 = src_of(d->dout, d->dout_stride);
+            pp.c1 = src_of(d->dout, d->dout_stride); pp.c2 = src_of(d->q, d->q_stride);
+            pp.n_vt = 2;
+            pp.stats = stats; pp.out = (uint4*)q_img;
+            pp.H = d->H; pp.L = d->Lq; pp.d = d->d; pp.n_tiles = g.n_q_tiles; pp.nc = g.nc; pp.ndb = g.ndb;
+            pp.tile_frags = (int)(g.q_tile_bytes / kFragBytes);
+            hipLaunchKernelGGL(pack_stream_kernel, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
+        }
     }
     {   // key stream: K, V, K^T  (K^T alone when dS is kept: the pass that reads it forms no scores)
         PackBwdParams pp;
         pp.a1 = src_of(d->k, d->k_stride); pp.a2 = src_of(d->v, d->v_stride);
         pp.c1 = src_of(d->k, d->k_stride); pp.c2 = PackSrc{nullptr, 0, 0, 0};
-        pp.n_vt = 1; pp.swz = 0;
+        pp.n_vt = 1;
         pp.stats = nullptr; pp.out = (uint4*)k_img;
         pp.H = d->H; pp.L = d->Lkv; pp.d = d->d; pp.n_tiles = g.n_k_tiles; pp.nc = g.spill ? 0 : g.nc; pp.ndb = g.ndb;
         pp.tile_frags = (int)(g.k_tile_bytes / kFragBytes);

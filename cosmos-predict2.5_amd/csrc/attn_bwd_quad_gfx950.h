@@ -27,7 +27,7 @@
 // or in LDS.  For both kinds of read to be free of bank conflicts the units of a part are stored in the order
 //     slot(q, cK, hK) = 16 (q/16 + 2 hK + 4 cK) + (q%4 + 4 ((q/4)%4 XOR (hK + 2 (cK%2)))):
 // the 16 lanes of a ds_read_b128 pass (16 consecutive rows, one cK, one hK) and the 32 lanes of a transposing pass (4 rows x
-// 2 chunks x 2 halves, both 8-byte halves of each unit) touch 256 consecutive-bank bytes each.  pack_stream_kernel writes the
+// 2 chunks x 2 halves, both 8-byte halves of each unit) touch 256 consecutive-bank bytes each.  pack_quad_stream_kernel writes the
 // image in that order; the direct-to-LDS fills copy it linearly.
 // LDS: rings of the two stream parts (Q 7 deep: fetched three steps before S1 uses it, kept until O2 has used it three steps
 // later; dO 5 deep), U and W hand-over (two stages each), statistics ring (6).  All fills are issued by the O wavefronts (five

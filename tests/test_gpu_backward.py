@@ -50,6 +50,23 @@ def test_bwd_ragged_small(pkg, oracle, gpu, Lq, Lkv):
     run_bwd(pkg, oracle, gpu, (1, 2, Lq, 128), (1, 2, Lkv, 128), seed=Lq + Lkv)
 
 
+@pytest.mark.parametrize("Lq", [1, 31, 32, 33, 63, 165])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_bwd_query_stream_layouts(pkg, oracle, gpu, Lq, dtype):
+    """The fused re-tiling of q, dout and the row sums dout . o: full, ragged and single-row tiles, with the three tensors in three
+    different layouts, with dS kept and with the dQ kernel that reads the row sums from memory (same tolerances as above)."""
+    q, k, v, _, _, _ = oracle.make_inputs((2, 3, Lq, 128), (2, 3, 70, 128), seed=Lq, dtype=dtype)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(Lq)).to(dtype)
+    want = oracle.grads_closed_form(q, k, v, dout)
+    qd, kd, vd = q.transpose(1, 2).contiguous().to(gpu).transpose(1, 2), k.to(gpu), v.to(gpu)
+    wide = torch.zeros(2, 3, Lq, 136, dtype=dtype, device=gpu)
+    wide[..., :128] = dout.to(gpu)
+    o, _, lse = pkg.fwd_jvp(qd, kd, vd)
+    for max_ds_mib in (None, -1):
+        for name, got, ref in zip(("dq", "dk", "dv"), pkg.ops.bwd(qd, kd, vd, o, lse, wide[..., :128], max_ds_mib=max_ds_mib), want):
+            check(oracle, name, got, ref)
+
+
 @pytest.mark.parametrize("L", [128, 999, 1024])
 def test_bwd_self_attention_d128(pkg, oracle, gpu, L):
     run_bwd(pkg, oracle, gpu, (1, 2, L, 128), seed=L)
