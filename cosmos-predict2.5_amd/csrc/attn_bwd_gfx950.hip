@@ -238,6 +238,20 @@ __global__ void __launch_bounds__(kPackThreads) pack_quad_stream_kernel(const Pa
     if (threadIdx.x >= 16 && threadIdx.x < 64) dst[2 * NC * 64 + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);   // the fragment's unused rest
 }
 
+// K^T alone, for attn_dq_from_ds_kernel: a run of kKtTiles tiles of one head per workgroup.  HBM-bound; pack_stream_kernel, which
+// gathers a unit from eight 2-byte loads, took 87 - 99 us at 16 heads x 24640 rows, this 58; at 512 rows 11 and 5.6.
+constexpr int kKtTiles = 4;
+__global__ void __launch_bounds__(kPackThreads) pack_kt_kernel(const PackSrc k, uint4* out, int H, int L, int d, int n_tiles, int ndb) {
+    const int bh = blockIdx.y, b = bh / H, h = bh % H, t0 = blockIdx.x * kKtTiles;
+    const int quads = 8 * ndb, per_tile = 4 * quads, tiles = n_tiles - t0 < kKtTiles ? n_tiles - t0 : kKtTiles;
+    const uint16_t* head = k.ptr + (int64_t)b * k.sb + (int64_t)h * k.sh;
+    uint4* dst = out + ((size_t)bh * n_tiles + t0) * (size_t)(2 * ndb * (kFragBytes / 16));
+    for (int u = threadIdx.x; u < tiles * per_tile; u += kPackThreads) {
+        const int t = u / per_tile, w = u - t * per_tile, quad = w % quads, ch = w / quads;
+        transpose_units(head, k.sl, (t0 + t) * kRows, L, d, quad, ch & 1, ch >> 1, dst + (size_t)t * (2 * ndb * (kFragBytes / 16)));
+    }
+}
+
 // ---------------------------------------------------------------------------------------------- main kernels
 struct BwdParams {
     const void *st1, *st2;             // stationary operands: rows of (q, dout) for dQ, of (k, v) for dK/dV
@@ -1127,13 +1141,16 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
             hipLaunchKernelGGL(pack_stream_kernel, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
         }
     }
-    {   // key stream: K, V, K^T  (K^T alone when dS is kept: the pass that reads it forms no scores)
+    if (g.spill) {   // key stream: K^T alone (the pass that reads it forms no scores)
+        hipLaunchKernelGGL(pack_kt_kernel, dim3((g.n_k_tiles + kKtTiles - 1) / kKtTiles, BH), dim3(kPackThreads), 0, stream,
+                           src_of(d->k, d->k_stride), (uint4*)k_img, d->H, d->Lkv, d->d, g.n_k_tiles, g.ndb);
+    } else {         // key stream: K, V, K^T
         PackBwdParams pp;
         pp.a1 = src_of(d->k, d->k_stride); pp.a2 = src_of(d->v, d->v_stride);
         pp.c1 = src_of(d->k, d->k_stride); pp.c2 = PackSrc{nullptr, 0, 0, 0};
         pp.n_vt = 1;
         pp.stats = nullptr; pp.out = (uint4*)k_img;
-        pp.H = d->H; pp.L = d->Lkv; pp.d = d->d; pp.n_tiles = g.n_k_tiles; pp.nc = g.spill ? 0 : g.nc; pp.ndb = g.ndb;
+        pp.H = d->H; pp.L = d->Lkv; pp.d = d->d; pp.n_tiles = g.n_k_tiles; pp.nc = g.nc; pp.ndb = g.ndb;
         pp.tile_frags = (int)(g.k_tile_bytes / kFragBytes);
         hipLaunchKernelGGL(pack_stream_kernel, dim3(g.n_k_tiles, BH), dim3(kPackThreads), 0, stream, pp);
     }

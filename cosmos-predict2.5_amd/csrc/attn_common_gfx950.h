@@ -90,6 +90,30 @@ __device__ __forceinline__ void issue_part(__amdgpu_buffer_rsrc_t rsrc, char* ds
     if (LOADS > 3) lds_load<3 * kFragBytes>(rsrc, dst, lane_off, src);
 }
 
+// Four units of a V^T-type section (channels 4 quad .. + 3, key chunk c, lane half hh of the 32-key tile at row key0): eight 8-byte
+// loads, one per key, of which 32 neighbouring threads cover whole rows of 128 channels, transposed in registers into four 16-byte
+// stores side by side.  Channels past `width` and rows past `rows` become zeros.
+__device__ __forceinline__ void transpose_units(const uint16_t* head, int64_t row_stride, int key0, int rows, int width, int quad, int c, int hh, uint4* section) {
+    const int d = 4 * quad;
+    uint2 r[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const int key = key0 + 16 * c + 8 * (s >> 2) + 4 * hh + (s & 3);
+        r[s] = key < rows && d < width ? *reinterpret_cast<const uint2*>(head + (int64_t)key * row_stride + d) : make_uint2(0u, 0u);
+    }
+    uint4* dst = section + (2 * (d >> 5) + c) * (kFragBytes / 16) + 32 * hh + (d & 31);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t a = j < 2 ? r[2 * i].x : r[2 * i].y, b = j < 2 ? r[2 * i + 1].x : r[2 * i + 1].y;
+            w[i] = j & 1 ? (a >> 16) | (b & 0xFFFF0000u) : (a & 0xFFFFu) | (b << 16);
+        }
+        dst[j] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per (device, kernel).  A kernel's LDS size is a compile-time
 // constant of its instantiation, so the call never needs repeating; keeping it out of the steady state also keeps
 // the entry points usable while a stream is being captured into a graph.  (Needs <mutex>, <set>, <utility>.)

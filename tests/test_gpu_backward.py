@@ -67,6 +67,12 @@ def test_bwd_query_stream_layouts(pkg, oracle, gpu, Lq, dtype):
             check(oracle, name, got, ref)
 
 
+@pytest.mark.parametrize("Lkv", [1, 33, 96, 128, 130, 260])
+def test_bwd_key_stream_tiles(pkg, oracle, gpu, Lkv):
+    """Runs of four re-tiled K^T tiles: fewer than one, one and several, ragged last tiles and last runs."""
+    run_bwd(pkg, oracle, gpu, (1, 2, 70, 128), (1, 2, Lkv, 128), seed=Lkv)
+
+
 @pytest.mark.parametrize("L", [128, 999, 1024])
 def test_bwd_self_attention_d128(pkg, oracle, gpu, L):
     run_bwd(pkg, oracle, gpu, (1, 2, L, 128), seed=L)
