@@ -88,7 +88,8 @@ _FUSED_MODULATION_ROWS = 64
 
 def _bare(m: nn.Module) -> bool:
     """Is calling m the same as computing its forward?"""
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__)
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
+                or nn.modules.module._has_any_global_hook())
 
 
 class GPT2FeedForward(nn.Module):

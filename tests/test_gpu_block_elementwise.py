@@ -177,6 +177,9 @@ def test_modulation_dispatch(pkg, gpu):
         handle = m.adaln_modulation_mlp[1].register_forward_hook(lambda mod, a, out: out * 2)
         assert m._fused_modulations(emb, lora, x) is None
         handle.remove()
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, a, out: None)
+        assert m._fused_modulations(emb, lora, x) is None
+        handle.remove()
         assert m._fused_modulations(emb, lora, x) is not None
         m.adaln_modulation_mlp[0] = torch.nn.GELU()
         assert m._fused_modulations(emb, lora, x) is None
