@@ -85,9 +85,17 @@ struct PackParams {
     int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
     uint4* out;
     int H, Lkv, dqk, dv, n_tiles;
+    int run;                           // tiles per workgroup
 };
 
-// grid (ceil(n_tiles / 2), B*H); every 16-byte unit of a tile image is produced by one thread.
+// grid (ceil(n_tiles / run), B*H, parts); every 16-byte unit of a tile image is produced by one thread, a workgroup makes the
+// units of one part of a run of tiles.  HBM-bound, in short calls bound by the chain of load and store that a thread goes through
+// for each of its units: two units per thread (kPackUnits) are fast throughout.  Measured (16 heads, d = 128, forward only, us, two tiles
+// per workgroup and so eight units per thread -> two units): 512 keys 5.5 -> 3.5, 1560 7.0 -> 5.7, 3520 10.9 -> 10.2,
+// 37440 114 -> 112 (5.5 TB/s), 84480 251 -> 248; d = 256, 512 keys, 8.7 -> 4.6.  One unit per thread is slower where there are
+// many (d = 64, 3520 keys: two units 5.8, one 6.6).  Not faster: V^T from 8-byte loads of whole rows, transposed in registers (37440 keys: 121),
+// as its stores leave 16 bytes in every 64.
+constexpr int kPackUnits = 2;
 __global__ void __launch_bounds__(kPackThreads) pack_kv_kernel(const PackParams p) {
     const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H;
     const bool full = p.tk != nullptr;
@@ -95,11 +103,11 @@ __global__ void __launch_bounds__(kPackThreads) pack_kv_kernel(const PackParams 
     const int64_t k_off = (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
     const int64_t v_off = (int64_t)b * p.v_sb + (int64_t)h * p.v_sh;
     const int units = g.tile_frags * 64;
-    for (int tt = 0; tt < 2; ++tt) {
-        const int t = blockIdx.x * 2 + tt;
+    for (int tt = 0; tt < p.run; ++tt) {
+        const int t = blockIdx.x * p.run + tt;
         if (t >= p.n_tiles) break;
         uint4* dst = p.out + ((size_t)bh * p.n_tiles + t) * (size_t)(g.tile_frags * (kFragBytes / 16));
-        for (int u = threadIdx.x; u < units; u += kPackThreads) {
+        for (int u = blockIdx.z * kPackThreads + threadIdx.x; u < units; u += gridDim.z * kPackThreads) {
             int frag = u >> 6;
             const int l = u & 63, i = l & 31, hh = l >> 5;
             uint4 val = make_uint4(0u, 0u, 0u, 0u);
@@ -1674,7 +1682,10 @@ COSMOS_ATTN_API int cosmos_attn_pack_kv(const cosmos_attn_desc* d, void* workspa
     pp.v_sb = d->v_stride[0]; pp.v_sh = d->v_stride[1]; pp.v_sl = d->v_stride[2];
     pp.out = (uint4*)workspace;
     pp.H = d->H; pp.Lkv = d->Lkv; pp.dqk = d->d_qk; pp.dv = d->d_v; pp.n_tiles = n_tiles_of(d);
-    hipLaunchKernelGGL(pack_kv_kernel, dim3((pp.n_tiles + 1) / 2, d->B * d->H), dim3(kPackThreads), 0, (hipStream_t)stream, pp);
+    const int frags = (int)(tile_bytes_of(d) / kFragBytes), frags_per_part = kPackUnits * kPackThreads / 64;
+    pp.run = frags < frags_per_part ? 2 : 1;                             // (small head dims: a tile is less than a workgroup's share)
+    const int parts = frags < frags_per_part ? 1 : frags / frags_per_part;
+    hipLaunchKernelGGL(pack_kv_kernel, dim3((pp.n_tiles + pp.run - 1) / pp.run, d->B * d->H, parts), dim3(kPackThreads), 0, (hipStream_t)stream, pp);
     return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
 }
 

@@ -490,6 +490,50 @@ def test_autograd_function_contract(pkg, oracle, gpu):
         o.sum().backward()
 
 
+def _kv_image(k, v):
+    """The re-tiled image of one head by its definition: per tile of 32 keys, fragments of 64 lanes x 8 elements."""
+    (L, dk), dv = k.shape, v.shape[1]
+    tiles, ndb = -(-L // 32), -(-dv // 32)
+    kp, vp = np.zeros((tiles, 32, dk), np.int16), np.zeros((tiles, 32, 32 * ndb), np.int16)
+    kp.reshape(-1, dk)[:L] = k
+    vp.reshape(-1, 32 * ndb)[:L, :dv] = v
+    # K-type [c][half][row][8]; V^T-type [db][c][half][column][s / 4][s % 4], key 16 c + 8 (s / 4) + 4 half + s % 4
+    return (kp.reshape(tiles, 32, dk // 16, 2, 8).transpose(0, 2, 3, 1, 4).reshape(tiles, -1),
+            vp.reshape(tiles, 2, 2, 2, 4, ndb, 32).transpose(0, 5, 1, 3, 6, 2, 4).reshape(tiles, -1))
+
+
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("Lkv,d_qk,d_v", [(1, 16, 16), (31, 32, 128), (33, 64, 32), (64, 128, 128), (65, 128, 64), (97, 256, 256), (130, 128, 16), (300, 16, 256)])
+def test_packed_image(pkg, oracle, gpu, Lkv, d_qk, d_v, full):
+    """The re-tiled K/V image, byte for byte: every head dim and section, ragged and odd numbers of tiles, strided views."""
+    L, lib = pkg._lib, pkg._lib.load_library()
+    B, H = 2, 3
+    g = torch.Generator().manual_seed(Lkv + d_qk)
+    mk = lambda d: torch.randn((B, Lkv, H, d), generator=g).to(torch.bfloat16).to(gpu).transpose(1, 2)
+    k, v, tk, tv = mk(d_qk), mk(d_v), mk(d_qk), mk(d_v)
+    q, o = torch.zeros((B, H, 5, d_qk), device=gpu, dtype=k.dtype), torch.zeros((B, H, 5, d_v), device=gpu, dtype=k.dtype)
+    D = L.AttnDesc()
+    D.abi_version, D.dtype = L.ABI_VERSION, L.DTYPE_BF16
+    D.B, D.H, D.Lq, D.Lkv, D.d_qk, D.d_v, D.causal, D.sm_scale = B, H, 5, Lkv, d_qk, d_v, 0, 1.0
+    D.q, D.k, D.v, D.o = (x.data_ptr() for x in (q, k, v, o))
+    D.tq, D.tk, D.tv, D.to = (x.data_ptr() if full else None for x in (q, tk, tv, o))
+    s3 = lambda x: (ctypes.c_int64 * 3)(x.stride(0), x.stride(1), x.stride(2))
+    D.q_stride, D.k_stride, D.v_stride, D.o_stride = s3(q), s3(k), s3(v), s3(o)
+    n = lib.cosmos_attn_packed_bytes(ctypes.byref(D))
+    image = torch.full((n // 2 + 64,), 0x5A5A, device=gpu, dtype=torch.int16)
+    assert lib.cosmos_attn_pack_kv(ctypes.byref(D), image.data_ptr(), n, torch.cuda.current_stream().cuda_stream) == 0
+    got = image.cpu().numpy()
+    host = lambda x: x.contiguous().cpu().view(torch.int16).numpy()
+    k, v, tk, tv = (host(x) for x in (k, v, tk, tv))
+    want = []
+    for b in range(B):
+        for h in range(H):
+            parts = [_kv_image(k[b, h], v[b, h])] + ([_kv_image(tk[b, h], tv[b, h])] if full else [])
+            want.append(np.concatenate([p[0] for p in parts] + [p[1] for p in parts], axis=1).reshape(-1))
+    want = np.concatenate(want)
+    assert np.array_equal(got[:want.size], want) and (got[want.size:] == 0x5A5A).all()
+
+
 def test_c_abi_two_stage_equals_one_call(pkg, oracle, gpu):
     """cosmos_attn_pack_kv + cosmos_attn_run called directly through ctypes == cosmos_attn_fwd_jvp; workspace reuse across
     two runs with different q (the cross-attention / fixed-context use)."""
