@@ -399,7 +399,9 @@ __global__ void __launch_bounds__(kThreads) ln_modulate_bwd_kernel(const LnModBw
         block_sums<3 * R>(s, red2);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const float rs = rsqrtf(s[3 * r] * inv_d + p.eps), m1 = s[3 * r + 1] * inv_d, m2 = s[3 * r + 2] * inv_d * rs;
+            // a row past the end has no variance: with eps = 0 its rsqrt is inf, and 0 inf would reach the column sums
+            const float rs = row0 + r < hi ? rsqrtf(s[3 * r] * inv_d + p.eps) : 0.f;
+            const float m1 = s[3 * r + 1] * inv_d, m2 = s[3 * r + 2] * inv_d * rs;
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
                 const int off = 8 * ((int)threadIdx.x + kThreads * c);

@@ -127,6 +127,20 @@ def test_reverse_mode(pkg, gpu, rows, rpg, D, dtype):
     check("dgate", got[1], dgate, dtype)
 
 
+@pytest.mark.parametrize("rows,rpg,D", [(17, 17, 264), (66, 33, 2048), (5, 1, 64), (34, 17, 2056), (33, 33, 4104)])
+def test_reverse_mode_without_eps(pkg, gpu, rows, rpg, D):
+    """eps = 0, runs that end inside the rows that are in flight together (four up to 2048 columns, two up to 4096): the rows past
+    the end, which have no variance, stay out of the column sums.  Bounds as in test_reverse_mode."""
+    dtype, g = torch.bfloat16, torch.Generator().manual_seed(rows + D)
+    x, dy, sc = rnd(g, dtype, rows, D, std=2.0, mean=0.5), rnd(g, dtype, rows, D), rnd(g, dtype, rows // rpg, D, std=0.3)
+    rep = lambda m: m.repeat_interleave(rpg, dim=0)
+    xr, scr, shr = (t.double().requires_grad_(True) for t in (x, sc, torch.zeros_like(sc)))
+    y = torch.nn.functional.layer_norm(xr, (D,), eps=0.0) * (1 + rep(scr)) + rep(shr)
+    want = torch.autograd.grad(y, (xr, shr, scr), dy.double())
+    for name, got, ref in zip(("dx", "dshift", "dscale"), pkg.ops.ln_modulate_bwd(x.to(gpu), sc.to(gpu), dy.to(gpu), eps=0.0), want):
+        check(name, got, ref, dtype)
+
+
 @pytest.mark.parametrize("rows,K,hidden,D", [(1, 32, 32, 16), (3, 2048, 256, 2048), (8, 256, 64, 48), (16, 288, 32, 80), (17, 5120, 256, 128), (40, 96, 96, 32)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_modulation(pkg, gpu, rows, K, hidden, D, dtype):
