@@ -138,11 +138,14 @@ inline bool allow_lds(const void* fn, size_t bytes) {
 // (1 = leave it) of the least cost in microseconds, where
 //   * a round of workgroups takes `steps` barrier steps of step_us each and range_us to start and end;
 //   * the step of a round that fills only a part of the chip is faster, as the part then clocks higher under its power limit:
-//     0.7 of the full chip's time for a few workgroups, growing with the square of the filled part (forward only, one round,
-//     384-row steps: 1.86 us at 112 of 256 workgroups, 1.95 at 160, 2.34 at 224, 2.66 in full rounds);
+//     `alone` (0.7 at head dim 128) of the full chip's time for a few workgroups, growing with the square of the filled part
+//     (forward only, one round, 384-row steps: 1.86 us at 112 of 256 workgroups, 1.95 at 160, 2.34 at 224, 2.66 in full rounds);
+//     smaller head dims draw less power: 0.9;
 //   * every range leaves slot_bytes of partial results, written once and read once by the merge kernel: 3.8 MB of them cost a
 //     microsecond, the merge kernel's launch three.
-// The constants are fits to B*H = 16 .. 80, 255 .. 17600 positions and S = 1 .. 16, every S measured.  What the rule that
+// The constants are fits to B*H = 16 .. 80, 255 .. 17600 positions and S = 1 .. 16, every S measured (the forward's at head dims 16 .. 128
+// each, beside plan_split; the backward's step at 128, taken down with the head dim: at 16 .. 64, B*H = 16 and 40, 700 .. 9000 positions, its
+// choice takes 1.014 times the best S on average, 1.11 at most).  What the rule that
 // counted rounds alone chose, and this one (us, forward + tangents unless said, head dim 128, with the re-tiling):
 //   1 x 16 x 1560: S = 11 243, S = 1 77;   1 x 40 x 512: S = 3 64, S = 1 40;   1 x 16 x 7040: S = 16 1093, S = 2 1012;
 //   forward only 1 x 16 x 3520: S = 8 222, S = 1 133;   1 x 16 x 5000: S = 8 388, S = 1 217;
@@ -151,13 +154,19 @@ inline bool allow_lds(const void* fn, size_t bytes) {
 constexpr int kNumCUs = 256;          // MI355X
 constexpr int kMaxSplits = 16;
 constexpr int kMinStepsPerSplit = 4;
-struct StepCost { double step_us, range_us; };   // a barrier step in full rounds, and what a workgroup costs besides its steps
+struct StepCost { double step_us, range_us, alone = 0.7; };   // a barrier step in full rounds, and what a workgroup costs besides its steps
 // `pairs` workgroups of n_steps / S steps each, in rounds
 inline double rounds_cost(int64_t pairs, double n_steps, StepCost c) {
     if (pairs <= 0) return 0.0;
     const int64_t rounds = (pairs + kNumCUs - 1) / kNumCUs;
     const double filled = (double)pairs / (double)(rounds * kNumCUs);
-    return (double)rounds * (n_steps * c.step_us * (0.7 + 0.3 * filled * filled) + c.range_us);
+    return (double)rounds * (n_steps * c.step_us * (c.alone + (1.0 - c.alone) * filled * filled) + c.range_us);
+}
+// a value measured at head dims 16, 32, 64 and 128, and on the line between two of them for calls of unequal head dims
+inline double by_head_dim(const double (&at)[4], double d) {
+    const int i = d > 64.0 ? 2 : d > 32.0 ? 1 : 0;
+    const double lo = (double)(16 << i);
+    return at[i] + (at[i + 1] - at[i]) * (d - lo) / lo;
 }
 inline double split_cost(int rem, int n_steps, int S, StepCost c, double slot_bytes) {
     return rounds_cost((int64_t)rem * S, (double)n_steps / S, c) + (S > 1 ? 3.0 + (double)rem * S * slot_bytes / 3.8e6 : 0.0);

@@ -1531,19 +1531,26 @@ size_t tiles_bytes_of(const cosmos_attn_desc* d) { return (size_t)d->B * d->H * 
 // a head dim of 256 goes to attn_wide_kernel
 bool is_wide(const cosmos_attn_desc* d) { return d->d_qk == 256 || d->d_v == 256; }
 struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // us: estimated time of the launches
+// Barrier steps in full rounds at head dims 16, 32, 64, 128 (us): below 64 the exponentials and the step's fixed instructions are
+// most of it.  Fits to 500 .. 9000 positions and 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, S = 1 .. 16, every S measured: the S
+// chosen with them takes 1.0035 to 1.011 times the best one's time on average, 1.13 at most.  (A step that shrinks in proportion to the
+// head dim, which had been assumed, cut too few: forward only, us, 16 x 700 at head dim 16 23.0 -> 20.3, 40 x 1100 36.8 -> 32.9, 40 x 9000 at 32
+// 889 -> 789.)
+constexpr double kStepUs[3][4] = {{1.36, 1.37, 1.77, 2.66}, {0.54, 0.56, 0.68, 0.86}, {0.54, 0.60, 0.82, 1.21}};   // MODE_FWD, MODE_JVP_Q, MODE_JVP_FULL
+constexpr double kStepAlone[4] = {0.9, 0.9, 0.9, 0.7};
+constexpr double kPairUs[4] = {5.0, 5.0, 5.0, 13.0};          // what a workgroup that is a whole pair costs besides its steps
 SplitPlan plan_split(const cosmos_attn_desc* d) {
     SplitPlan s;
     const bool fwd = mode_of(d) == MODE_FWD;
-    // (smaller head dims: fewer matrix instructions per step, the same exponentials; tangent on q only: two thirds of them)
-    const double part = 0.3 + 0.7 * (d->d_qk + d->d_v) / 256.0;
-    const StepCost c = fwd ? StepCost{2.66 * part, 13.0} : StepCost{(mode_of(d) == MODE_JVP_Q ? 0.86 : 1.21) * part, 8.0};
+    const double dim = 0.5 * (d->d_qk + d->d_v);
+    const StepCost c{by_head_dim(kStepUs[mode_of(d)], dim), fwd && dim > 64.0 ? 13.0 : 8.0, by_head_dim(kStepAlone, dim)};
     const int n_steps = fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d);   // barrier steps: 64 keys forward only, 32 with tangents
     s.block_m = fwd ? kSymBlockM : kBlockM;
     s.n_qt = (d->Lq + s.block_m - 1) / s.block_m;
     s.n_pairs = s.n_qt * d->B * d->H;
     s.n_rem = 0; s.splits = 1; s.n_full = s.n_pairs;
     const int rem = s.n_pairs % kNumCUs;
-    const StepCost alone = StepCost{c.step_us, 13.0};                    // (a workgroup that is a whole pair also starts and ends it)
+    const StepCost alone{c.step_us, by_head_dim(kPairUs, dim), c.alone};
     s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
     if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
     const double slot_bytes = (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4));
@@ -1556,14 +1563,21 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
 // of compute units (every unit gets the same number of equal pieces).  It is chosen where the units' share of query blocks, at
-// block_us + tile_us per key tile each, comes out faster than the other kernels' rounds: a finished block costs it little, a key
-// tile costs it more than the forward-only kernel (which has three wavefronts per SIMD).  Measured (us, stream / other kernel,
-// 16 heads; B*H = 40 and the lengths between alike): tangent on q 3520 x 512 keys 45 / 62, 7040 x 512 78 / 109, 37440 x 2048
-// 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  With all tangents the
+// block_us + tile_us per key tile each and start_us once, comes out faster than the other kernels' rounds: a finished block costs it
+// little, a key tile costs it more than the forward-only kernel (which has three wavefronts per SIMD).  Measured (us, stream / other kernel,
+// 16 heads): tangent on q 3520 x 512 keys 45 / 62, 7040 x 512 78 / 109, 37440 x 2048
+// 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  Forward only at small head
+// dims the stream pays only while a unit has one block (head dim 32: 1560 x 512 16 / 19, 3520 x 512 24 / 20, 40 heads 1560 x 512 33 / 22).
+// The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: the way chosen takes
+// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  With all tangents the
 // two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
 // cosmos_attn_set_stream_override() replaces the choice (tuning and tests); nothing in the per-call path reads the environment.
 constexpr int kStreamMaxTiles = 64;       // up to 2048 keys
 constexpr int kStreamGroupsPerCU = 1;       // one workgroup fills a compute unit (8 wavefronts, 2 per SIMD at 256 registers): a single round
+// forward only, tangent on q: at head dims 16, 32, 64, 128
+constexpr double kStreamTileUs[2][4] = {{0.32, 0.32, 0.44, 0.63}, {0.58, 0.62, 0.60, 0.79}};
+constexpr double kStreamBlockUs[2][4] = {{2.5, 2.0, 0.5, 1.0}, {3.5, 2.5, 0.5, 6.0}};
+constexpr double kStreamStartUs[4] = {5.0, 5.0, 5.0, 0.0};
 constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
 std::atomic<int> g_stream_groups{0};      // number of workgroups, 0 = the library's own choice
@@ -1582,11 +1596,10 @@ int stream_groups_of(const cosmos_attn_desc* d) {
     if (pairs < kStreamMinPairs) return 0;
     const int groups = kNumCUs * kStreamGroupsPerCU;
     const int mode = mode_of(d);
-    const double part = 0.3 + 0.7 * d->d_qk / 128.0;
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
-    const double tile_us = (mode == MODE_FWD ? 0.575 : 0.79) * part, block_us = mode == MODE_FWD ? 2.4 : 6.0;
-    const double stream_us = (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
-    return stream_us <= 1.03 * plan_split(d).us ? groups : 0;     // (40 heads, 7040 x 512 keys, forward only: 109 us against 117)
+    const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
+    const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
+    return stream_us <= plan_split(d).us ? groups : 0;
 }
 // LDS of attn_qstream_kernel: the layout of attn_fwd_jvp_kernel (AttnCfg::LDS_BYTES) + the per-block statistics slots
 size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {

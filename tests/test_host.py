@@ -109,6 +109,23 @@ def test_key_range_plan(pkg, H, L, tangents, ranges):
     assert extra == (0 if ranges == 1 else rem * ranges * block * (128 * (2 if tangents else 1) * 4 + 16))
 
 
+@pytest.mark.parametrize("d,H,L,ranges", [
+    (16, 16, 700, 2),         # forward only: 32 pairs of 11 steps
+    (16, 40, 1100, 2),        # 120 pairs
+    (32, 40, 9000, 4),        # 960 pairs: 192 of a fourth round
+    (64, 40, 1100, 2),        # 120 pairs
+    (64, 16, 5000, 1),        # 224 pairs in one round
+])
+def test_key_range_plan_below_head_dim_128(pkg, d, H, L, ranges):
+    """As above, forward only: a step costs more than its share of matrix instructions there, so that more calls are worth cutting."""
+    lib = pkg._lib.load_library()
+    D = good_desc(pkg, B=1, H=H, Lq=L, Lkv=L, d_qk=d, d_v=d, tq=None, tk=None, tv=None, to=None)
+    rem = (L + 383) // 384 * H % 256
+    extra = lib.cosmos_attn_workspace_bytes(ctypes.byref(D)) - lib.cosmos_attn_packed_bytes(ctypes.byref(D))
+    acc = rem * ranges * 384 * d * 4
+    assert extra == (0 if ranges == 1 else (acc + 255) // 256 * 256 + rem * ranges * 384 * 16)
+
+
 def good_bwd_desc(pkg, **over):
     D = pkg._lib.AttnBwdDesc()
     D.abi_version, D.dtype = pkg._lib.ABI_VERSION, pkg._lib.DTYPE_BF16
