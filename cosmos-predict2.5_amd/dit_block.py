@@ -241,6 +241,8 @@ class Block(nn.Module):
             return None
         if any(w.shape != (w1[0].shape[0], K) for w in w1) or any(w.shape != (3 * D, w1[0].shape[0]) for w in w2):
             return None
+        if not all(ops._is_dense16(w) for w in (*w1, *w2)):     # (views of a flat buffer: the library's layers read them where they are)
+            return None
         return ops.modulation(emb, lora, w1, w2, temb, tlora, tangent)
 
     def _fp32_region(self, t: torch.Tensor):

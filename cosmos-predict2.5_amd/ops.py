@@ -448,8 +448,14 @@ def as_stacked(x: torch.Tensor, tx: torch.Tensor) -> Optional[torch.Tensor]:
     return None
 
 
+def _is_dense16(t: torch.Tensor) -> bool:
+    return t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
 def _dense16(t: torch.Tensor) -> torch.Tensor:
-    return t if (t.is_contiguous() and t.data_ptr() % 16 == 0) else t.contiguous()
+    """``t``, or a copy where it is not contiguous or does not start at 16 bytes (``.contiguous()`` returns a contiguous slice of a
+    larger buffer as it is, wherever that starts)."""
+    return t if _is_dense16(t) else t.clone(memory_format=torch.contiguous_format)
 
 
 def _check_elementwise(x: torch.Tensor) -> None:

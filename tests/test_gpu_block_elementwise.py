@@ -170,6 +170,40 @@ def test_modulation(pkg, gpu, rows, K, hidden, D, dtype):
         check("tout", tout, twant, dtype, flip)
 
 
+def off16(t):
+    """t's values, contiguous, but one element past a 16-byte boundary (a slice of a larger buffer)."""
+    v = torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
+    assert v.is_contiguous() and v.data_ptr() % 16 == t.element_size()
+    return v
+
+
+def test_inputs_that_start_off_16_bytes(pkg, gpu):
+    """Gradients, embeddings and weights that are contiguous slices of larger buffers: the same bits as from aligned ones.  Weights
+    like that go to the modules (the fused call would copy them every time)."""
+    g = torch.Generator().manual_seed(3)
+    x, dy, dskip, res = (rnd(g, torch.bfloat16, 12, 264).to(gpu) for _ in range(4))
+    sc = rnd(g, torch.bfloat16, 3, 264, std=0.3).to(gpu)
+    same = lambda a, b: all(p is None and q is None or torch.equal(p, q) for p, q in zip(a, b))
+    assert same(pkg.ops.ln_modulate_bwd(off16(x), off16(sc), off16(dy), off16(dskip)), pkg.ops.ln_modulate_bwd(x, sc, dy, dskip))
+    assert same(pkg.ops.gated_residual_bwd(off16(res), off16(sc), off16(dy)), pkg.ops.gated_residual_bwd(res, sc, dy))
+
+    torch.manual_seed(0)
+    m = pkg.Block(256, 64, 2, use_adaln_lora=True, adaln_lora_dim=32).to(gpu, torch.bfloat16).eval()
+    for p in m.parameters():
+        torch.nn.init.normal_(p, std=p.shape[-1] ** -0.5)
+    x, emb, lora, ctx = (torch.randn(*s, device=gpu).bfloat16() for s in ((1, 2, 2, 4, 256), (1, 2, 256), (1, 2, 768), (1, 8, 64)))
+    temb, tlora = torch.randn_like(emb), torch.randn_like(lora)
+    run = lambda e, l, te, tl: (m(x, e, ctx, None, l), *m.forward_jvp(x, x, e, te, ctx, None, l, tl))
+    with torch.no_grad():
+        want = run(emb, lora, temb, tlora)
+        assert same(run(off16(emb), off16(lora), off16(temb), off16(tlora)), want)
+        for layer in (m.adaln_modulation_mlp[1], m.adaln_modulation_mlp[2]):
+            layer.weight = torch.nn.Parameter(off16(layer.weight.detach()))
+            assert m._fused_modulations(emb, lora, x) is None
+        for a, b in zip(run(emb, lora, temb, tlora), want):      # the modules round the modulation vectors once more
+            assert float((a.float() - b.float()).norm()) <= 1e-2 * float(b.float().norm())
+
+
 def test_modulation_dispatch(pkg, gpu):
     """The block takes the fused call only for the plain MLPs of one 16-bit type; otherwise the modules themselves, which agree."""
     torch.manual_seed(0)

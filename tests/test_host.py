@@ -585,3 +585,15 @@ def test_checkpoint_configuration_and_kept_attention_results_bookkeeping(pkg):
         with att.replay_attention_results([("o", "lse")]):
             pass
     assert att._kept.replay is None
+
+
+@pytest.mark.parametrize("first", [0, 1, 4, 8])
+def test_dense16_copies_what_starts_off_16_bytes(pkg, first):
+    """A contiguous slice of a larger buffer is contiguous wherever it starts; the elementwise kernels need it to start at 16 bytes."""
+    buf = torch.arange(64, dtype=torch.float32).bfloat16()
+    assert buf.data_ptr() % 16 == 0
+    t = buf[first:first + 48].view(6, 8)
+    got = pkg.ops._dense16(t)
+    assert got.is_contiguous() and got.data_ptr() % 16 == 0 and torch.equal(got, t)
+    assert (got is t) == (first % 8 == 0)
+    assert torch.equal(pkg.ops._dense16(t.t()), t.t()) and pkg.ops._dense16(t.t()).is_contiguous()
