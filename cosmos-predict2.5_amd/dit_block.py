@@ -27,6 +27,32 @@ from . import ops
 from .dit_attention import Attention, I2VCrossAttention
 
 
+def _per_row(m, like):
+    """The modulation vectors m, one per group of consecutive rows, repeated to the shape of ``like``."""
+    D = like.shape[-1]
+    groups = m.reshape(-1, 1, D)
+    return groups.expand(-1, like.numel() // D // groups.shape[0], D).reshape(like.shape)
+
+
+def _per_group(t, m):
+    """The sum of t's rows over each group of the modulation vector m, in m's shape and type."""
+    D = t.shape[-1]
+    return t.reshape(m.numel() // D, -1, D).sum(1).reshape(m.shape).to(m.dtype)
+
+
+def _ln_modulate_bwd_differentiable(x, scale, dy, dskip, eps):
+    """``ops.ln_modulate_bwd`` in differentiable tensor-library ops (fp32)."""
+    mean = lambda t: t.mean(-1, keepdim=True)
+    xc = x.float() - mean(x.float())
+    r = (mean(xc * xc) + eps).rsqrt()
+    n, dyf = xc * r, dy.float()
+    dn = dyf * (1 + _per_row(scale.float(), dyf))
+    dx = r * (dn - mean(dn) - n * mean(dn * n))
+    if dskip is not None:
+        dx = dx + dskip.float()
+    return dx.to(x.dtype), _per_group(dyf, scale), _per_group(dyf * n, scale)
+
+
 class _LnModulateFn(torch.autograd.Function):
     """``LayerNorm(x) * (1 + scale) + shift`` as the fused pass, differentiable (x ``[B, T, H, W, D]``, shift / scale
     ``[B, T, 1, 1, D]``).  Returns x as well, for the residual connection around what follows: both gradients of x then meet in
@@ -46,7 +72,10 @@ class _LnModulateFn(torch.autograd.Function):
         x, scale = ctx.saved_tensors
         if dy is None:
             return dskip, None, None, None
-        dx, dshift, dscale = ops.ln_modulate_bwd(x, scale, dy, dskip, eps=ctx.eps)
+        if torch.is_grad_enabled():      # create_graph: the gradients are differentiated again
+            dx, dshift, dscale = _ln_modulate_bwd_differentiable(x, scale, dy, dskip, ctx.eps)
+        else:
+            dx, dshift, dscale = ops.ln_modulate_bwd(x, scale, dy, dskip, eps=ctx.eps)
         return dx, dshift.reshape(scale.shape), dscale.reshape(scale.shape), None
 
 
@@ -62,7 +91,10 @@ class _GatedResidualFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         res, gate = ctx.saved_tensors
-        dres, dgate = ops.gated_residual_bwd(res, gate, dy)
+        if torch.is_grad_enabled():      # create_graph, as above
+            dres, dgate = dy * _per_row(gate, dy), _per_group(dy.float() * res.float(), gate)
+        else:
+            dres, dgate = ops.gated_residual_bwd(res, gate, dy)
         return dy, dres, dgate.reshape(gate.shape)
 
 

@@ -170,6 +170,39 @@ def test_block_reverse_mode(pkg, oracle, nr_oracle, gpu):
         assert prm.grad is not None and torch.isfinite(prm.grad.float()).all(), name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gradients_of_the_elementwise_steps_differentiate_again(pkg, gpu, dtype):
+    """create_graph=True: a penalty on the gradients of LayerNorm + modulation and of the gated residual, against the same in 64 bits.
+    Bound: the first gradients are rounded to 16 bits, the penalty's gradient again, and for bf16 an inner product of two rounded
+    factors adds their errors: 4 units of 2^-9 (bf16) / 2^-12 (fp16) in the 2-norm."""
+    from importlib import import_module
+    db = import_module(pkg.__name__ + ".dit_block")
+    g = torch.Generator().manual_seed(7)
+    r = lambda *s: torch.randn(*s, generator=g).to(dtype)
+    x, res, dy, vx = (r(2, 3, 2, 4, 64) for _ in range(4))
+    shift, scale, gate, vs = (0.5 * r(2, 3, 1, 1, 64) for _ in range(4))
+
+    def penalty(first, outs, ins, grad_out, weights):
+        grads = torch.autograd.grad(outs, ins, grad_out, create_graph=True)
+        assert all(gr.requires_grad for gr in grads)
+        return torch.autograd.grad(sum((gr * w).sum() for gr, w in zip(grads, weights)), first)
+
+    def both(ln, gated, to):
+        t = lambda z: z.to(to) if isinstance(to, torch.device) else z.double()
+        leaf = lambda z: t(z).requires_grad_(True)
+        xl, sh, sc, rl, gl, d1, d2 = leaf(x), leaf(shift), leaf(scale), leaf(res), leaf(gate), leaf(dy), leaf(dy)
+        a = penalty((xl, sc, d1), ln(xl, sh, sc), (xl, sc), d1, (t(vx), t(vs)))
+        b = penalty((rl, gl, d2), gated(t(x), rl, gl), (rl, gl), d2, (t(vx), t(vs)))
+        return (*a, *b)
+
+    got = both(lambda a, b, c: db._LnModulateFn.apply(a, b, c, 1e-6)[0], db._GatedResidualFn.apply, gpu)
+    want = both(lambda a, b, c: torch.nn.functional.layer_norm(a, (64,), eps=1e-6) * (1 + c) + b, lambda a, b, c: a + c * b, None)
+    for name, p, q in zip(("x", "scale", "dy", "res", "gate", "dy of the residual"), got, want):
+        rel = float((p.double().cpu() - q).norm() / q.norm())
+        print(f"  {name}: rel_l2={rel:.2e}", flush=True)
+        assert rel <= 4 * 2.0 ** (-9 if dtype == torch.bfloat16 else -12), name
+
+
 def test_block_with_image_context_reverse_mode(pkg, oracle, nr_oracle, block_oracle, gpu):
     """Reverse mode through the image-conditioned cross-attention (two attention calls summed): the gradient of x
     against torch autograd of the block oracle."""
