@@ -112,6 +112,44 @@ class _GeluFn(torch.autograd.Function):
         return torch.ops.aten.gelu_backward(dy, h, approximate="none")
 
 
+class _ModulationFn(torch.autograd.Function):
+    """The modulation vectors as ``ops.modulation`` makes them (values), differentiable in emb, lora and the six weights.  The
+    backward pass forms the two small activations again; the gradients of emb and lora are summed over the three MLPs in fp32."""
+
+    @staticmethod
+    def forward(ctx, emb, lora, *w):
+        ctx.save_for_backward(emb, *w)
+        ctx.lora_shape = lora.shape
+        return ops.modulation(emb, lora, w[:3], w[3:])[0]
+
+    @staticmethod
+    def backward(ctx, dout):
+        emb, *w = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        e = emb.reshape(-1, emb.shape[-1])
+        a, rows = F.silu(e), e.shape[0]
+        cat = lambda m: m.transpose(0, 1).reshape(rows, -1)          # [3, rows, D] -> [rows, 3 D]
+        dw1, dw2, da = [None] * 3, [None] * 3, 0
+        for i in range(3):
+            dm = cat(dout[i])
+            if need[5 + i]:
+                dw2[i] = dm.t() @ (a @ w[i].t())
+            if need[0] or need[2 + i]:
+                dh = dm @ w[3 + i]
+                if need[2 + i]:
+                    dw1[i] = dh.t() @ a
+                if need[0]:
+                    da = da + (dh @ w[i]).float()
+        demb = dlora = None
+        if need[0]:
+            ef = e.float()
+            sig = torch.sigmoid(ef)
+            demb = (da * (sig * (1 + ef * (1 - sig)))).to(emb.dtype).reshape(emb.shape)
+        if need[1]:
+            dlora = cat(dout.float().sum(0)).to(dout.dtype).reshape(ctx.lora_shape)
+        return (demb, dlora, *dw1, *dw2)
+
+
 # A call of up to this many rows (twice as many with tangents) forms the modulation vectors in two launches of its own kernels;
 # those read the weights again for every 16 rows, so that many rows are the library's (5120 channels, us: 64 rows 45 against 100,
 # 128 rows 76 against 112; with tangents 64 rows 76 against 344).
@@ -249,8 +287,9 @@ class Block(nn.Module):
         return cut(m), cut(tm)
 
     def _fused_modulations(self, emb, lora, like, temb=None, tlora=None, tangent=False):
-        """All three sub-layers' modulation vectors in two launches: ``[3, 3, rows, D]`` (sub-layer; shift, scale, gate) and its
-        tangent, or None where the modules compute something else than the plain MLPs of one 16-bit type, or for many rows."""
+        """All three sub-layers' modulation vectors in two launches: ``[3, 3, rows, D]`` (sub-layer; shift, scale, gate), through its
+        autograd rule where grad mode is on, and its tangent; or None where the modules compute something else than the plain MLPs
+        of one 16-bit type, or for many rows."""
         if not self.use_adaln_lora or self.use_wan_fp32_strategy or lora is None or torch.is_autocast_enabled("cuda"):
             return None
         mods = (self.adaln_modulation_self_attn, self.adaln_modulation_cross_attn, self.adaln_modulation_mlp)
@@ -275,7 +314,16 @@ class Block(nn.Module):
             return None
         if not all(ops._is_dense16(w) for w in (*w1, *w2)):     # (views of a flat buffer: the library's layers read them where they are)
             return None
+        if torch.is_grad_enabled() and not tangent:
+            return _ModulationFn.apply(emb, lora, *w1, *w2), None
         return ops.modulation(emb, lora, w1, w2, temb, tlora, tangent)
+
+    def _modulations(self, emb, lora, like):
+        """(shift, scale, gate) of one sub-layer after the other; modules are called when their turn comes."""
+        fused = self._fused_modulations(emb, lora, like)
+        vectors = None if fused is None else fused[0].flatten(0, 1).unbind(0)
+        for i, m in enumerate((self.adaln_modulation_self_attn, self.adaln_modulation_cross_attn, self.adaln_modulation_mlp)):
+            yield self._modulation(m, emb, lora, like) if fused is None else vectors[3 * i:3 * i + 3]
 
     def _fp32_region(self, t: torch.Tensor):
         return torch.autocast(t.device.type, enabled=self.use_wan_fp32_strategy, dtype=torch.float32)
@@ -313,14 +361,13 @@ class Block(nn.Module):
         return self._forward_autograd(x, emb_B_T_D, crossattn_emb, rope_emb_L_1_1_D, adaln_lora_B_T_3D)
 
     def _forward_autograd(self, x, emb, crossattn_emb, rope, lora):
-        """The differentiable path: the same kernels as the inference path (so both give the same bits), each behind an
-        autograd rule: attention, RMSNorm + RoPE, LayerNorm + modulation and the gated residuals through their HIP backward
-        kernels."""
+        """The differentiable path: the same kernels as the inference path (so both give the same bits, as long as the attention
+        call does not cut its keys into ranges, which the inference path's cross-attention never does), each behind an autograd
+        rule: attention, RMSNorm + RoPE, LayerNorm + modulation and the gated residuals through their HIP backward kernels."""
         B, T, H, W, D = x.shape
-        for name, norm, sub in (("self_attn", self.layer_norm_self_attn, self.self_attn),
-                                ("cross_attn", self.layer_norm_cross_attn, self.cross_attn),
-                                ("mlp", self.layer_norm_mlp, self.mlp)):
-            shift, scale, gate = self._modulation(getattr(self, "adaln_modulation_" + name), emb, lora, x)
+        for name, norm, sub, (shift, scale, gate) in zip(("self_attn", "cross_attn", "mlp"),
+                                                         (self.layer_norm_self_attn, self.layer_norm_cross_attn, self.layer_norm_mlp),
+                                                         (self.self_attn, self.cross_attn, self.mlp), self._modulations(emb, lora, x)):
             n, x = _LnModulateFn.apply(x, shift, scale, norm.eps)
             if name == "mlp":
                 r = sub(n)
@@ -334,14 +381,9 @@ class Block(nn.Module):
         one fused HIP pass instead of a chain of tensor-library ops."""
         B, T, H, W, D = x.shape
         flat2 = lambda m: m.reshape(-1, D)
-        fused = self._fused_modulations(emb, lora, x)
-        for i, (name, norm, sub) in enumerate((("self_attn", self.layer_norm_self_attn, self.self_attn),
-                                               ("cross_attn", self.layer_norm_cross_attn, self.cross_attn),
-                                               ("mlp", self.layer_norm_mlp, self.mlp))):
-            if fused is not None:
-                shift, scale, gate = fused[0][i].unbind(0)
-            else:
-                shift, scale, gate = self._modulation(getattr(self, "adaln_modulation_" + name), emb, lora, x)
+        for name, norm, sub, (shift, scale, gate) in zip(("self_attn", "cross_attn", "mlp"),
+                                                         (self.layer_norm_self_attn, self.layer_norm_cross_attn, self.layer_norm_mlp),
+                                                         (self.self_attn, self.cross_attn, self.mlp), self._modulations(emb, lora, x)):
             n, _ = ops.ln_modulate(x, flat2(shift), flat2(scale), eps=norm.eps)
             if name == "mlp":
                 r = sub(n)

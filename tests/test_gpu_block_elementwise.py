@@ -170,6 +170,36 @@ def test_modulation(pkg, gpu, rows, K, hidden, D, dtype):
         check("tout", tout, twant, dtype, flip)
 
 
+@pytest.mark.parametrize("rows,K,hidden,D", [(1, 32, 32, 16), (24, 256, 64, 48), (40, 96, 96, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_modulation_reverse_mode(pkg, gpu, rows, K, hidden, D, dtype):
+    """Gradients of emb, lora and the six weights, and the gradients of a penalty on emb's, against 64 bits.  Bound: a gradient goes
+    through at most four 16-bit roundings of relative size 2^-9 (bf16) / 2^-12 (fp16), the penalty's through twice as many."""
+    from importlib import import_module
+    fn = import_module(pkg.__name__ + ".dit_block")._ModulationFn
+    g = torch.Generator().manual_seed(rows)
+    ins = [rnd(g, dtype, rows, K), rnd(g, dtype, rows, 3 * D, std=0.3)]
+    for s in ((hidden, K), (3 * D, hidden)):
+        ins += [rnd(g, dtype, *s, std=s[1] ** -0.5) for _ in range(3)]
+    dout, v = rnd(g, dtype, 3, 3, rows, D), rnd(g, dtype, rows, K)
+
+    def grads(f, to):
+        leaves = [to(t).requires_grad_(True) for t in ins]
+        first = torch.autograd.grad(f(*leaves), leaves, to(dout), create_graph=True)
+        return *first, *torch.autograd.grad((first[0] * to(v)).sum(), (leaves[0], leaves[2], leaves[5]))
+
+    def ref(emb, lora, *w):
+        a = torch.nn.functional.silu(emb)
+        return torch.stack([(a @ w[i].T @ w[3 + i].T + lora).reshape(rows, 3, D).transpose(0, 1) for i in range(3)])
+
+    unit = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
+    got, want = grads(fn.apply, lambda t: t.to(gpu)), grads(ref, lambda t: t.double())
+    for i, (a, b) in enumerate(zip(got, want)):
+        rel = float((a.detach().double().cpu() - b.detach()).norm() / b.detach().norm())
+        print(f"  gradient {i}: rel_l2={rel:.2e}", flush=True)
+        assert a.dtype == dtype and rel <= (4 if i < 8 else 8) * unit, i
+
+
 def off16(t):
     """t's values, contiguous, but one element past a 16-byte boundary (a slice of a larger buffer)."""
     v = torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)[1:].view(t.shape).copy_(t)
@@ -212,6 +242,7 @@ def test_modulation_dispatch(pkg, gpu):
         torch.nn.init.normal_(p, std=p.shape[-1] ** -0.5)
     emb, lora = (torch.randn(2, 3, n, device=gpu).bfloat16() for n in (256, 768))
     x = torch.randn(2, 3, 2, 2, 256, device=gpu).bfloat16()
+    assert m._fused_modulations(emb, lora, x)[0].requires_grad
     with torch.no_grad():
         got, _ = m._fused_modulations(emb, lora, x)
         for i, name in enumerate(("self_attn", "cross_attn", "mlp")):

@@ -63,7 +63,7 @@ def run(pkg, oracle, nr_oracle, block_oracle, gpu, B, T, Hh, W, D, H, Mk, Kc, lo
     check(oracle, "tout - tx", tout.float().cpu() - tx.float(), twant - tx.float(), rel_l2=2e-2)
 
 
-@pytest.mark.parametrize("lora_dim", [0, 16])
+@pytest.mark.parametrize("lora_dim", [0, 16, 32])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_block_small(pkg, oracle, nr_oracle, block_oracle, gpu, lora_dim, dtype):
     run(pkg, oracle, nr_oracle, block_oracle, gpu, B=2, T=2, Hh=4, W=6, D=256, H=2, Mk=20, Kc=96, lora_dim=lora_dim, dtype=dtype, seed=lora_dim)
@@ -81,15 +81,16 @@ def test_block_14b_widths_reduced_length(pkg, oracle, nr_oracle, block_oracle, g
     run(pkg, oracle, nr_oracle, block_oracle, gpu, B=1, T=2, Hh=6, W=8, D=5120, H=40, Mk=64, Kc=1024, lora_dim=256, seed=4)
 
 
-def test_block_with_image_context(pkg, oracle, nr_oracle, block_oracle, gpu):
+@pytest.mark.parametrize("lora_dim", [16, 32])
+def test_block_with_image_context(pkg, oracle, nr_oracle, block_oracle, gpu, lora_dim):
     """image_context_dim: the cross-attention also attends to an image context (minimal_v4_dit.py:451-493)."""
     B, T, Hh, W, D, H, Mk, Kc, Mi, Ki = 2, 2, 4, 6, 256, 2, 20, 96, 12, 80
     torch.manual_seed(7)
-    m = pkg.Block(D, Kc, H, use_adaln_lora=True, adaln_lora_dim=16, image_context_dim=Ki)
+    m = pkg.Block(D, Kc, H, use_adaln_lora=True, adaln_lora_dim=lora_dim, image_context_dim=Ki)
     m.init_weights()
     with torch.no_grad():
         for mod in (m.adaln_modulation_self_attn, m.adaln_modulation_cross_attn, m.adaln_modulation_mlp):
-            mod[-1].weight.copy_(torch.randn_like(mod[-1].weight) / 4.0)
+            mod[-1].weight.copy_(torch.randn_like(mod[-1].weight) / lora_dim ** 0.5)
     m = m.to(device=gpu, dtype=torch.bfloat16).eval()
     assert "cross_attn.k_img.weight" in m.state_dict() and "cross_attn.k_img_norm.weight" in m.state_dict()
     g = torch.Generator().manual_seed(8)
@@ -111,21 +112,24 @@ def test_block_with_image_context(pkg, oracle, nr_oracle, block_oracle, gpu):
     check(oracle, "out - x", out.float().cpu() - x.float(), want - x.float(), rel_l2=2e-2)
 
 
-def test_inference_path_matches_autograd_path(pkg, oracle, nr_oracle, gpu):
-    """Under no_grad the block runs the fused elementwise passes; with autograd it runs tensor-library ops around the same
-    kernels.  Same arithmetic up to the 16-bit roundings between the unfused ops."""
-    B, T, Hh, W, D, H, Mk, Kc = 1, 2, 4, 8, 256, 2, 24, 96
-    m = build(pkg, gpu, D, Kc, H, 16, torch.bfloat16, 21)
+@pytest.mark.parametrize("B,lora_dim,dtype", [(1, 0, torch.bfloat16), (1, 16, torch.float16), (1, 32, torch.bfloat16), (2, 32, torch.bfloat16), (2, 32, torch.float16),
+                                             (2, 64, torch.bfloat16)])
+def test_inference_path_matches_autograd_path(pkg, nr_oracle, gpu, B, lora_dim, dtype):
+    """With autograd the block runs the kernels of the inference path, each behind an autograd rule: the same bits, as a block that
+    is run again for its backward pass needs.  (Modulation vectors by their own kernels from 32 hidden units on, else by the modules.)"""
+    T, Hh, W, D, H, Mk, Kc = 2, 4, 8, 256, 2, 24, 96
+    m = build(pkg, gpu, D, Kc, H, lora_dim, dtype, 21)
     g = torch.Generator().manual_seed(22)
-    r = lambda *s: torch.randn(*s, generator=g).bfloat16().to(gpu)
+    r = lambda *s: torch.randn(*s, generator=g).to(gpu, dtype)
     x, emb, ctx, lora = r(B, T, Hh, W, D), r(B, T, D), r(B, Mk, Kc), 0.3 * r(B, T, 3 * D)
+    assert (m._fused_modulations(emb, lora, x) is not None) == (lora_dim >= 32)
     hd = D // H
     rope = torch.from_numpy(nr_oracle.rope_angles_3d(T, Hh, W, hd)).reshape(-1, 1, 1, hd).to(gpu)
     with torch.no_grad():
         fused = m(x, emb, ctx, rope, lora)
     with torch.enable_grad():
         plain = m(x.clone().requires_grad_(True), emb, ctx, rope, lora)
-    check(oracle, "fused vs autograd path", fused, plain.detach().float().cpu(), rel_l2=1e-2)
+    assert plain.requires_grad and torch.equal(fused, plain)
 
 
 def test_fresh_block_is_the_identity(pkg, nr_oracle, gpu):

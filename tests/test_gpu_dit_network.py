@@ -236,11 +236,12 @@ def test_consistency_distillation_step(pkg, oracle, net_oracle, gpu):
     print(f"  weight gradients: worst rel-L2 {worst[1]:.3e} ({worst[0]})", flush=True)
 
 
-def test_activation_checkpointing_gives_the_same_gradients(pkg, gpu):
+@pytest.mark.parametrize("lora_dim", [16, 32])      # modulation vectors from the modules, and from their own kernels
+def test_activation_checkpointing_gives_the_same_gradients(pkg, gpu, lora_dim):
     """sac_config (minimal_v4_dit.py:1660-1686): blocks keep their inputs and their attention results and run again in the
     backward pass (without launching the forward attention kernels again); the recomputation is deterministic, so the
     output, the gradient of x and the gradients of the blocks' weights are the bits of the plain run."""
-    kw = dict(SMALL, use_adaln_lora=True, adaln_lora_dim=16)
+    kw = dict(SMALL, use_adaln_lora=True, adaln_lora_dim=lora_dim)
     plain = build(pkg, gpu, torch.bfloat16, 37, in_channels=4, **kw).train()
     ckpt = build(pkg, gpu, torch.bfloat16, 37, in_channels=4, sac_config=dict(mode="predict2_2b_720_aggressive", every_n_blocks=1), **kw).train()
     ckpt.load_state_dict(plain.state_dict())
