@@ -1530,7 +1530,7 @@ size_t tiles_bytes_of(const cosmos_attn_desc* d) { return (size_t)d->B * d->H * 
 // workgroups are cut along the keys, and a small second kernel merges the ranges.
 // a head dim of 256 goes to attn_wide_kernel
 bool is_wide(const cosmos_attn_desc* d) { return d->d_qk == 256 || d->d_v == 256; }
-struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // us: estimated time of the launches
+struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us, uncut_us; };   // estimated time of the launches, and without cuts
 // Barrier steps in full rounds at head dims 16, 32, 64, 128 (us): below 64 the exponentials and the step's fixed instructions are
 // most of it.  Fits to 500 .. 9000 positions and 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, S = 1 .. 16, every S measured: the S
 // chosen with them takes 1.0035 to 1.011 times the best one's time on average, 1.13 at most.  (A step that shrinks in proportion to the
@@ -1551,7 +1551,7 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
     s.n_rem = 0; s.splits = 1; s.n_full = s.n_pairs;
     const int rem = s.n_pairs % kNumCUs;
     const StepCost alone{c.step_us, by_head_dim(kPairUs, dim), c.alone};
-    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
+    s.us = s.uncut_us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
     if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
     const double slot_bytes = (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4));
     const int splits = choose_splits(rem, n_steps, c, slot_bytes);
@@ -1569,7 +1569,9 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
 // 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  Forward only at small head
 // dims the stream pays only while a unit has one block (head dim 32: 1560 x 512 16 / 19, 3520 x 512 24 / 20, 40 heads 1560 x 512 33 / 22).
 // The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: the way chosen takes
-// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  With all tangents the
+// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  The two-stage run never cuts key ranges (can_cut false), so that its
+// other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121; forward only 6500 x 1024
+// 80 / 97, 6800 x 1536 116 / 133 (one call, which cuts, with its re-tiling: 67, 101, 87, 116).  With all tangents the
 // two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
 // cosmos_attn_set_stream_override() replaces the choice (tuning and tests); nothing in the per-call path reads the environment.
 constexpr int kStreamMaxTiles = 64;       // up to 2048 keys
@@ -1581,7 +1583,7 @@ constexpr double kStreamStartUs[4] = {5.0, 5.0, 5.0, 0.0};
 constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
 std::atomic<int> g_stream_groups{0};      // number of workgroups, 0 = the library's own choice
-int stream_groups_of(const cosmos_attn_desc* d) {
+int stream_groups_of(const cosmos_attn_desc* d, bool can_cut) {
     if (d->causal || d->d_qk != d->d_v || n_tiles_of(d) > kStreamMaxTiles) return 0;
     // the kernel addresses q and o inside a head with 32-bit byte offsets
     if ((int64_t)d->Lq * d->q_stride[2] >= ((int64_t)1 << 30) || (int64_t)d->Lq * d->o_stride[2] >= ((int64_t)1 << 30)) return 0;
@@ -1599,7 +1601,8 @@ int stream_groups_of(const cosmos_attn_desc* d) {
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
     const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
     const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
-    return stream_us <= plan_split(d).us ? groups : 0;
+    const SplitPlan other = plan_split(d);
+    return stream_us <= (can_cut ? other.us : other.uncut_us) ? groups : 0;
 }
 // LDS of attn_qstream_kernel: the layout of attn_fwd_jvp_kernel (AttnCfg::LDS_BYTES) + the per-block statistics slots
 size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {
@@ -1733,8 +1736,9 @@ int run_wide(const cosmos_attn_desc* d, const void* workspace, void* stream) {
     return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
 }
 // `scratch`: where key-range partial results may go (null: never split).  cosmos_attn_run only reads its workspace, so
-// that several runs may share one re-tiled K/V image; the one-call entry point owns the workspace and passes its tail.
-int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* scratch, void* stream) {
+// that several runs may share one re-tiled K/V image (can_cut false); the one-call entry point owns the workspace and passes its tail
+// (or null where the call needs none).
+int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* scratch, bool can_cut, void* stream) {
     const int st = validate(d);
     if (st != COSMOS_ATTN_OK) return st;
     // the two-stage run never cuts key ranges: it needs the image only
@@ -1759,7 +1763,7 @@ int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_
     ap.BH = d->B * d->H; ap.q_chunk = 0;
     ap.n_qt = (d->Lq + kBlockM - 1) / kBlockM; ap.n_full = ap.n_rem = 0; ap.splits = 1;
     ap.part_acc = nullptr; ap.part_stat = nullptr;
-    if (const int groups = stream_groups_of(d)) {   // short key sequences: `groups` workgroups stream the query blocks
+    if (const int groups = stream_groups_of(d, can_cut)) {   // short key sequences: `groups` workgroups stream the query blocks
         attn_kernel_t sfn = d->dtype == COSMOS_ATTN_BF16 ? pick_stream<__bf16>(d->d_qk, d->d_v, mode)
                                                          : pick_stream<_Float16>(d->d_qk, d->d_v, mode);
         if (sfn) {
@@ -1800,14 +1804,14 @@ int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_
 extern "C" {
 
 COSMOS_ATTN_API int cosmos_attn_run(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* stream) {
-    return run_impl(d, workspace, workspace_bytes, nullptr, stream);
+    return run_impl(d, workspace, workspace_bytes, nullptr, false, stream);
 }
 
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
     const int st = cosmos_attn_pack_kv(d, workspace, workspace_bytes, stream);
     if (st != COSMOS_ATTN_OK) return st;
     void* scratch = partial_bytes_of(d) ? (char*)workspace + align256(tiles_bytes_of(d)) : nullptr;
-    return run_impl(d, workspace, workspace_bytes, scratch, stream);
+    return run_impl(d, workspace, workspace_bytes, scratch, true, stream);
 }
 
 }  // extern "C"

@@ -268,8 +268,8 @@ def test_single_valid_key(pkg, oracle, gpu):
 
 
 # ------------------------------------------------------------------ short key sequences: the query-streaming kernels
-# The library sends a call to the streaming kernels only when it has a thousand (query block, head) pairs or more; the
-# library's hook cosmos_attn_set_stream_override (query blocks per workgroup; the `stream_override` fixture) forces them on small ones.
+# The library sends a call to the streaming kernels where its measured costs say that they are faster, and never below 128 (query block,
+# head) pairs; the library's hook cosmos_attn_set_stream_override (query blocks per workgroup; the `stream_override` fixture) forces them on small ones.
 @pytest.mark.parametrize("chunk", [2, 3, 16])
 @pytest.mark.parametrize("tangents", ["q", "none", "full"])
 def test_streaming_kernels_key_tile_counts(pkg, oracle, gpu, stream_override, chunk, tangents):
@@ -316,6 +316,27 @@ def test_streaming_kernels_random_shapes(pkg, oracle, gpu, stream_override, chun
         stream_override(groups=rng.choice([8, 16, 24, 40, 64, 256]))
         run_case(pkg, oracle, gpu, (B, H, Lq, d), (B, H, Lkv, d), tangents=tangents, dtype=dtype, key_lens=lens,
                  seed=9000 + 100 * chunk + it)
+
+
+@pytest.mark.parametrize("tangents,Lq,Lkv", [("q", 2120, 1024), ("none", 6500, 1024)])
+def test_packed_run_is_compared_with_the_uncut_kernel(pkg, oracle, gpu, stream_override, tangents, Lq, Lkv):
+    """The two-stage run never cuts key ranges: it streams where streaming beats the uncut kernel (by 16 % at both sizes), also where
+    the one-call form, which may cut, does not.  Told apart by their bits; all ways within the ordinary tolerance of each other."""
+    g = torch.Generator(device=gpu).manual_seed(Lq)
+    q, tq = (torch.randn(1, 16, Lq, 128, device=gpu, generator=g).bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, 16, Lkv, 128, device=gpu, generator=g).bfloat16() for _ in range(2))
+    t = (tq,) if tangents == "q" else ()
+    packed, outs = pkg.pack_kv(k, v), {}
+    for name, steer in (("chosen", {}), ("stream", dict(groups=256)), ("uncut", dict(chunk=1))):
+        stream_override(**steer)
+        outs[name] = pkg.run_packed(q, packed, *t)
+    stream_override()
+    outs["one call"] = pkg.ops.fwd_jvp(q, k, v, *t)
+    same = lambda a, b: all(torch.equal(x, y) for x, y in zip(outs[a], outs[b]) if x is not None)
+    assert same("chosen", "stream") and not same("chosen", "uncut") and not same("chosen", "one call")
+    for name in ("uncut", "one call"):
+        for x, y in zip(outs["chosen"], outs[name]):
+            assert x is None or float((x.float() - y.float()).norm() / y.float().norm()) <= 1e-2, name
 
 
 @pytest.mark.parametrize("d", [16, 32, 64, 128])
