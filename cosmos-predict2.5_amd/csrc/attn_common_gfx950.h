@@ -171,11 +171,11 @@ inline double by_head_dim(const double (&at)[4], double d) {
 inline double split_cost(int rem, int n_steps, int S, StepCost c, double slot_bytes) {
     return rounds_cost((int64_t)rem * S, (double)n_steps / S, c) + (S > 1 ? 3.0 + (double)rem * S * slot_bytes / 3.8e6 : 0.0);
 }
-inline int choose_splits(int rem, int n_steps, StepCost c, double slot_bytes) {
+inline int choose_splits(int rem, int n_steps, StepCost c, double slot_bytes, int most = kMaxSplits) {
     if (rem <= 0) return 1;
     int best = 1;
     double best_cost = 0.95 * split_cost(rem, n_steps, 1, c, slot_bytes);
-    for (int S = 2; S <= kMaxSplits && S * kMinStepsPerSplit <= n_steps; ++S) {
+    for (int S = 2; S <= most && S * kMinStepsPerSplit <= n_steps; ++S) {
         const double cost = split_cost(rem, n_steps, S, c, slot_bytes);
         if (cost < best_cost) { best_cost = cost; best = S; }
     }

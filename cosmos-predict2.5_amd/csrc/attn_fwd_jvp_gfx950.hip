@@ -1530,7 +1530,7 @@ size_t tiles_bytes_of(const cosmos_attn_desc* d) { return (size_t)d->B * d->H * 
 // workgroups are cut along the keys, and a small second kernel merges the ranges.
 // a head dim of 256 goes to attn_wide_kernel
 bool is_wide(const cosmos_attn_desc* d) { return d->d_qk == 256 || d->d_v == 256; }
-struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us, uncut_us; };   // estimated time of the launches, and without cuts
+struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // us: estimated time of the launches
 // Barrier steps in full rounds at head dims 16, 32, 64, 128 (us): below 64 the exponentials and the step's fixed instructions are
 // most of it.  Fits to 500 .. 9000 positions and 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, S = 1 .. 16, every S measured: the S
 // chosen with them takes 1.0035 to 1.011 times the best one's time on average, 1.13 at most.  (A step that shrinks in proportion to the
@@ -1539,7 +1539,18 @@ struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us,
 constexpr double kStepUs[3][4] = {{1.36, 1.37, 1.77, 2.66}, {0.54, 0.56, 0.68, 0.86}, {0.54, 0.60, 0.82, 1.21}};   // MODE_FWD, MODE_JVP_Q, MODE_JVP_FULL
 constexpr double kStepAlone[4] = {0.9, 0.9, 0.9, 0.7};
 constexpr double kPairUs[4] = {5.0, 5.0, 5.0, 13.0};          // what a workgroup that is a whole pair costs besides its steps
-SplitPlan plan_split(const cosmos_attn_desc* d) {
+size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+// partial results of the split pairs: fp32 accumulators (O, and T with tangents), then the row statistics
+size_t partial_acc_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
+    const size_t per_row = (size_t)d->d_v * (mode_of(d) == MODE_FWD ? 1 : 2) * sizeof(float);
+    return align256((size_t)s.n_rem * s.splits * s.block_m * per_row);
+}
+size_t partial_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
+    return s.splits < 2 ? 0 : partial_acc_bytes(d, s) + align256((size_t)s.n_rem * s.splits * s.block_m * sizeof(float4));
+}
+// `room`: bytes there are for partial results (0: never split)
+constexpr size_t kNoLimit = ~(size_t)0;
+SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     SplitPlan s;
     const bool fwd = mode_of(d) == MODE_FWD;
     const double dim = 0.5 * (d->d_qk + d->d_v);
@@ -1551,13 +1562,15 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
     s.n_rem = 0; s.splits = 1; s.n_full = s.n_pairs;
     const int rem = s.n_pairs % kNumCUs;
     const StepCost alone{c.step_us, by_head_dim(kPairUs, dim), c.alone};
-    s.us = s.uncut_us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
+    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
     if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
     const double slot_bytes = (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4));
-    const int splits = choose_splits(rem, n_steps, c, slot_bytes);
-    if (splits < 2) return s;
-    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + split_cost(rem, n_steps, splits, c, slot_bytes);
-    s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = splits;
+    const SplitPlan uncut = s;
+    s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
+    while (s.splits > 1 && partial_bytes(d, s) > room) --s.splits;
+    s.splits = choose_splits(rem, n_steps, c, slot_bytes, s.splits);
+    if (s.splits < 2) return uncut;
+    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + split_cost(rem, n_steps, s.splits, c, slot_bytes);
     return s;
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
@@ -1569,7 +1582,7 @@ SplitPlan plan_split(const cosmos_attn_desc* d) {
 // 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  Forward only at small head
 // dims the stream pays only while a unit has one block (head dim 32: 1560 x 512 16 / 19, 3520 x 512 24 / 20, 40 heads 1560 x 512 33 / 22).
 // The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: the way chosen takes
-// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  The two-stage run never cuts key ranges (can_cut false), so that its
+// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  The two-stage run never cuts key ranges (no room), so that its
 // other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121; forward only 6500 x 1024
 // 80 / 97, 6800 x 1536 116 / 133 (one call, which cuts, with its re-tiling: 67, 101, 87, 116).  With all tangents the
 // two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
@@ -1583,7 +1596,7 @@ constexpr double kStreamStartUs[4] = {5.0, 5.0, 5.0, 0.0};
 constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
 std::atomic<int> g_stream_groups{0};      // number of workgroups, 0 = the library's own choice
-int stream_groups_of(const cosmos_attn_desc* d, bool can_cut) {
+int stream_groups_of(const cosmos_attn_desc* d, const SplitPlan& other) {
     if (d->causal || d->d_qk != d->d_v || n_tiles_of(d) > kStreamMaxTiles) return 0;
     // the kernel addresses q and o inside a head with 32-bit byte offsets
     if ((int64_t)d->Lq * d->q_stride[2] >= ((int64_t)1 << 30) || (int64_t)d->Lq * d->o_stride[2] >= ((int64_t)1 << 30)) return 0;
@@ -1601,8 +1614,7 @@ int stream_groups_of(const cosmos_attn_desc* d, bool can_cut) {
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
     const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
     const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
-    const SplitPlan other = plan_split(d);
-    return stream_us <= (can_cut ? other.us : other.uncut_us) ? groups : 0;
+    return stream_us <= other.us ? groups : 0;
 }
 // LDS of attn_qstream_kernel: the layout of attn_fwd_jvp_kernel (AttnCfg::LDS_BYTES) + the per-block statistics slots
 size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {
@@ -1613,17 +1625,6 @@ size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {
     const int dvp = d->d_v < 32 ? d->d_v : 32 * ((d->d_v + 31) / 32);
     const size_t xp = mode == MODE_JVP_FULL ? 0 : (size_t)4 * (mode == MODE_FWD ? 1 : 2) * 32 * dvp * 2;   // StreamStores::XP_BYTES per wavefront pair
     return kRingK * kp + kRingV * vp + 2 * 4 * ph + 2 * 4 * 256 + 2 * 2 * 4 * 256 + xp;
-}
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-// partial results of the split pairs: fp32 accumulators (O, and T with tangents), then the row statistics
-size_t partial_acc_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
-    const size_t per_row = (size_t)d->d_v * (mode_of(d) == MODE_FWD ? 1 : 2) * sizeof(float);
-    return align256((size_t)s.n_rem * s.splits * s.block_m * per_row);
-}
-size_t partial_bytes_of(const cosmos_attn_desc* d) {
-    const SplitPlan s = plan_split(d);
-    if (s.splits < 2) return 0;
-    return partial_acc_bytes(d, s) + align256((size_t)s.n_rem * s.splits * s.block_m * sizeof(float4));
 }
 
 int validate(const cosmos_attn_desc* d) {
@@ -1678,7 +1679,7 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
 
 COSMOS_ATTN_API size_t cosmos_attn_workspace_bytes(const cosmos_attn_desc* d) {
     if (validate(d) != COSMOS_ATTN_OK) return 0;
-    return align256(tiles_bytes_of(d)) + partial_bytes_of(d);
+    return align256(tiles_bytes_of(d)) + partial_bytes(d, plan_split(d, kNoLimit));
 }
 
 COSMOS_ATTN_API size_t cosmos_attn_packed_bytes(const cosmos_attn_desc* d) {
@@ -1735,15 +1736,14 @@ int run_wide(const cosmos_attn_desc* d, const void* workspace, void* stream) {
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kWideWaves), 0, (hipStream_t)stream, ap, (int)d->d_qk, (int)d->d_v);
     return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
 }
-// `scratch`: where key-range partial results may go (null: never split).  cosmos_attn_run only reads its workspace, so
-// that several runs may share one re-tiled K/V image (can_cut false); the one-call entry point owns the workspace and passes its tail
-// (or null where the call needs none).
-int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* scratch, bool can_cut, void* stream) {
+// `room`: bytes behind the re-tiled K/V image that key-range partial results may take.  cosmos_attn_run only reads its workspace, so
+// that several runs may share one image: 0, never split.
+int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, size_t room, void* stream) {
     const int st = validate(d);
     if (st != COSMOS_ATTN_OK) return st;
-    // the two-stage run never cuts key ranges: it needs the image only
-    const size_t need = scratch ? cosmos_attn_workspace_bytes(d) : align256(tiles_bytes_of(d));
-    if (!workspace || workspace_bytes < need || !aligned16(workspace)) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
+    const SplitPlan sp = plan_split(d, room);
+    const size_t image_bytes = align256(tiles_bytes_of(d));
+    if (!workspace || workspace_bytes < image_bytes + partial_bytes(d, sp) || !aligned16(workspace)) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
     if (!device_is_whole_mi355x()) return COSMOS_ATTN_WRONG_DEVICE;
     const int mode = mode_of(d);
     if (is_wide(d)) return run_wide(d, workspace, stream);
@@ -1763,7 +1763,7 @@ int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_
     ap.BH = d->B * d->H; ap.q_chunk = 0;
     ap.n_qt = (d->Lq + kBlockM - 1) / kBlockM; ap.n_full = ap.n_rem = 0; ap.splits = 1;
     ap.part_acc = nullptr; ap.part_stat = nullptr;
-    if (const int groups = stream_groups_of(d, can_cut)) {   // short key sequences: `groups` workgroups stream the query blocks
+    if (const int groups = stream_groups_of(d, sp)) {   // short key sequences: `groups` workgroups stream the query blocks
         attn_kernel_t sfn = d->dtype == COSMOS_ATTN_BF16 ? pick_stream<__bf16>(d->d_qk, d->d_v, mode)
                                                          : pick_stream<_Float16>(d->d_qk, d->d_v, mode);
         if (sfn) {
@@ -1776,13 +1776,11 @@ int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_
     }
     const size_t lds = lds_bytes_of(d);
     if (!allow_lds((const void*)fn, lds)) return COSMOS_ATTN_LAUNCH_FAILED;
-    SplitPlan sp = plan_split(d);
-    if (!scratch) { sp.n_full = sp.n_pairs; sp.n_rem = 0; sp.splits = 1; }
     ap.n_qt = sp.n_qt; ap.n_full = sp.n_full; ap.n_rem = sp.n_rem; ap.splits = sp.splits;
     ap.part_acc = nullptr; ap.part_stat = nullptr;
     if (sp.splits > 1) {
-        ap.part_acc = (float*)scratch;
-        ap.part_stat = (float4*)((char*)scratch + partial_acc_bytes(d, sp));
+        ap.part_acc = (float*)((char*)workspace + image_bytes);
+        ap.part_stat = (float4*)((char*)workspace + image_bytes + partial_acc_bytes(d, sp));
     }
     const int64_t blocks = (int64_t)sp.n_full + (int64_t)sp.n_rem * sp.splits;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymWaves : kAttnThreads), lds, (hipStream_t)stream, ap);
@@ -1804,14 +1802,13 @@ int run_impl(const cosmos_attn_desc* d, const void* workspace, size_t workspace_
 extern "C" {
 
 COSMOS_ATTN_API int cosmos_attn_run(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* stream) {
-    return run_impl(d, workspace, workspace_bytes, nullptr, false, stream);
+    return run_impl(d, const_cast<void*>(workspace), workspace_bytes, 0, stream);     // (no room: not written)
 }
 
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
     const int st = cosmos_attn_pack_kv(d, workspace, workspace_bytes, stream);
     if (st != COSMOS_ATTN_OK) return st;
-    void* scratch = partial_bytes_of(d) ? (char*)workspace + align256(tiles_bytes_of(d)) : nullptr;
-    return run_impl(d, workspace, workspace_bytes, scratch, true, stream);
+    return run_impl(d, workspace, workspace_bytes, kNoLimit, stream);
 }
 
 }  // extern "C"
@@ -1849,13 +1846,15 @@ COSMOS_ATTN_API size_t cosmos_attn_static_scratch_bytes(void) { return kStaticSc
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp_static(const cosmos_attn_desc* d, void* stream) {
     const int st = validate(d);
     if (st != COSMOS_ATTN_OK) return st;
-    const size_t need = cosmos_attn_workspace_bytes(d);
-    if (need > kStaticScratchBytes) return COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED;
+    const size_t image_bytes = align256(tiles_bytes_of(d));
+    if (image_bytes > kStaticScratchBytes) return COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED;
     void* const ws = static_scratch_ptr();
     if (!ws) return COSMOS_ATTN_LAUNCH_FAILED;
     // nothing in the workspace has to start at zero: the re-tiling kernel writes every byte of the image (padding
     // included) and every key range writes its whole slot of partial results before the merge kernel reads it
-    return cosmos_attn_fwd_jvp(d, ws, need, stream);
+    const int packed = cosmos_attn_pack_kv(d, ws, kStaticScratchBytes, stream);
+    // where the key ranges that cosmos_attn_fwd_jvp would cut leave more partial results than fit, fewer are cut
+    return packed != COSMOS_ATTN_OK ? packed : run_impl(d, ws, kStaticScratchBytes, kStaticScratchBytes - image_bytes, stream);
 }
 
 }  // extern "C"

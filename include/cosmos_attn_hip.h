@@ -40,7 +40,7 @@ enum cosmos_attn_status {
     COSMOS_ATTN_UNSUPPORTED = 4,    /* dtype / head-dim combination not built */
     COSMOS_ATTN_WORKSPACE_TOO_SMALL = 5,
     COSMOS_ATTN_LAUNCH_FAILED = 6,  /* hipGetLastError() != hipSuccess after a launch */
-    COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED = 7,  /* cosmos_attn_fwd_jvp_static: workspace need > COSMOS_ATTN_STATIC_SCRATCH_BYTES */
+    COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED = 7,  /* cosmos_attn_fwd_jvp_static: the re-tiled K/V image > COSMOS_ATTN_STATIC_SCRATCH_BYTES */
     COSMOS_ATTN_WRONG_DEVICE = 8    /* the current device does not report 256 compute units (a partitioned MI355X, another part):
                                        checked once per device at the first attention launch */
 };
@@ -118,8 +118,9 @@ COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc *desc, void *work
  * No counterpart in the reference.  It is for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  The call itself calls no hipMalloc / hipFree and no
  * allocating library routine; inputs and outputs are the caller's, as in cosmos_attn_fwd_jvp, and results are bitwise
- * those of cosmos_attn_fwd_jvp.
- * A problem whose cosmos_attn_workspace_bytes() exceeds the array is refused with COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED
+ * those of cosmos_attn_fwd_jvp where cosmos_attn_workspace_bytes() fits the array.  Where only the re-tiled K/V image
+ * (cosmos_attn_packed_bytes()) and a part of the partial results do, the keys are cut into fewer ranges, or not cut.
+ * A problem whose cosmos_attn_packed_bytes() exceeds the array is refused with COSMOS_ATTN_STATIC_SCRATCH_EXCEEDED
  * (the text cross-attention of the 2B DiT, B=2 H=16 Lkv=512 d=128, needs 8 MiB; self-attention at L=84480 does not fit).
  * All calls on one GPU share that GPU's array: calls that overlap in time on one GPU (different streams or threads)
  * race on it; calls on one stream are ordered and safe.

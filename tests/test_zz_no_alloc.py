@@ -83,6 +83,33 @@ def test_static_scratch_entry_point_refuses_what_does_not_fit(pkg, oracle, gpu):
     assert lib.cosmos_attn_fwd_jvp_static(ctypes.byref(D), None) == L.ST_BAD_ARG
 
 
+@pytest.mark.parametrize("d,H,L,tangents", [(32, 20, 16000, "none"), (16, 64, 10000, "q"), (16, 64, 9000, "q")])
+def test_static_scratch_entry_point_cuts_fewer_ranges_where_not_all_fit(pkg, oracle, gpu, d, H, L, tangents):
+    """The K/V image fits the array, the partial results of the key ranges that the other entry point cuts do not: the call is taken
+    all the same.  Bound: both ways round a sum of fp32 partial sums to bf16 once, 2^-9 each at most, and P to bf16 for maxima of
+    their own (2^-9 each)."""
+    lib, mod = pkg._lib.load_library(), pkg._lib
+    g = torch.Generator(device=gpu).manual_seed(L)
+    q, k, v, tq = (torch.randn(1, H, L, d, device=gpu, generator=g).bfloat16() for _ in range(4))
+    tq = tq if tangents == "q" else None
+    outs, st = [], torch.cuda.current_stream().cuda_stream
+    for static in (False, True):
+        o, lse = torch.full_like(q, float("nan")), torch.full((1, H, L), float("nan"), device=gpu)
+        to = None if tq is None else torch.full_like(q, float("nan"))
+        D = _desc(mod, q, k, v, tq, None, None, o, to, lse)
+        assert lib.cosmos_attn_packed_bytes(ctypes.byref(D)) <= lib.cosmos_attn_static_scratch_bytes() < lib.cosmos_attn_workspace_bytes(ctypes.byref(D))
+        if static:
+            rc = lib.cosmos_attn_fwd_jvp_static(ctypes.byref(D), st)
+        else:
+            ws = torch.empty(lib.cosmos_attn_workspace_bytes(ctypes.byref(D)), device=gpu, dtype=torch.uint8)
+            rc = lib.cosmos_attn_fwd_jvp(ctypes.byref(D), ws.data_ptr(), ws.numel(), st)
+        assert rc == 0, mod.status_string(rc)
+        torch.cuda.synchronize()
+        outs.append([x for x in (o, to, lse) if x is not None])
+    for a, b in zip(*outs):
+        assert float((a.float() - b.float()).norm() / a.float().norm()) <= 4 * 2.0 ** -9
+
+
 def test_static_scratch_entry_point_under_graph_capture(pkg, oracle, gpu, stream_override):
     """What the entry point is for: a HIP graph captured around it (no allocation inside the capture: the outputs exist
     already), replayed with new input contents and eager work in between, matches eager calls bit for bit.  The streaming
