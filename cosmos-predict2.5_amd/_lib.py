@@ -18,6 +18,7 @@ LIB_PATH = os.environ.get("COSMOS_ATTN_LIB") or _BUILT_LIB_PATH
 
 ABI_VERSION = 2
 DTYPE_BF16, DTYPE_FP16 = 0, 1
+NORM_ROPE_WEIGHT_16 = 0x100     # flag in a norm_rope descriptor's dtype
 
 ST_OK, ST_BAD_ARG, ST_BAD_SHAPE, ST_BAD_STRIDE, ST_UNSUPPORTED, ST_WORKSPACE, ST_LAUNCH, ST_STATIC_SCRATCH, ST_WRONG_DEVICE = range(9)
 
@@ -98,7 +99,7 @@ class NormRopeDesc(ctypes.Structure):
         ("H", ctypes.c_int32),
         ("D", ctypes.c_int32),
         ("eps", ctypes.c_float),
-        ("weight_type", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
         ("x", ctypes.c_void_p),
         ("tx", ctypes.c_void_p),
         ("weight", ctypes.c_void_p),
@@ -121,7 +122,7 @@ class NormRopeBwdDesc(ctypes.Structure):
         ("H", ctypes.c_int32),
         ("D", ctypes.c_int32),
         ("eps", ctypes.c_float),
-        ("weight_type", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
         ("x", ctypes.c_void_p),
         ("dy", ctypes.c_void_p),
         ("weight", ctypes.c_void_p),

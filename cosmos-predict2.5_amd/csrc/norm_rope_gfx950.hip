@@ -420,6 +420,8 @@ UnitPlan plan_units(int B, int S, int H, int D) {
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
+int element_type(int32_t dtype) { return dtype & ~COSMOS_NORM_ROPE_WEIGHT_16; }
+int weight16(int32_t dtype) { return dtype & COSMOS_NORM_ROPE_WEIGHT_16 ? 1 : 0; }
 bool strides_ok(const int64_t* s) { return s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0; }
 
 }  // namespace
@@ -431,16 +433,15 @@ COSMOS_ATTN_API int cosmos_norm_rope(const cosmos_norm_rope_desc* d, void* strea
     if (d->B <= 0 || d->S <= 0 || d->H <= 0) return COSMOS_ATTN_BAD_ARG;
     if (!d->x || !d->y || (d->tx != nullptr) != (d->ty != nullptr)) return COSMOS_ATTN_BAD_ARG;
     if (!(d->eps >= 0.f)) return COSMOS_ATTN_BAD_ARG;
-    if (d->dtype != COSMOS_ATTN_BF16 && d->dtype != COSMOS_ATTN_FP16) return COSMOS_ATTN_UNSUPPORTED;
+    if (element_type(d->dtype) != COSMOS_ATTN_BF16 && element_type(d->dtype) != COSMOS_ATTN_FP16) return COSMOS_ATTN_UNSUPPORTED;
     if (d->D != 16 && d->D != 32 && d->D != 64 && d->D != 128 && d->D != 256) return COSMOS_ATTN_BAD_SHAPE;
     if (!aligned16(d->x) || !aligned16(d->y) || (d->tx && (!aligned16(d->tx) || !aligned16(d->ty)))) return COSMOS_ATTN_BAD_STRIDE;
     if (d->angles && !aligned16(d->angles)) return COSMOS_ATTN_BAD_STRIDE;
-    if (d->weight_type != 0 && d->weight_type != 1) return COSMOS_ATTN_BAD_ARG;
-    if (d->weight && d->weight_type && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
+    if (d->weight && weight16(d->dtype) && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
     if (!strides_ok(d->x_stride) || !strides_ok(d->y_stride)) return COSMOS_ATTN_BAD_STRIDE;
     NormRopeParams p;
     p.x = (const uint16_t*)d->x; p.tx = (const uint16_t*)d->tx; p.y = (uint16_t*)d->y; p.ty = (uint16_t*)d->ty;
-    p.weight = d->weight; p.weight16 = d->weight_type; p.angles = d->angles;
+    p.weight = d->weight; p.weight16 = weight16(d->dtype); p.angles = d->angles;
     p.x_sb = d->x_stride[0]; p.x_ss = d->x_stride[1]; p.x_sh = d->x_stride[2];
     p.y_sb = d->y_stride[0]; p.y_ss = d->y_stride[1]; p.y_sh = d->y_stride[2];
     p.B = d->B; p.S = d->S; p.H = d->H; p.D = d->D;
@@ -449,7 +450,7 @@ COSMOS_ATTN_API int cosmos_norm_rope(const cosmos_norm_rope_desc* d, void* strea
     p.heads_per_unit = u.heads_per_unit; p.head_groups = u.head_groups; p.units = u.units;
     const int64_t blocks = u.blocks;
     if (blocks > 0x7FFFFFFF) return COSMOS_ATTN_BAD_SHAPE;
-    const bool bf16 = d->dtype == COSMOS_ATTN_BF16;
+    const bool bf16 = element_type(d->dtype) == COSMOS_ATTN_BF16;
     norm_rope_kernel_t fn = d->tx ? (bf16 ? pick<true, true>(d->D) : pick<true, false>(d->D))
                                   : (bf16 ? pick<false, true>(d->D) : pick<false, false>(d->D));
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
@@ -461,11 +462,10 @@ static int validate_norm_rope_bwd(const cosmos_norm_rope_bwd_desc* d) {
     if (d->B <= 0 || d->S <= 0 || d->H <= 0) return COSMOS_ATTN_BAD_ARG;
     if (!d->x || !d->dy || !d->dx) return COSMOS_ATTN_BAD_ARG;
     if (!(d->eps >= 0.f)) return COSMOS_ATTN_BAD_ARG;
-    if (d->dtype != COSMOS_ATTN_BF16 && d->dtype != COSMOS_ATTN_FP16) return COSMOS_ATTN_UNSUPPORTED;
+    if (element_type(d->dtype) != COSMOS_ATTN_BF16 && element_type(d->dtype) != COSMOS_ATTN_FP16) return COSMOS_ATTN_UNSUPPORTED;
     if (d->D != 16 && d->D != 32 && d->D != 64 && d->D != 128 && d->D != 256) return COSMOS_ATTN_BAD_SHAPE;
     if (!aligned16(d->x) || !aligned16(d->dy) || !aligned16(d->dx)) return COSMOS_ATTN_BAD_STRIDE;
-    if (d->weight_type != 0 && d->weight_type != 1) return COSMOS_ATTN_BAD_ARG;
-    if (d->weight && d->weight_type && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
+    if (d->weight && weight16(d->dtype) && (reinterpret_cast<uintptr_t>(d->weight) & 7u)) return COSMOS_ATTN_BAD_STRIDE;
     if (d->angles && !aligned16(d->angles)) return COSMOS_ATTN_BAD_STRIDE;
     if (!strides_ok(d->x_stride) || !strides_ok(d->dy_stride) || !strides_ok(d->dx_stride)) return COSMOS_ATTN_BAD_STRIDE;
     if (plan_units(d->B, d->S, d->H, d->D).blocks > 0x7FFFFFFF) return COSMOS_ATTN_BAD_SHAPE;
@@ -486,7 +486,7 @@ COSMOS_ATTN_API int cosmos_norm_rope_bwd(const cosmos_norm_rope_bwd_desc* d, voi
     if (need && !aligned16(workspace)) return COSMOS_ATTN_BAD_STRIDE;
     NormRopeBwdParams p;
     p.x = (const uint16_t*)d->x; p.dy = (const uint16_t*)d->dy; p.dx = (uint16_t*)d->dx;
-    p.weight = d->weight; p.weight16 = d->weight_type; p.angles = d->angles;
+    p.weight = d->weight; p.weight16 = weight16(d->dtype); p.angles = d->angles;
     p.partials = d->dweight ? (float*)workspace : nullptr;
     p.x_sb = d->x_stride[0]; p.x_ss = d->x_stride[1]; p.x_sh = d->x_stride[2];
     p.g_sb = d->dy_stride[0]; p.g_ss = d->dy_stride[1]; p.g_sh = d->dy_stride[2];
@@ -494,7 +494,7 @@ COSMOS_ATTN_API int cosmos_norm_rope_bwd(const cosmos_norm_rope_bwd_desc* d, voi
     p.B = d->B; p.S = d->S; p.H = d->H; p.D = d->D;
     p.eps = d->eps;
     p.heads_per_unit = u.heads_per_unit; p.head_groups = u.head_groups; p.units = u.units;
-    norm_rope_bwd_kernel_t fn = d->dtype == COSMOS_ATTN_BF16 ? pick_bwd<true>(d->D) : pick_bwd<false>(d->D);
+    norm_rope_bwd_kernel_t fn = element_type(d->dtype) == COSMOS_ATTN_BF16 ? pick_bwd<true>(d->D) : pick_bwd<false>(d->D);
     hipLaunchKernelGGL(fn, dim3((unsigned)u.blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
     if (hipGetLastError() != hipSuccess) return COSMOS_ATTN_LAUNCH_FAILED;
     if (d->dweight) {

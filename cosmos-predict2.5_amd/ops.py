@@ -327,6 +327,10 @@ def _norm_weight(weight: Optional[torch.Tensor], x: torch.Tensor) -> Optional[to
     return weight.to(device=x.device, dtype=torch.float32).contiguous()
 
 
+def _norm_rope_dtype(x: torch.Tensor, weight: Optional[torch.Tensor]) -> int:
+    return _DTYPES[x.dtype] | (_lib.NORM_ROPE_WEIGHT_16 if weight is not None and weight.dtype == x.dtype else 0)
+
+
 def norm_rope(
     x: torch.Tensor,
     weight: Optional[torch.Tensor] = None,
@@ -370,10 +374,10 @@ def norm_rope(
 
     desc = _lib.NormRopeDesc()
     desc.abi_version = _lib.ABI_VERSION
-    desc.dtype = _DTYPES[x.dtype]
+    desc.dtype = _norm_rope_dtype(x, weight)
     desc.B, desc.S, desc.H, desc.D = B, S, H, D
     desc.eps = float(eps)
-    desc.weight_type = int(weight is not None and weight.dtype != torch.float32)
+    desc.reserved = 0
     desc.x, desc.tx = x.data_ptr(), (tx.data_ptr() if tx is not None else None)
     desc.weight = weight.data_ptr() if weight is not None else None
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None
@@ -416,10 +420,10 @@ def norm_rope_bwd(
 
     desc = _lib.NormRopeBwdDesc()
     desc.abi_version = _lib.ABI_VERSION
-    desc.dtype = _DTYPES[x.dtype]
+    desc.dtype = _norm_rope_dtype(x, weight)
     desc.B, desc.S, desc.H, desc.D = B, S, H, D
     desc.eps = float(eps)
-    desc.weight_type = int(weight is not None and weight.dtype != torch.float32)
+    desc.reserved = 0
     desc.x, desc.dy, desc.dx = x.data_ptr(), dy.data_ptr(), dx.data_ptr()
     desc.weight = weight.data_ptr() if weight is not None else None
     desc.angles = rope_emb.data_ptr() if rope_emb is not None else None

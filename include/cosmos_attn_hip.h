@@ -185,14 +185,17 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc *desc, void *work
  * x, tx: [B, S, H, D] addressed through element strides (batch, sequence, head), innermost stride 1; y, ty likewise with
  * their own strides (so the result can be written heads-first).  One kernel launch; no workspace.
  */
+/* flag in a norm_rope descriptor's dtype: weight has the element type (8-byte aligned) */
+#define COSMOS_NORM_ROPE_WEIGHT_16 0x100
+
 typedef struct cosmos_norm_rope_desc {
     int32_t abi_version;     /* COSMOS_ATTN_ABI_VERSION */
-    int32_t dtype;           /* enum cosmos_attn_dtype: element type of x, tx, y, ty */
+    int32_t dtype;           /* enum cosmos_attn_dtype: element type of x, tx, y, ty; | COSMOS_NORM_ROPE_WEIGHT_16 */
     int32_t B, S, H, D;      /* D in {16,32,64,128,256} */
     float eps;               /* 1e-6 in the DiT */
-    int32_t weight_type;     /* 0: weight is fp32; 1: weight has the element type */
+    int32_t reserved;        /* not looked at */
     const void *x, *tx;      /* device; tx may be NULL (then ty must be NULL) */
-    const void *weight;      /* [D] (RMSNorm's gamma), device; NULL = ones */
+    const void *weight;      /* [D] (RMSNorm's gamma), device, fp32 unless dtype says otherwise; NULL = ones */
     const float *angles;     /* [S, D] fp32 contiguous, device; NULL = no rotation (cross-attention keys, :409) */
     void *y, *ty;            /* outputs, device */
     int64_t x_stride[3];     /* (batch, sequence, head) element strides of x and tx */
@@ -213,12 +216,12 @@ COSMOS_ATTN_API int cosmos_norm_rope(const cosmos_norm_rope_desc *desc, void *st
  */
 typedef struct cosmos_norm_rope_bwd_desc {
     int32_t abi_version;     /* COSMOS_ATTN_ABI_VERSION */
-    int32_t dtype;           /* element type of x, dy, dx */
+    int32_t dtype;           /* element type of x, dy, dx; | COSMOS_NORM_ROPE_WEIGHT_16 */
     int32_t B, S, H, D;
     float eps;
-    int32_t weight_type;     /* 0: weight is fp32; 1: weight has the element type */
+    int32_t reserved;        /* not looked at */
     const void *x, *dy;      /* device */
-    const void *weight;      /* [D] or NULL = ones */
+    const void *weight;      /* [D], fp32 unless dtype says otherwise, or NULL = ones */
     const float *angles;     /* [S, D] fp32 or NULL = no rotation */
     void *dx;                /* device */
     float *dweight;          /* [D] fp32, device; NULL = not wanted */

@@ -203,6 +203,10 @@ def test_norm_rope_desc_layout_and_status_codes(pkg):
         (dict(tx=0x7F0000200000), L.ST_BAD_ARG),          # a tangent in without a tangent out
         (dict(eps=-1.0), L.ST_BAD_ARG),
         (dict(dtype=5), L.ST_UNSUPPORTED),
+        (dict(dtype=5 | L.NORM_ROPE_WEIGHT_16), L.ST_UNSUPPORTED),
+        (dict(reserved=7, weight=0x7F0000300004, D=48), L.ST_BAD_SHAPE),      # what the field holds is not looked at
+        (dict(reserved=7, weight=0x7F0000300004, y_stride=(ctypes.c_int64 * 3)(4 * 2 * 66, 2 * 66, 66)), L.ST_BAD_STRIDE),
+        (dict(dtype=L.DTYPE_FP16 | L.NORM_ROPE_WEIGHT_16, weight=0x7F0000300004), L.ST_BAD_STRIDE),      # a 16-bit weight: 8 bytes
         (dict(D=512), L.ST_BAD_SHAPE),
         (dict(D=48), L.ST_BAD_SHAPE),
         (dict(x=0x7F0000000004), L.ST_BAD_STRIDE),
@@ -235,8 +239,12 @@ def test_norm_rope_bwd_desc_layout_and_status_codes(pkg):
     assert ws(desc()) == 13 * 64 * 4
     assert ws(desc(dweight=None)) == 0
     assert run(desc()) == L.ST_WORKSPACE
+    for held in (1, 7, -1):      # what the reserved field holds is not looked at: the weight is fp32, and needs no more than its own alignment
+        assert run(desc(reserved=held, weight=0x7F0000400004)) == L.ST_WORKSPACE, held
+    assert run(desc(dtype=L.DTYPE_BF16 | L.NORM_ROPE_WEIGHT_16, weight=0x7F0000400008)) == L.ST_WORKSPACE
     cases = [
         (dict(abi_version=1), L.ST_BAD_ARG),
+        (dict(dtype=L.DTYPE_BF16 | L.NORM_ROPE_WEIGHT_16, weight=0x7F0000400004), L.ST_BAD_STRIDE),
         (dict(H=0), L.ST_BAD_ARG),
         (dict(dy=None), L.ST_BAD_ARG),
         (dict(dtype=5), L.ST_UNSUPPORTED),
