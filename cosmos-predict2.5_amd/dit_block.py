@@ -150,9 +150,12 @@ class _ModulationFn(torch.autograd.Function):
         return (demb, dlora, *dw1, *dw2)
 
 
-# A call of up to this many rows (twice as many with tangents) forms the modulation vectors in two launches of its own kernels;
-# those read the weights again for every 16 rows, so that many rows are the library's (5120 channels, us: 64 rows 45 against 100,
-# 128 rows 76 against 112; with tangents 64 rows 76 against 344).
+# A call of up to this many rows (one per batch row and frame; with tangents as many again) forms the modulation vectors in two
+# launches of its own kernels.  Those read the weights again for every 16 rows, the library's products once, so that many rows are
+# the library's.  Measured, us, own kernels / modules, values only: in a replayed graph 5120 channels 64 rows 45 / 73, 128 rows
+# 75 / 80, 192 rows 107 / 86; 2048 channels 64 rows 21 / 52, 256 rows 57 / 66, 512 rows 101 / 77.  With tangents, 64 rows: 76 / 291
+# and 36 / 203.  Launched one by one the modules take 200, with tangents 910, at any of these sizes.  The line lies where the own
+# kernels take at most two thirds of the modules' time on the GPU at both widths; at 5120 channels they stop winning at some 140 rows.
 _FUSED_MODULATION_ROWS = 64
 
 
