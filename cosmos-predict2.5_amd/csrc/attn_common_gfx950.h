@@ -39,6 +39,11 @@ constexpr int kFragBytes = 1024;   // one MFMA A-operand fragment: 64 lanes x 16
 // the accumulators, which otherwise runs in nearly every one of a sweep's first dozens of steps (in every step of a short
 // sweep), runs about once per sweep.
 constexpr float kMaxSlack = 6.0f;
+// Whether a score lies that far above the max is read off the row sums: a lane's sum of the exponentials of its 16 keys of a tile is at least
+// its largest one, and is formed anyway.  A tile whose lane sums all stay within kMaxTileSum is done; otherwise (or if a sum is no number)
+// the max moves up to the tile's scores and the tile's softmax is done again from them.  A max over the scores before the exponentials
+// (10 dependent instructions and the wait for the last score MFMA in front of them) costs 5 % of the forward-only kernel.
+constexpr float kMaxTileSum = 64.0f;       // 2^kMaxSlack
 // With tangents H = p dS s is rounded to the 16-bit type as well, and fp16 has the range for |dS s| up to 65504 only while
 // p <= 1 (the reference's range, flash_attention_jvp_triton.py:114,141); a p of up to 2^6 would overflow from |dS s| ~ 1e3 on.
 // So fp16 with tangents keeps the exact running max; bf16 (8 exponent bits) and the forward-only kernels use the slack.
@@ -139,16 +144,15 @@ inline bool allow_lds(const void* fn, size_t bytes) {
 //   * a round of workgroups takes `steps` barrier steps of step_us each and range_us to start and end;
 //   * the step of a round that fills only a part of the chip is faster, as the part then clocks higher under its power limit:
 //     `alone` (0.7 at head dim 128) of the full chip's time for a few workgroups, growing with the square of the filled part
-//     (forward only, one round, 384-row steps: 1.86 us at 112 of 256 workgroups, 1.95 at 160, 2.34 at 224, 2.66 in full rounds);
+//     (forward only, 384-row steps: 1.74 us for a few workgroups, 2.42 in full rounds);
 //     smaller head dims draw less power: 0.9;
 //   * every range leaves slot_bytes of partial results, written once and read once by the merge kernel: 3.8 MB of them cost a
 //     microsecond, the merge kernel's launch three.
 // The constants are fits to B*H = 16 .. 80, 255 .. 17600 positions and S = 1 .. 16, every S measured (the forward's at head dims 16 .. 128
-// each, beside plan_split; the backward's step at 128, taken down with the head dim: at 16 .. 64, B*H = 16 and 40, 700 .. 9000 positions, its
+// each, beside kSymShapes and plan_split; the backward's step at 128, taken down with the head dim: at 16 .. 64, B*H = 16 and 40, 700 .. 9000 positions, its
 // choice takes 1.014 times the best S on average, 1.11 at most).  What the rule that
 // counted rounds alone chose, and this one (us, forward + tangents unless said, head dim 128, with the re-tiling):
 //   1 x 16 x 1560: S = 11 243, S = 1 77;   1 x 40 x 512: S = 3 64, S = 1 40;   1 x 16 x 7040: S = 16 1093, S = 2 1012;
-//   forward only 1 x 16 x 3520: S = 8 222, S = 1 133;   1 x 16 x 5000: S = 8 388, S = 1 217;
 //   backward 1 x 16 x 1560: S = 11 267, S = 1 113.
 // The cost of a split has to come out at least a twentieth lower: the fits are no better than that.
 constexpr int kNumCUs = 256;          // MI355X

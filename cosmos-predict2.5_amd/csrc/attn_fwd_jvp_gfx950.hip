@@ -36,8 +36,8 @@
 //     the output wavefronts; hand-over slots; 146 KB at d = 128 with tangents.  One bare s_barrier per 32-key step
 //     publishes fills and hand-over (a __syncthreads() would also drain every wavefront's LDS operand prefetch).
 //   * Forward only (no tangents) runs a different, symmetric kernel (attn_fwd_sym_kernel below): there the softmax
-//     VALU work per MFMA is three times higher and a wavefront's state is small, so 12 wavefronts (three per SIMD)
-//     each do everything for their own 32 rows and P^T never leaves registers.
+//     VALU work per MFMA is three times higher and a wavefront's state is small, so 8 or 12 wavefronts (two or three per
+//     SIMD) each do everything for their own 32 rows and P^T never leaves registers.
 //   * Query-tile index is the fastest grid dimension, so the 256 workgroups in flight sweep the same
 //     head's K/V images and share them through the per-XCD L2s and the Infinity Cache; workgroups of
 //     one XCD start their (order-free) sweep a few tiles apart so they do not hit one L2 channel at once.
@@ -148,7 +148,7 @@ struct AttnParams {
     float sm_scale, scale_log2;
     // 1-D grid: workgroups [0, n_full) each own a (query block, head) pair; the remaining n_rem pairs are cut into
     // `splits` key ranges, one workgroup each, which leave unnormalised partial results for attn_combine_kernel.
-    // slot = (pair - n_full) * splits + split; block_m = query rows per workgroup (128, or 384 forward only)
+    // slot = (pair - n_full) * splits + split; block_m = query rows per workgroup (128; forward only 128, 256 or 384)
     int n_qt, n_full, n_rem, splits;
     // attn_qstream_kernel: BH = batch * heads (the kernel deals the (query block, head) pairs out over its workgroups itself)
     int BH, q_chunk;
@@ -1114,39 +1114,55 @@ attn_qstream_kernel(const AttnParams p) {
 
 // ---------------------------------------------------------------------------------------------------------------
 // Forward only.  Without tangents a wavefront's whole state (Q fragments, one 32 x d_v accumulator, two score sets)
-// fits the 256 registers that two wavefronts per SIMD leave it, and the softmax VALU work per MFMA is three times
-// that of the tangent modes -- too much for one score wavefront per pair.  So all 8 wavefronts do the same thing,
-// each for its own 32 query rows (256 per workgroup): score MFMAs of the next 32 keys interleaved with the softmax of
-// the current ones, then the P.V MFMAs, with P^T never leaving registers.  The workgroup synchronises (and refills
-// the LDS rings) once per 64 keys: a step is two such half steps.
-constexpr int kSymWaves = 12;        // wavefronts per workgroup, three per SIMD
-constexpr int kSymBlockM = 32 * kSymWaves;     // query rows per workgroup
-constexpr int kSymRing = 4;         // LDS ring depth in steps (pairs of packed tiles), K slots and V slots
-
-template <int DQK, int DV>
+// fits the 168 registers that three wavefronts per SIMD leave it, and the softmax VALU work per MFMA is three times
+// that of the tangent modes -- too much for one score wavefront per pair.  So all wavefronts do the same thing,
+// each for its own 32 query rows, with P^T never leaving registers.
+//
+// What bounds it: a SIMD issues one VALU or MFMA instruction in 4 cycles.  A tile of 32 keys costs a wavefront 16 MFMAs (512 cycles of
+// the matrix unit) and some 125 such turns, 64 of them in 16 exponentials; in long calls the part's power limit on top (74 % MFMA duty
+// at 1.70 GHz).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
+// formed where it did not move (kMaxTileSum).  Measured, us, before either / with the softmax between the MFMAs / with both: 16 heads,
+// d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120.
+// Not faster: v_mfma_f32_16x16x32 (less energy, but twice the MFMA instructions to issue: 37440 9450, 3520 142), operand fetches three
+// groups ahead, the fills spread over the step.
+//
+// A workgroup is RG groups of 32 query rows x KG groups of keys: of every KG tiles of 32 keys a wavefront takes one, and the KG partial
+// results of a row group (accumulator, running max, row sum) are merged through LDS at the end.  Large calls take 12 x 1; 8 x 1 and 4 x 2
+// keep more compute units busy, and each workgroup's chain of steps shorter, where there are few rows (kSymShapes).
+template <int DQK, int DV, int RG, int KG>
 struct SymCfg {
-    static constexpr int NC = DQK / 16, NDB = (DV + 31) / 32;
+    static constexpr int NC = DQK / 16, NDB = (DV + 31) / 32, NW = RG * KG;
+    static constexpr int TPS = KG == 1 ? 2 : KG;                           // packed tiles per barrier step
+    static constexpr int RING = 4;                           // LDS ring depth in steps, K slots and V slots
     static constexpr int K_FR = NC, VT_FR = 2 * NDB;                       // fragments per packed tile
     static constexpr int KP_BYTES = K_FR * kFragBytes, VP_BYTES = VT_FR * kFragBytes, TILE_BYTES = KP_BYTES + VP_BYTES;
-    static constexpr int KS_BYTES = 2 * KP_BYTES, VS_BYTES = 2 * VP_BYTES;   // ring slots: the parts of two packed tiles
-    static constexpr int K_LOADS = (2 * K_FR + 7) / 8, V_LOADS = (2 * VT_FR + 7) / 8;   // per wavefront per step
-    static_assert(K_LOADS <= 2 && V_LOADS <= 2 && (K_LOADS == 1 || K_FR % 2 == 0) && (V_LOADS == 1 || VT_FR % 2 == 0), "runs stay inside a tile");
+    static constexpr int KS_BYTES = TPS * KP_BYTES, VS_BYTES = TPS * VP_BYTES;   // ring slots: the parts of a step's tiles
+    static constexpr int FW = KG == 1 && NW > 8 ? 8 : NW;                  // wavefronts that fill the rings
+    static constexpr int K_LOADS = (TPS * K_FR + FW - 1) / FW, V_LOADS = (TPS * VT_FR + FW - 1) / FW;   // per filling wavefront and step
+    static_assert(K_LOADS <= 4 && V_LOADS <= 4 && K_FR % K_LOADS == 0 && VT_FR % V_LOADS == 0, "runs stay inside a tile");
     static constexpr int GROUP_LOADS = K_LOADS + V_LOADS;
-    static constexpr int KRING_OFF = 0, VRING_OFF = kSymRing * KS_BYTES;
-    static constexpr int LDS_BYTES = VRING_OFF + kSymRing * VS_BYTES;
+    static constexpr int KRING_OFF = 0, VRING_OFF = RING * KS_BYTES;
+    static constexpr int RING_BYTES = VRING_OFF + RING * VS_BYTES;
+    // merge of the key groups, in the place of the rings: accumulator blocks of the wavefronts that do not own them, (max, sum) of all
+    static constexpr int BLK_BYTES = 4 * kFragBytes, STAT_OFF = (KG - 1) * RG * NDB * BLK_BYTES;
+    static constexpr int MERGE_BYTES = KG == 1 ? 0 : STAT_OFF + NW * 64 * 8;
+    static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
 };
 
 template <typename T, int DQK, int DV>
 struct SymWave {
-    typedef SymCfg<DQK, DV> C;
     typedef typename VecOf<T>::v8 V8;
-    static constexpr int NC = C::NC, NDB = C::NDB;
+    typedef T V2 __attribute__((ext_vector_type(2)));
+    static constexpr int NC = DQK / 16, NDB = (DV + 31) / 32;
     static constexpr int NB = 2 * NDB;      // P.V MFMA groups of a tile, (c, db) at index c * NDB + db
     static constexpr int PD = COSMOS_ATTN_PREFETCH_GROUPS;
 
     V8 qf[NC];
     f32x16 acc[NDB];
     float m_run, l_run, scale_log2;
+    float l_tile;                           // the current tile's share of the row sum (this lane's keys)
+    float p_even;
+    uint32_t pw[8];                         // P^T of the current tile, two values each (B operand c of the P.V MFMAs: words 4 c .. + 3)
     int lane;
 
     __device__ __forceinline__ V8 lds_frag(const char* base, int frag) const {
@@ -1167,20 +1183,12 @@ struct SymWave {
             s[e] = ok ? s[e] : -INFINITY;
         }
     }
-    // fold the lane-local max of a tile's scores into the running max; returns the rescale factor (1 if no row moved)
-    __device__ __forceinline__ float update_max(float mx) {
-        {   // max with lane ^ 32 (the other half of the same query column)
-            float lo, hi;
-            both_halves(mx, lo, hi);
-            mx = fmaxf(lo, hi);
-        }
-        const float m_new = fmaxf(m_run, mx * scale_log2);
-        float alpha = 1.0f;
-        if (__any(m_new > m_run + kMaxSlack)) {
-            alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-            m_run = m_new;
-        }
+    // Move the running max up to a tile's scores; returns the rescale factor of everything accumulated so far.
+    __device__ __forceinline__ float raise_max(const f32x16& x) {
+        float lo, hi;   // max with lane ^ 32 (the other half of the same query column)
+        both_halves(lane_max(x) * scale_log2, lo, hi);
+        const float m_new = fmaxf(m_run, fmaxf(lo, hi)), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
         return alpha;
     }
     __device__ __forceinline__ void scores_plain(f32x16& x, const char* kpart) const {
@@ -1189,13 +1197,34 @@ struct SymWave {
 #pragma unroll
         for (int c = 0; c < NC; ++c) x = mfma32(lds_frag(kpart, c), qf[c], x);
     }
+    // Softmax of n elements of x from e0 on (already folded into m_run).  The empty asm statements keep the arithmetic where it is
+    // written, between the MFMAs: the compiler would otherwise put all of it behind the next branch, where no MFMA of this wavefront covers it.
+    __device__ __forceinline__ void softmax_elems(const f32x16& x, int e0, int n) {
+#pragma unroll
+        for (int k = 0; k < n; ++k) {
+            const int e = e0 + k;
+            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], scale_log2, -m_run));
+            if (e & 1) {
+                l_tile += p_even;                // (an instruction between the exponential and its first use)
+                asm volatile("" : "+v"(l_tile));
+                const V2 both = {(T)p_even, (T)p};
+                pw[e >> 1] = __builtin_bit_cast(uint32_t, both);
+                l_tile += p;
+                asm volatile("" : "+v"(pw[e >> 1]), "+v"(l_tile));
+            } else {
+                p_even = p;
+                asm volatile("" : "+v"(p_even));
+            }
+        }
+    }
 
-    // Half a step (32 keys).  Stage A: scores of the next tile (K part `kpart`) into `xn`, interleaved with the softmax
-    // of the current one (`x`, already folded into m_run) into the 16-bit operands P^T.  Then rescale by `alpha`
-    // (the factor that goes with `x`) if some row's max moved, and stage B: O^T += V^T P^T over the V part `vpart`.
-    __device__ __forceinline__ void half_step(const f32x16& x, f32x16& xn, const char* kpart, const char* vpart, float alpha) {
-        V8 pf[2];
-        constexpr int EPC = 16 / NC;   // softmax elements dealt out per d chunk
+    // One tile of 32 keys.  Stage A: scores of the next tile (K part `kpart`) into `xn`, interleaved with the softmax of the second
+    // half of the current one (`x`).  Its exponentials referred to the max of earlier tiles (kMaxTileSum): where a lane's sum of them is too
+    // large, which is rare after a sweep's first tiles, the max moves up to this tile's and the tile's softmax is done again.
+    // Stage B: O^T += V^T P^T over the V part `vpart`, interleaved with the softmax of the first half of `xn`.
+    template <class Mask>
+    __device__ __forceinline__ void tile_step(const f32x16& x, f32x16& xn, const char* kpart, const char* vpart, int t_next, Mask mask) {
+        constexpr int EPC = 8 / NC, EPB = 8 / NB;   // softmax elements dealt out per d chunk / per P.V group
         V8 fa[NC];
 #pragma unroll
         for (int i = 0; i < PD && i < NC; ++i) fa[i] = lds_frag(kpart, i);
@@ -1207,25 +1236,28 @@ struct SymWave {
             if (c + PD < NC) fa[c + PD] = lds_frag(kpart, c + PD);
             SCHED_FENCE();
             xn = mfma32(fa[c], qf[c], xn);
-#pragma unroll
-            for (int k = 0; k < EPC; ++k) {
-                const int e = c * EPC + k;
-                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(x[e], scale_log2, -m_run));
-                l_run += p;
-                pf[e >> 3][e & 7] = (T)p;
-            }
+            softmax_elems(x, 8 + c * EPC, EPC);
         }
         SCHED_FENCE();
-        V8 fv[NB];
+        V8 pf[2], fv[NB];
 #pragma unroll
         for (int i = 0; i < PD && i < NB; ++i) fv[i] = lds_frag(vpart, 2 * (i % NDB) + i / NDB);
-        if (__any(alpha != 1.0f)) {
+        if (__any(!(l_tile <= kMaxTileSum))) {
+            const float alpha = raise_max(x);
+            l_run *= alpha;
 #pragma unroll
             for (int i = 0; i < NDB; ++i) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][e] *= alpha;
+                acc[i] *= alpha;
+                asm volatile("" : "+v"(acc[i]));
             }
+            l_tile = 0.f;
+            softmax_elems(x, 0, 16);
         }
+        l_run += l_tile;
+        l_tile = 0.f;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) pf[c] = __builtin_bit_cast(V8, make_uint4(pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]));
+        mask(xn, t_next);
 #pragma unroll
         for (int g = 0; g < NB; ++g) {
             const int c = g / NDB, db = g % NDB;
@@ -1233,25 +1265,25 @@ struct SymWave {
             if (g + PD < NB) fv[g + PD] = lds_frag(vpart, 2 * ((g + PD) % NDB) + (g + PD) / NDB);
             SCHED_FENCE();
             acc[db] = mfma32(fv[g], pf[c], acc[db]);
+            softmax_elems(xn, g * EPB, EPB);
         }
         SCHED_FENCE();
     }
 };
 
-template <typename T, int DQK, int DV>
-__global__ void __attribute__((amdgpu_flat_work_group_size(64 * kSymWaves, 64 * kSymWaves), amdgpu_waves_per_eu(3, 3)))
+template <typename T, int DQK, int DV, int RG, int KG>
+__global__ void __attribute__((amdgpu_flat_work_group_size(64 * RG * KG, 64 * RG * KG), amdgpu_waves_per_eu(RG * KG / 4, RG * KG / 4)))
 attn_fwd_sym_kernel(const AttnParams p) {
-    typedef SymCfg<DQK, DV> C;
+    typedef SymCfg<DQK, DV, RG, KG> C;
     typedef SymWave<T, DQK, DV> W;
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
-    constexpr int NC = C::NC, NDB = C::NDB;
-    constexpr int TILE_BYTES = C::TILE_BYTES, KS_BYTES = C::KS_BYTES, VS_BYTES = C::VS_BYTES;
-    // K(s), V(s): the K parts / V parts of the two packed tiles at sweep position s ("step tile" g = tiles 2g, 2g+1).
-    // Step s: half step 0 = scores of tile (s,1) | softmax and P.V of tile (s,0); half step 1 = scores of tile (s+1,0) |
-    // softmax and P.V of tile (s,1).  It reads K(s), K(s+1), V(s) and issues the fills of K(s+3), V(s+3) into the slots
-    // of K(s-1), V(s-1), dead since the barrier.  At the top of step s the fills issued up to step s-2 must have
-    // landed; those of step s-1 may be in flight.
+    constexpr int NC = C::NC, NDB = C::NDB, BLOCK_M = 32 * RG;
+    constexpr int TILE_BYTES = C::TILE_BYTES, KS_BYTES = C::KS_BYTES, VS_BYTES = C::VS_BYTES, TPS = C::TPS, RING = C::RING;
+    // K(s), V(s): the K parts / V parts of the TPS packed tiles at sweep position s ("step tile" t = tiles TPS t .. TPS t + TPS - 1).
+    // KG = 1: a wavefront does the two tiles of a step one after the other; KG = 2: one of them.  Step s reads K(s), K(s+1), V(s) and
+    // issues the fills of K(s+3), V(s+3) into the slots of K(s-1), V(s-1), dead since the barrier.  At the top of step s the fills issued
+    // up to step s-2 must have landed; those of step s-1 may be in flight.
     constexpr int IN_FLIGHT = C::GROUP_LOADS;
     constexpr int WAIT_FILLS = (IN_FLIGHT & 15) | ((IN_FLIGHT >> 4) << 14) | 0x0F70;
 
@@ -1263,22 +1295,24 @@ attn_fwd_sym_kernel(const AttnParams p) {
     const int qt = pair % p.n_qt, bh = pair / p.n_qt, b = bh / p.H, h = bh % p.H;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rg = wave % RG, kg = wave / RG;
     const int j = lane & 31, hh = lane >> 5;
-    const int row0 = qt * kSymBlockM + wave * 32;   // first query row of this wavefront
+    const int row0 = qt * BLOCK_M + rg * 32;        // first query row of this wavefront
     const int row = row0 + j;                       // this lane's query row (lanes l and l^32 share it)
 
     int kv_len = p.Lkv;
     if (p.key_lens) { const int kl = p.key_lens[b]; kv_len = kl < kv_len ? (kl < 0 ? 0 : kl) : kv_len; }
-    int n_tiles = (kv_len + kBlockN - 1) / kBlockN;
-    if (p.causal) { const int lim = (qt * kSymBlockM + kSymBlockM + kBlockN - 1) / kBlockN; n_tiles = n_tiles < lim ? n_tiles : lim; }
-    const int n_steps_all = (n_tiles + 1) / 2;   // (a last step tile that sticks out past n_tiles is masked like any tail)
+    const int n_tiles_valid = (kv_len + kBlockN - 1) / kBlockN;
+    int n_tiles = n_tiles_valid;
+    if (p.causal) { const int lim = (qt * BLOCK_M + BLOCK_M + kBlockN - 1) / kBlockN; n_tiles = n_tiles < lim ? n_tiles : lim; }
+    const int n_steps_all = (n_tiles + TPS - 1) / TPS;   // (a last step tile that sticks out past n_tiles is masked like any tail)
     // this workgroup's share of the sweep: positions [u_lo, u_lo + n_steps)
     const int u_lo = partial ? (int)((int64_t)split * n_steps_all / p.splits) : 0;
     const int n_steps = partial ? (int)((int64_t)(split + 1) * n_steps_all / p.splits) - u_lo : n_steps_all;
 
     char* const kring = smem + C::KRING_OFF;
     char* const vring = smem + C::VRING_OFF;
-    // reads past the end of the buffer (second tile of a last, odd step) return zeros
+    // reads past the end of the buffer (later tiles of a last step) return zeros
     const __amdgpu_buffer_rsrc_t kv_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<char*>(p.kv) + (size_t)bh * p.n_tiles * TILE_BYTES, 0, p.n_tiles * TILE_BYTES, 0x00020000);
     // sweep order (in step tiles): see attn_fwd_jvp_kernel
@@ -1287,16 +1321,21 @@ attn_fwd_sym_kernel(const AttnParams p) {
     auto tile_at = [&](int u) { return __builtin_amdgcn_readfirstlane((u_lo + u + shift) % n_sweep); };
     auto wrap_inc = [&](int t) { ++t; return t >= n_sweep ? t - n_sweep : t; };
     // this wavefront's run of fragments inside a K slot / V slot (never crosses a packed tile)
-    const int kf0 = (wave * C::K_LOADS) % (2 * C::K_FR), vf0 = (wave * C::V_LOADS) % (2 * C::VT_FR);
+    const int kf0 = (wave * C::K_LOADS) % (TPS * C::K_FR), vf0 = (wave * C::V_LOADS) % (TPS * C::VT_FR);
     const int k_src_run = (kf0 / C::K_FR) * TILE_BYTES + (kf0 % C::K_FR) * kFragBytes;
     const int v_src_run = (vf0 / C::VT_FR) * TILE_BYTES + C::KP_BYTES + (vf0 % C::VT_FR) * kFragBytes;
-    auto fill = [&](int g, int u) {
-        if (wave >= 8) return;   // eight wavefronts cover a slot
-        issue_part<C::K_LOADS>(kv_rsrc, kring + (u % kSymRing) * KS_BYTES + kf0 * kFragBytes, lane * 16, g * 2 * TILE_BYTES + k_src_run);
-        issue_part<C::V_LOADS>(kv_rsrc, vring + (u % kSymRing) * VS_BYTES + vf0 * kFragBytes, lane * 16, g * 2 * TILE_BYTES + v_src_run);
+    auto fill_k = [&](int t, int u) {
+        if (wave < C::FW) issue_part<C::K_LOADS>(kv_rsrc, kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + k_src_run);
     };
+    auto fill_v = [&](int t, int u) {
+        if (wave < C::FW) issue_part<C::V_LOADS>(kv_rsrc, vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + v_src_run);
+    };
+    constexpr int PRE = RING - 1;
 #pragma unroll
-    for (int u = 0; u < 3; ++u) fill(tile_at(u), u);
+    for (int u = 0; u < PRE; ++u) {
+        fill_k(tile_at(u), u);
+        fill_v(tile_at(u), u);
+    }
 
     W w;
     w.lane = lane;
@@ -1316,55 +1355,114 @@ attn_fwd_sym_kernel(const AttnParams p) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) w.acc[i][e] = 0.f;
     }
-    w.m_run = -INFINITY;
+    // (a key group's tiles may all be masked for a while, or throughout: its max starts at a number, so that exp2(-inf - max) is 0)
+    w.m_run = KG == 1 ? -INFINITY : -3.0e38f;
     w.l_run = 0.f;
 
     const bool causal = p.causal != 0;
     auto need_mask = [&](int t) { return (t * kBlockN + kBlockN > kv_len) || (causal && (t * kBlockN + kBlockN - 1 > row0)); };
-    float alpha = 1.0f;
-    // fold the scores of packed tile pt into the running max (masking them first where the tile needs it)
-    auto fold = [&](f32x16& x, int pt) {
-        if (need_mask(pt)) W::mask_scores(x, pt * kBlockN + 4 * hh, kv_len, causal, row);
-        alpha = w.update_max(W::lane_max(x));
-    };
-    f32x16 sc0, sc1;   // scores of the current / next tile, swapping roles every half step
+    auto mask = [&](f32x16& x, int t) { if (need_mask(t)) W::mask_scores(x, t * kBlockN + 4 * hh, kv_len, causal, row); };
+    f32x16 sc0, sc1;   // scores of the current / next tile, swapping roles every tile
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): Q and this wavefront's share of the first fills are here
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    w.scores_plain(sc0, kring);
-    if (n_steps > 0) fold(sc0, 2 * tile_at(0));
-    int g_cur = tile_at(0), g_nxt = tile_at(1), g_fill = tile_at(3);
-    for (int s = 0; s < n_steps; ++s) {
-        __builtin_amdgcn_s_waitcnt(WAIT_FILLS);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        fill(g_fill, s + 3);
-        const char* kslot = kring + (s % kSymRing) * KS_BYTES;
-        const char* vslot = vring + (s % kSymRing) * VS_BYTES;
-        {
-            const float a = alpha;
-            w.half_step(sc0, sc1, kslot + C::KP_BYTES, vslot, a);
-            fold(sc1, 2 * g_cur + 1);
-        }
-        {
-            const float a = alpha;
-            w.half_step(sc1, sc0, kring + ((s + 1) % kSymRing) * KS_BYTES, vslot + C::VP_BYTES, a);
-            if (s + 1 < n_steps) fold(sc0, 2 * g_nxt);
-        }
-        g_cur = g_nxt; g_nxt = wrap_inc(g_nxt); g_fill = wrap_inc(g_fill);
+    w.scores_plain(sc0, kring + kg * C::KP_BYTES);
+    w.l_tile = 0.f;
+    if (n_steps > 0) {
+        mask(sc0, TPS * tile_at(0) + kg);
+        w.raise_max(sc0);
+        w.softmax_elems(sc0, 0, 8);
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);   // drain the (unused) trailing fills before the LDS is released
+    // past the last position there is no next tile: whatever scores are formed for it are masked, so that they add nothing
+    if constexpr (KG == 1) {
+        int g_cur = tile_at(0), g_nxt = tile_at(1), g_fill = tile_at(3);
+        for (int s = 0; s < n_steps; ++s) {
+            __builtin_amdgcn_s_waitcnt(WAIT_FILLS);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            fill_k(g_fill, s + 3);
+            fill_v(g_fill, s + 3);
+            const char* kslot = kring + (s % RING) * KS_BYTES;
+            const char* vslot = vring + (s % RING) * VS_BYTES;
+            w.tile_step(sc0, sc1, kslot + C::KP_BYTES, vslot, 2 * g_cur + 1, mask);
+            w.tile_step(sc1, sc0, kring + ((s + 1) % RING) * KS_BYTES, vslot + C::VP_BYTES, s + 1 < n_steps ? 2 * g_nxt : n_tiles_valid, mask);
+            g_cur = g_nxt; g_nxt = wrap_inc(g_nxt); g_fill = wrap_inc(g_fill);
+        }
+    } else {
+        int g_nxt = tile_at(1), g_fill = tile_at(RING - 1), slot = 0;
+        auto body = [&](int s, f32x16& x, f32x16& xn) {
+            __builtin_amdgcn_s_waitcnt(WAIT_FILLS);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int next = slot + 1 < RING ? slot + 1 : 0, prev = slot > 0 ? slot - 1 : RING - 1;
+            fill_k(g_fill, prev);
+            fill_v(g_fill, prev);
+            w.tile_step(x, xn, kring + next * KS_BYTES + kg * C::KP_BYTES, vring + slot * VS_BYTES + kg * C::VP_BYTES,
+                        s + 1 < n_steps ? TPS * g_nxt + kg : n_tiles_valid, mask);
+            slot = next;
+            g_nxt = wrap_inc(g_nxt); g_fill = wrap_inc(g_fill);
+        };
+        for (int s = 0; s < n_steps; s += 2) {
+            body(s, sc0, sc1);
+            if (s + 1 < n_steps) body(s + 1, sc1, sc0);
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // drain the (unused) trailing fills before the LDS is released or reused
 
     // ---- epilogue: O = acc / l ; LSE = (m + log2 l) ln 2 ----
-    const float l_tot = w.l_run + __shfl_xor(w.l_run, 32);
+    float l_tot = w.l_run + __shfl_xor(w.l_run, 32);
+    if constexpr (KG > 1) {
+        // merge the key groups: the wavefront of key group db % KG finishes 32-channel block db; the others hand it theirs
+        __syncthreads();
+        float2* const stat = reinterpret_cast<float2*>(smem + C::STAT_OFF) + lane;
+        auto block_at = [&](int src, int db) {   // slot of key group src's block db
+            const int i = (src - db % KG + KG) % KG - 1;
+            return reinterpret_cast<float4*>(smem + ((i * RG + rg) * NDB + db) * C::BLK_BYTES) + lane;
+        };
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+            if (db % KG == kg) continue;
+            float4* dst = block_at(kg, db);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) dst[64 * g] = make_float4(w.acc[db][4 * g], w.acc[db][4 * g + 1], w.acc[db][4 * g + 2], w.acc[db][4 * g + 3]);
+        }
+        stat[64 * wave] = make_float2(w.m_run, l_tot);
+        __syncthreads();
+        float wgt[KG], m_all = w.m_run;
+        float2 st[KG];
+#pragma unroll
+        for (int k = 0; k < KG; ++k) { st[k] = stat[64 * (k * RG + rg)]; m_all = fmaxf(m_all, st[k].x); }
+        l_tot = 0.f;
+#pragma unroll
+        for (int k = 0; k < KG; ++k) { wgt[k] = __builtin_amdgcn_exp2f(st[k].x - m_all); l_tot += st[k].y * wgt[k]; }
+        const float own = __builtin_amdgcn_exp2f(w.m_run - m_all);
+        w.m_run = m_all;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+            if (db % KG != kg) continue;
+            w.acc[db] *= own;
+#pragma unroll
+            for (int k = 0; k < KG; ++k) {
+                if (k == kg) continue;
+                const float4* src = block_at(k, db);
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 a = src[64 * g];
+                    w.acc[db][4 * g] += a.x * wgt[k]; w.acc[db][4 * g + 1] += a.y * wgt[k];
+                    w.acc[db][4 * g + 2] += a.z * wgt[k]; w.acc[db][4 * g + 3] += a.w * wgt[k];
+                }
+            }
+        }
+    }
     if (partial) {
         // a key range only: leave acc, m, l as they are for attn_combine_kernel (rows past Lq are written too and
         // never combined)
         const int64_t slot = (int64_t)(pair - p.n_full) * p.splits + split;
-        const int wrow = wave * 32 + j;
-        float* pa = p.part_acc + (slot * kSymBlockM + wrow) * DV;
+        const int wrow = rg * 32 + j;
+        float* pa = p.part_acc + (slot * BLOCK_M + wrow) * DV;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
+            if (KG > 1 && db % KG != kg) continue;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d = 32 * db + 8 * g + 4 * hh;
@@ -1372,7 +1470,7 @@ attn_fwd_sym_kernel(const AttnParams p) {
                     *reinterpret_cast<float4*>(pa + d) = make_float4(w.acc[db][4 * g], w.acc[db][4 * g + 1], w.acc[db][4 * g + 2], w.acc[db][4 * g + 3]);
             }
         }
-        if (hh == 0) p.part_stat[slot * kSymBlockM + wrow] = make_float4(w.m_run, l_tot, 0.f, 0.f);
+        if (kg == 0 && hh == 0) p.part_stat[slot * BLOCK_M + wrow] = make_float4(w.m_run, l_tot, 0.f, 0.f);
         return;
     }
     const float inv_l = 1.0f / l_tot;
@@ -1380,6 +1478,7 @@ attn_fwd_sym_kernel(const AttnParams p) {
         T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
+            if (KG > 1 && db % KG != kg) continue;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d = 32 * db + 8 * g + 4 * hh;   // registers 4g..4g+3 are 4 consecutive d
@@ -1391,7 +1490,7 @@ attn_fwd_sym_kernel(const AttnParams p) {
                 }
             }
         }
-        if (p.lse && hh == 0) p.lse[(int64_t)bh * p.Lq + row] = (w.m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
+        if (p.lse && kg == 0 && hh == 0) p.lse[(int64_t)bh * p.Lq + row] = (w.m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
     }
 }
 
@@ -1446,34 +1545,54 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnParams p, i
 // ------------------------------------------------------------------------------------------------ host
 typedef void (*attn_kernel_t)(const AttnParams);
 
+// Workgroups of attn_fwd_sym_kernel, groups of 32 query rows x groups of keys, and what they cost at head dims 16, 32, 64, 128 (StepCost):
+// the least estimate is taken (plan_split).  Fits to 255 .. 13000 positions and 600 .. 37440 x 512 .. 2048, B*H = 16 and 40, S = 1 .. 16, each
+// shape with each S measured; the choice takes 1.003 to 1.008 times the best one's time on average, 1.07 at most.  us, 12 x 1 / 8 x 1 /
+// 4 x 2, uncut, d = 128, with the re-tiling: 16 heads 255 positions 19.4 / 18.3 / 15.5, 700 35.2 / 30.0 / 25.9, 1560 61 / 53 / 41, 3520
+// 137 / 120 / 135, 5000 219 / 285 / 262; 40 heads 1000 51 / 45 / 59, 1560 82 / 108 / 109.  (Three key groups are no faster than two.)
+// The smaller shapes are for calls that fit into one round of them.  Past that 12 x 1 with its last round cut, or the query-streaming kernel, is
+// as fast but at single sizes (16 heads 7040 x 1024: 8 x 1 87, 12 x 1 93; 40 heads 3520: 282, 298).
+struct SymShape { int rg, kg; double step_us[4], alone[4], range_us[4]; };
+constexpr SymShape kSymShapes[] = {
+    {12, 1, {1.09, 1.12, 1.55, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
+    {8, 1, {0.82, 0.85, 1.10, 1.73}, {1.0, 1.0, 0.94, 0.78}, {4.6, 5.1, 6.6, 10.6}},
+    {4, 2, {0.45, 0.46, 0.60, 0.94}, {1.0, 1.0, 1.0, 0.99}, {4.1, 4.8, 6.0, 9.0}},
+};
+constexpr int kNumSymShapes = sizeof(kSymShapes) / sizeof(kSymShapes[0]);
+
 template <typename T, int DQK, int DV>
-attn_kernel_t pick_mode(int mode) {
+attn_kernel_t pick_mode(int mode, int shape) {
     switch (mode) {
-        case MODE_FWD: return attn_fwd_sym_kernel<T, DQK, DV>;
+        case MODE_FWD:
+            switch (shape) {
+                case 0: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[0].rg, kSymShapes[0].kg>;
+                case 1: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[1].rg, kSymShapes[1].kg>;
+                default: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[2].rg, kSymShapes[2].kg>;
+            }
         case MODE_JVP_Q: return attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q>;
         default: return attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL>;
     }
 }
 template <typename T, int DQK>
-attn_kernel_t pick_dv(int dv, int mode) {
+attn_kernel_t pick_dv(int dv, int mode, int shape) {
     switch (dv) {
-        case 16: return pick_mode<T, DQK, 16>(mode);
-        case 32: return pick_mode<T, DQK, 32>(mode);
-        case 64: return pick_mode<T, DQK, 64>(mode);
-        case 128: return pick_mode<T, DQK, 128>(mode);
+        case 16: return pick_mode<T, DQK, 16>(mode, shape);
+        case 32: return pick_mode<T, DQK, 32>(mode, shape);
+        case 64: return pick_mode<T, DQK, 64>(mode, shape);
+        case 128: return pick_mode<T, DQK, 128>(mode, shape);
         default: return nullptr;
     }
 }
 template <typename T>
-attn_kernel_t pick_dqk(int dqk, int dv, int mode) {
+attn_kernel_t pick_dqk(int dqk, int dv, int mode, int shape) {
 #ifdef COSMOS_ATTN_ONLY_D128   // development builds: instantiate the d=128 kernels only
-    return (dqk == 128 && dv == 128) ? pick_mode<T, 128, 128>(mode) : nullptr;
+    return (dqk == 128 && dv == 128) ? pick_mode<T, 128, 128>(mode, shape) : nullptr;
 #endif
     switch (dqk) {
-        case 16: return pick_dv<T, 16>(dv, mode);
-        case 32: return pick_dv<T, 32>(dv, mode);
-        case 64: return pick_dv<T, 64>(dv, mode);
-        case 128: return pick_dv<T, 128>(dv, mode);
+        case 16: return pick_dv<T, 16>(dv, mode, shape);
+        case 32: return pick_dv<T, 32>(dv, mode, shape);
+        case 64: return pick_dv<T, 64>(dv, mode, shape);
+        case 128: return pick_dv<T, 128>(dv, mode, shape);
         default: return nullptr;
     }
 }
@@ -1513,12 +1632,17 @@ size_t tile_bytes_of(const cosmos_attn_desc* d) {
     const TileGeom g(d->d_qk, d->d_v, mode_of(d) == MODE_JVP_FULL);
     return (size_t)g.tile_frags * kFragBytes;
 }
-// LDS of the attention kernel: K ring, V ring, P^T/H^T hand-over buffers, rescale factors (AttnCfg::LDS_BYTES)
-size_t lds_bytes_of(const cosmos_attn_desc* d) {
+// LDS of the attention kernels: K ring, V ring, P^T/H^T hand-over buffers, rescale factors (AttnCfg::LDS_BYTES); forward only the
+// rings or, with key groups, what merging them takes (SymCfg::LDS_BYTES)
+size_t lds_bytes_of(const cosmos_attn_desc* d, int shape) {
     const int mode = mode_of(d);
     const TileGeom g(d->d_qk, d->d_v, mode == MODE_JVP_FULL);
     const size_t kp = (size_t)g.kpart_frags * kFragBytes, vp = (size_t)(g.tile_frags - g.kpart_frags) * kFragBytes;
-    if (mode == MODE_FWD) return (size_t)kSymRing * 2 * (kp + vp);   // SymCfg::LDS_BYTES
+    if (mode == MODE_FWD) {
+        const SymShape w = kSymShapes[shape];
+        const size_t rings = (size_t)4 * 2 * (kp + vp), merge = w.kg == 1 ? 0 : (size_t)(w.kg - 1) * w.rg * g.ndb * 4 * kFragBytes + (size_t)w.rg * w.kg * 64 * 8;
+        return rings > merge ? rings : merge;
+    }
     const size_t ph = 4 * kFragBytes;
     return kRingK * kp + kRingV * vp + 2 * 4 * ph + 2 * 4 * 256;
 }
@@ -1530,13 +1654,11 @@ size_t tiles_bytes_of(const cosmos_attn_desc* d) { return (size_t)d->B * d->H * 
 // workgroups are cut along the keys, and a small second kernel merges the ranges.
 // a head dim of 256 goes to attn_wide_kernel
 bool is_wide(const cosmos_attn_desc* d) { return d->d_qk == 256 || d->d_v == 256; }
-struct SplitPlan { int block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // us: estimated time of the launches
-// Barrier steps in full rounds at head dims 16, 32, 64, 128 (us): below 64 the exponentials and the step's fixed instructions are
+struct SplitPlan { int shape, block_m, n_qt, n_pairs, n_full, n_rem, splits; double us; };   // shape: of kSymShapes; us: estimated time of the launches
+// With tangents: barrier steps in full rounds at head dims 16, 32, 64, 128 (us): below 64 the exponentials and the step's fixed instructions are
 // most of it.  Fits to 500 .. 9000 positions and 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, S = 1 .. 16, every S measured: the S
-// chosen with them takes 1.0035 to 1.011 times the best one's time on average, 1.13 at most.  (A step that shrinks in proportion to the
-// head dim, which had been assumed, cut too few: forward only, us, 16 x 700 at head dim 16 23.0 -> 20.3, 40 x 1100 36.8 -> 32.9, 40 x 9000 at 32
-// 889 -> 789.)
-constexpr double kStepUs[3][4] = {{1.36, 1.37, 1.77, 2.66}, {0.54, 0.56, 0.68, 0.86}, {0.54, 0.60, 0.82, 1.21}};   // MODE_FWD, MODE_JVP_Q, MODE_JVP_FULL
+// chosen with them takes 1.0035 to 1.011 times the best one's time on average, 1.13 at most.
+constexpr double kStepUs[2][4] = {{0.54, 0.56, 0.68, 0.86}, {0.54, 0.60, 0.82, 1.21}};   // MODE_JVP_Q, MODE_JVP_FULL
 constexpr double kStepAlone[4] = {0.9, 0.9, 0.9, 0.7};
 constexpr double kPairUs[4] = {5.0, 5.0, 5.0, 13.0};          // what a workgroup that is a whole pair costs besides its steps
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1550,28 +1672,49 @@ size_t partial_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
 }
 // `room`: bytes there are for partial results (0: never split)
 constexpr size_t kNoLimit = ~(size_t)0;
-SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
+// The best cut for workgroups of block_m rows and n_steps barrier steps: `whole` is what a pair that is not cut costs, `cut` one of
+// which S ranges may be made.
+SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int block_m, int n_steps, StepCost whole, StepCost cut) {
     SplitPlan s;
-    const bool fwd = mode_of(d) == MODE_FWD;
-    const double dim = 0.5 * (d->d_qk + d->d_v);
-    const StepCost c{by_head_dim(kStepUs[mode_of(d)], dim), fwd && dim > 64.0 ? 13.0 : 8.0, by_head_dim(kStepAlone, dim)};
-    const int n_steps = fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d);   // barrier steps: 64 keys forward only, 32 with tangents
-    s.block_m = fwd ? kSymBlockM : kBlockM;
+    s.shape = shape;
+    s.block_m = block_m;
     s.n_qt = (d->Lq + s.block_m - 1) / s.block_m;
     s.n_pairs = s.n_qt * d->B * d->H;
     s.n_rem = 0; s.splits = 1; s.n_full = s.n_pairs;
     const int rem = s.n_pairs % kNumCUs;
-    const StepCost alone{c.step_us, by_head_dim(kPairUs, dim), c.alone};
-    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + (rem ? rounds_cost(rem, n_steps, alone) : 0.0);
+    const double full_us = rounds_cost(s.n_pairs - rem, n_steps, whole);
+    s.us = full_us + rounds_cost(rem, n_steps, whole);
     if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
-    const double slot_bytes = (double)s.block_m * (d->d_v * (fwd ? 1 : 2) * sizeof(float) + sizeof(float4));
+    const double slot_bytes = (double)s.block_m * (d->d_v * (mode_of(d) == MODE_FWD ? 1 : 2) * sizeof(float) + sizeof(float4));
     const SplitPlan uncut = s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
     while (s.splits > 1 && partial_bytes(d, s) > room) --s.splits;
-    s.splits = choose_splits(rem, n_steps, c, slot_bytes, s.splits);
+    s.splits = choose_splits(rem, n_steps, cut, slot_bytes, s.splits);
     if (s.splits < 2) return uncut;
-    s.us = rounds_cost(s.n_pairs - rem, n_steps, alone) + split_cost(rem, n_steps, s.splits, c, slot_bytes);
+    s.us = full_us + split_cost(rem, n_steps, s.splits, cut, slot_bytes);
     return s;
+}
+SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
+    const int mode = mode_of(d), n_tiles = n_tiles_of(d);
+    const double dim = 0.5 * (d->d_qk + d->d_v);
+    if (mode != MODE_FWD || is_wide(d)) {                          // a barrier step is 32 keys
+        const int m = mode == MODE_JVP_Q ? 0 : 1;
+        const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
+        return plan_shape(d, room, 0, kBlockM, n_tiles, StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+    }
+    SplitPlan best;
+    double best_us = 0.0;
+    for (int i = 0; i < kNumSymShapes; ++i) {                      // 64 keys
+        const SymShape& w = kSymShapes[i];
+        const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
+        const SplitPlan s = plan_shape(d, room, i, 32 * w.rg, (n_tiles + 1) / 2, c, c);
+        if (i > 0 && s.n_pairs > kNumCUs) continue;
+        // (a cut has to come out a twentieth better than no cut, of another shape as well: so what the two-stage run takes, which
+        // never cuts, is what the one-call form takes wherever that does not cut either)
+        const double us = s.splits > 1 ? s.us : 0.95 * s.us;
+        if (i == 0 || us < best_us) { best = s; best_us = us; }
+    }
+    return best;
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
@@ -1747,8 +1890,8 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
     if (!device_is_whole_mi355x()) return COSMOS_ATTN_WRONG_DEVICE;
     const int mode = mode_of(d);
     if (is_wide(d)) return run_wide(d, workspace, stream);
-    attn_kernel_t fn = d->dtype == COSMOS_ATTN_BF16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode)
-                                                    : pick_dqk<_Float16>(d->d_qk, d->d_v, mode);
+    attn_kernel_t fn = d->dtype == COSMOS_ATTN_BF16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode, sp.shape)
+                                                    : pick_dqk<_Float16>(d->d_qk, d->d_v, mode, sp.shape);
     if (!fn) return COSMOS_ATTN_UNSUPPORTED;
     AttnParams ap;
     ap.q = d->q; ap.tq = d->tq;
@@ -1774,7 +1917,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
             return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
         }
     }
-    const size_t lds = lds_bytes_of(d);
+    const size_t lds = lds_bytes_of(d, sp.shape);
     if (!allow_lds((const void*)fn, lds)) return COSMOS_ATTN_LAUNCH_FAILED;
     ap.n_qt = sp.n_qt; ap.n_full = sp.n_full; ap.n_rem = sp.n_rem; ap.splits = sp.splits;
     ap.part_acc = nullptr; ap.part_stat = nullptr;
@@ -1783,7 +1926,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
         ap.part_stat = (float4*)((char*)workspace + image_bytes + partial_acc_bytes(d, sp));
     }
     const int64_t blocks = (int64_t)sp.n_full + (int64_t)sp.n_rem * sp.splits;
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymWaves : kAttnThreads), lds, (hipStream_t)stream, ap);
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymShapes[sp.shape].rg * kSymShapes[sp.shape].kg : kAttnThreads), lds, (hipStream_t)stream, ap);
     if (hipGetLastError() != hipSuccess) return COSMOS_ATTN_LAUNCH_FAILED;
     if (sp.splits > 1) {
         const int rows_per_block = 256 / (d->d_v / 4);

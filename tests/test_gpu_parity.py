@@ -108,7 +108,7 @@ def test_many_workgroups_rotated_sweeps(pkg, oracle, gpu):
     run_case(pkg, oracle, gpu, (1, 8, 1024, 64), (1, 8, 700, 64), seed=12, tangents="q")
 
 
-# ------------------------------------------------------------------ forward only (its own kernel: 384-row workgroups)
+# ------------------------------------------------------------------ forward only (its own kernel: 128-, 256- or 384-row workgroups)
 @pytest.mark.parametrize("Lq,Lkv", [(1, 1), (50, 37), (383, 65), (385, 64), (129, 1), (5, 300), (800, 96)])
 def test_forward_only_ragged(pkg, oracle, gpu, Lq, Lkv):
     run_case(pkg, oracle, gpu, (1, 2, Lq, 128), (1, 2, Lkv, 128), seed=Lq + Lkv, tangents="none")
@@ -166,6 +166,41 @@ def test_forward_only_key_range_split(pkg, oracle, gpu, shape_q, Lkv, ranges):
     # same inputs, same plan: bitwise repeatable
     o_again, _, lse_again = pkg.fwd_jvp(q, k, v)
     assert torch.equal(o_again, o_ref) and torch.equal(lse_again, lse_ref)
+
+
+@pytest.mark.parametrize("shape_q,Lkv,dtype", [
+    ((2, 8, 255, 128), 1, torch.bfloat16),         # 128 rows x 2 key groups: the second has no key at all,
+    ((2, 8, 255, 128), 33, torch.float16),         # one key,
+    ((1, 2, 129, 128), 64, torch.bfloat16),        # as many as the first,
+    ((1, 2, 128, 128), 97, torch.float16),         # one tile less,
+    ((1, 3, 31, 16), 65, torch.bfloat16),          # a masked tile at a sweep's end; the smallest head dim
+    ((1, 40, 993, 128), 1000, torch.bfloat16),     # 256 rows
+    ((1, 40, 1000, 128), 65, torch.float16),
+    ((2, 20, 770, 64), 300, torch.bfloat16),
+    ((1, 40, 1560, 128), 700, torch.bfloat16),     # 384 rows
+])
+def test_forward_only_workgroup_shapes(pkg, oracle, gpu, stream_override, shape_q, Lkv, dtype):
+    """Calls for each of the three workgroup shapes of the forward-only kernel, at the edges of its key groups."""
+    stream_override(chunk=1)                       # never the query-streaming kernel
+    run_case(pkg, oracle, gpu, shape_q, (*shape_q[:2], Lkv, shape_q[3]), seed=Lkv, dtype=dtype, tangents="none")
+
+
+@pytest.mark.parametrize("order", ["rising", "falling", "spike"])
+@pytest.mark.parametrize("shape_q,Lkv,dtype", [((1, 2, 300, 128), 333, torch.bfloat16), ((1, 2, 129, 32), 333, torch.float16),
+                                               ((1, 40, 993, 128), 200, torch.bfloat16)])
+def test_forward_only_scores_that_move_the_max(pkg, oracle, gpu, stream_override, order, shape_q, Lkv, dtype):
+    """Scores that outgrow the running max by far more than its slack, in tile after tile, in one late key, or not at all."""
+    stream_override(chunk=1)
+    B, H, Lq, d = shape_q
+    q, k, v, _, _, _ = oracle.make_inputs(shape_q, (B, H, Lkv, d), seed=Lkv + d, dtype=dtype)
+    top = {"rising": torch.linspace(-60, 60, Lkv), "falling": torch.linspace(60, -60, Lkv),
+           "spike": torch.where(torch.arange(Lkv) == Lkv - 3, 60.0, 0.0)}[order]      # scores: about those, the same for every query
+    q = (0.1 * q.float() + 1.0).to(dtype)
+    k = (0.1 * k.float() + (top * d ** -0.5).view(1, 1, Lkv, 1)).to(dtype)
+    o, _, lse = pkg.fwd_jvp(q.to(gpu), k.to(gpu), v.to(gpu))
+    o_ref, _, lse_ref = oracle.closed_form(q, k, v)
+    check(oracle, "o", o, o_ref)
+    assert oracle.error_metrics(lse.cpu(), lse_ref)[0] <= LSE_ABS * 4      # (log-sum-exp of 60: 4 bits fewer behind the point)
 
 
 @pytest.mark.parametrize("chunk", range(4))
