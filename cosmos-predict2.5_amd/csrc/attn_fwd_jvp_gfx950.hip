@@ -42,6 +42,7 @@
 //     head's K/V images and share them through the per-XCD L2s and the Infinity Cache; workgroups of
 //     one XCD start their (order-free) sweep a few tiles apart so they do not hit one L2 channel at once.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <stdint.h>
 #include <stddef.h>
 #include <stdlib.h>
@@ -1554,7 +1555,7 @@ typedef void (*attn_kernel_t)(const AttnParams);
 // as fast but at single sizes (16 heads 7040 x 1024: 8 x 1 87, 12 x 1 93; 40 heads 3520: 282, 298).
 struct SymShape { int rg, kg; double step_us[4], alone[4], range_us[4]; };
 constexpr SymShape kSymShapes[] = {
-    {12, 1, {1.09, 1.12, 1.55, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
+    {12, 1, {1.09, 1.12, 1.58, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
     {8, 1, {0.82, 0.85, 1.10, 1.73}, {1.0, 1.0, 0.94, 0.78}, {4.6, 5.1, 6.6, 10.6}},
     {4, 2, {0.45, 0.46, 0.60, 0.94}, {1.0, 1.0, 1.0, 0.99}, {4.1, 4.8, 6.0, 9.0}},
 };
@@ -1694,6 +1695,12 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     s.us = full_us + split_cost(rem, n_steps, s.splits, cut, slot_bytes);
     return s;
 }
+SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {     // forward only: a barrier step is 64 keys
+    const SymShape& w = kSymShapes[shape];
+    const double dim = 0.5 * (d->d_qk + d->d_v);
+    const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
+    return plan_shape(d, room, shape, 32 * w.rg, (n_tiles_of(d) + 1) / 2, c, c);
+}
 SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     const int mode = mode_of(d), n_tiles = n_tiles_of(d);
     const double dim = 0.5 * (d->d_qk + d->d_v);
@@ -1704,10 +1711,8 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     }
     SplitPlan best;
     double best_us = 0.0;
-    for (int i = 0; i < kNumSymShapes; ++i) {                      // 64 keys
-        const SymShape& w = kSymShapes[i];
-        const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
-        const SplitPlan s = plan_shape(d, room, i, 32 * w.rg, (n_tiles + 1) / 2, c, c);
+    for (int i = 0; i < kNumSymShapes; ++i) {
+        const SplitPlan s = plan_sym(d, room, i);
         if (i > 0 && s.n_pairs > kNumCUs) continue;
         // (a cut has to come out a twentieth better than no cut, of another shape as well: so what the two-stage run takes, which
         // never cuts, is what the one-call form takes wherever that does not cut either)
@@ -1715,6 +1720,12 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
         if (i == 0 || us < best_us) { best = s; best_us = us; }
     }
     return best;
+}
+// Room for partial results that a caller is asked for: what the chosen plan needs, and forward only no less than the 12 x 32-row workgroups'
+// does (the sizes that callers have planned with hold whichever shape is chosen).
+size_t planned_partial_bytes(const cosmos_attn_desc* d) {
+    const size_t chosen = partial_bytes(d, plan_split(d, kNoLimit));
+    return mode_of(d) == MODE_FWD && !is_wide(d) ? std::max(chosen, partial_bytes(d, plan_sym(d, kNoLimit, 0))) : chosen;
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
@@ -1822,7 +1833,7 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
 
 COSMOS_ATTN_API size_t cosmos_attn_workspace_bytes(const cosmos_attn_desc* d) {
     if (validate(d) != COSMOS_ATTN_OK) return 0;
-    return align256(tiles_bytes_of(d)) + partial_bytes(d, plan_split(d, kNoLimit));
+    return align256(tiles_bytes_of(d)) + planned_partial_bytes(d);
 }
 
 COSMOS_ATTN_API size_t cosmos_attn_packed_bytes(const cosmos_attn_desc* d) {
