@@ -163,6 +163,23 @@ class GatedResidualDesc(ctypes.Structure):
     ]
 
 
+class GatedResidualLnModulateDesc(ctypes.Structure):
+    """Mirror of ``struct cosmos_gated_residual_ln_modulate_desc``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32), ("dtype", ctypes.c_int32),
+        ("D", ctypes.c_int32), ("rows_per_group", ctypes.c_int32),
+        ("eps", ctypes.c_float), ("reserved", ctypes.c_int32),
+        ("rows", ctypes.c_int64),
+        ("x", ctypes.c_void_p), ("tx", ctypes.c_void_p), ("res", ctypes.c_void_p), ("tres", ctypes.c_void_p),
+        ("gate", ctypes.c_void_p), ("tgate", ctypes.c_void_p),
+        ("shift", ctypes.c_void_p), ("scale", ctypes.c_void_p),
+        ("tshift", ctypes.c_void_p), ("tscale", ctypes.c_void_p),
+        ("out", ctypes.c_void_p), ("tout", ctypes.c_void_p),
+        ("y", ctypes.c_void_p), ("ty", ctypes.c_void_p),
+    ]
+
+
 class GeluDesc(ctypes.Structure):
     """Mirror of ``struct cosmos_gelu_desc``."""
 
@@ -228,6 +245,7 @@ EXPORTS = {
     "cosmos_norm_rope_bwd": (ctypes.c_int, [ctypes.POINTER(NormRopeBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_ln_modulate": (ctypes.c_int, [ctypes.POINTER(LnModulateDesc), ctypes.c_void_p]),
     "cosmos_gated_residual": (ctypes.c_int, [ctypes.POINTER(GatedResidualDesc), ctypes.c_void_p]),
+    "cosmos_gated_residual_ln_modulate": (ctypes.c_int, [ctypes.POINTER(GatedResidualLnModulateDesc), ctypes.c_void_p]),
     "cosmos_ln_modulate_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(LnModulateBwdDesc)]),
     "cosmos_ln_modulate_bwd": (ctypes.c_int, [ctypes.POINTER(LnModulateBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_gated_residual_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(GatedResidualBwdDesc)]),

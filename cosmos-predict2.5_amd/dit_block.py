@@ -342,6 +342,15 @@ class Block(nn.Module):
         return y, ty
 
     @staticmethod
+    def _residual_modulate_jvp(norm_layer, x, tx, res, tres, gates, mod, tmod):
+        """The gated residual of the sub-layer before (``gates``: its modulation and tangent) and :meth:`_modulate_jvp` of it."""
+        (shift, scale, _), (tshift, tscale, _) = mod, tmod
+        y, ty = ops.stacked_pair(x.shape, x.dtype, x.device)
+        flat = lambda m: m.reshape(-1, m.shape[-1])
+        return ops.gated_residual_ln_modulate(x, res, flat(gates[0][2]), flat(shift), flat(scale), tx, tres, flat(gates[1][2]), flat(tshift),
+                                              flat(tscale), eps=norm_layer.eps, y=y, ty=ty)
+
+    @staticmethod
     def _gated_residual_jvp(x, tx, res, tres, mod, tmod):
         flat = lambda m: m.reshape(-1, m.shape[-1])
         return ops.gated_residual(x, res, flat(mod[2]), tx, tres, flat(tmod[2]))
@@ -387,13 +396,16 @@ class Block(nn.Module):
         for name, norm, sub, (shift, scale, gate) in zip(("self_attn", "cross_attn", "mlp"),
                                                          (self.layer_norm_self_attn, self.layer_norm_cross_attn, self.layer_norm_mlp),
                                                          (self.self_attn, self.cross_attn, self.mlp), self._modulations(emb, lora, x)):
-            n, _ = ops.ln_modulate(x, flat2(shift), flat2(scale), eps=norm.eps)
+            if name == "self_attn":
+                n, _ = ops.ln_modulate(x, flat2(shift), flat2(scale), eps=norm.eps)
+            else:
+                x, _, n, _ = ops.gated_residual_ln_modulate(x, r, r_gate, flat2(shift), flat2(scale), eps=norm.eps)
             if name == "mlp":
                 r = sub(n)
             else:
                 r = sub(n.reshape(B, T * H * W, D), None if name == "self_attn" else crossattn_emb, rope_emb=rope)
-            x, _ = ops.gated_residual(x, r.reshape(x.shape), flat2(gate))
-        return x
+            r, r_gate = r.reshape(x.shape), flat2(gate)
+        return ops.gated_residual(x, r, r_gate)[0]
 
     # ------------------------------------------------------------------ forward mode
     @torch.no_grad()
@@ -428,15 +440,13 @@ class Block(nn.Module):
         mod, tmod = modulation(0, self.adaln_modulation_self_attn)
         n, tn = self._modulate_jvp(self.layer_norm_self_attn, x, tx, mod, tmod)
         r, tr = self.self_attn.forward_jvp(flat(n), flat(tn), rope_emb=rope_emb_L_1_1_D)
-        x, tx = self._gated_residual_jvp(x, tx, vid(r), vid(tr), mod, tmod)
 
-        mod, tmod = modulation(1, self.adaln_modulation_cross_attn)
-        n, tn = self._modulate_jvp(self.layer_norm_cross_attn, x, tx, mod, tmod)
+        gates, (mod, tmod) = (mod, tmod), modulation(1, self.adaln_modulation_cross_attn)
+        x, tx, n, tn = self._residual_modulate_jvp(self.layer_norm_cross_attn, x, tx, vid(r), vid(tr), gates, mod, tmod)
         r, tr = self.cross_attn.forward_jvp(flat(n), flat(tn), crossattn_emb, None, rope_emb=rope_emb_L_1_1_D)
-        x, tx = self._gated_residual_jvp(x, tx, vid(r), vid(tr), mod, tmod)
 
-        mod, tmod = modulation(2, self.adaln_modulation_mlp)
-        n, tn = self._modulate_jvp(self.layer_norm_mlp, x, tx, mod, tmod)
+        gates, (mod, tmod) = (mod, tmod), modulation(2, self.adaln_modulation_mlp)
+        x, tx, n, tn = self._residual_modulate_jvp(self.layer_norm_mlp, x, tx, vid(r), vid(tr), gates, mod, tmod)
         r, tr = self.mlp.forward_jvp(n, tn)
         x, tx = self._gated_residual_jvp(x, tx, r, tr, mod, tmod)
         return x, tx

@@ -537,6 +537,41 @@ def gated_residual(x, res, gate, tx=None, tres=None, tgate=None, inplace: bool =
     return out, tout
 
 
+def gated_residual_ln_modulate(x, res, gate, shift, scale, tx=None, tres=None, tgate=None, tshift=None, tscale=None,
+                               eps: float = 1e-6, y=None, ty=None):
+    """:func:`gated_residual` and :func:`ln_modulate` of its result in one pass (two, where ``gate`` and ``shift`` have different
+    ``G``): ``(out, tout, y, ty)``.  ``y`` / ``ty``: optional preallocated outputs."""
+    _check_elementwise(x)
+    D = x.shape[-1]
+    if gate.numel() != shift.numel():
+        out, tout = gated_residual(x, res, gate, tx, tres, tgate)
+        return out, tout, *ln_modulate(out, shift, scale, tout, tshift, tscale, eps=eps, out=y, tout=ty)
+    assert res.shape == x.shape and res.dtype == x.dtype
+    x, res = _dense16(x), _dense16(res)
+    rows = x.numel() // D
+    vector = lambda m: None if m is None else _dense16(m.to(x.dtype)).reshape(-1, D)
+    gate, shift, scale = vector(gate), vector(shift), vector(scale)
+    assert gate.shape == shift.shape == scale.shape and rows % gate.shape[0] == 0
+    if tx is not None:
+        assert tres is not None and tx.shape == x.shape == tres.shape and tx.dtype == x.dtype == tres.dtype
+        tx, tres, tgate, tshift, tscale = _dense16(tx), _dense16(tres), vector(tgate), vector(tshift), vector(tscale)
+        assert all(t is None or t.shape == gate.shape for t in (tgate, tshift, tscale))
+    else:
+        tres = tgate = tshift = tscale = ty = None
+    out, tout = torch.empty_like(x), None if tx is None else torch.empty_like(x)
+    y = torch.empty_like(x) if y is None else y
+    ty = torch.empty_like(x) if ty is None and tx is not None else ty
+    assert y.is_contiguous() and y.shape == x.shape and (ty is None or (ty.is_contiguous() and ty.shape == x.shape))
+    d = _lib.GatedResidualLnModulateDesc()
+    d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[x.dtype]
+    d.D, d.rows_per_group, d.eps, d.reserved, d.rows = D, rows // gate.shape[0], float(eps), 0, rows
+    d.x, d.tx, d.res, d.tres, d.gate, d.tgate = _ptr(x), _ptr(tx), _ptr(res), _ptr(tres), _ptr(gate), _ptr(tgate)
+    d.shift, d.scale, d.tshift, d.tscale = _ptr(shift), _ptr(scale), _ptr(tshift), _ptr(tscale)
+    d.out, d.tout, d.y, d.ty = _ptr(out), _ptr(tout), _ptr(y), _ptr(ty)
+    _launch("cosmos_gated_residual_ln_modulate", d, x.device)
+    return out, tout, y, ty
+
+
 def _launch_with_workspace(fn_name: str, desc, device) -> None:
     lib = _lib.load_library()
     fn, n = getattr(lib, fn_name), getattr(lib, fn_name + "_workspace_bytes")(ctypes.byref(desc))

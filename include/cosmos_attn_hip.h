@@ -267,6 +267,19 @@ typedef struct cosmos_gated_residual_desc {
     void *out, *tout;
 } cosmos_gated_residual_desc;
 
+/* Both, where the gated residual is what the LayerNorm reads:  out = x + gate res,  y = LayerNorm(out) (1 + scale) + shift. */
+typedef struct cosmos_gated_residual_ln_modulate_desc {
+    int32_t abi_version, dtype;
+    int32_t D, rows_per_group;         /* D % 8 == 0, D <= 8192; rows % rows_per_group == 0 */
+    float eps;
+    int32_t reserved;
+    int64_t rows;
+    const void *x, *tx, *res, *tres;   /* [rows, D]; tx, tres, tout, ty NULL together */
+    const void *gate, *tgate;          /* [rows / rows_per_group, D], as shift, scale, tshift, tscale; the tangents may be NULL */
+    const void *shift, *scale, *tshift, *tscale;
+    void *out, *tout, *y, *ty;         /* [rows, D] */
+} cosmos_gated_residual_ln_modulate_desc;
+
 typedef struct cosmos_gelu_desc {
     int32_t abi_version, dtype;
     int64_t n;                         /* elements, n % 8 == 0 */
@@ -276,6 +289,7 @@ typedef struct cosmos_gelu_desc {
 
 COSMOS_ATTN_API int cosmos_ln_modulate(const cosmos_ln_modulate_desc *desc, void *stream);
 COSMOS_ATTN_API int cosmos_gated_residual(const cosmos_gated_residual_desc *desc, void *stream);
+COSMOS_ATTN_API int cosmos_gated_residual_ln_modulate(const cosmos_gated_residual_ln_modulate_desc *desc, void *stream);
 COSMOS_ATTN_API int cosmos_gelu(const cosmos_gelu_desc *desc, void *stream);
 
 /*

@@ -101,6 +101,34 @@ def test_gated_residual(pkg, block_oracle, gpu, dtype, rows, D, rpg):
     check("tout (fixed gate, in place)", t3, twant3, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,D,rpg", [(1, 8, 1), (30, 264, 5), (9, 520, 3), (64, 2048, 16), (7, 5120, 7), (6, 8192, 2)])
+def test_gated_residual_ln_modulate(pkg, block_oracle, gpu, dtype, rows, D, rpg):
+    """One pass against the two it stands for, and the LayerNorm against the oracle of the residual that was stored."""
+    g = torch.Generator().manual_seed(rows + D)
+    x, res, tx, tres = (rnd(g, dtype, rows, D) for _ in range(4))
+    gate, sc, sh, tgate, tsc, tsh = (rnd(g, dtype, rows // rpg, D, std=s) for s in (1.0, 0.3, 1.0, 0.3, 0.1, 0.3))
+    d = lambda *ts: [t.to(gpu) for t in ts]
+    for moving in (None, False, True):       # values only; a tangent with a modulation that does not move; one that does
+        t, mt = ((tx, tres) if moving is not None else (None, None)), ((tgate, tsh, tsc) if moving else (None, None, None))
+        dt, dmt = [None if v is None else v.to(gpu) for v in t], [None if v is None else v.to(gpu) for v in mt]
+        (dx, dres, dg, dsh, dsc) = d(x, res, gate, sh, sc)
+        out, tout, y, ty = pkg.ops.gated_residual_ln_modulate(dx, dres, dg, dsh, dsc, *dt, *dmt)
+        ref = pkg.gated_residual(dx, dres, dg, *dt, dmt[0])
+        assert torch.equal(out, ref[0]) and (tout is None) == (ref[1] is None) == (moving is None)
+        assert torch.equal(dx.cpu(), x) and (tout is None or torch.equal(tout, ref[1]))
+        want, twant = block_oracle.ln_modulate_torch(out.cpu(), sh, sc, None if tout is None else tout.cpu(), mt[1], mt[2], rows_per_group=rpg)
+        check(f"y ({moving})", y, want, dtype)
+        if moving is None:
+            assert ty is None
+        elif rows * D > 8:                    # (rows of 8 elements: the tangent of n is a difference of near-equal terms)
+            check(f"ty ({moving})", ty, twant, dtype)
+    # modulations of different groups go through the two passes
+    out, _, y, _ = pkg.ops.gated_residual_ln_modulate(dx, dres, dg[:1], dsh, dsc)
+    ref, _ = pkg.gated_residual(dx, dres, dg[:1])
+    assert torch.equal(out, ref) and torch.equal(y, pkg.ln_modulate(ref, dsh, dsc)[0])
+
+
 @pytest.mark.parametrize("rows,rpg,D", [(24, 4, 8), (17, 17, 264), (66, 33, 2048), (8, 1, 2056), (90, 45, 4104), (40, 40, 5120), (21, 21, 8192),
                                         (9000, 4500, 64)])      # (the last: rows enough for runs longer than the shortest)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -344,6 +344,22 @@ def test_block_elementwise_desc_layouts_and_status_codes(pkg):
         pkg.gelu(torch.zeros(8, dtype=torch.bfloat16))
 
 
+def test_gated_residual_ln_modulate_desc_layout_and_status_codes(pkg):
+    L, lib = pkg._lib, pkg._lib.load_library()
+    assert ctypes.sizeof(L.GatedResidualLnModulateDesc) == 24 + 8 + 14 * 8 and L.GatedResidualLnModulateDesc.x.offset == 32
+    P = 0x7F0000000000   # never dereferenced: every case below is rejected on the host
+    for over, want in [(dict(abi_version=1), L.ST_BAD_ARG), (dict(rows=0), L.ST_BAD_ARG), (dict(gate=None), L.ST_BAD_ARG), (dict(out=None), L.ST_BAD_ARG),
+                       (dict(eps=-1.0), L.ST_BAD_ARG), (dict(tx=P), L.ST_BAD_ARG), (dict(tx=P, tres=P, tout=P), L.ST_BAD_ARG), (dict(tgate=P), L.ST_BAD_ARG),
+                       (dict(dtype=7), L.ST_UNSUPPORTED), (dict(D=8200), L.ST_UNSUPPORTED), (dict(D=252), L.ST_BAD_SHAPE),
+                       (dict(rows_per_group=5), L.ST_BAD_SHAPE), (dict(res=P + 2), L.ST_BAD_STRIDE), (dict(out=P + 8), L.ST_BAD_STRIDE)]:
+        d = L.GatedResidualLnModulateDesc()
+        d.abi_version, d.dtype, d.D, d.rows_per_group, d.eps, d.rows = L.ABI_VERSION, L.DTYPE_BF16, 256, 4, 1e-6, 16
+        d.x, d.res, d.gate, d.shift, d.scale, d.out, d.y = (P + 0x10000 * i for i in range(7))
+        for k, v in over.items():
+            setattr(d, k, v)
+        assert lib.cosmos_gated_residual_ln_modulate(ctypes.byref(d), None) == want, over
+
+
 def test_block_reverse_mode_desc_layouts_and_status_codes(pkg):
     L, lib = pkg._lib, pkg._lib.load_library()
     assert ctypes.sizeof(L.LnModulateBwdDesc) == 24 + 8 + 7 * 8 and L.LnModulateBwdDesc.x.offset == 32
