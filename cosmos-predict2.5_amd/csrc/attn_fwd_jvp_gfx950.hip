@@ -1673,6 +1673,10 @@ size_t partial_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
 }
 // `room`: bytes there are for partial results (0: never split)
 constexpr size_t kNoLimit = ~(size_t)0;
+// key ranges of equal work only, not too short; not for head dim 256
+bool may_cut(const cosmos_attn_desc* d, int n_steps) {
+    return n_steps >= 2 * kMinStepsPerSplit && !d->causal && !d->key_lens && !is_wide(d);
+}
 // The best cut for workgroups of block_m rows and n_steps barrier steps: `whole` is what a pair that is not cut costs, `cut` one of
 // which S ranges may be made.
 SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int block_m, int n_steps, StepCost whole, StepCost cut) {
@@ -1685,7 +1689,7 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     const int rem = s.n_pairs % kNumCUs;
     const double full_us = rounds_cost(s.n_pairs - rem, n_steps, whole);
     s.us = full_us + rounds_cost(rem, n_steps, whole);
-    if (d->causal || d->key_lens || is_wide(d)) return s;          // key ranges of equal work only; not for head dim 256
+    if (!may_cut(d, n_steps)) return s;
     const double slot_bytes = (double)s.block_m * (d->d_v * (mode_of(d) == MODE_FWD ? 1 : 2) * sizeof(float) + sizeof(float4));
     const SplitPlan uncut = s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
@@ -1701,7 +1705,8 @@ SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {     // f
     const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
     return plan_shape(d, room, shape, 32 * w.rg, (n_tiles_of(d) + 1) / 2, c, c);
 }
-SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
+// `large`, where given: the 12 x 32-row plan of a forward-only call
+SplitPlan plan_split(const cosmos_attn_desc* d, size_t room, SplitPlan* large = nullptr) {
     const int mode = mode_of(d), n_tiles = n_tiles_of(d);
     const double dim = 0.5 * (d->d_qk + d->d_v);
     if (mode != MODE_FWD || is_wide(d)) {                          // a barrier step is 32 keys
@@ -1712,8 +1717,9 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     SplitPlan best;
     double best_us = 0.0;
     for (int i = 0; i < kNumSymShapes; ++i) {
+        if (i > 0 && (int64_t)((d->Lq + 32 * kSymShapes[i].rg - 1) / (32 * kSymShapes[i].rg)) * d->B * d->H > kNumCUs) continue;
         const SplitPlan s = plan_sym(d, room, i);
-        if (i > 0 && s.n_pairs > kNumCUs) continue;
+        if (i == 0 && large) *large = s;
         // (a cut has to come out a twentieth better than no cut, of another shape as well: so what the two-stage run takes, which
         // never cuts, is what the one-call form takes wherever that does not cut either)
         const double us = s.splits > 1 ? s.us : 0.95 * s.us;
@@ -1724,8 +1730,11 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
 // Room for partial results that a caller is asked for: what the chosen plan needs, and forward only no less than the 12 x 32-row workgroups'
 // does (the sizes that callers have planned with hold whichever shape is chosen).
 size_t planned_partial_bytes(const cosmos_attn_desc* d) {
-    const size_t chosen = partial_bytes(d, plan_split(d, kNoLimit));
-    return mode_of(d) == MODE_FWD && !is_wide(d) ? std::max(chosen, partial_bytes(d, plan_sym(d, kNoLimit, 0))) : chosen;
+    const bool fwd = mode_of(d) == MODE_FWD;
+    if (!may_cut(d, fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d))) return 0;
+    SplitPlan large;
+    const size_t chosen = partial_bytes(d, plan_split(d, kNoLimit, &large));
+    return fwd ? std::max(chosen, partial_bytes(d, large)) : chosen;
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
