@@ -469,6 +469,12 @@ def _check_elementwise(x: torch.Tensor) -> None:
         raise NotImplementedError(f"dtype={x.dtype} is not supported (bf16 / fp16)")
 
 
+def _check_outputs(x: torch.Tensor, *outs: Optional[torch.Tensor]) -> None:
+    """Outputs that a caller may have preallocated: the kernels write ``x.numel()`` elements of ``x``'s type there."""
+    for t in outs:
+        assert t is None or (t.is_contiguous() and t.shape == x.shape and t.dtype == x.dtype and t.device == x.device)
+
+
 def _launch(fn_name: str, desc, device) -> None:
     fn = getattr(_lib.load_library(), fn_name)
     _lib.raise_for_status(_on_device(device, lambda stream: fn(ctypes.byref(desc), stream)))
@@ -497,7 +503,7 @@ def ln_modulate(x, shift, scale, tx=None, tshift=None, tscale=None, eps: float =
         assert (tshift is None or tshift.shape == shift.shape) and (tscale is None or tscale.shape == shift.shape)
     y = torch.empty_like(x) if out is None else out
     ty = (torch.empty_like(x) if tout is None else tout) if tx is not None else None
-    assert y.is_contiguous() and y.shape == x.shape and (ty is None or (ty.is_contiguous() and ty.shape == x.shape))
+    _check_outputs(x, y, ty)
     d = _lib.LnModulateDesc()
     d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[x.dtype]
     d.D, d.rows_per_group, d.eps, d.reserved, d.rows = D, rows // shift.shape[0], float(eps), 0, rows
@@ -561,7 +567,7 @@ def gated_residual_ln_modulate(x, res, gate, shift, scale, tx=None, tres=None, t
     out, tout = torch.empty_like(x), None if tx is None else torch.empty_like(x)
     y = torch.empty_like(x) if y is None else y
     ty = torch.empty_like(x) if ty is None and tx is not None else ty
-    assert y.is_contiguous() and y.shape == x.shape and (ty is None or (ty.is_contiguous() and ty.shape == x.shape))
+    _check_outputs(x, y, ty)
     d = _lib.GatedResidualLnModulateDesc()
     d.abi_version, d.dtype = _lib.ABI_VERSION, _DTYPES[x.dtype]
     d.D, d.rows_per_group, d.eps, d.reserved, d.rows = D, rows // gate.shape[0], float(eps), 0, rows

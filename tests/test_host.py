@@ -360,6 +360,28 @@ def test_gated_residual_ln_modulate_desc_layout_and_status_codes(pkg):
         assert lib.cosmos_gated_residual_ln_modulate(ctypes.byref(d), None) == want, over
 
 
+@pytest.mark.parametrize("wrong", [dict(dtype=torch.int8), dict(dtype=torch.float32), dict(dtype=torch.float16), dict(device="meta")])
+@pytest.mark.parametrize("which", ["y", "ty"])
+def test_given_outputs_of_another_type_or_device_are_refused(pkg, monkeypatch, wrong, which):
+    """A preallocated output is written as x's type on x's device: of a narrower type, the kernel would write past its end."""
+    launched = []
+    monkeypatch.setattr(pkg.ops, "_check_elementwise", lambda x: None)      # (nothing is launched: CPU tensors do)
+    monkeypatch.setattr(pkg.ops, "_launch", lambda name, desc, device: launched.append(name))
+    x, res, tx, tres = (torch.zeros(4, 16, dtype=torch.bfloat16) for _ in range(4))
+    m = torch.zeros(2, 16, dtype=torch.bfloat16)
+    good, bad = torch.empty_like(x), torch.empty(4, 16, **{"dtype": x.dtype, **wrong})
+    out = {"y": good, "ty": good.clone(), which: bad}
+    with pytest.raises(AssertionError):
+        pkg.ops.gated_residual_ln_modulate(x, res, m, m, m, tx, tres, **out)
+    with pytest.raises(AssertionError):
+        pkg.ops.ln_modulate(x, m, m, tx, out=out["y"], tout=out["ty"])
+    assert not launched
+    out[which] = good.clone()
+    pkg.ops.gated_residual_ln_modulate(x, res, m, m, m, tx, tres, **out)
+    pkg.ops.ln_modulate(x, m, m, tx, out=out["y"], tout=out["ty"])
+    assert launched == ["cosmos_gated_residual_ln_modulate", "cosmos_ln_modulate"]
+
+
 def test_block_reverse_mode_desc_layouts_and_status_codes(pkg):
     L, lib = pkg._lib, pkg._lib.load_library()
     assert ctypes.sizeof(L.LnModulateBwdDesc) == 24 + 8 + 7 * 8 and L.LnModulateBwdDesc.x.offset == 32
