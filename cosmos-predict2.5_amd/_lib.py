@@ -54,6 +54,12 @@ class AttnDesc(ctypes.Structure):
     ]
 
 
+class AttnPlan(ctypes.Structure):
+    """Mirror of ``struct cosmos_attn_plan``."""
+
+    _fields_ = [(name, ctypes.c_int32) for name in ("streaming_workgroups", "query_rows", "key_groups", "whole_pairs", "cut_pairs", "key_ranges")]
+
+
 class AttnBwdDesc(ctypes.Structure):
     """Mirror of ``struct cosmos_attn_bwd_desc``."""
 
@@ -232,6 +238,7 @@ EXPORTS = {
     "cosmos_attn_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "cosmos_attn_set_stream_override": (None, [ctypes.c_int, ctypes.c_int]),
     "cosmos_attn_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnDesc)]),
+    "cosmos_attn_launch_plan": (ctypes.c_int, [ctypes.POINTER(AttnDesc), ctypes.c_size_t, ctypes.POINTER(AttnPlan)]),
     "cosmos_attn_fwd_jvp": (ctypes.c_int, [ctypes.POINTER(AttnDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_attn_static_scratch_bytes": (ctypes.c_size_t, []),
     "cosmos_attn_fwd_jvp_static": (ctypes.c_int, [ctypes.POINTER(AttnDesc), ctypes.c_void_p]),

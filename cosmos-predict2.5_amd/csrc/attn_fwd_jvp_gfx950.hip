@@ -42,7 +42,6 @@
 //     head's K/V images and share them through the per-XCD L2s and the Infinity Cache; workgroups of
 //     one XCD start their (order-free) sweep a few tiles apart so they do not hit one L2 channel at once.
 #include <hip/hip_runtime.h>
-#include <algorithm>
 #include <stdint.h>
 #include <stddef.h>
 #include <stdlib.h>
@@ -1705,8 +1704,7 @@ SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {     // f
     const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
     return plan_shape(d, room, shape, 32 * w.rg, (n_tiles_of(d) + 1) / 2, c, c);
 }
-// `large`, where given: the 12 x 32-row plan of a forward-only call
-SplitPlan plan_split(const cosmos_attn_desc* d, size_t room, SplitPlan* large = nullptr) {
+SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     const int mode = mode_of(d), n_tiles = n_tiles_of(d);
     const double dim = 0.5 * (d->d_qk + d->d_v);
     if (mode != MODE_FWD || is_wide(d)) {                          // a barrier step is 32 keys
@@ -1719,7 +1717,6 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room, SplitPlan* large = 
     for (int i = 0; i < kNumSymShapes; ++i) {
         if (i > 0 && (int64_t)((d->Lq + 32 * kSymShapes[i].rg - 1) / (32 * kSymShapes[i].rg)) * d->B * d->H > kNumCUs) continue;
         const SplitPlan s = plan_sym(d, room, i);
-        if (i == 0 && large) *large = s;
         // (a cut has to come out a twentieth better than no cut, of another shape as well: so what the two-stage run takes, which
         // never cuts, is what the one-call form takes wherever that does not cut either)
         const double us = s.splits > 1 ? s.us : 0.95 * s.us;
@@ -1727,14 +1724,10 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room, SplitPlan* large = 
     }
     return best;
 }
-// Room for partial results that a caller is asked for: what the chosen plan needs, and forward only no less than the 12 x 32-row workgroups'
-// does (the sizes that callers have planned with hold whichever shape is chosen).
+// Room for partial results that a caller is asked for: what the plan that runs needs (it stays the best of the plans that fit that room)
 size_t planned_partial_bytes(const cosmos_attn_desc* d) {
-    const bool fwd = mode_of(d) == MODE_FWD;
-    if (!may_cut(d, fwd ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d))) return 0;
-    SplitPlan large;
-    const size_t chosen = partial_bytes(d, plan_split(d, kNoLimit, &large));
-    return fwd ? std::max(chosen, partial_bytes(d, large)) : chosen;
+    if (!may_cut(d, mode_of(d) == MODE_FWD ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d))) return 0;      // (not planned only to see that)
+    return partial_bytes(d, plan_split(d, kNoLimit));
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
 // line of (query block, head) pairs into pieces of equal weight itself, so the launch is a small multiple of the number
@@ -1848,6 +1841,30 @@ COSMOS_ATTN_API size_t cosmos_attn_workspace_bytes(const cosmos_attn_desc* d) {
 COSMOS_ATTN_API size_t cosmos_attn_packed_bytes(const cosmos_attn_desc* d) {
     if (validate(d) != COSMOS_ATTN_OK) return 0;
     return align256(tiles_bytes_of(d));
+}
+
+COSMOS_ATTN_API int cosmos_attn_launch_plan(const cosmos_attn_desc* d, size_t workspace_bytes, cosmos_attn_plan* plan) {
+    const int st = validate(d);
+    if (st != COSMOS_ATTN_OK) return st;
+    if (!plan) return COSMOS_ATTN_BAD_ARG;
+    const size_t image_bytes = align256(tiles_bytes_of(d));
+    if (workspace_bytes < image_bytes) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
+    *plan = cosmos_attn_plan{};
+    if (is_wide(d)) {
+        plan->query_rows = 32; plan->key_groups = 1; plan->key_ranges = 1;
+        plan->whole_pairs = ((d->Lq + 31) / 32) * d->B * d->H;
+        return COSMOS_ATTN_OK;
+    }
+    const SplitPlan s = plan_split(d, workspace_bytes - image_bytes);
+    plan->streaming_workgroups = stream_groups_of(d, s);
+    plan->query_rows = s.block_m;
+    plan->key_groups = mode_of(d) == MODE_FWD && plan->streaming_workgroups == 0 ? kSymShapes[s.shape].kg : 1;
+    plan->whole_pairs = s.n_full; plan->cut_pairs = s.n_rem; plan->key_ranges = s.splits;
+    if (plan->streaming_workgroups) {
+        plan->query_rows = kBlockM; plan->key_ranges = 1; plan->cut_pairs = 0;
+        plan->whole_pairs = ((d->Lq + kBlockM - 1) / kBlockM) * d->B * d->H;
+    }
+    return COSMOS_ATTN_OK;
 }
 
 COSMOS_ATTN_API int cosmos_attn_pack_kv(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {

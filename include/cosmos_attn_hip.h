@@ -104,6 +104,18 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
 COSMOS_ATTN_API size_t cosmos_attn_workspace_bytes(const cosmos_attn_desc *desc);
 
 /*
+ * How a call with a workspace of `workspace_bytes` would be dealt out (SIZE_MAX: cosmos_attn_fwd_jvp; cosmos_attn_packed_bytes():
+ * cosmos_attn_run).  Values only, nothing is launched and no device is looked at; for tests and tuning.  A status code.
+ */
+typedef struct cosmos_attn_plan {
+    int32_t streaming_workgroups;      /* > 0: that many workgroups stream the query blocks (short key sequences); 0: as below */
+    int32_t query_rows, key_groups;    /* of a workgroup */
+    int32_t whole_pairs;               /* (query block, head) pairs that are one workgroup each */
+    int32_t cut_pairs, key_ranges;     /* pairs cut into key_ranges workgroups each, merged by a second kernel; key_ranges 1: none */
+} cosmos_attn_plan;
+COSMOS_ATTN_API int cosmos_attn_launch_plan(const cosmos_attn_desc *desc, size_t workspace_bytes, cosmos_attn_plan *plan);
+
+/*
  * Forward + JVP:  o = softmax(q k^T s) v ;  to = d/de o(q+e tq, k+e tk, v+e tv)|_{e=0} ;  lse.
  * Forward only when all tangent pointers are NULL.
  * Replaces `_attention.forward` -> `_attn_fwd[grid](...)`  (JVP:436-502, JVP:176-378) and, forward only,

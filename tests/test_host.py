@@ -88,42 +88,83 @@ def test_status_codes_for_bad_descriptors(pkg):
     assert L.status_string(0) == "ok"
 
 
-@pytest.mark.parametrize("H,L,tangents,ranges", [
-    (16, 1560, True, 1),      # 208 pairs in one round: a cut would only add partial results
-    (16, 2600, True, 3),      # 336 pairs: 80 of a second round, 3 ranges each
-    (16, 7040, True, 2),      # 880 pairs: 112 of a fourth round, 2 ranges each
-    (2, 2048, True, 6),       # 32 pairs, 64 steps: six ranges are as fast as the eight that fill the chip, with less to merge
-    (16, 3520, False, 1),     # forward only, 384 rows per pair: 160 pairs in one round
-    (16, 2000, False, 2),     # 96 pairs
-    (16, 37440, False, 8),    # 1568 pairs: 32 of a seventh round, 8 ranges each
-    (1, 100, False, 1),       # 2 steps: too short to cut
+def plan_of(pkg, D, workspace_bytes=ctypes.c_size_t(-1).value):
+    """(query rows, key groups, whole pairs, cut pairs, key ranges) of the launch; "streamed" where the query blocks are streamed."""
+    plan = pkg._lib.AttnPlan()
+    assert pkg._lib.load_library().cosmos_attn_launch_plan(ctypes.byref(D), workspace_bytes, ctypes.byref(plan)) == pkg._lib.ST_OK
+    if plan.streaming_workgroups:
+        return "streamed"
+    return plan.query_rows, plan.key_groups, plan.whole_pairs, plan.cut_pairs, plan.key_ranges
+
+
+def partial_result_bytes(plan, d_v, tangents):
+    """What the key ranges of a plan leave: fp32 accumulators (two with tangents), then 16 bytes of statistics per row."""
+    rows, _, _, cut, ranges = plan
+    up = lambda n: (n + 255) // 256 * 256
+    return 0 if ranges == 1 else up(cut * ranges * rows * d_v * (2 if tangents else 1) * 4) + up(cut * ranges * rows * 16)
+
+
+@pytest.mark.parametrize("H,L,tangents,plan", [
+    (16, 1560, True, (128, 1, 208, 0, 1)),      # 208 pairs in one round: a cut would only add partial results
+    (16, 2600, True, (128, 1, 256, 80, 3)),     # 336 pairs: 80 of a second round, 3 ranges each
+    (16, 7040, True, (128, 1, 768, 112, 2)),    # 880 pairs: 112 of a fourth round, 2 ranges each
+    (2, 2048, True, (128, 1, 0, 32, 6)),        # 32 pairs, 64 steps: six ranges are as fast as the eight that fill the chip, with less to merge
+    (16, 3520, False, (256, 1, 224, 0, 1)),     # forward only: 224 pairs of 256 rows in one round, of 384 rows 160
+    (16, 2000, False, (128, 2, 256, 0, 1)),     # a whole round of pairs of 128 rows and 2 key groups
+    (16, 37440, False, (384, 1, 1536, 32, 8)),  # 1568 pairs: 32 of a seventh round, 8 ranges each
+    (4, 4623, False, (256, 1, 0, 76, 3)),       # 76 pairs, 73 steps
+    (2, 1000, False, (128, 2, 0, 16, 4)),       # 16 pairs, 16 steps
+    (1, 100, False, (128, 2, 1, 0, 1)),         # 2 steps: too short to cut
 ])
-def test_key_range_plan(pkg, H, L, tangents, ranges):
-    """How many key ranges the pairs of a partly filled last round are cut into, read off the workspace for their partial results."""
+def test_key_range_plan(pkg, H, L, tangents, plan):
+    """What workgroups a call is dealt out to, how many key ranges the pairs of a partly filled last round are cut into, and that the
+    workspace asked for has room for their partial results and nothing else."""
     lib = pkg._lib.load_library()
     t = 0x8000000 if tangents else None
     D = good_desc(pkg, B=1, H=H, Lq=L, Lkv=L, d_v=128, tq=t, tk=t, tv=t, to=t)
-    block = 128 if tangents else 384
-    rem = (L + block - 1) // block * H % 256
+    assert plan_of(pkg, D) == plan
     extra = lib.cosmos_attn_workspace_bytes(ctypes.byref(D)) - lib.cosmos_attn_packed_bytes(ctypes.byref(D))
-    assert extra == (0 if ranges == 1 else rem * ranges * block * (128 * (2 if tangents else 1) * 4 + 16))
+    assert extra == partial_result_bytes(plan, 128, tangents)
 
 
-@pytest.mark.parametrize("d,H,L,ranges", [
-    (16, 16, 700, 2),         # forward only: 32 pairs of 11 steps
-    (16, 40, 1100, 2),        # 120 pairs
-    (32, 40, 9000, 4),        # 960 pairs: 192 of a fourth round
-    (64, 40, 1100, 2),        # 120 pairs
-    (64, 16, 5000, 1),        # 224 pairs in one round
+@pytest.mark.parametrize("d,H,L,plan", [
+    (16, 16, 700, (128, 2, 96, 0, 1)),          # forward only
+    (16, 40, 1100, (256, 1, 200, 0, 1)),
+    (32, 40, 9000, (384, 1, 768, 192, 4)),      # 960 pairs: 192 of a fourth round
+    (32, 1, 4000, (128, 2, 0, 32, 8)),          # 32 pairs, 63 steps
+    (64, 16, 5000, (384, 1, 224, 0, 1)),        # 224 pairs in one round
 ])
-def test_key_range_plan_below_head_dim_128(pkg, d, H, L, ranges):
+def test_key_range_plan_below_head_dim_128(pkg, d, H, L, plan):
     """As above, forward only: a step costs more than its share of matrix instructions there, so that more calls are worth cutting."""
     lib = pkg._lib.load_library()
-    D = good_desc(pkg, B=1, H=H, Lq=L, Lkv=L, d_qk=d, d_v=d, tq=None, tk=None, tv=None, to=None)
-    rem = (L + 383) // 384 * H % 256
+    D = good_desc(pkg, B=1, H=H, Lq=L, Lkv=L, d_qk=d, d_v=d)
+    assert plan_of(pkg, D) == plan
     extra = lib.cosmos_attn_workspace_bytes(ctypes.byref(D)) - lib.cosmos_attn_packed_bytes(ctypes.byref(D))
-    acc = rem * ranges * 384 * d * 4
-    assert extra == (0 if ranges == 1 else (acc + 255) // 256 * 256 + rem * ranges * 384 * 16)
+    assert extra == partial_result_bytes(plan, d, False)
+
+
+@pytest.mark.parametrize("tangents", [False, True])
+@pytest.mark.parametrize("d", [16, 32, 64, 128])
+def test_workspace_holds_the_plan_that_runs_and_no_more(pkg, d, tangents):
+    """Over sizes, every length of the query against every length of the keys: the bytes asked for are those of the plan that runs, that
+    plan is still the one chosen where there is no more room than that, and without room no keys are cut."""
+    lib = pkg._lib.load_library()
+    t = 0x8000000 if tangents else None
+    shapes = set()
+    for H in (1, 5, 16, 40):
+        for Lq in (1, 129, 226, 700, 993, 1560, 2000, 3520, 4623, 5000, 7040, 16100, 37440):
+            for Lkv in (1, 226, 449, 513, 1000, 2049, 4000, 9000):
+                D = good_desc(pkg, B=1, H=H, Lq=Lq, Lkv=Lkv, d_qk=d, d_v=d, tq=t, tk=t, tv=t, to=t)
+                plan, packed = plan_of(pkg, D), lib.cosmos_attn_packed_bytes(ctypes.byref(D))
+                bytes_ = lib.cosmos_attn_workspace_bytes(ctypes.byref(D))
+                assert plan_of(pkg, D, bytes_) == plan, (H, Lq, Lkv)
+                if plan == "streamed":      # (the size covers the launch that is not streamed as well)
+                    continue
+                assert bytes_ == packed + partial_result_bytes(plan, d, tangents), (H, Lq, Lkv)
+                shapes.add(plan[:2])
+                uncut = plan_of(pkg, D, packed)
+                assert uncut == "streamed" or uncut[3:] == (0, 1), (H, Lq, Lkv)
+    assert shapes == ({(128, 1)} if tangents else {(128, 2), (256, 1), (384, 1)})
 
 
 def good_bwd_desc(pkg, **over):
