@@ -237,6 +237,7 @@ EXPORTS = {
     "cosmos_attn_abi_version": (ctypes.c_int, []),
     "cosmos_attn_status_string": (ctypes.c_char_p, [ctypes.c_int]),
     "cosmos_attn_set_stream_override": (None, [ctypes.c_int, ctypes.c_int]),
+    "cosmos_attn_set_forward_override": (ctypes.c_int, [ctypes.c_int, ctypes.c_int]),
     "cosmos_attn_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnDesc)]),
     "cosmos_attn_launch_plan": (ctypes.c_int, [ctypes.POINTER(AttnDesc), ctypes.c_size_t, ctypes.POINTER(AttnPlan)]),
     "cosmos_attn_fwd_jvp": (ctypes.c_int, [ctypes.POINTER(AttnDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),

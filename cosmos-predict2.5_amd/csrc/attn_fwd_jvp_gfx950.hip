@@ -42,6 +42,7 @@
 //     head's K/V images and share them through the per-XCD L2s and the Infinity Cache; workgroups of
 //     one XCD start their (order-free) sweep a few tiles apart so they do not hit one L2 channel at once.
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <stdint.h>
 #include <stddef.h>
 #include <stdlib.h>
@@ -1676,6 +1677,8 @@ constexpr size_t kNoLimit = ~(size_t)0;
 bool may_cut(const cosmos_attn_desc* d, int n_steps) {
     return n_steps >= 2 * kMinStepsPerSplit && !d->causal && !d->key_lens && !is_wide(d);
 }
+// cosmos_attn_set_forward_override() (tuning and tests), 0 = the library's own choice: rows of a forward-only workgroup, key ranges
+std::atomic<int> g_sym_rows{0}, g_sym_ranges{0};
 // The best cut for workgroups of block_m rows and n_steps barrier steps: `whole` is what a pair that is not cut costs, `cut` one of
 // which S ranges may be made.
 SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int block_m, int n_steps, StepCost whole, StepCost cut) {
@@ -1693,7 +1696,9 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     const SplitPlan uncut = s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
     while (s.splits > 1 && partial_bytes(d, s) > room) --s.splits;
-    s.splits = choose_splits(rem, n_steps, cut, slot_bytes, s.splits);
+    const int asked = mode_of(d) == MODE_FWD ? g_sym_ranges.load(std::memory_order_relaxed) : 0;
+    if (asked > 0) s.splits = rem == 0 ? 1 : std::min({asked, s.splits, n_steps / kMinStepsPerSplit});
+    else s.splits = choose_splits(rem, n_steps, cut, slot_bytes, s.splits);
     if (s.splits < 2) return uncut;
     s.us = full_us + split_cost(rem, n_steps, s.splits, cut, slot_bytes);
     return s;
@@ -1712,9 +1717,11 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
         const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
         return plan_shape(d, room, 0, kBlockM, n_tiles, StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
     }
+    const int rows = g_sym_rows.load(std::memory_order_relaxed);
     SplitPlan best;
     double best_us = 0.0;
     for (int i = 0; i < kNumSymShapes; ++i) {
+        if (rows && rows == 32 * kSymShapes[i].rg) return plan_sym(d, room, i);
         if (i > 0 && (int64_t)((d->Lq + 32 * kSymShapes[i].rg - 1) / (32 * kSymShapes[i].rg)) * d->B * d->H > kNumCUs) continue;
         const SplitPlan s = plan_sym(d, room, i);
         // (a cut has to come out a twentieth better than no cut, of another shape as well: so what the two-stage run takes, which
@@ -1831,6 +1838,15 @@ COSMOS_ATTN_API const char* cosmos_attn_status_string(int status) {
 COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, int workgroups) {
     g_stream_chunk.store(blocks_per_workgroup > 0 ? blocks_per_workgroup : 0, std::memory_order_relaxed);
     g_stream_groups.store(workgroups > 0 ? workgroups : 0, std::memory_order_relaxed);
+}
+
+COSMOS_ATTN_API int cosmos_attn_set_forward_override(int query_rows, int key_ranges) {
+    bool known = query_rows == 0;
+    for (const SymShape& w : kSymShapes) known = known || query_rows == 32 * w.rg;
+    if (!known || key_ranges < 0) return COSMOS_ATTN_BAD_ARG;
+    g_sym_rows.store(query_rows, std::memory_order_relaxed);
+    g_sym_ranges.store(key_ranges, std::memory_order_relaxed);
+    return COSMOS_ATTN_OK;
 }
 
 COSMOS_ATTN_API size_t cosmos_attn_workspace_bytes(const cosmos_attn_desc* d) {

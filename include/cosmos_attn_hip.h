@@ -96,6 +96,14 @@ COSMOS_ATTN_API const char *cosmos_attn_status_string(int status);
 COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, int workgroups);
 
 /*
+ * Tuning and test hook, process-wide, like the one above, for the kernel that calls without tangents run where they are not streamed: workgroups of
+ * query_rows rows (128, 256 or 384; 0: the library's choice), and key_ranges for the pairs of a partly filled last round (1: never cut;
+ * n > 1: n, where the call may be cut at all, or as many as its length and the workspace allow; 0: the library's choice).  (0, 0) restores
+ * the default.  It steers sizes and launches alike: set it before the workspace is asked for.  A status code.
+ */
+COSMOS_ATTN_API int cosmos_attn_set_forward_override(int query_rows, int key_ranges);
+
+/*
  * Bytes of device workspace the call needs (K, V and their tangents re-tiled into the
  * kernel's LDS image).  0 on invalid descriptors.  The host allocates it however it likes
  * (the Python host uses torch's caching allocator) and may reuse it across calls on one stream.

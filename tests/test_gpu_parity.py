@@ -130,19 +130,34 @@ def test_forward_only_key_padding(pkg, oracle, gpu, lens):
     run_case(pkg, oracle, gpu, (2, 2, 450, 128), (2, 2, 512, 128), key_lens=lens, seed=sum(lens), tangents="none")
 
 
-@pytest.mark.parametrize("shape_q,Lkv,ranges", [
-    ((1, 2, 1000, 128), 1000, 4),      # 6 workgroup pairs, 16 steps of 64 keys: 4 key ranges each
-    ((1, 1, 1157, 32), 4000, 15),      # 4 pairs, 63 steps: 15 ranges of 4 or 5 steps
-    ((1, 3, 300, 128), 520, 2),        # 3 pairs, 9 steps: 2 ranges (4 + 5 steps); ragged last tile in the second
-    ((2, 8, 6500, 64), 700, 2),        # 272 pairs: 256 whole + 16 cut into ... 11 steps allow 2 ranges
-    ((1, 2, 400, 64), 250, 1),         # 4 steps only: too short to cut
+@pytest.mark.parametrize("shape_q,Lkv,rows,ranges", [      # rows of a workgroup, and key ranges, as (forced) or planned
+    ((1, 2, 1000, 128), 1000, 128, 4),       # 16 pairs, 16 steps of 64 keys: 4 key ranges each
+    ((1, 1, 1157, 32), 4000, 128, 15),       # 10 pairs, 63 steps: 15 ranges of 4 or 5 steps
+    ((1, 3, 300, 128), 520, (128,), (2,)),   # 9 steps: 2 ranges (4 + 5 steps); ragged last tile in the second
+    ((1, 3, 300, 128), 520, (256,), (2,)),
+    ((1, 3, 300, 128), 520, (384,), (2,)),
+    ((1, 4, 4623, 128), 900, (256,), (3,)),  # 76 pairs, 15 steps
+    ((1, 1, 1157, 32), 4001, (256,), (15,)), # 63 steps, one key in the last tile
+    ((1, 1, 1157, 32), 4001, (384,), (15,)),
+    ((1, 2, 900, 16), 600, (384,), (2,)),
+    ((2, 8, 6500, 64), 700, 384, 2),         # 272 pairs: 256 whole + 16 cut, 11 steps allow 2 ranges
+    ((2, 8, 4300, 64), 700, (256,), (2,)),   # the same of 256 rows,
+    ((2, 8, 2100, 64), 700, (128,), (2,)),   # of 128
+    ((80, 1, 226, 128), 1000, (256,), (3,)),
+    ((1, 2, 400, 64), 250, 128, 1),          # 4 steps only: too short to cut
 ])
-def test_forward_only_key_range_split(pkg, oracle, gpu, shape_q, Lkv, ranges):
-    """When the last round of forward-only workgroups (one per compute unit) is less than half full, its (query block,
-    head) pairs are cut along the keys and merged by a second kernel.  The one-call entry point (which may cut) and
+def test_forward_only_key_range_split(pkg, oracle, gpu, stream_override, forward_override, forward_plan, shape_q, Lkv, rows, ranges):
+    """The (query block, head) pairs of a partly filled last round of forward-only workgroups (one per compute unit) may be cut along
+    the keys and merged by a second kernel.  The one-call entry point (which may cut) and
     pack + run (which never does) must agree to rounding, and both with the oracle."""
-    del ranges   # documented above; the plan itself is internal
     B, H, Lq, d = shape_q
+    if isinstance(rows, tuple):
+        (rows,), (ranges,) = rows, ranges
+        forward_override(rows, ranges)
+        stream_override(chunk=1)
+    plan = forward_plan(shape_q, Lkv)
+    pairs = (Lq + rows - 1) // rows * B * H
+    assert plan == (rows, 2 if rows == 128 else 1, *((pairs, 0, 1) if ranges == 1 else (pairs - pairs % 256, pairs % 256, ranges)))
     run_case(pkg, oracle, gpu, shape_q, (B, H, Lkv, d), seed=Lq + Lkv, tangents="none")
     L, lib = pkg._lib, pkg._lib.load_library()
     q, k, v, _, _, _ = (x.to(gpu) for x in oracle.make_inputs(shape_q, (B, H, Lkv, d), seed=Lq + Lkv))
@@ -168,29 +183,73 @@ def test_forward_only_key_range_split(pkg, oracle, gpu, shape_q, Lkv, ranges):
     assert torch.equal(o_again, o_ref) and torch.equal(lse_again, lse_ref)
 
 
-@pytest.mark.parametrize("shape_q,Lkv,dtype", [
-    ((2, 8, 255, 128), 1, torch.bfloat16),         # 128 rows x 2 key groups: the second has no key at all,
-    ((2, 8, 255, 128), 33, torch.float16),         # one key,
-    ((1, 2, 129, 128), 64, torch.bfloat16),        # as many as the first,
-    ((1, 2, 128, 128), 97, torch.float16),         # one tile less,
-    ((1, 3, 31, 16), 65, torch.bfloat16),          # a masked tile at a sweep's end; the smallest head dim
-    ((1, 40, 993, 128), 1000, torch.bfloat16),     # 256 rows
-    ((1, 40, 1000, 128), 65, torch.float16),
-    ((2, 20, 770, 64), 300, torch.bfloat16),
-    ((1, 40, 1560, 128), 700, torch.bfloat16),     # 384 rows
+@pytest.mark.parametrize("shape_q,Lkv,dtype,rows", [
+    ((2, 8, 255, 128), 1, torch.bfloat16, 128),         # 128 rows x 2 key groups: the second has no key at all,
+    ((2, 8, 255, 128), 33, torch.float16, 128),         # one key,
+    ((1, 2, 129, 128), 64, torch.bfloat16, 128),        # as many as the first,
+    ((1, 2, 128, 128), 97, torch.float16, 128),         # one tile less,
+    ((1, 3, 31, 16), 65, torch.bfloat16, 128),          # a masked tile at a sweep's end; the smallest head dim
+    ((1, 40, 993, 128), 1000, torch.bfloat16, 256),
+    ((1, 40, 1000, 128), 65, torch.float16, 256),
+    ((2, 20, 770, 64), 300, torch.bfloat16, 256),
+    ((1, 40, 1560, 128), 700, torch.bfloat16, 384),
 ])
-def test_forward_only_workgroup_shapes(pkg, oracle, gpu, stream_override, shape_q, Lkv, dtype):
-    """Calls for each of the three workgroup shapes of the forward-only kernel, at the edges of its key groups."""
+def test_forward_only_workgroup_shapes(pkg, oracle, gpu, stream_override, forward_plan, shape_q, Lkv, dtype, rows):
+    """Calls for which the library picks each of the three workgroup shapes of the forward-only kernel, at the edges of its key groups."""
     stream_override(chunk=1)                       # never the query-streaming kernel
+    assert forward_plan(shape_q, Lkv)[0] == rows
     run_case(pkg, oracle, gpu, shape_q, (*shape_q[:2], Lkv, shape_q[3]), seed=Lkv, dtype=dtype, tangents="none")
 
 
+# what a workgroup shape can go wrong at, on each of them (a call is not moved to another one by the costs they are chosen by)
+each_shape = pytest.mark.parametrize("rows", [128, 256, 384])
+
+
+@each_shape
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_forward_only_each_shape_ragged(pkg, oracle, gpu, stream_override, forward_override, rows, dtype):
+    stream_override(chunk=1)
+    forward_override(rows)
+    for Lq, Lkv in [(1, 1), (50, 37), (rows - 1, 65), (rows + 1, 64), (129, 1), (5, 300), (2 * rows + 33, 96), (rows, 257)]:
+        run_case(pkg, oracle, gpu, (1, 2, Lq, 128), (1, 2, Lkv, 128), seed=Lq + Lkv, dtype=dtype, tangents="none")
+
+
+@each_shape
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_forward_only_each_shape_head_dims(pkg, oracle, gpu, stream_override, forward_override, rows, dtype):
+    stream_override(chunk=1)
+    forward_override(rows)
+    for dqk, dv in [(16, 16), (32, 32), (64, 64), (16, 128), (32, 64), (128, 32), (128, 16)]:
+        run_case(pkg, oracle, gpu, (2, 2, 400, dqk), (2, 2, 333, dqk), dv=dv, seed=dqk + dv, dtype=dtype, tangents="none")
+
+
+@each_shape
+@pytest.mark.parametrize("d", [16, 64, 128])
+def test_forward_only_each_shape_causal(pkg, oracle, gpu, forward_override, rows, d):
+    forward_override(rows)
+    for L in (1, 33, 128, 200, rows - 1, rows + 1, 515, 1000):
+        run_case(pkg, oracle, gpu, (1, 2, L, d), causal=True, seed=L, tangents="none")
+
+
+@each_shape
+@pytest.mark.parametrize("d", [32, 128])
+def test_forward_only_each_shape_key_padding(pkg, oracle, gpu, stream_override, forward_override, rows, d):
+    stream_override(chunk=1)
+    forward_override(rows)
+    for lens in ([64, 512], [7, 33], [300, 31], [1, 65], [97, 511]):
+        run_case(pkg, oracle, gpu, (2, 2, 450, d), (2, 2, 512, d), key_lens=lens, seed=sum(lens), tangents="none")
+
+
 @pytest.mark.parametrize("order", ["rising", "falling", "spike"])
-@pytest.mark.parametrize("shape_q,Lkv,dtype", [((1, 2, 300, 128), 333, torch.bfloat16), ((1, 2, 129, 32), 333, torch.float16),
-                                               ((1, 40, 993, 128), 200, torch.bfloat16)])
-def test_forward_only_scores_that_move_the_max(pkg, oracle, gpu, stream_override, order, shape_q, Lkv, dtype):
+@pytest.mark.parametrize("shape_q,Lkv,dtype,rows,ranges", [
+    ((1, 2, 300, 128), 333, torch.bfloat16, 128, 1), ((1, 2, 129, 32), 333, torch.float16, 128, 1), ((1, 40, 993, 128), 200, torch.bfloat16, 256, 1),
+    ((1, 2, 500, 32), 333, torch.float16, 256, 1), ((1, 2, 800, 128), 333, torch.bfloat16, 384, 1), ((1, 2, 400, 32), 333, torch.float16, 384, 1),
+    ((1, 2, 800, 128), 333, torch.float16, 384, 1), ((1, 2, 300, 128), 777, torch.bfloat16, 128, 3), ((1, 2, 300, 128), 777, torch.bfloat16, 256, 3),
+    ((1, 2, 800, 128), 777, torch.bfloat16, 384, 3)])
+def test_forward_only_scores_that_move_the_max(pkg, oracle, gpu, stream_override, forward_override, order, shape_q, Lkv, dtype, rows, ranges):
     """Scores that outgrow the running max by far more than its slack, in tile after tile, in one late key, or not at all."""
     stream_override(chunk=1)
+    forward_override(rows, ranges)
     B, H, Lq, d = shape_q
     q, k, v, _, _, _ = oracle.make_inputs(shape_q, (B, H, Lkv, d), seed=Lkv + d, dtype=dtype)
     top = {"rising": torch.linspace(-60, 60, Lkv), "falling": torch.linspace(60, -60, Lkv),

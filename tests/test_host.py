@@ -167,6 +167,25 @@ def test_workspace_holds_the_plan_that_runs_and_no_more(pkg, d, tangents):
     assert shapes == ({(128, 1)} if tangents else {(128, 2), (256, 1), (384, 1)})
 
 
+def test_forward_override_steers_plan_and_workspace(pkg, forward_override, forward_plan):
+    lib = pkg._lib.load_library()
+    for rows, ranges in ((64, 0), (-128, 0), (129, 0), (0, -1)):
+        assert lib.cosmos_attn_set_forward_override(rows, ranges) == pkg._lib.ST_BAD_ARG
+    default = forward_plan((1, 3, 300, 128), 520)
+    for rows, groups in ((128, 2), (256, 1), (384, 1)):
+        pairs = (300 + rows - 1) // rows * 3
+        for ranges, want in ((1, (pairs, 0, 1)), (2, (0, pairs, 2)), (9, (0, pairs, 2))):      # 9 steps of 64 keys: two ranges at most
+            forward_override(rows, ranges)
+            assert forward_plan((1, 3, 300, 128), 520) == (rows, groups, *want)
+            D = good_desc(pkg, H=3, Lq=300, Lkv=520, d_v=128)
+            extra = lib.cosmos_attn_workspace_bytes(ctypes.byref(D)) - lib.cosmos_attn_packed_bytes(ctypes.byref(D))
+            assert extra == partial_result_bytes((rows, groups, *want), 128, False)
+        assert forward_plan((1, 3, 300, 128), 300, causal=True) == (rows, groups, pairs, 0, 1)      # equal work only: never cut
+        assert forward_plan((1, 3, 300, 128), 520, padded=True) == (rows, groups, pairs, 0, 1)
+    forward_override()
+    assert forward_plan((1, 3, 300, 128), 520) == default
+
+
 def good_bwd_desc(pkg, **over):
     D = pkg._lib.AttnBwdDesc()
     D.abi_version, D.dtype = pkg._lib.ABI_VERSION, pkg._lib.DTYPE_BF16
