@@ -1559,42 +1559,50 @@ constexpr SymShape kSymShapes[] = {
     {8, 1, {0.82, 0.85, 1.10, 1.73}, {1.0, 1.0, 0.94, 0.78}, {4.6, 5.1, 6.6, 10.6}},
     {4, 2, {0.45, 0.46, 0.60, 0.94}, {1.0, 1.0, 1.0, 0.99}, {4.1, 4.8, 6.0, 9.0}},
 };
+constexpr int kSymStepTiles = 2;      // tiles of 32 keys per barrier step (SymCfg::TPS)
 constexpr int kNumSymShapes = sizeof(kSymShapes) / sizeof(kSymShapes[0]);
 
+struct Kernel { attn_kernel_t fn; int lds_bytes; };
+template <typename T, int DQK, int DV, int SHAPE>
+Kernel pick_sym() {
+    typedef SymCfg<DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg> C;
+    static_assert(C::TPS == kSymStepTiles, "plans count steps of that many tiles");
+    return {attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg>, C::LDS_BYTES};
+}
 template <typename T, int DQK, int DV>
-attn_kernel_t pick_mode(int mode, int shape) {
+Kernel pick_mode(int mode, int shape) {
     switch (mode) {
         case MODE_FWD:
             switch (shape) {
-                case 0: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[0].rg, kSymShapes[0].kg>;
-                case 1: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[1].rg, kSymShapes[1].kg>;
-                default: return attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[2].rg, kSymShapes[2].kg>;
+                case 0: return pick_sym<T, DQK, DV, 0>();
+                case 1: return pick_sym<T, DQK, DV, 1>();
+                default: return pick_sym<T, DQK, DV, 2>();
             }
-        case MODE_JVP_Q: return attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q>;
-        default: return attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL>;
+        case MODE_JVP_Q: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q>, AttnCfg<DQK, DV, MODE_JVP_Q>::LDS_BYTES};
+        default: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL>, AttnCfg<DQK, DV, MODE_JVP_FULL>::LDS_BYTES};
     }
 }
 template <typename T, int DQK>
-attn_kernel_t pick_dv(int dv, int mode, int shape) {
+Kernel pick_dv(int dv, int mode, int shape) {
     switch (dv) {
         case 16: return pick_mode<T, DQK, 16>(mode, shape);
         case 32: return pick_mode<T, DQK, 32>(mode, shape);
         case 64: return pick_mode<T, DQK, 64>(mode, shape);
         case 128: return pick_mode<T, DQK, 128>(mode, shape);
-        default: return nullptr;
+        default: return {};
     }
 }
 template <typename T>
-attn_kernel_t pick_dqk(int dqk, int dv, int mode, int shape) {
+Kernel pick_dqk(int dqk, int dv, int mode, int shape) {
 #ifdef COSMOS_ATTN_ONLY_D128   // development builds: instantiate the d=128 kernels only
-    return (dqk == 128 && dv == 128) ? pick_mode<T, 128, 128>(mode, shape) : nullptr;
+    return (dqk == 128 && dv == 128) ? pick_mode<T, 128, 128>(mode, shape) : Kernel{};
 #endif
     switch (dqk) {
         case 16: return pick_dv<T, 16>(dv, mode, shape);
         case 32: return pick_dv<T, 32>(dv, mode, shape);
         case 64: return pick_dv<T, 64>(dv, mode, shape);
         case 128: return pick_dv<T, 128>(dv, mode, shape);
-        default: return nullptr;
+        default: return {};
     }
 }
 
@@ -1632,20 +1640,6 @@ int mode_of(const cosmos_attn_desc* d) {
 size_t tile_bytes_of(const cosmos_attn_desc* d) {
     const TileGeom g(d->d_qk, d->d_v, mode_of(d) == MODE_JVP_FULL);
     return (size_t)g.tile_frags * kFragBytes;
-}
-// LDS of the attention kernels: K ring, V ring, P^T/H^T hand-over buffers, rescale factors (AttnCfg::LDS_BYTES); forward only the
-// rings or, with key groups, what merging them takes (SymCfg::LDS_BYTES)
-size_t lds_bytes_of(const cosmos_attn_desc* d, int shape) {
-    const int mode = mode_of(d);
-    const TileGeom g(d->d_qk, d->d_v, mode == MODE_JVP_FULL);
-    const size_t kp = (size_t)g.kpart_frags * kFragBytes, vp = (size_t)(g.tile_frags - g.kpart_frags) * kFragBytes;
-    if (mode == MODE_FWD) {
-        const SymShape w = kSymShapes[shape];
-        const size_t rings = (size_t)4 * 2 * (kp + vp), merge = w.kg == 1 ? 0 : (size_t)(w.kg - 1) * w.rg * g.ndb * 4 * kFragBytes + (size_t)w.rg * w.kg * 64 * 8;
-        return rings > merge ? rings : merge;
-    }
-    const size_t ph = 4 * kFragBytes;
-    return kRingK * kp + kRingV * vp + 2 * 4 * ph + 2 * 4 * 256;
 }
 int n_tiles_of(const cosmos_attn_desc* d) { return (d->Lkv + kBlockN - 1) / kBlockN; }
 // workspace = packed tiles [B*H][n_tiles][tile bytes]
@@ -1703,11 +1697,12 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     s.us = full_us + split_cost(rem, n_steps, s.splits, cut, slot_bytes);
     return s;
 }
-SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {     // forward only: a barrier step is 64 keys
+int sym_steps(const cosmos_attn_desc* d) { return (n_tiles_of(d) + kSymStepTiles - 1) / kSymStepTiles; }
+SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {
     const SymShape& w = kSymShapes[shape];
     const double dim = 0.5 * (d->d_qk + d->d_v);
     const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
-    return plan_shape(d, room, shape, 32 * w.rg, (n_tiles_of(d) + 1) / 2, c, c);
+    return plan_shape(d, room, shape, 32 * w.rg, sym_steps(d), c, c);
 }
 SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     const int mode = mode_of(d), n_tiles = n_tiles_of(d);
@@ -1733,7 +1728,7 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
 }
 // Room for partial results that a caller is asked for: what the plan that runs needs (it stays the best of the plans that fit that room)
 size_t planned_partial_bytes(const cosmos_attn_desc* d) {
-    if (!may_cut(d, mode_of(d) == MODE_FWD ? (n_tiles_of(d) + 1) / 2 : n_tiles_of(d))) return 0;      // (not planned only to see that)
+    if (!may_cut(d, mode_of(d) == MODE_FWD ? sym_steps(d) : n_tiles_of(d))) return 0;      // (not planned only to see that)
     return partial_bytes(d, plan_split(d, kNoLimit));
 }
 // Short key sequences go to attn_qstream_kernel: number of workgroups (0 = use the other kernels).  The kernel cuts the
@@ -1943,9 +1938,9 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
     if (!device_is_whole_mi355x()) return COSMOS_ATTN_WRONG_DEVICE;
     const int mode = mode_of(d);
     if (is_wide(d)) return run_wide(d, workspace, stream);
-    attn_kernel_t fn = d->dtype == COSMOS_ATTN_BF16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode, sp.shape)
-                                                    : pick_dqk<_Float16>(d->d_qk, d->d_v, mode, sp.shape);
-    if (!fn) return COSMOS_ATTN_UNSUPPORTED;
+    const Kernel kernel = d->dtype == COSMOS_ATTN_BF16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode, sp.shape)
+                                                       : pick_dqk<_Float16>(d->d_qk, d->d_v, mode, sp.shape);
+    if (!kernel.fn) return COSMOS_ATTN_UNSUPPORTED;
     AttnParams ap;
     ap.q = d->q; ap.tq = d->tq;
     ap.q_sb = d->q_stride[0]; ap.q_sh = d->q_stride[1]; ap.q_sl = d->q_stride[2];
@@ -1970,8 +1965,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
             return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
         }
     }
-    const size_t lds = lds_bytes_of(d, sp.shape);
-    if (!allow_lds((const void*)fn, lds)) return COSMOS_ATTN_LAUNCH_FAILED;
+    if (!allow_lds((const void*)kernel.fn, kernel.lds_bytes)) return COSMOS_ATTN_LAUNCH_FAILED;
     ap.n_qt = sp.n_qt; ap.n_full = sp.n_full; ap.n_rem = sp.n_rem; ap.splits = sp.splits;
     ap.part_acc = nullptr; ap.part_stat = nullptr;
     if (sp.splits > 1) {
@@ -1979,7 +1973,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
         ap.part_stat = (float4*)((char*)workspace + image_bytes + partial_acc_bytes(d, sp));
     }
     const int64_t blocks = (int64_t)sp.n_full + (int64_t)sp.n_rem * sp.splits;
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymShapes[sp.shape].rg * kSymShapes[sp.shape].kg : kAttnThreads), lds, (hipStream_t)stream, ap);
+    hipLaunchKernelGGL(kernel.fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymShapes[sp.shape].rg * kSymShapes[sp.shape].kg : kAttnThreads), kernel.lds_bytes, (hipStream_t)stream, ap);
     if (hipGetLastError() != hipSuccess) return COSMOS_ATTN_LAUNCH_FAILED;
     if (sp.splits > 1) {
         const int rows_per_block = 256 / (d->d_v / 4);
