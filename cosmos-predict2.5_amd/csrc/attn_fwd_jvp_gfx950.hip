@@ -1555,7 +1555,7 @@ typedef void (*attn_kernel_t)(const AttnParams);
 // as fast but at single sizes (16 heads 7040 x 1024: 8 x 1 87, 12 x 1 93; 40 heads 3520: 282, 298).
 struct SymShape { int rg, kg; double step_us[4], alone[4], range_us[4]; };
 constexpr SymShape kSymShapes[] = {
-    {12, 1, {1.09, 1.12, 1.58, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
+    {12, 1, {1.09, 1.12, 1.55, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
     {8, 1, {0.82, 0.85, 1.10, 1.73}, {1.0, 1.0, 0.94, 0.78}, {4.6, 5.1, 6.6, 10.6}},
     {4, 2, {0.45, 0.46, 0.60, 0.94}, {1.0, 1.0, 1.0, 0.99}, {4.1, 4.8, 6.0, 9.0}},
 };

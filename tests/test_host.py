@@ -133,6 +133,8 @@ def test_key_range_plan(pkg, H, L, tangents, plan):
     (32, 40, 9000, (384, 1, 768, 192, 4)),      # 960 pairs: 192 of a fourth round
     (32, 1, 4000, (128, 2, 0, 32, 8)),          # 32 pairs, 63 steps
     (64, 16, 5000, (384, 1, 224, 0, 1)),        # 224 pairs in one round
+    (64, 16, 2660, (384, 1, 0, 112, 2)),        # 112 pairs in halves 52.1 us, 176 pairs of 256 rows 54.3
+    (64, 40, 1100, (256, 1, 200, 0, 1)),        # 33.4 us; 120 pairs of 384 rows in halves 37.6
 ])
 def test_key_range_plan_below_head_dim_128(pkg, d, H, L, plan):
     """As above, forward only: a step costs more than its share of matrix instructions there, so that more calls are worth cutting."""
