@@ -32,21 +32,23 @@ __device__ __forceinline__ void both_halves(float x, float& lo, float& hi) {
 }
 
 constexpr int kFragBytes = 1024;   // one MFMA A-operand fragment: 64 lanes x 16 B
-// The running row max that the softmax exponentials refer to is allowed to lag the true one: it moves (and everything
+// The running row max that the softmax exponentials refer to is allowed to lag the true one.  In the kernels with a score role
+// (attn_fwd_jvp_kernel, attn_qstream_kernel) it moves (and everything
 // summed so far is rescaled) only when some row of the wavefront has a score more than kMaxSlack above it, in log2
 // units, so p = exp2(s c - m) stays below 2^kMaxSlack.  O = sum p v / sum p and LSE = m + log2 sum p hold for any
 // reference m, and 16-bit rounding of p is relative, so nothing is lost; what is gained is that the rescaling pass over
 // the accumulators, which otherwise runs in nearly every one of a sweep's first dozens of steps (in every step of a short
 // sweep), runs about once per sweep.
 constexpr float kMaxSlack = 6.0f;
-// Whether a score lies that far above the max is read off the row sums: a lane's sum of the exponentials of its 16 keys of a tile is at least
-// its largest one, and is formed anyway.  A tile whose lane sums all stay within kMaxTileSum is done; otherwise (or if a sum is no number)
-// the max moves up to the tile's scores and the tile's softmax is done again from them.  A max over the scores before the exponentials
-// (10 dependent instructions and the wait for the last score MFMA in front of them) costs 5 % of the forward-only kernel.
-constexpr float kMaxTileSum = 64.0f;       // 2^kMaxSlack
+// attn_fwd_sym_kernel reads whether the max has to move off the row sums instead: a lane's sum of the exponentials of its 16 keys of a tile is
+// at least its largest one, and is formed anyway.  A tile whose lane sums all stay within 2^kMaxSlack is done; otherwise (or if a sum is no
+// number) the max moves up to the tile's scores and the tile's softmax is done again from them.  That is the same bound on p; the max moves
+// earlier (sixteen scores 2 above it do), never later.  A max over the scores before the exponentials (10 dependent instructions and the wait
+// for the last score MFMA in front of them) costs that kernel 4 to 5 %.
+constexpr float kMaxTileSum = (float)(1 << (int)kMaxSlack);
 // With tangents H = p dS s is rounded to the 16-bit type as well, and fp16 has the range for |dS s| up to 65504 only while
 // p <= 1 (the reference's range, flash_attention_jvp_triton.py:114,141); a p of up to 2^6 would overflow from |dS s| ~ 1e3 on.
-// So fp16 with tangents keeps the exact running max; bf16 (8 exponent bits) and the forward-only kernels use the slack.
+// So fp16 with tangents keeps the exact running max; bf16 (8 exponent bits) and the forward-only mode of attn_qstream_kernel use the slack.
 template <typename T>
 __device__ __host__ constexpr float max_slack_of(bool with_tangents) {
     return (with_tangents && __is_same(T, _Float16)) ? 0.0f : kMaxSlack;

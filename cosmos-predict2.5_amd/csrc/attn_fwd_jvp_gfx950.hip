@@ -1120,8 +1120,8 @@ attn_qstream_kernel(const AttnParams p) {
 // each for its own 32 query rows, with P^T never leaving registers.
 //
 // What bounds it: a SIMD issues one VALU or MFMA instruction in 4 cycles.  A tile of 32 keys costs a wavefront 16 MFMAs (512 cycles of
-// the matrix unit) and some 125 such turns, 64 of them in 16 exponentials; in long calls the part's power limit on top (74 % MFMA duty
-// at 1.70 GHz).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
+// the matrix unit) and some 125 such turns, 64 of them in 16 exponentials; in long calls the part's power limit on top (80 % MFMA duty
+// at 1.56 GHz, 37440 positions; 66 % at 1.76 GHz before).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
 // formed where it did not move (kMaxTileSum).  Measured, us, before either / with the softmax between the MFMAs / with both: 16 heads,
 // d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120.
 // Not faster: v_mfma_f32_16x16x32 (less energy, but twice the MFMA instructions to issue: 37440 9450, 3520 142), operand fetches three
@@ -1548,11 +1548,15 @@ typedef void (*attn_kernel_t)(const AttnParams);
 
 // Workgroups of attn_fwd_sym_kernel, groups of 32 query rows x groups of keys, and what they cost at head dims 16, 32, 64, 128 (StepCost):
 // the least estimate is taken (plan_split).  Fits to 255 .. 13000 positions and 600 .. 37440 x 512 .. 2048, B*H = 16 and 40, S = 1 .. 16, each
-// shape with each S measured; the choice takes 1.003 to 1.008 times the best one's time on average, 1.07 at most.  us, 12 x 1 / 8 x 1 /
-// 4 x 2, uncut, d = 128, with the re-tiling: 16 heads 255 positions 19.4 / 18.3 / 15.5, 700 35.2 / 30.0 / 25.9, 1560 61 / 53 / 41, 3520
-// 137 / 120 / 135, 5000 219 / 285 / 262; 40 heads 1000 51 / 45 / 59, 1560 82 / 108 / 109.  (Three key groups are no faster than two.)
-// The smaller shapes are for calls that fit into one round of them.  Past that 12 x 1 with its last round cut, or the query-streaming kernel, is
-// as fast but at single sizes (16 heads 7040 x 1024: 8 x 1 87, 12 x 1 93; 40 heads 3520: 282, 298).
+// shape with each S measured.  us, 12 x 1 / 8 x 1 / 4 x 2, uncut, d = 128, with the re-tiling: 16 heads 255 positions 18.8 / 17.5 / 14.9,
+// 700 34.8 / 30.1 / 25.3, 1560 61 / 50 / 40, 3520 120 / 110 / 124, 5000 205 / 267 / 245; 40 heads 1000 49 / 41 / 56, 1560 75 / 98 / 100.
+// (Three key groups are no faster than two.)
+// The smaller shapes are chosen from only where a call fits into one round of them.  There the choice takes 1.003 times the best shape's time
+// on average and 1.08 at most (64 calls of those ranges at random, each shape uncut and with its own cut).  Past one round 12 x 1 is taken, whose
+// thin last round is cut: over 59 calls 1.012 on average, but 1.14 at most, since a last round of 64 .. 128 pairs is where two rounds of 8 x 1 can be
+// shorter (us, 12 x 1 cut / 8 x 1: 16 heads 7410 x 883 at head dim 32 43 / 38, 8120 x 1024 at 64 63 / 55, 2 x 16 heads 3520 225 / 215; the other way
+// 40 heads 3520 272 / 309, 16 heads 9452 at 64 409 / 488).  Where no keys are cut (two-stage runs, masks) such a call loses more: 16 heads 7040
+// 485 / 392, 2 x 16 heads 3520 262 / 215.  Causal calls are priced as if every workgroup walked all keys.
 struct SymShape { int rg, kg; double step_us[4], alone[4], range_us[4]; };
 constexpr SymShape kSymShapes[] = {
     {12, 1, {1.09, 1.12, 1.55, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
@@ -1737,12 +1741,14 @@ size_t planned_partial_bytes(const cosmos_attn_desc* d) {
 // block_us + tile_us per key tile each and start_us once, comes out faster than the other kernels' rounds: a finished block costs it
 // little, a key tile costs it more than the forward-only kernel (which has three wavefronts per SIMD).  Measured (us, stream / other kernel,
 // 16 heads): tangent on q 3520 x 512 keys 45 / 62, 7040 x 512 78 / 109, 37440 x 2048
-// 1162 / 1294; forward only 3520 x 512 33 / 41, 37440 x 512 212 / 236, x 1024 380 / 357, x 2048 728 / 603.  Forward only at small head
-// dims the stream pays only while a unit has one block (head dim 32: 1560 x 512 16 / 19, 3520 x 512 24 / 20, 40 heads 1560 x 512 33 / 22).
-// The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: the way chosen takes
-// 1.0000 to 1.008 times the better one's time on average, 1.12 at most.  The two-stage run never cuts key ranges (no room), so that its
-// other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121; forward only 6500 x 1024
-// 80 / 97, 6800 x 1536 116 / 133 (one call, which cuts, with its re-tiling: 67, 101, 87, 116).  With all tangents the
+// 1162 / 1294; forward only, with the re-tiling, 3520 x 512 29 / 31, 37440 x 512 206 / 220, x 1024 382 / 344, x 2048 738 / 591; at head dim 64
+// 8010 x 361 34 / 37, 6880 x 145 20 / 27, 6868 x 958 70 / 56; below that the forward-only kernel is the faster one (head dim 32: 1560 x 512 15 / 13,
+// 3520 x 512 23 / 16, 40 heads 1560 x 512 32 / 20).
+// The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: with a tangent the way chosen takes
+// 1.0000 to 1.008 times the better one's time on average, 1.12 at most; forward only 1.00 on average, 1.04 at most (68 calls, with all three
+// workgroup shapes on the other side).  The two-stage run never cuts key ranges (no room), so that its
+// other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121 (one call, which cuts, with its
+// re-tiling: 67, 101); forward only 6500 x 1024 80 / 88, 6800 x 1536 115 / 119 (one call 83, 110).  With all tangents the
 // two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
 // cosmos_attn_set_stream_override() replaces the choice (tuning and tests); nothing in the per-call path reads the environment.
 constexpr int kStreamMaxTiles = 64;       // up to 2048 keys

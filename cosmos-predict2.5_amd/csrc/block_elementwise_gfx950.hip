@@ -113,7 +113,9 @@ __device__ __forceinline__ void gated_sum(uint4 x, uint4 tx, uint4 res, uint4 tr
 // row stays in registers between the statistics and the output pass.
 // GATED: the row is the gated residual of the sub-layer before, formed, rounded and stored here, so that it is not read back from memory
 // (memory-bound, 4 tensors of traffic instead of 3 + 2, and 1 launch instead of 2; the same bits).  28 blocks on 3520 x 2048 rows, two such
-// pairs each: 18406 -> 18089 us, a block on 37440 rows 13558 -> 13467.
+// pairs each: 18406 -> 18089 us, a block on 37440 rows 13558 -> 13467.  One pair, us, two kernels -> this one: 17600 x 2048 rows 67 -> 52, with tangents
+// 148 -> 121; 17600 x 5120 179 -> 170, 398 -> 347; 3520 x 5120 39 -> 41, 86 -> 78.  Of a block with tangents the matrix products are so much that it
+// shows only where the two ways are timed in turn: 17600 rows 10110 -> 10081, 3520 1143 -> 1133, 1560 638 -> 627.
 template <int NCH, bool TANGENT, bool BF16, bool GATED>
 __global__ void __launch_bounds__(kThreads) ln_modulate_kernel(const LnModParams p) {
     const int lane = threadIdx.x & 63;

@@ -287,7 +287,8 @@ typedef struct cosmos_gated_residual_desc {
     void *out, *tout;
 } cosmos_gated_residual_desc;
 
-/* Both, where the gated residual is what the LayerNorm reads:  out = x + gate res,  y = LayerNorm(out) (1 + scale) + shift. */
+/* Both, where the gated residual is what the LayerNorm reads:  out = x + gate res,  y = LayerNorm(out) (1 + scale) + shift.
+ * Each of out, tout, y, ty may be x, tx, res or tres itself (what is written to has been read by then); the four are different buffers. */
 typedef struct cosmos_gated_residual_ln_modulate_desc {
     int32_t abi_version, dtype;
     int32_t D, rows_per_group;         /* D % 8 == 0, D <= 8192; rows % rows_per_group == 0 */

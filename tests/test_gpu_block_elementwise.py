@@ -129,6 +129,19 @@ def test_gated_residual_ln_modulate(pkg, block_oracle, gpu, dtype, rows, D, rpg)
     assert torch.equal(out, ref) and torch.equal(y, pkg.ln_modulate(ref, dsh, dsc)[0])
 
 
+@pytest.mark.parametrize("rows,D,rpg", [(30, 264, 5), (64, 2048, 16), (7, 5120, 7)])
+def test_gated_residual_ln_modulate_into_its_inputs(pkg, gpu, rows, D, rpg):
+    """Outputs that are inputs of the same call: the same bits as into buffers of their own."""
+    g = torch.Generator().manual_seed(rows + D)
+    big = [rnd(g, torch.bfloat16, rows, D).to(gpu) for _ in range(4)]                             # x, res, tx, tres
+    mod = [rnd(g, torch.bfloat16, rows // rpg, D, std=0.3).to(gpu) for _ in range(6)]             # gate, shift, scale and their tangents
+    call = lambda x, res, tx, tres, **outs: pkg.ops.gated_residual_ln_modulate(x, res, *mod[:3], tx, tres, *mod[3:], **outs)
+    want = call(*big)
+    for y, ty in ((0, 2), (1, 3), (3, 0)):
+        ins = [t.clone() for t in big]
+        assert all(torch.equal(a, b) for a, b in zip(call(*ins, y=ins[y], ty=ins[ty]), want))
+
+
 @pytest.mark.parametrize("rows,rpg,D", [(24, 4, 8), (17, 17, 264), (66, 33, 2048), (8, 1, 2056), (90, 45, 4104), (40, 40, 5120), (21, 21, 8192),
                                         (9000, 4500, 64)])      # (the last: rows enough for runs longer than the shortest)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
