@@ -114,8 +114,9 @@ __device__ __forceinline__ void gated_sum(uint4 x, uint4 tx, uint4 res, uint4 tr
 // GATED: the row is the gated residual of the sub-layer before, formed, rounded and stored here, so that it is not read back from memory
 // (memory-bound, 4 tensors of traffic instead of 3 + 2, and 1 launch instead of 2; the same bits).  28 blocks on 3520 x 2048 rows, two such
 // pairs each: 18406 -> 18089 us, a block on 37440 rows 13558 -> 13467.  One pair, us, two kernels -> this one: 17600 x 2048 rows 67 -> 52, with tangents
-// 148 -> 121; 17600 x 5120 179 -> 170, 398 -> 347; 3520 x 5120 39 -> 41, 86 -> 78.  Of a block with tangents the matrix products are so much that it
-// shows only where the two ways are timed in turn: 17600 rows 10110 -> 10081, 3520 1143 -> 1133, 1560 638 -> 627.
+// 148 -> 121; 17600 x 5120 180 -> 168, 399 -> 338; 3520 x 5120 37 -> 33
+// (inputs not in cache 40 -> 42), 80 -> 72; slower without tangents around 10000 x 5120, 96 -> 101.  Of a block with tangents the matrix products
+// are so much that it shows only where the two ways are timed in turn: 17600 rows 10110 -> 10081, 3520 1143 -> 1133, 1560 638 -> 627.
 template <int NCH, bool TANGENT, bool BF16, bool GATED>
 __global__ void __launch_bounds__(kThreads) ln_modulate_kernel(const LnModParams p) {
     const int lane = threadIdx.x & 63;
@@ -215,9 +216,13 @@ ln_kernel_t pick_ln(int d) {
     if (nch <= 4) return ln_modulate_kernel<4, TANGENT, BF16, GATED>;
     if (nch <= 8) return ln_modulate_kernel<8, TANGENT, BF16, GATED>;
     if (nch <= 10) return ln_modulate_kernel<10, TANGENT, BF16, GATED>;
-    if (nch <= 16) return ln_modulate_kernel<16, TANGENT, BF16, GATED>;
+    if constexpr (!GATED) if (nch <= 16) return ln_modulate_kernel<16, TANGENT, BF16, false>;
     return nullptr;
 }
+// Wider rows go through the two kernels.  16 chunks of a row take some 200 registers (340 with tangents), and one pass with its four streams is then
+// slower than two, but for calls so small that the launch counts (us, two kernels / one pass: 7040 rows of 5632 79 / 93, 37440 432 / 515, of 8192
+// 603 / 678, 1560 of 5632 24 / 20; with tangents either way within a tenth: 3520 of 5632 122 / 133, 10000 of 8192 470 / 445).
+constexpr int kMaxGatedLnD = 5120;
 
 // ------------------------------------------------------------------------------------------------ gated residual
 struct GatedResidualParams {
@@ -647,6 +652,21 @@ int launch_ln(const LnModParams& p, int dtype, void* stream) {
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
     return launched();
 }
+template <typename Desc>
+int launch_gated(const Desc* d, void* stream) {
+    GatedResidualParams p;
+    p.x = (const uint16_t*)d->x; p.tx = (const uint16_t*)d->tx; p.res = (const uint16_t*)d->res; p.tres = (const uint16_t*)d->tres;
+    p.gate = (const uint16_t*)d->gate; p.tgate = (const uint16_t*)d->tgate;
+    p.out = (uint16_t*)d->out; p.tout = (uint16_t*)d->tout;
+    p.chunks = d->rows * (d->D / 8); p.D = d->D; p.rows_per_group = d->rows_per_group;
+    const int64_t blocks = (p.chunks + kThreads - 1) / kThreads;
+    if (blocks > 0x7FFFFFFF) return COSMOS_ATTN_BAD_SHAPE;
+    const bool bf16 = d->dtype == COSMOS_ATTN_BF16;
+    auto fn = d->tx ? (bf16 ? gated_residual_kernel<true, true> : gated_residual_kernel<true, false>)
+                    : (bf16 ? gated_residual_kernel<false, true> : gated_residual_kernel<false, false>);
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
+    return launched();
+}
 int start_column_sums(ColumnSums& s, int64_t rows, int rows_per_group, int D, int vectors, void* out0, void* out1, void* workspace, size_t bytes) {
     plan_column_sums(s, rows, rows_per_group);
     s.out[0] = (uint16_t*)out0; s.out[1] = (uint16_t*)out1;
@@ -697,6 +717,11 @@ COSMOS_ATTN_API int cosmos_gated_residual_ln_modulate(const cosmos_gated_residua
     for (const void* q : ptrs) if (q && !aligned16(q)) return COSMOS_ATTN_BAD_STRIDE;
     LnModParams p = {};
     fill_ln(p, d);
+    if (d->D > kMaxGatedLnD) {
+        const int st = launch_gated(d, stream);
+        p.x = (const uint16_t*)d->out; p.tx = (const uint16_t*)d->tout;
+        return st == COSMOS_ATTN_OK ? launch_ln<false>(p, d->dtype, stream) : st;
+    }
     p.res = (const uint16_t*)d->res; p.tres = (const uint16_t*)d->tres;
     p.gate = (const uint16_t*)d->gate; p.tgate = (const uint16_t*)d->tgate;
     p.out = (uint16_t*)d->out; p.tout = (uint16_t*)d->tout;
@@ -713,18 +738,7 @@ COSMOS_ATTN_API int cosmos_gated_residual(const cosmos_gated_residual_desc* d, v
     if (d->D % 8 != 0 || d->rows % d->rows_per_group != 0) return COSMOS_ATTN_BAD_SHAPE;
     const void* ptrs[] = {d->x, d->tx, d->res, d->tres, d->gate, d->tgate, d->out, d->tout};
     for (const void* q : ptrs) if (q && !aligned16(q)) return COSMOS_ATTN_BAD_STRIDE;
-    GatedResidualParams p;
-    p.x = (const uint16_t*)d->x; p.tx = (const uint16_t*)d->tx; p.res = (const uint16_t*)d->res; p.tres = (const uint16_t*)d->tres;
-    p.gate = (const uint16_t*)d->gate; p.tgate = (const uint16_t*)d->tgate;
-    p.out = (uint16_t*)d->out; p.tout = (uint16_t*)d->tout;
-    p.chunks = d->rows * (d->D / 8); p.D = d->D; p.rows_per_group = d->rows_per_group;
-    const int64_t blocks = (p.chunks + kThreads - 1) / kThreads;
-    if (blocks > 0x7FFFFFFF) return COSMOS_ATTN_BAD_SHAPE;
-    const bool bf16 = d->dtype == COSMOS_ATTN_BF16;
-    auto fn = tangent ? (bf16 ? gated_residual_kernel<true, true> : gated_residual_kernel<true, false>)
-                      : (bf16 ? gated_residual_kernel<false, true> : gated_residual_kernel<false, false>);
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kThreads), 0, (hipStream_t)stream, p);
-    return launched();
+    return launch_gated(d, stream);
 }
 
 COSMOS_ATTN_API int cosmos_gelu(const cosmos_gelu_desc* d, void* stream) {

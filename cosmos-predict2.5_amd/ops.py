@@ -546,7 +546,7 @@ def gated_residual(x, res, gate, tx=None, tres=None, tgate=None, inplace: bool =
 def gated_residual_ln_modulate(x, res, gate, shift, scale, tx=None, tres=None, tgate=None, tshift=None, tscale=None,
                                eps: float = 1e-6, y=None, ty=None):
     """:func:`gated_residual` and :func:`ln_modulate` of its result in one pass (two, where ``gate`` and ``shift`` have different
-    ``G``): ``(out, tout, y, ty)``.  ``y`` / ``ty``: optional preallocated outputs."""
+    ``G``, or ``D > 5120``): ``(out, tout, y, ty)``.  ``y`` / ``ty``: optional preallocated outputs."""
     _check_elementwise(x)
     D = x.shape[-1]
     if gate.numel() != shift.numel():

@@ -287,7 +287,7 @@ typedef struct cosmos_gated_residual_desc {
     void *out, *tout;
 } cosmos_gated_residual_desc;
 
-/* Both, where the gated residual is what the LayerNorm reads:  out = x + gate res,  y = LayerNorm(out) (1 + scale) + shift.
+/* Both, where the gated residual is what the LayerNorm reads, in one launch (two where D > 5120):  out = x + gate res,  y = LayerNorm(out) (1 + scale) + shift.
  * Each of out, tout, y, ty may be x, tx, res or tres itself (what is written to has been read by then); the four are different buffers. */
 typedef struct cosmos_gated_residual_ln_modulate_desc {
     int32_t abi_version, dtype;
