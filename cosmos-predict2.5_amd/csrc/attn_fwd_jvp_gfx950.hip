@@ -1750,6 +1750,9 @@ size_t planned_partial_bytes(const cosmos_attn_desc* d) {
 // other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121 (one call, which cuts, with its
 // re-tiling: 67, 101); forward only 6500 x 1024 80 / 88, 6800 x 1536 115 / 119 (one call 83, 110).  With all tangents the
 // two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
+// Padded keys (key_lens, which the host does not read) are priced at their full length, so that a call at a tie may take the way that is slower on
+// its shorter rows: head dim 64, 700 x 700, 40 heads, stream / 4 x 2 (taken) 22.2 / 22.0, with half of the keys valid 15.7 / 17.9; 2 x 16 heads
+// 1000 x 1000 27.5 / 24.2 and 18.5 / 19.6.  (At head dims 16, 32 and 128 the way taken is no slower at any share of valid keys measured.)
 // cosmos_attn_set_stream_override() replaces the choice (tuning and tests); nothing in the per-call path reads the environment.
 constexpr int kStreamMaxTiles = 64;       // up to 2048 keys
 constexpr int kStreamGroupsPerCU = 1;       // one workgroup fills a compute unit (8 wavefronts, 2 per SIMD at 256 registers): a single round
