@@ -1121,7 +1121,7 @@ attn_qstream_kernel(const AttnParams p) {
 //
 // What bounds it: a SIMD issues one VALU or MFMA instruction in 4 cycles.  A tile of 32 keys costs a wavefront 16 MFMAs (512 cycles of
 // the matrix unit) and some 125 such turns, 64 of them in 16 exponentials; in long calls the part's power limit on top (80 % MFMA duty
-// at 1.56 GHz, 37440 positions; 66 % at 1.76 GHz before).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
+// at 1.53 GHz, 37440 positions; 66 % at 1.76 GHz before).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
 // formed where it did not move (kMaxTileSum).  Measured, us, before either / with the softmax between the MFMAs / with both: 16 heads,
 // d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120.
 // Not faster: v_mfma_f32_16x16x32 (less energy, but twice the MFMA instructions to issue: 37440 9450, 3520 142), operand fetches three
