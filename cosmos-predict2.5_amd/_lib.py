@@ -233,6 +233,21 @@ class ModulationDesc(ctypes.Structure):
     ]
 
 
+class GemmDesc(ctypes.Structure):
+    """Mirror of ``struct cosmos_attn_gemm_desc``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32), ("dtype", ctypes.c_int32), ("order", ctypes.c_int32), ("flags", ctypes.c_int32),
+        ("count", ctypes.c_int32), ("shape", ctypes.c_int32), ("rows", ctypes.c_int32), ("cols", ctypes.c_int32), ("depth", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("lda", ctypes.c_int64), ("ldb", ctypes.c_int64), ("ldc", ctypes.c_int64),
+        ("a", ctypes.c_void_p * 3), ("b", ctypes.c_void_p * 3), ("c", ctypes.c_void_p * 3),
+    ]
+
+
+GEMM_XWT, GEMM_XW, GEMM_XTX = 0, 1, 2
+GEMM_SUM = 1
+
 EXPORTS = {
     "cosmos_attn_abi_version": (ctypes.c_int, []),
     "cosmos_attn_status_string": (ctypes.c_char_p, [ctypes.c_int]),
@@ -260,6 +275,8 @@ EXPORTS = {
     "cosmos_gated_residual_bwd": (ctypes.c_int, [ctypes.POINTER(GatedResidualBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_ln_modulation_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(ModulationDesc)]),
     "cosmos_ln_modulation": (ctypes.c_int, [ctypes.POINTER(ModulationDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "cosmos_attn_gemm": (ctypes.c_int, [ctypes.POINTER(GemmDesc), ctypes.c_void_p]),
+    "cosmos_attn_gemm_preferred": (ctypes.c_int, [ctypes.POINTER(GemmDesc)]),
     "cosmos_gelu": (ctypes.c_int, [ctypes.POINTER(GeluDesc), ctypes.c_void_p]),
 }
 

@@ -1,4 +1,4 @@
-"""The DiT ``Attention`` module with ``backend="hip"``: projections (library GEMMs), fused RMSNorm + RoPE and the
+"""The DiT ``Attention`` module with ``backend="hip"``: projections (``linear.py``), fused RMSNorm + RoPE and the
 attention kernels of this package, with a forward that also carries a tangent.
 
 Reference: ``Attention`` in cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:286-440 -- same constructor
@@ -28,6 +28,7 @@ from torch import nn
 from . import ops
 from .attention import results_are_kept
 from .attn_op import HipAttnOp
+from .linear import linear
 
 
 class HeadRMSNormWeight(nn.Module):
@@ -138,12 +139,10 @@ class Attention(nn.Module):
         return both if both is not None else torch.cat([x, tx], dim=0)
 
     @staticmethod
-    def _apply_stacked(lin: nn.Linear, xs: torch.Tensor, has_tangent: bool):
-        y = lin(xs)
-        if not has_tangent:
-            return y, None
-        b = y.shape[0] // 2
-        return y[:b], y[b:]
+    def _apply_stacked(layers, xs: torch.Tensor, has_tangent: bool):
+        """(primal, tangent) of each layer on the stacked input."""
+        b = xs.shape[0] // 2
+        return [(y[:b], y[b:]) if has_tangent else (y, None) for y in linear(layers, xs)]
 
     def _norm_rope(self, t, norm: HeadRMSNormWeight, rope_emb, tt=None):
         rope = rope_emb if (self.is_selfattn and rope_emb is not None) else None   # only for self-attention (:409)
@@ -167,8 +166,9 @@ class Attention(nn.Module):
             hit = self._context_cache.get(slot)
             if hit is not None and hit[0]() is context and hit[1] == key:
                 return hit[2]
-        k, _ = self._norm_rope(self._heads(k_proj(context)), k_norm, None)
-        v = self._heads(v_proj(context))
+        k, v = linear([k_proj, v_proj], context)
+        k, _ = self._norm_rope(self._heads(k), k_norm, None)
+        v = self._heads(v)
         packed = ops.pack_kv(k.transpose(1, 2), v.transpose(1, 2))
         if cacheable:
             self._context_cache[slot] = (weakref.ref(context), key, packed)
@@ -190,25 +190,26 @@ class Attention(nn.Module):
     # ------------------------------------------------------------------ the reference's surface
     def compute_qkv(self, x, context=None, rope_emb=None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """q, k, v as ``[B, S, H, D]`` (q and k in heads-first memory, ready for the kernels)."""
-        context = x if context is None else context
-        q = self._heads(self.q_proj(x))
-        k = self._heads(self.k_proj(context))
-        v = self._heads(self.v_norm(self.v_proj(context)))
+        if context is None:
+            q, k, v = linear([self.q_proj, self.k_proj, self.v_proj], x)
+        else:
+            (q,), (k, v) = linear([self.q_proj], x), linear([self.k_proj, self.v_proj], context)
+        q, k, v = self._heads(q), self._heads(k), self._heads(self.v_norm(v))
         q, _ = self._norm_rope(q, self.q_norm, rope_emb)
         k, _ = self._norm_rope(k, self.k_norm, rope_emb)
         return q, k, v
 
     def compute_attention(self, q, k, v, video_size=None):
         result = self.attn_op(q, k, v, video_size=video_size)   # [B, S, H*D]
-        return self.output_dropout(self.output_proj(result))
+        return self.output_dropout(linear([self.output_proj], result)[0])
 
     def forward(self, x, context: Optional[torch.Tensor] = None, rope_emb: Optional[torch.Tensor] = None, video_size=None):
         """x: ``[B, Mq, K]`` (or ``[B, T, H, W, K]``); context: ``[B, Mk, Kc]`` or None for self-attention; rope_emb: the
         angles ``[Mq, 1, 1, D]`` (self-attention only).  Returns ``[B, Mq, K]`` in the shape of x."""
         if self._context_is_fixed(x, context):
-            q, _ = self._norm_rope(self._heads(self.q_proj(x)), self.q_norm, rope_emb)
+            q, _ = self._norm_rope(self._heads(linear([self.q_proj], x)[0]), self.q_norm, rope_emb)
             packed = self._packed_context("context", context, self.k_proj, self.k_norm, self.v_proj)
-            out = self.output_dropout(self.output_proj(self.attn_op.forward_packed(q, packed)))
+            out = self.output_dropout(linear([self.output_proj], self.attn_op.forward_packed(q, packed))[0])
             return out.reshape(*x.shape[:-1], out.shape[-1])
         q, k, v = self.compute_qkv(x, context, rope_emb=rope_emb)
         out = self.compute_attention(q, k, v, video_size=video_size)
@@ -226,27 +227,25 @@ class Attention(nn.Module):
         if isinstance(self.output_dropout, nn.Dropout) and self.training:
             raise NotImplementedError("forward_jvp with active dropout")
         xs = self._stack(x, tx)
-        q, tq = self._apply_stacked(self.q_proj, xs, True)
         if tcontext is None and self._context_is_fixed(x, context):
+            ((q, tq),) = self._apply_stacked([self.q_proj], xs, True)
             q, tq = self._norm_rope(self._heads(q), self.q_norm, rope_emb, self._heads(tq))
             packed = self._packed_context("context", context, self.k_proj, self.k_norm, self.v_proj)
             o, to = self.attn_op.forward_packed(q, packed, tq)
-            out, tout = self._apply_stacked(self.output_proj, self._stack(o, to), True)
+            ((out, tout),) = self._apply_stacked([self.output_proj], self._stack(o, to), True)
             shape = (*x.shape[:-1], out.shape[-1])
             return out.reshape(shape), tout.reshape(shape)
         if context is None:
-            k, tk = self._apply_stacked(self.k_proj, xs, True)
-            v, tv = self._apply_stacked(self.v_proj, xs, True)
+            (q, tq), (k, tk), (v, tv) = self._apply_stacked([self.q_proj, self.k_proj, self.v_proj], xs, True)
         else:
             assert tcontext is None or tcontext.shape == context.shape
-            cs = self._stack(context, tcontext)
-            k, tk = self._apply_stacked(self.k_proj, cs, tcontext is not None)
-            v, tv = self._apply_stacked(self.v_proj, cs, tcontext is not None)
+            ((q, tq),) = self._apply_stacked([self.q_proj], xs, True)
+            (k, tk), (v, tv) = self._apply_stacked([self.k_proj, self.v_proj], self._stack(context, tcontext), tcontext is not None)
         h = self._heads
         q, tq = self._norm_rope(h(q), self.q_norm, rope_emb, h(tq))
         k, tk = self._norm_rope(h(k), self.k_norm, rope_emb, None if tk is None else h(tk))
         o, to = self.attn_op.forward_jvp(q, k, h(v), tq, tk, None if tv is None else h(tv))
-        out, tout = self._apply_stacked(self.output_proj, self._stack(o, to), True)
+        ((out, tout),) = self._apply_stacked([self.output_proj], self._stack(o, to), True)
         shape = (*x.shape[:-1], out.shape[-1])
         return out.reshape(shape), tout.reshape(shape)
 
@@ -273,23 +272,23 @@ class I2VCrossAttention(Attention):
     def compute_qkv(self, x, context, rope_emb=None):
         text_context, img_context = context
         q, k, v = super().compute_qkv(x, text_context, rope_emb)
-        k_img, _ = self._norm_rope(self._heads(self.k_img(img_context)), self.k_img_norm, None)
-        v_img = self._heads(self.v_img(img_context))
-        return q, k, v, k_img, v_img
+        k_img, v_img = linear([self.k_img, self.v_img], img_context)
+        k_img, _ = self._norm_rope(self._heads(k_img), self.k_img_norm, None)
+        return q, k, v, k_img, self._heads(v_img)
 
     def compute_attention(self, q, k, v, k_img, v_img):
         result = self.attn_op(q, k, v)
         result_img = self.attn_op(q, k_img, v_img)
-        return self.output_dropout(self.output_proj(result + result_img))
+        return self.output_dropout(linear([self.output_proj], result + result_img)[0])
 
     def forward(self, x, context=None, rope_emb=None, video_size=None):
         del video_size
         if x.is_cuda and not torch.is_grad_enabled() and not results_are_kept():
             text_context, img_context = context
-            q, _ = self._norm_rope(self._heads(self.q_proj(x)), self.q_norm, rope_emb)
+            q, _ = self._norm_rope(self._heads(linear([self.q_proj], x)[0]), self.q_norm, rope_emb)
             result = self.attn_op.forward_packed(q, self._packed_context("text", text_context, self.k_proj, self.k_norm, self.v_proj))
             result_img = self.attn_op.forward_packed(q, self._packed_context("image", img_context, self.k_img, self.k_img_norm, self.v_img))
-            out = self.output_dropout(self.output_proj(result + result_img))
+            out = self.output_dropout(linear([self.output_proj], result + result_img)[0])
             return out.reshape(*x.shape[:-1], out.shape[-1])
         q, k, v, k_img, v_img = self.compute_qkv(x, context, rope_emb)
         out = self.compute_attention(q, k, v, k_img, v_img)
@@ -302,7 +301,7 @@ class I2VCrossAttention(Attention):
         assert tx is not None and tx.shape == x.shape
         text_context, img_context = context
         h = self._heads
-        q, tq = self._apply_stacked(self.q_proj, self._stack(x, tx), True)
+        ((q, tq),) = self._apply_stacked([self.q_proj], self._stack(x, tx), True)
         q, tq = self._norm_rope(h(q), self.q_norm, rope_emb, h(tq))
         if x.is_cuda:
             o, to = self.attn_op.forward_packed(q, self._packed_context("text", text_context, self.k_proj, self.k_norm, self.v_proj), tq)
@@ -315,6 +314,6 @@ class I2VCrossAttention(Attention):
             o2, to2 = self.attn_op.forward_jvp(q, k_img, v_img, tq)
         o.add_(o2)
         to.add_(to2)
-        out, tout = self._apply_stacked(self.output_proj, self._stack(o, to), True)
+        ((out, tout),) = self._apply_stacked([self.output_proj], self._stack(o, to), True)
         shape = (*x.shape[:-1], out.shape[-1])
         return out.reshape(shape), tout.reshape(shape)

@@ -25,6 +25,7 @@ from torch import nn
 
 from . import ops
 from .dit_attention import Attention, I2VCrossAttention
+from .linear import bare, linear
 
 
 def _per_row(m, like):
@@ -159,12 +160,6 @@ class _ModulationFn(torch.autograd.Function):
 _FUSED_MODULATION_ROWS = 64
 
 
-def _bare(m: nn.Module) -> bool:
-    """Is calling m the same as computing its forward?"""
-    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
-                or nn.modules.module._has_any_global_hook())
-
-
 class GPT2FeedForward(nn.Module):
     def __init__(self, d_model: int, d_ff: int):
         super().__init__()
@@ -186,20 +181,20 @@ class GPT2FeedForward(nn.Module):
         torch.nn.init.trunc_normal_(self.layer2.weight, std=std, a=-3 * std, b=3 * std)
 
     def forward(self, x: torch.Tensor):
-        h = self.layer1(x)
+        (h,) = linear([self.layer1], x)
         if h.is_cuda and h.numel() % 8 == 0 and h.dtype in (torch.bfloat16, torch.float16):
             if torch.is_grad_enabled() and h.requires_grad:
-                return self.layer2(_GeluFn.apply(h))
-            return self.layer2(ops.gelu(h, inplace=True)[0])      # inference: one fused pass, in place
+                return linear([self.layer2], _GeluFn.apply(h))[0]
+            return linear([self.layer2], ops.gelu(h, inplace=True)[0])[0]      # inference: one fused pass, in place
         return self.layer2(self.activation(h))
 
     @torch.no_grad()
     def forward_jvp(self, x: torch.Tensor, tx: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         b = x.shape[0]
         both = ops.as_stacked(x, tx)
-        h = self.layer1(both if both is not None else torch.cat([x, tx], dim=0))
+        (h,) = linear([self.layer1], both if both is not None else torch.cat([x, tx], dim=0))
         ops.gelu(h[:b], h[b:], inplace=True)       # a = gelu(h), ta = th gelu'(h), in place on the stacked buffer
-        y = self.layer2(h)
+        (y,) = linear([self.layer2], h)
         return y[:b], y[b:]
 
 
@@ -298,7 +293,7 @@ class Block(nn.Module):
         mods = (self.adaln_modulation_self_attn, self.adaln_modulation_cross_attn, self.adaln_modulation_mlp)
         w1, w2 = [], []
         for m in mods:
-            if type(m) is not nn.Sequential or len(m) != 3 or not _bare(m) or not all(_bare(c) for c in m):
+            if type(m) is not nn.Sequential or len(m) != 3 or not bare(m) or not all(bare(c) for c in m):
                 return None
             if type(m[0]) is not nn.SiLU or any(type(c) is not nn.Linear or c.bias is not None or type(c.weight) is not nn.Parameter for c in m[1:]):
                 return None

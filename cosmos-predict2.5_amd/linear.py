@@ -1,0 +1,91 @@
+"""Linear layers without bias (``nn.Linear``: the projections and the MLP of a block, cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:226-227,
+:349-358) on the package's own matrix products where those are faster, several layers of one input in a launch; ``nn.Linear`` itself elsewhere.
+
+The parameters stay where they are.  Whatever gives calling the module a meaning of its own (hooks, another class, a parametrization, autocast, function
+transforms, forward-mode AD, compilation, tensor subclasses) goes through the module.
+"""
+from __future__ import annotations
+
+from typing import Optional, Sequence
+
+import torch
+import torch.nn.functional as F
+from torch import nn
+from torch.autograd import forward_ad
+
+from . import ops
+
+
+def bare(m: nn.Module) -> bool:
+    """Is calling m the same as computing its forward?"""
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
+                or nn.modules.module._has_any_global_hook())
+
+
+def _weights(layers: Sequence[nn.Module], x: torch.Tensor) -> Optional[list]:
+    """The layers' weights, if their products with x may be formed by ``ops.gemm``."""
+    if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or type(x) is not torch.Tensor or x.numel() == 0:
+        return None
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0:
+        return None
+    if torch._C._functorch.is_functorch_wrapped_tensor(x) or not ops._is_dense16(x):
+        return None
+    ws = []
+    for m in layers:
+        if type(m) is not nn.Linear or m.bias is not None or not bare(m):
+            return None
+        w = m.weight
+        if type(w) is not nn.Parameter or torch._C._functorch.is_functorch_wrapped_tensor(w) or w.dtype != x.dtype or w.device != x.device or w.shape != layers[0].weight.shape or not ops._is_dense16(w):
+            return None
+        ws.append(w)
+    if ws[0].shape[1] != x.shape[-1]:
+        return None
+    return ws
+
+
+class _LinearFn(torch.autograd.Function):
+    """``x w_i^T`` for up to three weights of one shape: the outputs in one launch, their part of x's gradient summed in one, the weights' gradients in one."""
+
+    @staticmethod
+    def forward(ctx, made, x, *w):
+        ctx.save_for_backward(x, *w)
+        ctx.set_materialize_grads(False)
+        return tuple(made if made is not None else [F.linear(x, v) for v in w])
+
+    @staticmethod
+    def backward(ctx, *dy):
+        x, *w = ctx.saved_tensors
+        given = [i for i, g in enumerate(dy) if g is not None]
+        x2 = x.reshape(-1, x.shape[-1])
+        g2 = {i: dy[i].reshape(-1, dy[i].shape[-1]) for i in given}
+        dx, dw = None, [None] * len(w)
+        own = not torch.is_grad_enabled()        # (create_graph: the gradients are differentiated again)
+        if own:
+            g2 = {i: ops._dense16(g) for i, g in g2.items()}
+        if ctx.needs_input_grad[1] and given:
+            gs, ws = [g2[i] for i in given], [w[i] for i in given]
+            dx = ops.gemm("xw", gs, ws, total=True, if_preferred=True) if own else None
+            if dx is None:
+                for g, v in zip(gs, ws):
+                    dx = g @ v if dx is None else dx + g @ v
+            dx = dx.reshape(x.shape)
+        wanted = [i for i in given if ctx.needs_input_grad[2 + i]]
+        if wanted:
+            made = ops.gemm("xtx", [g2[i] for i in wanted], [x2] * len(wanted), if_preferred=True) if own else None
+            for k, i in enumerate(wanted):
+                dw[i] = made[k] if made is not None else g2[i].t() @ x2
+        return (None, dx, *dw)
+
+
+def linear(layers: Sequence[nn.Module], x: torch.Tensor) -> list:
+    """``[m(x) for m in layers]``: up to three layers without bias."""
+    ws = _weights(layers, x)
+    if ws is None:
+        return [m(x) for m in layers]
+    rows = x.numel() // x.shape[-1]
+    with torch.no_grad():
+        made = ops.gemm("xwt", [x.view(rows, -1)] * len(ws), ws, if_preferred=True, lead=x.shape[:-1])
+    if torch.is_grad_enabled() and (x.requires_grad or any(w.requires_grad for w in ws)):
+        # (the products of the backward pass are chosen there; below 256 rows they are the library's like these)
+        return list(_LinearFn.apply(made, x, *ws)) if made is not None or rows >= 256 else [m(x) for m in layers]
+    return made if made is not None else [m(x) for m in layers]

@@ -651,6 +651,52 @@ def modulation(emb, lora, w1, w2, temb=None, tlora=None, tangent: bool = False):
     return out, tout
 
 
+GEMM_ORDERS = {"xwt": _lib.GEMM_XWT, "xw": _lib.GEMM_XW, "xtx": _lib.GEMM_XTX}
+
+
+def _gemm_desc(order: str, a, b, total: bool, shape: int) -> "_lib.GemmDesc":
+    D = _lib.GemmDesc()
+    D.abi_version, D.dtype, D.order = _lib.ABI_VERSION, _DTYPES[a[0].dtype], GEMM_ORDERS[order]
+    D.flags, D.count, D.shape = (_lib.GEMM_SUM if total else 0), len(a), shape
+    D.rows, D.depth = a[0].shape if order != "xtx" else a[0].shape[::-1]
+    D.cols = b[0].shape[1] if order != "xwt" else b[0].shape[0]
+    D.lda, D.ldb, D.ldc = a[0].stride(0), b[0].stride(0), D.cols
+    for i in range(len(a)):
+        D.a[i], D.b[i] = a[i].data_ptr(), b[i].data_ptr()
+    return D
+
+
+def gemm(order: str, a, b, total: bool = False, shape: int = 0, if_preferred: bool = False, lead=None):
+    """Up to three matrix products of one shape in one launch, 16-bit matrices, fp32 sums.  ``order``: "xwt" ``a [rows, depth]`` by the transpose of
+    ``b [cols, depth]``; "xw" ``a [rows, depth]`` by ``b [depth, cols]``; "xtx" the transpose of ``a [depth, rows]`` by ``b [depth, cols]``.  Returns the
+    list of ``[rows, cols]`` products; with ``total`` their sum alone.  Lines are read where they are (any line stride that is a multiple of 8).
+    ``if_preferred``: None instead where the library's products are faster or the kernel does not take the matrices.  ``lead``: dimensions that the
+    outputs have in the place of their rows."""
+    assert 1 <= len(a) == len(b) <= 3
+    _check_elementwise(a[0])
+    for group, like in ((a, a[0]), (b, b[0])):
+        for t in group:
+            if t.dim() != 2 or t.shape != like.shape or t.stride() != like.stride() or t.stride(1) != 1:
+                raise ValueError("the matrices of a launch need one shape and one line stride, with elements of a line side by side")
+            if t.dtype != a[0].dtype or t.device != a[0].device:
+                raise ValueError("the matrices of a launch need one type and device")
+    D = _gemm_desc(order, a, b, total, shape)
+    depth = b[0].shape[1] if order == "xwt" else b[0].shape[0]
+    if D.depth != depth:
+        raise ValueError("the matrices' contractions differ")
+    n = 1 if total else len(a)
+    if if_preferred:
+        for i in range(n):
+            D.c[i] = 16            # (the outputs are allocated only where they are written)
+        if not _lib.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)):
+            return None
+    outs = [torch.empty((*(lead or (D.rows,)), D.cols), device=a[0].device, dtype=a[0].dtype) for _ in range(n)]
+    for i, o in enumerate(outs):
+        D.c[i] = o.data_ptr()
+    _launch("cosmos_attn_gemm", D, a[0].device)
+    return outs[0] if total else outs
+
+
 def gelu(h, th=None, inplace: bool = False):
     """Exact (erf) GELU and its tangent ``th * gelu'(h)`` in one pass (``nn.GELU()`` of
     cosmos_predict2/_src/predict2/networks/minimal_v4_dit.py:225).  Returns ``(a, ta)``."""

@@ -364,6 +364,35 @@ typedef struct cosmos_ln_modulation_desc {
 COSMOS_ATTN_API size_t cosmos_ln_modulation_workspace_bytes(const cosmos_ln_modulation_desc *desc);
 COSMOS_ATTN_API int cosmos_ln_modulation(const cosmos_ln_modulation_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * Matrix products of the linear layers (networks/minimal_v4_dit.py:226-227, :349-358: nn.Linear without bias), 16-bit operands, fp32 sums:
+ *     out[rows, cols] = sum over the contraction of A B       with A and B as a layer y = x w^T and its backward pass have them,
+ *     XWT: A [rows, depth], B [cols, depth]   (y = x w^T)
+ *     XW:  A [rows, depth], B [depth, cols]   (dx = dy w)
+ *     XTX: A [depth, rows], B [depth, cols]   (dw = dy^T x)
+ * Up to three products of one shape in a launch, each with its own output, or (COSMOS_GEMM_SUM) all summed into c[0].
+ * cols % 8 == 0; depth % 64 == 0 but for XTX, where rows % 8 == 0; lda, ldb, ldc (elements between the lines of an operand) % 8 == 0; all
+ * pointers at multiples of 16 bytes; an operand's last byte less than 4 GiB behind its first.  Writes nothing but the outputs; no workspace.
+ */
+enum cosmos_attn_gemm_order { COSMOS_GEMM_XWT = 0, COSMOS_GEMM_XW = 1, COSMOS_GEMM_XTX = 2 };
+#define COSMOS_GEMM_SUM 1
+typedef struct cosmos_attn_gemm_desc {
+    int32_t abi_version, dtype;
+    int32_t order;                     /* enum cosmos_attn_gemm_order */
+    int32_t flags;                     /* 0 or COSMOS_GEMM_SUM */
+    int32_t count;                     /* products, 1 .. 3 */
+    int32_t shape;                     /* 0: the library's choice of tiles; 1 .. 4 (tuning and tests): 256x256, 256x128, 128x256, 128x128 */
+    int32_t rows, cols, depth;
+    int32_t reserved;
+    int64_t lda, ldb, ldc;
+    const void *a[3], *b[3];
+    void *c[3];
+} cosmos_attn_gemm_desc;
+
+COSMOS_ATTN_API int cosmos_attn_gemm(const cosmos_attn_gemm_desc *desc, void *stream);
+/* 1 where cosmos_attn_gemm takes the call and is faster than the vendor library's product (or products and additions), 0 elsewhere.  Looks at sizes only. */
+COSMOS_ATTN_API int cosmos_attn_gemm_preferred(const cosmos_attn_gemm_desc *desc);
+
 #ifdef __cplusplus
 }
 #endif
