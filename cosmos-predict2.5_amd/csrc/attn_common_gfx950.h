@@ -97,6 +97,60 @@ __device__ __forceinline__ void issue_part(__amdgpu_buffer_rsrc_t rsrc, char* ds
     if (LOADS > 3) lds_load<3 * kFragBytes>(rsrc, dst, lane_off, src);
 }
 
+// ---- K and V read where they are (head dim 128): no re-tiling pass in front of a short call.
+// Parts of 32 keys in LDS, every load a run of whole 128-byte lines (a load whose lanes take 32 bytes of each of 32 rows, which would make the fragment order of the
+// re-tiled image, runs at half of the rate and costs a step 8 %):
+//   K: two halves of 32 rows x 128 bytes, 16-byte chunk c of row r at c XOR (r / 2) % 8: a K-type fragment is one ds_read_b128 per lane, from one of four lane addresses;
+//   V: 32 rows x 256 bytes, chunk c of row r at c XOR 4 (r % 4): a V^T fragment is two ds_read_b64_tr_b16 (within 16 lanes, lane i passes the address of 8 bytes, row
+//   i of a 16 x 4 matrix M, and receives M[i/4 + 4k][i%4], k = 0..3).
+// Neither has bank conflicts.
+typedef unsigned raw_u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned raw_u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kRawRow = 256;                     // bytes of a row
+struct RawFill {
+    __amdgpu_buffer_rsrc_t rsrc;                 // one (batch, head)'s rows: bytes behind the last row read as zeros
+    int row_bytes;                               // between rows
+    __device__ __forceinline__ RawFill(const void* head, int64_t row_stride, int rows)
+        : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(head), 0, (int)((rows - 1) * row_stride * 2) + kRawRow, 0x00020000)), row_bytes((int)row_stride * 2) {}
+    // K: the 1 KB blocks q .. q + N - 1 (half q / 4, rows 8 (q % 4) .. + 7) of the 32 keys from row `key` on
+    template <int N> __device__ __forceinline__ void k(char* dst, int key, int q, int lane) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int half = (q + i) >> 2, r8 = (q + i) & 3;
+            const int off = (key + 8 * r8 + (lane >> 3)) * row_bytes + half * 128 + (((lane & 7) ^ (4 * (r8 & 1) + (lane >> 4))) << 4);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + i * kFragBytes), 16, off, 0, 0, 0);
+        }
+    }
+    // V: 4 N rows from row `key` on
+    template <int N> __device__ __forceinline__ void v(char* dst, int key, int lane) const {
+        const int off = (key + (lane >> 4)) * row_bytes + (((lane & 15) ^ (4 * ((lane >> 4) & 3))) << 4);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(dst + i * kFragBytes), 16, off + 4 * i * row_bytes, 0, 0, 0);
+    }
+};
+// where this lane reads K-type fragment c % 4 of a K part's first half; that of the second half (c >= 4) lies 4096 behind
+__device__ __forceinline__ int raw_k_offset(int c, int lane) {
+    const int row = lane & 31;
+    return row * 128 + (((2 * c + (lane >> 5)) ^ ((row >> 1) & 7)) << 4);
+}
+// where this lane reads V^T fragment (db, 0) of a V part, from the part's start; fragment (db, c) lies 4096 c behind, its second half of keys 2048
+__device__ __forceinline__ unsigned raw_vt_offset(int db, int lane) {
+    const int i = lane & 15, key = 4 * (lane >> 5) + (i >> 2), chunk = 4 * db + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+    return (unsigned)(key * kRawRow + ((chunk ^ (4 * (i >> 2))) << 4) + 8 * (i & 1));
+}
+// a fragment on its way: valid behind a wait, made so by landed()
+struct RawVt {
+    raw_u32x2 lo, hi;
+    template <int OFF> __device__ __forceinline__ void read(unsigned a) {
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(lo) : "v"(a), "n"(OFF));
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(hi) : "v"(a), "n"(OFF + 8 * kRawRow));
+    }
+    __device__ __forceinline__ void landed() { asm volatile("" : "+v"(lo), "+v"(hi)); }
+    template <typename V8> __device__ __forceinline__ V8 get() const { return __builtin_bit_cast(V8, raw_u32x4{lo.x, lo.y, hi.x, hi.y}); }
+};
+template <int N> __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory"); }
+
 // Four units of a V^T-type section (channels 4 quad .. + 3, key chunk c, lane half hh of the 32-key tile at row key0): eight 8-byte
 // loads, one per key, of which 32 neighbouring threads cover whole rows of 128 channels, transposed in registers into four 16-byte
 // stores side by side.  Channels past `width` and rows past `rows` become zeros.

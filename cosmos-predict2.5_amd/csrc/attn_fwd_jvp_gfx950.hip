@@ -144,6 +144,8 @@ struct AttnParams {
     int64_t o_sb, o_sh, o_sl;
     float* lse;
     const char* kv;            // packed tiles [B*H][n_tiles][tile bytes]
+    const uint16_t *k, *v, *tk, *tv;                 // or (RAW kernels) the tensors themselves
+    int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl;
     const int32_t* key_lens;   // nullable
     int H, Lq, Lkv, n_tiles, causal;
     float sm_scale, scale_log2;
@@ -199,7 +201,7 @@ __device__ __forceinline__ void issue_group(const LoadJob& j) {
 // Score wavefront: owns 32 query rows' Q, dQ fragments and softmax statistics.  Per step it issues the score
 // MFMAs of the NEXT tile interleaved with the softmax VALU work of the current one, and hands P^T, H^T (16-bit
 // MFMA B operands) and the rescale factor of the tile to its output wavefront through LDS.
-template <typename T, int DQK, int DV, int MODE>
+template <typename T, int DQK, int DV, int MODE, bool RAW = false>
 struct ScoreWave {
     typedef AttnCfg<DQK, DV, MODE> C;
     typedef typename VecOf<T>::v8 V8;
@@ -218,6 +220,11 @@ struct ScoreWave {
 
     __device__ __forceinline__ V8 lds_frag(const char* base, int frag) const {
         return *reinterpret_cast<const V8*>(base + frag * kFragBytes + lane * 16);
+    }
+
+    int k_off[RAW ? 4 : 1];                 // RAW: raw_k_offset
+    __device__ __forceinline__ V8 k_frag(const char* base, int c) const {
+        return RAW ? *reinterpret_cast<const V8*>(base + k_off[c & 3] + (c >> 2) * 4096) : lds_frag(base, c);
     }
 
     __device__ __forceinline__ static float lane_max(const Scores& x) {
@@ -281,14 +288,14 @@ struct ScoreWave {
         V8 fa[NC], fb[NC];
         asm volatile("ds_write_b32 %0, %1" ::"v"(alpha_out + 4 * lane), "v"(alpha) : "memory");
 #pragma unroll
-        for (int i = 0; i < PD && i < NC; ++i) { fa[i] = lds_frag(kpart, i); if (FULL) fb[i] = lds_frag(kpart + C::DK_OFF, i); }
+        for (int i = 0; i < PD && i < NC; ++i) { fa[i] = k_frag(kpart, i); if (FULL) fb[i] = k_frag(kpart + C::DK_OFF, i); }
 #pragma unroll
         for (int e = 0; e < 16; ++e) { xn.s[e] = 0.f; xn.ds[e] = 0.f; }
         constexpr int EPC = 16 / NC;   // softmax elements dealt out per chunk (NC <= 8)
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             SCHED_FENCE();
-            if (c + PD < NC) { fa[c + PD] = lds_frag(kpart, c + PD); if (FULL) fb[c + PD] = lds_frag(kpart + C::DK_OFF, c + PD); }
+            if (c + PD < NC) { fa[c + PD] = k_frag(kpart, c + PD); if (FULL) fb[c + PD] = k_frag(kpart + C::DK_OFF, c + PD); }
             SCHED_FENCE();
             xn.s = mfma32(fa[c], qf[c], xn.s);
 #pragma unroll
@@ -328,10 +335,10 @@ struct ScoreWave {
         for (int e = 0; e < 16; ++e) { x.s[e] = 0.f; x.ds[e] = 0.f; }
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            const V8 kf = lds_frag(kpart, c);
+            const V8 kf = k_frag(kpart, c);
             if (JVP) x.ds = mfma32(kf, tqf[c], x.ds);
             x.s = mfma32(kf, qf[c], x.s);
-            if (FULL) x.ds = mfma32(lds_frag(kpart + C::DK_OFF, c), qf[c], x.ds);
+            if (FULL) x.ds = mfma32(k_frag(kpart + C::DK_OFF, c), qf[c], x.ds);
         }
     }
 };
@@ -339,7 +346,7 @@ struct ScoreWave {
 // ---------------------------------------------------------------------------------------------------------------
 // Output wavefront: owns the fp32 accumulators O^T and T^T (= (P dV + H V)^T; the reference keeps the two terms
 // apart, JVP:134-146, but only ever uses their sum, JVP:369) of the same 32 query rows.
-template <typename T, int DQK, int DV, int MODE>
+template <typename T, int DQK, int DV, int MODE, bool RAW = false>
 struct OutputWave {
     typedef AttnCfg<DQK, DV, MODE> C;
     typedef typename VecOf<T>::v8 V8;
@@ -358,6 +365,63 @@ struct OutputWave {
         const int c = g / NDB, db = g % NDB;
         a = lds_frag(vpart, 2 * db + c);
         if (FULL) b = lds_frag(vpart + C::DVT_OFF, 2 * db + c);
+    }
+
+    // The same with V and dV in rows (RAW): every LDS read of the step is asm with its own waits, as the transposing reads are (the compiler's count of
+    // outstanding reads does not know of them), kRawAhead groups of four ahead.
+    static constexpr int kRawAhead = 3;
+    unsigned vt_off[RAW ? NDB : 1];
+    template <int G> __device__ __forceinline__ void read_vt(RawVt* fa, RawVt* fb, unsigned vpart) const {
+        if constexpr (G < NB) {
+            const unsigned at = vpart + vt_off[G % NDB];
+            fa[G].template read<(G / NDB) * 16 * kRawRow>(at);
+            fb[G].template read<(G / NDB) * 16 * kRawRow + C::DVT_OFF>(at);
+        }
+    }
+    template <int G> __device__ __forceinline__ void raw_groups(RawVt* fa, RawVt* fb, const raw_u32x4* ph, unsigned vpart) {
+        if constexpr (G < NB) {
+            constexpr int AHEAD = NB - 1 - G < kRawAhead ? NB - 1 - G : kRawAhead, c = G / NDB, db = G % NDB;
+            SCHED_FENCE();
+            read_vt<G + kRawAhead>(fa, fb, vpart);
+            wait_lds<4 * AHEAD>();
+            fa[G].landed();
+            fb[G].landed();
+            SCHED_FENCE();
+            const V8 pf = __builtin_bit_cast(V8, ph[c]), hf = __builtin_bit_cast(V8, ph[2 + c]), a = fa[G].template get<V8>();
+            acc[db] = mfma32(a, pf, acc[db]);
+            acct[db] = mfma32(a, hf, acct[db]);
+            acct[db] = mfma32(fb[G].template get<V8>(), pf, acct[db]);
+            raw_groups<G + 1>(fa, fb, ph, vpart);
+        }
+    }
+    __device__ __forceinline__ void raw_step(unsigned vpart, unsigned ph_in, unsigned alpha_in) {
+        static_assert(!RAW || FULL, "built for all tangents");
+        float alpha;
+        raw_u32x4 ph[4];
+        const unsigned pa = ph_in + 16 * lane;
+        asm volatile("ds_read_b32 %0, %1" : "=v"(alpha) : "v"(alpha_in + 4 * lane));
+        asm volatile("ds_read_b128 %0, %1" : "=v"(ph[0]) : "v"(pa));
+        asm volatile("ds_read_b128 %0, %1 offset:1024" : "=v"(ph[1]) : "v"(pa));
+        asm volatile("ds_read_b128 %0, %1 offset:2048" : "=v"(ph[2]) : "v"(pa));
+        asm volatile("ds_read_b128 %0, %1 offset:3072" : "=v"(ph[3]) : "v"(pa));
+        RawVt fa[NB], fb[NB];
+        read_vt<0>(fa, fb, vpart);
+        read_vt<1>(fa, fb, vpart);
+        read_vt<2>(fa, fb, vpart);
+        wait_lds<4 * kRawAhead>();
+        asm volatile("" : "+v"(alpha), "+v"(ph[0]), "+v"(ph[1]), "+v"(ph[2]), "+v"(ph[3]));
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int i = 0; i < NDB; ++i) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {       // (v_mul_legacy_f32 as in step())
+                    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(acc[i][e]) : "v"(alpha), "v"(acc[i][e]));
+                    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(acct[i][e]) : "v"(alpha), "v"(acct[i][e]));
+                }
+            }
+        }
+        raw_groups<0>(fa, fb, ph, vpart);
+        SCHED_FENCE();
     }
 
     // One step: O^T = alpha O^T + V^T P^T ;  T^T = alpha T^T + V^T H^T + dV^T P^T
@@ -396,13 +460,14 @@ struct OutputWave {
     }
 };
 
-template <typename T, int DQK, int DV, int MODE>
+template <typename T, int DQK, int DV, int MODE, bool RAW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kAttnThreads, kAttnThreads), amdgpu_waves_per_eu(2, 2)))
 attn_fwd_jvp_kernel(const AttnParams p) {
     static_assert(MODE != MODE_FWD, "forward only is attn_fwd_sym_kernel's job");
+    static_assert(!RAW || (DQK == 128 && DV == 128 && MODE == MODE_JVP_FULL), "rows of 256 bytes");
     typedef AttnCfg<DQK, DV, MODE> C;
-    typedef ScoreWave<T, DQK, DV, MODE> SW;
-    typedef OutputWave<T, DQK, DV, MODE> OW;
+    typedef ScoreWave<T, DQK, DV, MODE, RAW> SW;
+    typedef OutputWave<T, DQK, DV, MODE, RAW> OW;
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
     constexpr int NC = C::NC, NDB = C::NDB;
@@ -465,7 +530,18 @@ attn_fwd_jvp_kernel(const AttnParams p) {
     // (positions past the end of the sweep wrap around: that data is loaded but never used, so that every
     // wavefront always issues the same number of loads)
     // The output wavefronts issue all fills (their instruction stream has room; the score wavefronts' has not).
-    if (!score_role) {
+    // RAW: wavefront pairs 0, 1 fill halves of K and V, 2, 3 of dK and dV
+    const RawFill raw_k((qw < 2 ? p.k : p.tk) + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh, p.k_sl, p.Lkv),
+                  raw_v((qw < 2 ? p.v : p.tv) + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh, p.v_sl, p.Lkv);
+    auto raw_fill_k = [&](int t, int u) { raw_k.template k<4>(kring + (u % kRingK) * KP_BYTES + k_run, t * kBlockN, 4 * (qw & 1), lane); };
+    auto raw_fill_v = [&](int t, int u) { raw_v.template v<4>(vring + (u % kRingV) * VP_BYTES + v_run, t * kBlockN + 16 * (qw & 1), lane); };
+    if constexpr (RAW) {
+        if (!score_role) {
+            for (int u = 0; u < 3; ++u) raw_fill_k(tile_at(u), u);
+            raw_fill_v(tile_at(0), 0);
+            raw_fill_k(tile_at(3), 3);
+        }
+    } else if (!score_role) {
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
             const LoadJob jb = make_job(tile_at(u), u, 0, 0);
@@ -485,6 +561,10 @@ attn_fwd_jvp_kernel(const AttnParams p) {
     if (score_role) {
         SW w;
         w.lane = lane;
+        if constexpr (RAW) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w.k_off[i] = raw_k_offset(i, lane);
+        }
         w.scale_log2 = p.scale_log2;
         w.sm_scale = p.sm_scale;
         {   // Q (and dQ) fragments: B operand of S^T = K Q^T; lane holds Q[row][16 c + 8 hh .. +7]
@@ -556,6 +636,10 @@ attn_fwd_jvp_kernel(const AttnParams p) {
     } else {
         OW w;
         w.lane = lane;
+        if constexpr (RAW) {
+#pragma unroll
+            for (int i = 0; i < NDB; ++i) w.vt_off[i] = raw_vt_offset(i, lane);
+        }
 #pragma unroll
         for (int i = 0; i < NDB; ++i) {
 #pragma unroll
@@ -569,10 +653,18 @@ attn_fwd_jvp_kernel(const AttnParams p) {
             __builtin_amdgcn_s_waitcnt(WAIT_FILLS);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            issue_group<C>(make_job(t_k, s + 4, t_v, s + 1));
-            if (s > 0)
-                w.step(vring + ((s - 1) % kRingV) * VP_BYTES, smem + ph_base + ((s - 1) & 1) * 4 * C::PH_BYTES,
-                       smem + alpha_base + ((s - 1) & 1) * 4 * 256);
+            if constexpr (RAW) {
+                raw_fill_v(t_v, s + 1);
+                raw_fill_k(t_k, s + 4);
+                if (s > 0)
+                    w.raw_step(lds0 + C::VRING_OFF + ((s - 1) % kRingV) * VP_BYTES, lds0 + ph_base + ((s - 1) & 1) * 4 * C::PH_BYTES,
+                               lds0 + alpha_base + ((s - 1) & 1) * 4 * 256);
+            } else {
+                issue_group<C>(make_job(t_k, s + 4, t_v, s + 1));
+                if (s > 0)
+                    w.step(vring + ((s - 1) % kRingV) * VP_BYTES, smem + ph_base + ((s - 1) & 1) * 4 * C::PH_BYTES,
+                           smem + alpha_base + ((s - 1) & 1) * 4 * 256);
+            }
             t_v = wrap_inc(t_v); t_k = wrap_inc(t_k);
         }
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1150,7 +1242,7 @@ struct SymCfg {
     static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
 };
 
-template <typename T, int DQK, int DV>
+template <typename T, int DQK, int DV, bool RAW = false>
 struct SymWave {
     typedef typename VecOf<T>::v8 V8;
     typedef T V2 __attribute__((ext_vector_type(2)));
@@ -1165,6 +1257,28 @@ struct SymWave {
     float p_even;
     uint32_t pw[8];                         // P^T of the current tile, two values each (B operand c of the P.V MFMAs: words 4 c .. + 3)
     int lane;
+    unsigned vt_off[RAW ? NDB : 1];         // RAW: raw_vt_offset of each channel block, raw_k_offset of each fragment
+    int k_off[RAW ? 4 : 1];
+    __device__ __forceinline__ V8 k_frag(const char* base, int c) const {
+        return RAW ? *reinterpret_cast<const V8*>(base + k_off[c & 3] + (c >> 2) * 4096) : lds_frag(base, c);
+    }
+    template <int G> __device__ __forceinline__ void read_vt(RawVt* fv, unsigned vpart) const {
+        if constexpr (G < NB) fv[G].template read<(G / NDB) * 16 * kRawRow>(vpart + vt_off[G % NDB]);
+    }
+    // stage B of tile_step with V in rows: the same groups, the transposing reads PD groups ahead
+    template <int G> __device__ __forceinline__ void raw_groups(RawVt* fv, const V8* pf, unsigned vpart, const f32x16& xn) {
+        if constexpr (G < NB) {
+            constexpr int AHEAD = NB - 1 - G < PD ? NB - 1 - G : PD, EPB = 8 / NB;
+            SCHED_FENCE();
+            read_vt<G + PD>(fv, vpart);
+            wait_lds<2 * AHEAD>();
+            fv[G].landed();
+            SCHED_FENCE();
+            acc[G % NDB] = mfma32(fv[G].template get<V8>(), pf[G / NDB], acc[G % NDB]);
+            softmax_elems(xn, G * EPB, EPB);
+            raw_groups<G + 1>(fv, pf, vpart, xn);
+        }
+    }
 
     __device__ __forceinline__ V8 lds_frag(const char* base, int frag) const {
         return *reinterpret_cast<const V8*>(base + frag * kFragBytes + lane * 16);
@@ -1196,7 +1310,7 @@ struct SymWave {
 #pragma unroll
         for (int e = 0; e < 16; ++e) x[e] = 0.f;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) x = mfma32(lds_frag(kpart, c), qf[c], x);
+        for (int c = 0; c < NC; ++c) x = mfma32(k_frag(kpart, c), qf[c], x);
     }
     // Softmax of n elements of x from e0 on (already folded into m_run).  The empty asm statements keep the arithmetic where it is
     // written, between the MFMAs: the compiler would otherwise put all of it behind the next branch, where no MFMA of this wavefront covers it.
@@ -1228,21 +1342,29 @@ struct SymWave {
         constexpr int EPC = 8 / NC, EPB = 8 / NB;   // softmax elements dealt out per d chunk / per P.V group
         V8 fa[NC];
 #pragma unroll
-        for (int i = 0; i < PD && i < NC; ++i) fa[i] = lds_frag(kpart, i);
+        for (int i = 0; i < PD && i < NC; ++i) fa[i] = k_frag(kpart, i);
 #pragma unroll
         for (int e = 0; e < 16; ++e) xn[e] = 0.f;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             SCHED_FENCE();
-            if (c + PD < NC) fa[c + PD] = lds_frag(kpart, c + PD);
+            if (c + PD < NC) fa[c + PD] = k_frag(kpart, c + PD);
             SCHED_FENCE();
             xn = mfma32(fa[c], qf[c], xn);
             softmax_elems(x, 8 + c * EPC, EPC);
         }
         SCHED_FENCE();
         V8 pf[2], fv[NB];
+        RawVt rv[RAW ? NB : 1];
+        const unsigned vrows = RAW ? (unsigned)(uintptr_t)(__attribute__((address_space(3))) const char*)vpart : 0u;
+        if constexpr (RAW) {
+            static_assert(PD == 2, "the groups read ahead");
+            read_vt<0>(rv, vrows);
+            read_vt<1>(rv, vrows);
+        } else {
 #pragma unroll
-        for (int i = 0; i < PD && i < NB; ++i) fv[i] = lds_frag(vpart, 2 * (i % NDB) + i / NDB);
+            for (int i = 0; i < PD && i < NB; ++i) fv[i] = lds_frag(vpart, 2 * (i % NDB) + i / NDB);
+        }
         if (__any(!(l_tile <= kMaxTileSum))) {
             const float alpha = raise_max(x);
             l_run *= alpha;
@@ -1259,24 +1381,29 @@ struct SymWave {
 #pragma unroll
         for (int c = 0; c < 2; ++c) pf[c] = __builtin_bit_cast(V8, make_uint4(pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]));
         mask(xn, t_next);
+        if constexpr (RAW) {
+            raw_groups<0>(rv, pf, vrows, xn);
+        } else {
 #pragma unroll
-        for (int g = 0; g < NB; ++g) {
-            const int c = g / NDB, db = g % NDB;
-            SCHED_FENCE();
-            if (g + PD < NB) fv[g + PD] = lds_frag(vpart, 2 * ((g + PD) % NDB) + (g + PD) / NDB);
-            SCHED_FENCE();
-            acc[db] = mfma32(fv[g], pf[c], acc[db]);
-            softmax_elems(xn, g * EPB, EPB);
+            for (int g = 0; g < NB; ++g) {
+                const int c = g / NDB, db = g % NDB;
+                SCHED_FENCE();
+                if (g + PD < NB) fv[g + PD] = lds_frag(vpart, 2 * ((g + PD) % NDB) + (g + PD) / NDB);
+                SCHED_FENCE();
+                acc[db] = mfma32(fv[g], pf[c], acc[db]);
+                softmax_elems(xn, g * EPB, EPB);
+            }
         }
         SCHED_FENCE();
     }
 };
 
-template <typename T, int DQK, int DV, int RG, int KG>
+template <typename T, int DQK, int DV, int RG, int KG, bool RAW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * RG * KG, 64 * RG * KG), amdgpu_waves_per_eu(RG * KG / 4, RG * KG / 4)))
 attn_fwd_sym_kernel(const AttnParams p) {
     typedef SymCfg<DQK, DV, RG, KG> C;
-    typedef SymWave<T, DQK, DV> W;
+    typedef SymWave<T, DQK, DV, RAW> W;
+    static_assert(!RAW || (DQK == 128 && DV == 128), "rows of 256 bytes");
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
     constexpr int NC = C::NC, NDB = C::NDB, BLOCK_M = 32 * RG;
@@ -1325,10 +1452,19 @@ attn_fwd_sym_kernel(const AttnParams p) {
     const int kf0 = (wave * C::K_LOADS) % (TPS * C::K_FR), vf0 = (wave * C::V_LOADS) % (TPS * C::VT_FR);
     const int k_src_run = (kf0 / C::K_FR) * TILE_BYTES + (kf0 % C::K_FR) * kFragBytes;
     const int v_src_run = (vf0 / C::VT_FR) * TILE_BYTES + C::KP_BYTES + (vf0 % C::VT_FR) * kFragBytes;
+    const RawFill raw_k(p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh, p.k_sl, p.Lkv), raw_v(p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh, p.v_sl, p.Lkv);
     auto fill_k = [&](int t, int u) {
+        if constexpr (RAW) {
+            raw_k.template k<C::K_LOADS>(kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, (t * TPS + kf0 / C::K_FR) * kBlockN, kf0 % C::K_FR, lane);
+            return;
+        }
         if (wave < C::FW) issue_part<C::K_LOADS>(kv_rsrc, kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + k_src_run);
     };
     auto fill_v = [&](int t, int u) {
+        if constexpr (RAW) {
+            raw_v.template v<C::V_LOADS>(vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, (t * TPS + vf0 / C::VT_FR) * kBlockN + 4 * (vf0 % C::VT_FR), lane);
+            return;
+        }
         if (wave < C::FW) issue_part<C::V_LOADS>(kv_rsrc, vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + v_src_run);
     };
     constexpr int PRE = RING - 1;
@@ -1341,6 +1477,10 @@ attn_fwd_sym_kernel(const AttnParams p) {
     W w;
     w.lane = lane;
     w.scale_log2 = p.scale_log2;
+    if constexpr (RAW) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { w.vt_off[i] = raw_vt_offset(i, lane); w.k_off[i] = raw_k_offset(i, lane); }
+    }
     {
         const int64_t off = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)row * p.q_sl + 8 * hh;
         const T* qp = reinterpret_cast<const T*>(p.q) + off;
@@ -1567,11 +1707,11 @@ constexpr int kSymStepTiles = 2;      // tiles of 32 keys per barrier step (SymC
 constexpr int kNumSymShapes = sizeof(kSymShapes) / sizeof(kSymShapes[0]);
 
 struct Kernel { attn_kernel_t fn; int lds_bytes; };
-template <typename T, int DQK, int DV, int SHAPE>
+template <typename T, int DQK, int DV, int SHAPE, bool RAW = false>
 Kernel pick_sym() {
     typedef SymCfg<DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg> C;
     static_assert(C::TPS == kSymStepTiles, "plans count steps of that many tiles");
-    return {attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg>, C::LDS_BYTES};
+    return {attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg, RAW>, C::LDS_BYTES};
 }
 template <typename T, int DQK, int DV>
 Kernel pick_mode(int mode, int shape) {
@@ -1582,9 +1722,15 @@ Kernel pick_mode(int mode, int shape) {
                 case 1: return pick_sym<T, DQK, DV, 1>();
                 default: return pick_sym<T, DQK, DV, 2>();
             }
-        case MODE_JVP_Q: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q>, AttnCfg<DQK, DV, MODE_JVP_Q>::LDS_BYTES};
-        default: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL>, AttnCfg<DQK, DV, MODE_JVP_FULL>::LDS_BYTES};
+        case MODE_JVP_Q: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q, false>, AttnCfg<DQK, DV, MODE_JVP_Q>::LDS_BYTES};
+        default: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL, false>, AttnCfg<DQK, DV, MODE_JVP_FULL>::LDS_BYTES};
     }
+}
+// the kernels that read K and V where they are
+template <typename T>
+Kernel pick_raw(int mode, int shape) {
+    if (mode == MODE_JVP_FULL) return {attn_fwd_jvp_kernel<T, 128, 128, MODE_JVP_FULL, true>, AttnCfg<128, 128, MODE_JVP_FULL>::LDS_BYTES};
+    return shape == 1 ? pick_sym<T, 128, 128, 1, true>() : pick_sym<T, 128, 128, 2, true>();
 }
 template <typename T, int DQK>
 Kernel pick_dv(int dv, int mode, int shape) {
@@ -1936,21 +2082,46 @@ int run_wide(const cosmos_attn_desc* d, const void* workspace, void* stream) {
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * kWideWaves), 0, (hipStream_t)stream, ap, (int)d->d_qk, (int)d->d_v);
     return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
 }
+// One-call forms at head dim 128 read K and V where they are (RAW kernels: the same results, bit for bit) instead of re-tiling them first where there are few
+// query rows: the re-tiling costs by keys, what the RAW kernels lose (twice the LDS read instructions for V, an address per four K fragments) 5 % of the
+// sweep, by rows times keys, so that the line is a number of rows.  Measured, us, re-tiled / in place: forward only 2 x 16 heads 255 positions 19.6 / 17.0, 16 heads
+// 700 26.5 / 18.6, 3520 120 / 113, 40 heads 1000 46 / 38; all tangents 16 heads 255 24.1 / 21.5, 704 39.6 / 34.6, 1560 81.5 / 77.6, 3520 290 / 290,
+// 7040 999 / 1011, 37440 25870 / 27185, 40 heads 1560 191 / 179.  (Forward only the larger calls take 12 x 32 rows a workgroup, which has no registers left for it.)
+constexpr int kInPlaceRows[2] = {6144, 3072};       // forward only, all tangents
+bool reads_in_place(const cosmos_attn_desc* d, const SplitPlan& sp) {
+    const int mode = mode_of(d);
+    if (d->d_qk != 128 || d->d_v != 128 || mode == MODE_JVP_Q || d->Lq > kInPlaceRows[mode == MODE_FWD ? 0 : 1]) return false;
+    if ((mode == MODE_FWD && sp.shape == 0) || stream_groups_of(d, sp)) return false;
+    for (const int64_t stride : {d->k_stride[2], d->v_stride[2]})       // 32-bit buffer offsets, also of the rows behind the last one
+        if (stride < 0 || stride >= (int64_t)1 << 30 || (d->Lkv + 4 * kBlockN) * stride * 2 >= (int64_t)1 << 31) return false;
+    return true;
+}
 // `room`: bytes behind the re-tiled K/V image that key-range partial results may take.  cosmos_attn_run only reads its workspace, so
-// that several runs may share one image: 0, never split.
-int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, size_t room, void* stream) {
+// that several runs may share one image: 0, never split.  one_call: K and V are re-tiled here, or read where they are.
+int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, size_t room, void* stream, bool one_call) {
     const int st = validate(d);
     if (st != COSMOS_ATTN_OK) return st;
     const SplitPlan sp = plan_split(d, room);
+    const bool raw = one_call && reads_in_place(d, sp);
+    if (one_call && !raw) {
+        const int packed = cosmos_attn_pack_kv(d, workspace, workspace_bytes, stream);
+        if (packed != COSMOS_ATTN_OK) return packed;
+    }
     const size_t image_bytes = align256(tiles_bytes_of(d));
     if (!workspace || workspace_bytes < image_bytes + partial_bytes(d, sp) || !aligned16(workspace)) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
     if (!device_is_whole_mi355x()) return COSMOS_ATTN_WRONG_DEVICE;
     const int mode = mode_of(d);
     if (is_wide(d)) return run_wide(d, workspace, stream);
-    const Kernel kernel = d->dtype == COSMOS_ATTN_BF16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode, sp.shape)
-                                                       : pick_dqk<_Float16>(d->d_qk, d->d_v, mode, sp.shape);
+    const bool bf16 = d->dtype == COSMOS_ATTN_BF16;
+    const Kernel kernel = raw ? (bf16 ? pick_raw<__bf16>(mode, sp.shape) : pick_raw<_Float16>(mode, sp.shape))
+                          : bf16 ? pick_dqk<__bf16>(d->d_qk, d->d_v, mode, sp.shape) : pick_dqk<_Float16>(d->d_qk, d->d_v, mode, sp.shape);
     if (!kernel.fn) return COSMOS_ATTN_UNSUPPORTED;
-    AttnParams ap;
+    AttnParams ap = {};
+    if (raw) {
+        ap.k = (const uint16_t*)d->k; ap.v = (const uint16_t*)d->v; ap.tk = (const uint16_t*)d->tk; ap.tv = (const uint16_t*)d->tv;
+        ap.k_sb = d->k_stride[0]; ap.k_sh = d->k_stride[1]; ap.k_sl = d->k_stride[2];
+        ap.v_sb = d->v_stride[0]; ap.v_sh = d->v_stride[1]; ap.v_sl = d->v_stride[2];
+    }
     ap.q = d->q; ap.tq = d->tq;
     ap.q_sb = d->q_stride[0]; ap.q_sh = d->q_stride[1]; ap.q_sl = d->q_stride[2];
     ap.o = d->o; ap.to = d->to;
@@ -1988,7 +2159,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
         const int rows_per_block = 256 / (d->d_v / 4);
         const int64_t rows = (int64_t)sp.n_rem * sp.block_m;
         const dim3 cgrid((unsigned)((rows + rows_per_block - 1) / rows_per_block));
-        const bool bf16 = d->dtype == COSMOS_ATTN_BF16, jvp = mode != MODE_FWD;
+        const bool jvp = mode != MODE_FWD;
         auto cfn = jvp ? (bf16 ? attn_combine_kernel<__bf16, true> : attn_combine_kernel<_Float16, true>)
                        : (bf16 ? attn_combine_kernel<__bf16, false> : attn_combine_kernel<_Float16, false>);
         hipLaunchKernelGGL(cfn, cgrid, dim3(256), 0, (hipStream_t)stream, ap, d->d_v, sp.block_m);
@@ -2001,13 +2172,11 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
 extern "C" {
 
 COSMOS_ATTN_API int cosmos_attn_run(const cosmos_attn_desc* d, const void* workspace, size_t workspace_bytes, void* stream) {
-    return run_impl(d, const_cast<void*>(workspace), workspace_bytes, 0, stream);     // (no room: not written)
+    return run_impl(d, const_cast<void*>(workspace), workspace_bytes, 0, stream, false);     // (no room: not written)
 }
 
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
-    const int st = cosmos_attn_pack_kv(d, workspace, workspace_bytes, stream);
-    if (st != COSMOS_ATTN_OK) return st;
-    return run_impl(d, workspace, workspace_bytes, kNoLimit, stream);
+    return run_impl(d, workspace, workspace_bytes, kNoLimit, stream, true);
 }
 
 }  // extern "C"
@@ -2050,10 +2219,9 @@ COSMOS_ATTN_API int cosmos_attn_fwd_jvp_static(const cosmos_attn_desc* d, void* 
     void* const ws = static_scratch_ptr();
     if (!ws) return COSMOS_ATTN_LAUNCH_FAILED;
     // nothing in the workspace has to start at zero: the re-tiling kernel writes every byte of the image (padding
-    // included) and every key range writes its whole slot of partial results before the merge kernel reads it
-    const int packed = cosmos_attn_pack_kv(d, ws, kStaticScratchBytes, stream);
-    // where the key ranges that cosmos_attn_fwd_jvp would cut leave more partial results than fit, fewer are cut
-    return packed != COSMOS_ATTN_OK ? packed : run_impl(d, ws, kStaticScratchBytes, kStaticScratchBytes - image_bytes, stream);
+    // included) and every key range writes its whole slot of partial results before the merge kernel reads it.
+    // Where the key ranges that cosmos_attn_fwd_jvp would cut leave more partial results than fit, fewer are cut.
+    return run_impl(d, ws, kStaticScratchBytes, kStaticScratchBytes - image_bytes, stream, true);
 }
 
 }  // extern "C"

@@ -1,0 +1,66 @@
+"""Attention calls that read K and V where they are (head dim 128, few query rows): the same bits as the same kernels on the re-tiled image (without
+tangents), and parity with the oracle (with all tangents), where what lies behind the last row is not a number."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(g, B, L, H, dtype, scale, layout):
+    """[B, H, L, 128] view of memory whose rows behind the last one are not numbers."""
+    shape = (B, L + 70, H, 128) if layout == "blhd" else (B, H, L + 70, 128)
+    m = torch.full(shape, float("nan"), device="cuda", dtype=dtype)
+    x = (torch.randn(B, H, L, 128, device="cuda", generator=g) * scale).to(dtype)
+    view = m[:, :L].transpose(1, 2) if layout == "blhd" else m[:, :, :L]
+    view.copy_(x)
+    return view
+
+
+# keys: one, a tile's edge, a step's edge, ragged; 128-row workgroups of two key groups (few rows) and 256-row ones
+@pytest.mark.parametrize("dtype, layout", [(torch.bfloat16, "blhd"), (torch.float16, "bhld")])
+@pytest.mark.parametrize("B, H, Lq, Lkv, causal, lens", [
+    (1, 2, 1, 1, False, None), (2, 3, 129, 32, False, None), (1, 2, 300, 33, False, None), (1, 16, 255, 255, False, None), (2, 16, 520, 520, True, None),
+    (1, 40, 1000, 1000, False, None), (1, 40, 1100, 65, False, None), (2, 16, 513, 700, False, (1, 411)),
+])
+def test_forward_gives_the_bits_of_the_re_tiled_image(pkg, B, H, Lq, Lkv, causal, lens, dtype, layout):
+    ops = pkg.ops
+    g = torch.Generator(device="cuda").manual_seed(Lq + Lkv)
+    q = _rows(g, B, Lq, H, dtype, 1.0, layout)
+    k, v = _rows(g, B, Lkv, H, dtype, 2.0, layout), _rows(g, B, Lkv, H, dtype, 1.0, layout)
+    lens = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda")
+    o, _, lse = ops.fwd_jvp(q, k, v, causal=causal, key_lens=lens)
+    assert torch.isfinite(o).all() and torch.isfinite(lse).all()
+    if causal:
+        s = (q.double() @ k.double().transpose(-1, -2)) * 128 ** -0.5
+        s.masked_fill_(torch.ones(Lq, Lkv, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+        want = s.softmax(-1) @ v.double()
+        assert (o.double() - want).norm() / want.norm() < (5e-3 if dtype == torch.bfloat16 else 5e-3 / 8)      # limit of the parity tests; fp16 rounds 8 times finer
+        return
+    want, _, want_lse = ops.run_packed(q, ops.pack_kv(k, v), key_lens=lens)
+    # (a two-stage run may stream its query blocks or take 384-row workgroups: the same sums in another order then)
+    if torch.equal(lse, want_lse):
+        assert torch.equal(o, want)
+    else:
+        assert (lse - want_lse).abs().max() < 1e-4 and (o.double() - want.double()).norm() / want.double().norm() < (5e-3 if dtype == torch.bfloat16 else 5e-3 / 8)
+
+
+@pytest.mark.parametrize("dtype, layout", [(torch.bfloat16, "blhd"), (torch.float16, "bhld")])
+@pytest.mark.parametrize("B, H, Lq, Lkv, lens", [(1, 2, 1, 1, None), (1, 3, 127, 33, None), (2, 2, 300, 256, None), (1, 16, 255, 255, None), (2, 4, 385, 1100, (3, 1100))])
+def test_all_tangents(pkg, B, H, Lq, Lkv, lens, dtype, layout):
+    ops = pkg.ops
+    g = torch.Generator(device="cuda").manual_seed(Lq + Lkv)
+    mk = lambda L, scale: _rows(g, B, L, H, dtype, scale, layout)
+    q, k, v, tq, tk, tv = mk(Lq, 1.0), mk(Lkv, 1.0), mk(Lkv, 1.0), mk(Lq, 0.1), mk(Lkv, 0.1), mk(Lkv, 0.1)
+    dev = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda")
+    o, to, _ = ops.fwd_jvp(q, k, v, tq, tk, tv, key_lens=dev)
+    assert torch.isfinite(o).all() and torch.isfinite(to).all()
+    d = lambda x: x.double()
+    s, ds = d(q) @ d(k).transpose(-1, -2) * 128 ** -0.5, (d(tq) @ d(k).transpose(-1, -2) + d(q) @ d(tk).transpose(-1, -2)) * 128 ** -0.5
+    if lens is not None:
+        out = torch.arange(Lkv, device="cuda")[None, None, None] >= dev[:, None, None, None]
+        s = s.masked_fill(out, float("-inf"))
+    p = s.softmax(-1)
+    want = p @ d(v)
+    twant = (p * ds) @ d(v) - (p * ds).sum(-1, keepdim=True) * want + p @ d(tv)
+    limit = 5e-3 if dtype == torch.bfloat16 else 5e-3 / 8                 # limit of the parity tests; fp16 rounds 8 times finer
+    assert (d(o) - want).norm() / want.norm() < limit and (d(to) - twant).norm() / twant.norm() < limit
