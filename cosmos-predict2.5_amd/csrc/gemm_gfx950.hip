@@ -529,7 +529,7 @@ COSMOS_ATTN_API int cosmos_attn_gemm_preferred(const cosmos_attn_gemm_desc* d) {
     if (d->order == COSMOS_GEMM_XTX) return d->depth >= 256 && !(shape == 3 && d->depth > 32768);
     if (d->rows < 1024) return 0;
     if (d->order == COSMOS_GEMM_XW) return d->count > 1 ? us <= d->count * (one / 1.25e9 + 10.0) : rate >= 1.02e9 || (one <= 6e10 && rate >= 0.55e9);
-    if (d->count > 1) return us <= d->count * (one / 1.35e9 + 8.0);
+    if (d->count > 1) return us <= d->count * (one / 1.35e9 + 12.0);
     return d->rows >= 8192 || (int64_t)d->cols * d->depth <= (int64_t)1 << 22;
 }
 
