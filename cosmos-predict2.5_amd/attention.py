@@ -112,9 +112,12 @@ def attention(
         raise NotImplementedError(f"attention(): dropout_p={dropout_p} is not supported by the HIP kernels (pass 0.0)")
     del q_lens, k_lens, deterministic
 
-    q = q.to(dtype)
-    k = k.to(dtype)
-    v = v.to(dtype)
+    if q.dtype != dtype:
+        q = q.to(dtype)
+    if k.dtype != dtype:
+        k = k.to(dtype)
+    if v.dtype != dtype:
+        v = v.to(dtype)
     if q_scale is not None:
         q = q * q_scale
 
@@ -127,6 +130,10 @@ def attention(
             raise RuntimeError("more attention calls in the recomputation than were recorded")
         return _kept.replay.pop(0)[0].transpose(1, 2)
     recording = _kept.record is not None
+    if not recording:
+        o = ops.forward_in_place(q, k, v, causal, softmax_scale)
+        if o is not None:
+            return o
     o, _, lse = ops.fwd_jvp(
         q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2),
         causal=causal, sm_scale=softmax_scale, out_layout="blhd", need_lse=recording,

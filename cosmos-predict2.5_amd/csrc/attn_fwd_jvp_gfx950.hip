@@ -2108,7 +2108,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
         if (packed != COSMOS_ATTN_OK) return packed;
     }
     const size_t image_bytes = align256(tiles_bytes_of(d));
-    if (!workspace || workspace_bytes < image_bytes + partial_bytes(d, sp) || !aligned16(workspace)) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
+    if (!(raw && sp.splits < 2) && (!workspace || workspace_bytes < image_bytes + partial_bytes(d, sp) || !aligned16(workspace))) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
     if (!device_is_whole_mi355x()) return COSMOS_ATTN_WRONG_DEVICE;
     const int mode = mode_of(d);
     if (is_wide(d)) return run_wide(d, workspace, stream);
@@ -2175,7 +2175,18 @@ COSMOS_ATTN_API int cosmos_attn_run(const cosmos_attn_desc* d, const void* works
     return run_impl(d, const_cast<void*>(workspace), workspace_bytes, 0, stream, false);     // (no room: not written)
 }
 
+COSMOS_ATTN_API int cosmos_attn_fwd_in_place(const cosmos_attn_desc* d, void* stream) {
+    const int st = validate(d);
+    if (st != COSMOS_ATTN_OK) return st;
+    if (!reads_in_place(d, plan_split(d, 0))) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
+    // (a call whose keys would be cut into ranges, given room for their results, is left to cosmos_attn_fwd_jvp)
+    if (planned_partial_bytes(d)) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
+    return run_impl(d, nullptr, 0, 0, stream, true);
+}
+
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!workspace || !aligned16(workspace)) { const int st = validate(d); return st != COSMOS_ATTN_OK ? st : COSMOS_ATTN_WORKSPACE_TOO_SMALL; }
+    if (validate(d) == COSMOS_ATTN_OK && workspace_bytes < align256(tiles_bytes_of(d))) return COSMOS_ATTN_WORKSPACE_TOO_SMALL;
     return run_impl(d, workspace, workspace_bytes, kNoLimit, stream, true);
 }
 

@@ -132,6 +132,10 @@ COSMOS_ATTN_API int cosmos_attn_launch_plan(const cosmos_attn_desc *desc, size_t
  */
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
 
+/* cosmos_attn_fwd_jvp for the calls that read k and v where they are and cut nothing (head dim 128, few query rows; the same results): no workspace.
+ * COSMOS_ATTN_WORKSPACE_TOO_SMALL, and nothing launched, for every other valid call. */
+COSMOS_ATTN_API int cosmos_attn_fwd_in_place(const cosmos_attn_desc *desc, void *stream);
+
 /*
  * cosmos_attn_fwd_jvp without a workspace argument and without any allocation: the workspace is a static device array
  * inside the library (COSMOS_ATTN_STATIC_SCRATCH_BYTES = 64 MiB per GPU, held until the process ends).

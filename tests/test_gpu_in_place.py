@@ -64,3 +64,36 @@ def test_all_tangents(pkg, B, H, Lq, Lkv, lens, dtype, layout):
     twant = (p * ds) @ d(v) - (p * ds).sum(-1, keepdim=True) * want + p @ d(tv)
     limit = 5e-3 if dtype == torch.bfloat16 else 5e-3 / 8                 # limit of the parity tests; fp16 rounds 8 times finer
     assert (d(o) - want).norm() / want.norm() < limit and (d(to) - twant).norm() / twant.norm() < limit
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B, S, H, Lkv, causal, scale, how", [
+    (2, 255, 16, 255, False, None, "dense"), (1, 300, 3, 300, True, 0.2, "heads first"), (1, 6144, 1, 64, False, None, "dense"), (1, 6145, 1, 64, False, None, "dense"),
+    (1, 130, 2, 77, False, 1.0, "unaligned"), (1, 130, 2, 77, False, None, "strided"), (1, 64, 2, 64, False, None, "expanded"), (1, 256, 4, 2000, False, None, "dense"),
+])
+def test_attention_is_the_general_call(pkg, B, S, H, Lkv, causal, scale, how, dtype):
+    """``attention`` takes a shorter way on the host for these calls: the same bits as ``fwd_jvp`` for every layout, its refusals for what it refuses."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+
+    def make(L):
+        x = torch.randn(B, L, H, 128, device="cuda", generator=g).to(dtype)
+        if how == "heads first":
+            return x.transpose(1, 2).contiguous().transpose(1, 2)
+        if how == "unaligned":
+            return torch.empty(x.numel() + 4, device="cuda", dtype=dtype)[4:].view(x.shape).copy_(x)
+        if how == "strided":
+            return torch.empty(B, L, H, 256, device="cuda", dtype=dtype)[..., ::2].copy_(x)
+        if how == "expanded":
+            return x[:, :1].expand(B, L, H, 128)
+        return x
+
+    q, k, v = make(S), make(Lkv), make(Lkv)
+    t = lambda x: x.transpose(1, 2)
+    with torch.no_grad():
+        got = pkg.attention_forward(q, k, v, softmax_scale=scale, causal=causal, dtype=dtype)
+    want = pkg.ops.fwd_jvp(t(q), t(k), t(v), causal=causal, sm_scale=scale, out_layout="blhd", need_lse=False)[0].transpose(1, 2)
+    assert got.is_contiguous() and got.dtype == dtype and torch.equal(got, want)
+    with torch.no_grad(), pytest.raises(AssertionError):
+        pkg.attention_forward(q, k[:, :-1], v, dtype=dtype)
+    with torch.no_grad(), pytest.raises((RuntimeError, NotImplementedError)):
+        pkg.attention_forward(q.cpu(), k.cpu(), v.cpu(), dtype=dtype)
