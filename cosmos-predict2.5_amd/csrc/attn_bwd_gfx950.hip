@@ -798,6 +798,9 @@ __global__ void __launch_bounds__(256) bwd_combine_kernel(const BwdParams p, int
 // group of 16 lanes, lane i passes the address of 8 bytes (row i of a 16 x 4 matrix M of 16-bit values) and receives
 // M[i/4 + 4k][i%4], k = 0..3.  A row of M here is one key's dS for 4 consecutive queries, so lane (query, half hh) gets, for
 // key chunk c and read t, the keys 16 c + 8 t + 4 hh + k -- the order in which a V^T-type fragment of K^T holds them.
+// One workgroup fills a compute unit (144 KB of ring), so where the queries give more blocks than units each workgroup walks several, the next block's
+// first loads in flight while the last steps and the stores of the one before run: at 512 keys (16 steps a block) of 16 heads x 37440 queries 192 -> 171 us
+// (4.5 TB/s), at 37440 keys the same time.  Causal blocks have unequal lengths, which a fixed share would not balance: one workgroup each.
 constexpr int kDsLoadPolicy = 2;     // cache policy bits of the dS loads: non-temporal (each tile is read once; 4 % faster than plain loads)
 constexpr int kDsRing = 6;            // steps of dS / K^T in flight per workgroup
 constexpr int kDqWaves = 8;           // query tiles per workgroup
@@ -810,7 +813,7 @@ struct DqFromDsParams {
     const char* kt_img;                // K^T stream: [B*H][n_k_tiles][2 NDB fragments]
     void* dq;
     int64_t o_sb, o_sh, o_sl;
-    int H, Lq, Lkv, n_q_tiles, n_k_tiles, n_blk, bh0, causal;
+    int H, Lq, Lkv, n_q_tiles, n_k_tiles, n_blk, bh0, heads, causal;      // heads: of this launch, from bh0 on
     float sm_scale;
 };
 
@@ -833,38 +836,47 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
     constexpr int NDB = C::NDB;
-    // vmcnt(n): the loads of the newest kDsRing - 2 steps may still be in flight
-    constexpr int IN_FLIGHT = C::LOADS * (kDsRing - 2);
-    constexpr int WAIT_LOADS = (IN_FLIGHT & 15) | ((IN_FLIGHT >> 4) << 14) | 0x0F70;
+    static_assert(D % 32 == 0, "every store of a row is issued");
+    // vmcnt(n): the loads of the newest kDsRing - 2 steps may still be in flight, and behind a query block's end its stores, issued between them
+    constexpr int STORES = 4 * NDB, IN_FLIGHT = C::LOADS * (kDsRing - 2);
+    auto wait_imm = [](int n) constexpr { return (n & 15) | ((n >> 4) << 14) | 0x0F70; };
+    constexpr int WAIT_LOADS = wait_imm(IN_FLIGHT), WAIT_BEHIND_STORES = wait_imm(IN_FLIGHT + STORES);
+    static_assert(IN_FLIGHT + STORES < 64, "vmcnt");
 
-    const int blk = blockIdx.x % p.n_blk, bhl = blockIdx.x / p.n_blk, bh = p.bh0 + bhl, b = bh / p.H, h = bh % p.H;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 31, hh = lane >> 5;
-    const int qt = blk * kDqWaves + wave;          // this wavefront's query tile
-    const bool live_tile = qt < p.n_q_tiles;
-    const int row = qt * kRows + j;
+    const int n_items = p.n_blk * p.heads;         // query blocks of all heads; this workgroup's: blockIdx.x, + gridDim.x, ...
+    // key tiles of a query block: all, or up to its last query's diagonal when causal
+    auto steps_of = [&](int blk) { const int lim = blk * kDqWaves + kDqWaves; return p.causal && lim < p.n_k_tiles ? lim : p.n_k_tiles; };
 
-    // key tiles this workgroup walks: all, or up to its last query's diagonal when causal
-    int n_steps = p.n_k_tiles;
-    if (p.causal) { const int lim = blk * kDqWaves + kDqWaves; n_steps = n_steps < lim ? n_steps : lim; }
-
-    // this wavefront's run of dS tiles (one query tile, all key tiles: contiguous), and the head's K^T stream
-    const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(p.ds) + (int64_t)bhl * p.ds_head_bytes + (int64_t)(live_tile ? qt : 0) * p.n_kt_pad * C::W_BYTES, 0,
-        live_tile ? p.n_kt_pad * C::W_BYTES : 0, 0x00020000);   // no tile: every load returns zeros
-    const __amdgpu_buffer_rsrc_t rs_k = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(p.kt_img) + (size_t)bh * p.n_k_tiles * C::KT_BYTES, 0, p.n_k_tiles * C::KT_BYTES, 0x00020000);
+    // The loads run kDsRing - 1 steps ahead, over the ends of query blocks: this wavefront's run of dS tiles (one query tile, all key tiles: contiguous),
+    // and the head's K^T stream.  (Behind the last block they are issued all the same, of buffers of no bytes; so are a query tile's that is not there: zeros.)
     const int kfrag = wave % C::KT_FR;             // the K^T fragment this wavefront copies (copied redundantly when there are fewer than 8)
-    auto issue = [&](int u) {                      // loads of sweep position u (clamped: positions past the end repeat the last tile, unused)
-        const int t = __builtin_amdgcn_readfirstlane(u < n_steps ? u : n_steps - 1);
-        char* slot = smem + (u % kDsRing) * C::SLOT_BYTES;
-        lds_load<0, kDsLoadPolicy>(rs_w, slot + wave * C::W_BYTES, lane * 16, t * C::W_BYTES);
-        lds_load<kFragBytes, kDsLoadPolicy>(rs_w, slot + wave * C::W_BYTES, lane * 16, t * C::W_BYTES);
-        lds_load<0>(rs_k, slot + kDqWaves * C::W_BYTES + kfrag * kFragBytes, lane * 16, t * C::KT_BYTES + kfrag * kFragBytes);
+    __amdgpu_buffer_rsrc_t rs_w, rs_k;
+    int l_item = blockIdx.x, l_u = 0, l_steps = 0, l_slot = 0;
+    auto open_block = [&]() {
+        const bool any = l_item < n_items;
+        const int blk = l_item % p.n_blk, bhl = any ? l_item / p.n_blk : 0, qt = blk * kDqWaves + wave;
+        const bool live = any && qt < p.n_q_tiles;
+        rs_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.ds) + (int64_t)bhl * p.ds_head_bytes + (int64_t)(live ? qt : 0) * p.n_kt_pad * C::W_BYTES, 0,
+                                                 live ? p.n_kt_pad * C::W_BYTES : 0, 0x00020000);
+        rs_k = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.kt_img) + (size_t)(p.bh0 + bhl) * p.n_k_tiles * C::KT_BYTES, 0,
+                                                 any ? p.n_k_tiles * C::KT_BYTES : 0, 0x00020000);
+        l_u = 0;
+        l_steps = steps_of(blk);
+    };
+    open_block();
+    auto issue = [&]() {
+        char* slot = smem + l_slot * C::SLOT_BYTES;
+        lds_load<0, kDsLoadPolicy>(rs_w, slot + wave * C::W_BYTES, lane * 16, l_u * C::W_BYTES);
+        lds_load<kFragBytes, kDsLoadPolicy>(rs_w, slot + wave * C::W_BYTES, lane * 16, l_u * C::W_BYTES);
+        lds_load<0>(rs_k, slot + kDqWaves * C::W_BYTES + kfrag * kFragBytes, lane * 16, l_u * C::KT_BYTES + kfrag * kFragBytes);
+        l_slot = l_slot + 1 < kDsRing ? l_slot + 1 : 0;
+        if (++l_u == l_steps) { l_item += gridDim.x; open_block(); }
     };
 #pragma unroll
-    for (int u = 0; u < kDsRing - 1; ++u) issue(u);
+    for (int u = 0; u < kDsRing - 1; ++u) issue();
 
     f32x16 acc[NDB];
 #pragma unroll
@@ -881,12 +893,13 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
     const int g16 = lane >> 4, r16 = lane & 15;
     const unsigned tr_off = (unsigned)(256 * (g16 >> 1) + 128 * (g16 & 1) + 64 * (r16 & 1) + 16 * (r16 >> 2) + 8 * ((r16 & 3) >> 1));
 
-    auto step = [&](int s) {
-        const char* slot = smem + (s % kDsRing) * C::SLOT_BYTES;
+    int r_slot = 0;
+    auto step = [&](int s, int qt, bool live_tile) {
+        const char* slot = smem + r_slot * C::SLOT_BYTES;
         // (written out: the compiler takes the builtin of this read for an access that may alias the direct-to-LDS loads in
         // flight and puts vmcnt(0) in front of it, which would end the prefetch; it does not see through the asm, so the
         // wait for the four results is in the block as well)
-        const unsigned wt = lds0 + (unsigned)((s % kDsRing) * C::SLOT_BYTES + wave * C::W_BYTES) + tr_off;
+        const unsigned wt = lds0 + (unsigned)(r_slot * C::SLOT_BYTES + wave * C::W_BYTES) + tr_off;
         s16x4 t00, t01, t10, t11;
         asm volatile("ds_read_b64_tr_b16 %0, %4\n\t"
                      "ds_read_b64_tr_b16 %1, %4 offset:512\n\t"
@@ -917,22 +930,29 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
                 acc[db] = mfma32(*reinterpret_cast<const V8*>(kt + (2 * db + c) * kFragBytes), wf[c], acc[db]);
         }
     };
-    for (int s = 0; s < n_steps; ++s) {
-        __builtin_amdgcn_s_waitcnt(WAIT_LOADS);
-        __builtin_amdgcn_s_barrier();          // everybody's loads of step s have landed, everybody is done reading step s - 1
-        asm volatile("" ::: "memory");
-        issue(s + kDsRing - 1);                // into the slot of step s - 1
-        step(s);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);        // drain the trailing loads before the LDS is released
-    if (live_tile && row < p.Lq) {
-        T* o1 = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl;
+    int since_stores = kDsRing - 1;            // steps since a block's stores
+    for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+        const int blk = item % p.n_blk, bh = p.bh0 + item / p.n_blk, b = bh / p.H, h = bh % p.H;
+        const int qt = blk * kDqWaves + wave;      // this wavefront's query tile
+        const bool live_tile = qt < p.n_q_tiles;
+        const int n_steps = steps_of(blk);
+        for (int s = 0; s < n_steps; ++s) {
+            if (since_stores < kDsRing - 1) { __builtin_amdgcn_s_waitcnt(WAIT_BEHIND_STORES); ++since_stores; }
+            else __builtin_amdgcn_s_waitcnt(WAIT_LOADS);
+            __builtin_amdgcn_s_barrier();          // everybody's loads of this step have landed, everybody is done reading the step before
+            asm volatile("" ::: "memory");
+            issue();                               // into the slot of the step before
+            step(s, qt, live_tile);
+            r_slot = r_slot + 1 < kDsRing ? r_slot + 1 : 0;
+        }
+        const int row = qt * kRows + j;
+        if (live_tile && row < p.Lq) {             // (a tile that is there has its first row, so all its stores are issued and counted)
+            T* o1 = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
+            for (int db = 0; db < NDB; ++db) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * db + 8 * g + 4 * hh;   // registers 4g..4g+3 are 4 consecutive channels
-                if (d < D) {
+                for (int g = 0; g < 4; ++g) {
+                    const int d = 32 * db + 8 * g + 4 * hh;   // registers 4g..4g+3 are 4 consecutive channels
                     V4 v1;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v1[r] = (T)(acc[db][4 * g + r] * p.sm_scale);
@@ -940,7 +960,14 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
                 }
             }
         }
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
+        }
+        if (live_tile) since_stores = 0;
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);        // drain the trailing loads before the LDS is released
 }
 
 // ------------------------------------------------------------------------------------------------ host
@@ -1186,8 +1213,9 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
             const BwdGeom::Plan pl = heads == g.group ? g.dkdv : BwdGeom::plan(g.dkdv.n_blk, heads, g.n_q_tiles, d->causal != 0, d->d, true);
             bp.bh0 = bh0;
             if (!launch(k_spill, lds_dkdv, pl, bp, true)) return COSMOS_ATTN_LAUNCH_FAILED;
-            qp.bh0 = bh0;
-            hipLaunchKernelGGL(k_ds, dim3((unsigned)(qp.n_blk * heads)), dim3(kDqThreads), lds_ds, stream, qp);
+            qp.bh0 = bh0; qp.heads = heads;
+            const int items = qp.n_blk * heads, grid = !d->causal && items > kNumCUs ? kNumCUs : items;
+            hipLaunchKernelGGL(k_ds, dim3((unsigned)grid), dim3(kDqThreads), lds_ds, stream, qp);
         }
         return hipGetLastError() == hipSuccess ? COSMOS_ATTN_OK : COSMOS_ATTN_LAUNCH_FAILED;
     }

@@ -125,6 +125,13 @@ def test_bwd_many_workgroups(pkg, oracle, gpu):
     run_bwd(pkg, oracle, gpu, (2, 4, 1024, 128), (2, 4, 1500, 128), seed=11)
 
 
+@pytest.mark.parametrize("Lkv", [1, 33, 70, 160, 200, 515])
+def test_bwd_several_query_blocks_per_workgroup(pkg, oracle, gpu, Lkv):
+    """The kept-dS dQ pass with more query blocks (of 256) than compute units: its loads run 5 key tiles ahead over the ends of blocks.  One key tile,
+    fewer than 5, 5 and more, ragged; the last block of a head has wavefronts with a whole, a partly filled and no query tile (same tolerances)."""
+    run_bwd(pkg, oracle, gpu, (5, 13, 1070, 128), (5, 13, Lkv, 128), seed=Lkv)
+
+
 def test_bwd_through_autograd_function(pkg, oracle, gpu):
     """`attention(q, k, v, tq, tk, tv, causal, sm_scale)[0].backward(dout)` like the reference's procedure."""
     q, k, v, tq, tk, tv = oracle.make_inputs((1, 2, 300, 64), (1, 2, 300, 64), seed=3, primal_std=0.5)
