@@ -115,11 +115,10 @@ __global__ void __launch_bounds__(kPackThreads) bwd_stats_kernel(const StatsPara
 }
 
 // ---------------------------------------------------------------------------------------------- stream re-tiling
-// Order of the 16-byte units (row q of the tile, 16-channel chunk cK, half hK: 8 channels) inside a K-type section of the
-// query stream of attn_dkdv_quad_kernel, which reads the same units linearly (ds_read_b128, lane = row) and transposed
-// (ds_read_b64_tr_b16): both without bank conflicts in this order (attn_bwd_quad_gfx950.h).
-__host__ __device__ constexpr int quad_unit_slot(int q, int cK, int hK) {
-    return 16 * ((q >> 4) + 2 * hK + 4 * cK) + ((q & 3) + 4 * (((q >> 2) & 3) ^ (hK + 2 * (cK & 1))));
+// Order of the 16-byte units (row r, chunk C of 8 channels) of a stream part of attn_dkdv_quad_kernel in LDS: read with ds_read_b128
+// (lane = row) and with transposing reads (ds_read_b64_tr_b16) without bank conflicts, and filled four whole rows a load (attn_bwd_quad_gfx950.h).
+__host__ __device__ constexpr int quad_unit_slot(int r, int C) {
+    return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ ((r >> 2) & 3));
 }
 
 struct PackSrc { const uint16_t* ptr; int64_t sb, sh, sl; };
@@ -182,34 +181,37 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
     }
 }
 
-// The query stream of attn_dkdv_quad_kernel in one pass over q, dout and o (head dim 128): both K-type sections in its unit order
-// and the statistics fragment, whose row sums dout . o come from the rows just read.  HBM-bound; as bwd_stats_kernel followed by
-// pack_stream_kernel, dout was read twice and a row's 256 bytes by 16 threads that were not neighbours.  Eight threads per row,
-// two 16-byte units of each tensor per thread, rows read whole.  grid (n_tiles, B*H).
-// Measured at 16 heads x 37440 rows (bf16): 79 + 114 -> 145 us = 5.4 TB/s; x 24640 rows 52 + 87 -> 93 us.
-struct PackQuadParams {
+// What attn_dkdv_quad_kernel streams beside Q and dO (head dim 128): per tile of 32 queries 32 values LSE log2 e, then 32 row sums dout . o.  With COPY also
+// rows of q and dout, one behind the other, for a call whose own rows the kernel does not read.  HBM-bound; eight threads per row, two 16-byte units of each tensor
+// per thread, rows read whole.  grid (n_tiles, B*H).
+constexpr int kQuadStatBytes = 2 * kRows * (int)sizeof(float);
+struct QuadStatsParams {
     PackSrc q, g, o;             // q, dout, o
     const float* lse;            // [B,H,L]
-    float2* stats;               // [B*H][L] : (LSE log2 e, D)
-    char* out;
+    float2* stats;               // [B*H][L] : (LSE log2 e, D); null: nobody reads it
+    char* tile_stats;            // [B*H][n_tiles][kQuadStatBytes]
+    uint4 *q_rows, *g_rows;      // COPY: [B*H][32 n_tiles][16 units]
     int H, L, n_tiles;
 };
-template <bool BF16>
-__global__ void __launch_bounds__(kPackThreads) pack_quad_stream_kernel(const PackQuadParams p) {
+template <bool BF16, bool COPY>
+__global__ void __launch_bounds__(kPackThreads) quad_stats_kernel(const QuadStatsParams p) {
     static_assert(kPackThreads == 8 * kRows, "eight threads per row of a tile");
-    constexpr int NC = 8;        // 16-channel chunks of a row
     const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H, t = blockIdx.x;
     const int r = threadIdx.x >> 3, part = threadIdx.x & 7, row = t * kRows + r;
     const bool live = row < p.L;
-    uint4* dst = reinterpret_cast<uint4*>(p.out) + ((size_t)bh * p.n_tiles + t) * (size_t)((2 * NC + 1) * (kFragBytes / 16));
-    uint4 q[2], g[2], o[2];
+    uint4 g[2], o[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int c = 8 * (part + 8 * i);
         auto unit = [&](const PackSrc& s) {
             return live ? *reinterpret_cast<const uint4*>(s.ptr + (int64_t)b * s.sb + (int64_t)h * s.sh + (int64_t)row * s.sl + c) : make_uint4(0u, 0u, 0u, 0u);
         };
-        q[i] = unit(p.q); g[i] = unit(p.g); o[i] = unit(p.o);
+        g[i] = unit(p.g); o[i] = unit(p.o);
+        if (COPY) {
+            const int64_t at = (((int64_t)bh * p.n_tiles + t) * kRows + r) * 16 + part + 8 * i;
+            p.q_rows[at] = unit(p.q);
+            p.g_rows[at] = g[i];
+        }
     }
     float lse = INFINITY;        // rows past the end: LSE = +inf (so P = 0) and D = 0
     if (live) lse = p.lse[(int64_t)bh * p.L + row] * 1.4426950408889634f;
@@ -222,20 +224,16 @@ __global__ void __launch_bounds__(kPackThreads) pack_quad_stream_kernel(const Pa
             acc += half_bits_to_float((uint16_t)(ow[k] & 0xFFFF), BF16) * half_bits_to_float((uint16_t)(gw[k] & 0xFFFF), BF16);
             acc += half_bits_to_float((uint16_t)(ow[k] >> 16), BF16) * half_bits_to_float((uint16_t)(gw[k] >> 16), BF16);
         }
-        const int C = part + 8 * i, slot = quad_unit_slot(r, C >> 1, C & 1);
-        dst[slot] = q[i];
-        dst[NC * 64 + slot] = g[i];
     }
     acc += __shfl_xor(acc, 1); acc += __shfl_xor(acc, 2); acc += __shfl_xor(acc, 4);
-    float* st = reinterpret_cast<float*>(dst + 2 * NC * 64);
     if (part == 0) {
-        if (live) p.stats[(int64_t)bh * p.L + row] = make_float2(lse, acc);
-        // statistics fragment: 32 LSE values, then 32 D values, each half wavefront's 16 streamed rows together
+        if (live && p.stats) p.stats[(int64_t)bh * p.L + row] = make_float2(lse, acc);
+        // 32 LSE values, then 32 D values, each half wavefront's 16 streamed rows together
+        float* st = reinterpret_cast<float*>(p.tile_stats + ((size_t)bh * p.n_tiles + t) * kQuadStatBytes);
         const int idx = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
         st[idx] = lse;
         st[32 + idx] = acc;
     }
-    if (threadIdx.x >= 16 && threadIdx.x < 64) dst[2 * NC * 64 + threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);   // the fragment's unused rest
 }
 
 // K^T alone, for attn_dq_from_ds_kernel: a run of kKtTiles tiles of one head per workgroup.  HBM-bound; pack_stream_kernel, which
@@ -253,13 +251,15 @@ __global__ void __launch_bounds__(kPackThreads) pack_kt_kernel(const PackSrc k, 
 }
 
 // ---------------------------------------------------------------------------------------------- main kernels
+struct QuadRows { const char* ptr; int64_t sb, sh; int row; };   // bytes between batches, heads, rows
 struct BwdParams {
     const void *st1, *st2;             // stationary operands: rows of (q, dout) for dQ, of (k, v) for dK/dV
     int64_t s1_sb, s1_sh, s1_sl, s2_sb, s2_sh, s2_sl;
     void *out1, *out2;                 // dq | dv, dk
     int64_t o1_sb, o1_sh, o1_sl, o2_sb, o2_sh, o2_sl;
     const float2* stats;               // [B*H][Lq]
-    const char* stream;                // packed stream tiles [B*H][n_tiles][tile bytes]
+    const char* stream;                // packed stream tiles [B*H][n_tiles][tile bytes]; attn_dkdv_quad_kernel: their statistics alone
+    QuadRows rows_q, rows_do;          // attn_dkdv_quad_kernel: Q and dO
     int H, L_stat, L_stream, n_tiles, causal;
     float sm_scale, scale_log2;
     // 1-D grid: workgroups [0, n_full) each own a (block of 128 stationary rows, head) pair; the remaining n_rem pairs
@@ -1090,6 +1090,15 @@ int validate_bwd(const cosmos_attn_bwd_desc* d) {
     return COSMOS_ATTN_OK;
 }
 
+// Does attn_dkdv_quad_kernel read Q and dO where they are?  It addresses a head's rows with 31-bit offsets, and rows past the end have to lie past the buffer.  Where
+// it can it does: a row's 256 bytes are whole cache lines wherever they lie, and a copy is two more passes over both.  Backward, us, copied / in place (bf16, rows 4 KB
+// apart): 16 heads x 37440 queries x 512 keys 654 / 578, 84480 x 300 1200 / 985, 3520 x 512 86 / 80, 1560 x 1560 107 / 104, 17600 x 17600 6983 / 6958.
+bool quad_in_place(const cosmos_attn_bwd_desc* d) {
+    const int64_t n = (int64_t)(d->Lq + kRows - 1) / kRows * kRows;
+    auto addressed = [&](const int64_t* s) { return s[2] >= d->d && s[2] * 2 <= ((int64_t)1 << 31) / n - 1; };
+    return addressed(d->q_stride) && addressed(d->dout_stride);
+}
+
 PackSrc src_of(const void* ptr, const int64_t* s) { return PackSrc{(const uint16_t*)ptr, s[0], s[1], s[2]}; }
 
 }  // namespace
@@ -1143,11 +1152,22 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
         return true;
     };
 
-    if (g.quad) {   // query stream of attn_dkdv_quad_kernel: Q, dO, statistics
-        PackQuadParams pp;
+    BwdParams bp{};
+    if (g.quad) {   // query stream of attn_dkdv_quad_kernel: Q and dO where they are, statistics
+        const bool copy = !quad_in_place(d);
+        const size_t rows_bytes = (size_t)BH * g.n_q_tiles * kRows * 256;
+        QuadStatsParams pp;
         pp.q = src_of(d->q, d->q_stride); pp.g = src_of(d->dout, d->dout_stride); pp.o = src_of(d->o, d->o_stride);
-        pp.lse = d->lse; pp.stats = stats; pp.out = q_img; pp.H = d->H; pp.L = d->Lq; pp.n_tiles = g.n_q_tiles;
-        hipLaunchKernelGGL(bf16 ? pack_quad_stream_kernel<true> : pack_quad_stream_kernel<false>, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
+        pp.q_rows = (uint4*)q_img; pp.g_rows = (uint4*)(q_img + rows_bytes); pp.tile_stats = q_img + 2 * rows_bytes;
+        pp.lse = d->lse; pp.stats = g.spill ? nullptr : stats; pp.H = d->H; pp.L = d->Lq; pp.n_tiles = g.n_q_tiles;
+        auto fn = bf16 ? (copy ? quad_stats_kernel<true, true> : quad_stats_kernel<true, false>) : (copy ? quad_stats_kernel<false, true> : quad_stats_kernel<false, false>);
+        hipLaunchKernelGGL(fn, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
+        auto rows = [&](const void* ptr, const int64_t* s, const uint4* copied) {
+            const int64_t head = (int64_t)g.n_q_tiles * kRows * 256;
+            return copy ? QuadRows{(const char*)copied, d->H * head, head, 256} : QuadRows{(const char*)ptr, 2 * s[0], 2 * s[1], (int)(2 * s[2])};
+        };
+        bp.rows_q = rows(d->q, d->q_stride, pp.q_rows); bp.rows_do = rows(d->dout, d->dout_stride, pp.g_rows);
+        q_img = pp.tile_stats;
     } else {
         {   // per-query statistics
             StatsParams sp;
@@ -1183,7 +1203,6 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
     }
     if (hipGetLastError() != hipSuccess) return COSMOS_ATTN_LAUNCH_FAILED;
 
-    BwdParams bp;
     bp.stats = stats; bp.H = d->H; bp.causal = d->causal;
     bp.sm_scale = d->sm_scale; bp.scale_log2 = d->sm_scale * 1.4426950408889634f;
     bp.bh0 = 0; bp.ds = nullptr; bp.ds_head_bytes = 0; bp.n_kt_pad = 0;

@@ -19,16 +19,15 @@
 // Pipeline, step s (tile = sweep position):   S1: MFMAs S(s+1) | U(s)      S2: MFMAs dP(s) | W(s-1)
 //                                             O1: tile s-1                 O2: tile s-2
 //
-// One copy of the stream.  A tile is [Q | dO | LSE log2e, D]: 32 rows x 128 channels of each tensor as 16-byte units
-// (row q, 16-channel chunk cK, half hK: 8 channels).  S1 / S2 read them as MFMA A operands with ds_read_b128 (lane = row);
-// O1 / O2 need the transposed operands (lane = channel, 8 rows per lane) and get them from the SAME units with the
-// transposing read ds_read_b64_tr_b16 (within 16 lanes, lane i passes the address of 8 bytes -- row i of a 16 x 4 matrix M of
-// 16-bit values -- and receives M[i/4 + 4k][i%4], k = 0..3): no second, transposed copy of the tile in memory, in the fills
-// or in LDS.  For both kinds of read to be free of bank conflicts the units of a part are stored in the order
-//     slot(q, cK, hK) = 16 (q/16 + 2 hK + 4 cK) + (q%4 + 4 ((q/4)%4 XOR (hK + 2 (cK%2)))):
-// the 16 lanes of a ds_read_b128 pass (16 consecutive rows, one cK, one hK) and the 32 lanes of a transposing pass (4 rows x
-// 2 chunks x 2 halves, both 8-byte halves of each unit) touch 256 consecutive-bank bytes each.  pack_quad_stream_kernel writes the
-// image in that order; the direct-to-LDS fills copy it linearly.
+// One copy of the stream.  A part of a tile in LDS is 32 rows x 128 channels as 16-byte units (row r, chunk C of 8 channels).  S1 / S2
+// read them as MFMA A operands with ds_read_b128 (lane = row); O1 / O2 need the transposed operands (lane = channel, 8 rows per
+// lane) and get them from the SAME units with the transposing read ds_read_b64_tr_b16 (within 16 lanes, lane i passes the address
+// of 8 bytes -- row i of a 16 x 4 matrix M of 16-bit values -- and receives M[i/4 + 4k][i%4], k = 0..3): no second, transposed copy
+// of the tile in memory, in the fills or in LDS.  The unit (r, C) lies at
+//     slot(r, C) = 64 (r/4) + 16 (C/4) + 4 (r%4) + (C%4 XOR (r/4)%4):
+// the 16 lanes of a ds_read_b128 pass (16 consecutive rows, one C) and the 32 lanes of a transposing pass (4 rows x 4 chunks, both
+// 8-byte halves of each unit) touch 256 consecutive-bank bytes each, and a direct-to-LDS load of 64 units is four whole rows, so
+// that the fills read Q and dO rows where they are (or in the copy that is made of rows which they cannot address).
 // LDS: rings of the two stream parts (Q 7 deep: fetched three steps before S1 uses it, kept until O2 has used it three steps
 // later; dO 5 deep), U and W hand-over (two stages each), statistics ring (6).  All fills are issued by the O wavefronts (five
 // 1 KB loads per wavefront and step); one s_barrier per step.  The O wavefronts' LDS reads are written as asm (the compiler
@@ -40,9 +39,6 @@ struct QuadCfg {
     static_assert(D == 128, "built for head dim 128");
     static constexpr int NC = D / 16, NDB = D / 32;
     static constexpr int KP_BYTES = NC * kFragBytes;          // Q part, dO part of a tile
-    static constexpr int Q_SRC = 0, DO_SRC = KP_BYTES, ST_SRC = 2 * KP_BYTES;
-    static constexpr int TILE_FRAGS = 2 * NC + 1;
-    static constexpr int TILE_BYTES = TILE_FRAGS * kFragBytes;
     static constexpr int RQ = 7, RDO = 5, RST = 6;
     static constexpr int HO_BYTES = 4 * kFragBytes;           // hand-over of one group and stage: 64 keys x 32 queries, 16 bit
     static constexpr int Q_OFF = 0;
@@ -51,7 +47,7 @@ struct QuadCfg {
     static constexpr int W_OFF = U_OFF + 4 * HO_BYTES;
     static constexpr int ST_OFF = W_OFF + 4 * HO_BYTES;
     static constexpr int LDS_BYTES = ST_OFF + RST * kFragBytes;
-    static constexpr int LOADS = 5;                           // per O wavefront and step: 2 fragments of each part + the statistics
+    static constexpr int LOADS = 5;                           // per O wavefront and step: 4 rows twice of each part + the statistics
     static constexpr int IN_FLIGHT = 2 * LOADS;               // at the top of a step: all but the loads of the last two steps must have landed
 };
 
@@ -94,24 +90,37 @@ attn_dkdv_quad_kernel(const BwdParams p) {
     auto tile_at = [&](int u) { return __builtin_amdgcn_readfirstlane(t_lo + (u + shift) % n_sweep); };
     auto wrap_inc = [&](int t) { ++t; return t >= t_lo + n_sweep ? t - n_sweep : t; };
 
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(p.stream) + (size_t)bh * p.n_tiles * C::TILE_BYTES, 0, p.n_tiles * C::TILE_BYTES, 0x00020000);
+    auto rows_of = [&](const QuadRows& r) {   // a head's rows; behind the last one zeros are read
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(r.ptr) + (int64_t)b * r.sb + (int64_t)h * r.sh, 0, (p.L_stream - 1) * r.row + 2 * D, 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t rsrc_q = rows_of(p.rows_q), rsrc_do = rows_of(p.rows_do);
+    const __amdgpu_buffer_rsrc_t rsrc_st = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(p.stream) + (size_t)bh * p.n_tiles * kQuadStatBytes, 0, p.n_tiles * kQuadStatBytes, 0x00020000);
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     auto frag = [&](const char* base, int f) { return *reinterpret_cast<const V8*>(base + f * kFragBytes + lane * 16); };
     // A fragment cK of a stream part (lane = row j, half hh): byte offset of this lane's unit, for even / odd cK
-    const int a_off[2] = {16 * quad_unit_slot(j, 0, hh), 16 * quad_unit_slot(j, 1, hh) - kFragBytes};
-    auto afrag = [&](const char* part, int cK) { return *reinterpret_cast<const V8*>(part + cK * kFragBytes + a_off[cK & 1]); };
+    const int a_off[2] = {16 * quad_unit_slot(j, hh), 16 * quad_unit_slot(j, 2 + hh)};
+    auto afrag = [&](const char* part, int cK) { return *reinterpret_cast<const V8*>(part + 256 * (cK >> 1) + a_off[cK & 1]); };
 
-    // ---- fills (O wavefronts): this wavefront's two fragments of a part of tile t into ring slot u
-    const int run = 2 * ow * kFragBytes;
-    auto fill_part = [&](int src_off, int dst_off, int part_bytes, int ring, int t, int u) {
-        issue_part<2>(rsrc, smem + dst_off + (u % ring) * part_bytes + run, lane * 16, t * C::TILE_BYTES + src_off + run);
+    // ---- fills (O wavefronts): this wavefront's eight rows 8 ow .. + 7 of a part of tile t into ring slot u, four rows a load
+    int off_q[2], off_do[2];                      // what this lane reads of them
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 8 * ow + 4 * i + ((lane >> 2) & 3), unit = 4 * (lane >> 4) + ((lane & 3) ^ ((2 * ow + i) & 3));
+        off_q[i] = r * p.rows_q.row + 16 * unit;
+        off_do[i] = r * p.rows_do.row + 16 * unit;
+    }
+    auto fill_part = [&](__amdgpu_buffer_rsrc_t rsrc, const int* off, int row, int part, int t) {
+        char* dst = smem + part + 2 * ow * kFragBytes;
+        lds_load<0>(rsrc, dst, off[0] + t * (kRows * row), 0);
+        lds_load<0>(rsrc, dst + kFragBytes, off[1] + t * (kRows * row), 0);
     };
     auto fill_q = [&](int t, int u) {
-        fill_part(C::Q_SRC, C::Q_OFF, C::KP_BYTES, C::RQ, t, u);
-        lds_load<0>(rsrc, smem + C::ST_OFF + (u % C::RST) * kFragBytes, lane * 16, t * C::TILE_BYTES + C::ST_SRC);
+        fill_part(rsrc_q, off_q, p.rows_q.row, C::Q_OFF + (u % C::RQ) * C::KP_BYTES, t);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_st, (__attribute__((address_space(3))) void*)(smem + C::ST_OFF + (u % C::RST) * kFragBytes), 4, lane * 4,
+                                                 t * kQuadStatBytes, 0, 0);
     };
-    auto fill_do = [&](int t, int u) { fill_part(C::DO_SRC, C::DO_OFF, C::KP_BYTES, C::RDO, t, u); };
+    auto fill_do = [&](int t, int u) { fill_part(rsrc_do, off_do, p.rows_do.row, C::DO_OFF + (u % C::RDO) * C::KP_BYTES, t); };
     if (!s_role) {   // what the steps before step 0 would have issued
         fill_q(tile_at(0), 0);
 #pragma unroll
@@ -345,16 +354,16 @@ attn_dkdv_quad_kernel(const BwdParams p) {
         const int lag = second ? 2 : 1;                       // O1 accumulates tile s-1, O2 tile s-2
         // Transposing reads.  Lane (group g = lane / 16, r = lane % 16) is channel 16 (g%2) + r of a 32-channel block and key-index
         // half g/2 of the MFMA A operand; as a supplier of addresses it passes, for fragment (db, c) and read t, the 8 bytes of row
-        // q = 16 c + 8 t + 4 (g/2) + r/4, channels 32 db + 16 (g%2) + 4 (r%4) .. + 3: unit (q, cK = 2 db + g%2, hK = (r%4)/2), its
-        // second half when r is odd.  Byte offset in the part = 256 c + 2048 db + tr_off[t].
-        const int g16 = lane >> 4, r16 = lane & 15, hK = (r16 & 3) >> 1;
+        // q = 16 c + 8 t + 4 (g/2) + r/4, channels 32 db + 16 (g%2) + 4 (r%4) .. + 3: unit (q, C = 4 db + 2 (g%2) + (r%4)/2), its
+        // second half when r is odd.  Byte offset in the part = 4096 c + 256 db + tr_off[t].
+        const int g16 = lane >> 4, r16 = lane & 15;
         unsigned tr_off[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
-            tr_off[t] = (unsigned)(512 * hK + 1024 * (g16 & 1) + 16 * (r16 >> 2) + 64 * ((2 * t + (g16 >> 1)) ^ (hK + 2 * (g16 & 1))) + 8 * (r16 & 1));
-// one MFMA group's A operand: fragment (db, c) = two transposing reads (t = 0, 1); IMM = 256 c + 2048 db
+            tr_off[t] = (unsigned)(16 * quad_unit_slot(8 * t + 4 * (g16 >> 1) + (r16 >> 2), 2 * (g16 & 1) + ((r16 & 3) >> 1)) + 8 * (r16 & 1));
+// one MFMA group's A operand: fragment (db, c) = two transposing reads (t = 0, 1); IMM = 4096 c + 256 db
 #define QUAD_TR_PAIR(g) asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%4\n\tds_read_b64_tr_b16 %1, %3 offset:%4" \
-                                     : "=&v"(lo[g]), "=&v"(hi[g]) : "v"(ta0), "v"(ta1), "n"(256 * ((g) / NDB) + 2048 * ((g) % NDB)) : "memory")
+                                     : "=&v"(lo[g]), "=&v"(hi[g]) : "v"(ta0), "v"(ta1), "n"(4096 * ((g) / NDB) + 256 * ((g) % NDB)) : "memory")
 // wait until at most N of this wavefront's LDS reads are outstanding; ties the registers the wait makes valid
 #define QUAD_WAIT(N, g) asm volatile("s_waitcnt lgkmcnt(" #N ")" : "+v"(lo[g]), "+v"(hi[g]), "+v"(bf[0][0]), "+v"(bf[0][1]), "+v"(bf[1][0]), "+v"(bf[1][1]) :: "memory")
 #define QUAD_GROUP(g) do { \

@@ -132,6 +132,34 @@ def test_bwd_several_query_blocks_per_workgroup(pkg, oracle, gpu, Lkv):
     run_bwd(pkg, oracle, gpu, (5, 13, 1070, 128), (5, 13, Lkv, 128), seed=Lkv)
 
 
+@pytest.mark.parametrize("Lq", [1, 32, 45, 300])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("which", ["q", "dout", "far"])
+def test_bwd_query_rows_the_kernel_does_not_address(pkg, oracle, gpu, Lq, dtype, which):
+    """Rows that lie less than a row's bytes apart (one row for all queries), or so far apart that a head's rows span 2 GiB, are copied first: the gradients are
+    those of the same values in ordinary rows, byte for byte, and within the tolerances above."""
+    q, k, v, _, _, _ = oracle.make_inputs((2, 3, Lq, 128), (2, 3, 70, 128), seed=Lq, dtype=dtype)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(Lq)).to(dtype)
+    if which == "q":
+        q = q[:, :, :1].expand(q.shape)
+    elif which == "dout":
+        dout = dout[:, :, :1].expand(q.shape)
+    qd, dd, kd, vd = q.to(gpu), dout.to(gpu), k.to(gpu), v.to(gpu)
+    if which == "q":
+        qd = qd[:, :, :1].expand(q.shape)
+    elif which == "dout":
+        dd = dd[:, :, :1].expand(q.shape)
+    else:
+        stride = max(2 ** 30 // (32 * ((Lq + 31) // 32)), 6 * 128)
+        qd = torch.empty(Lq * stride, dtype=dtype, device=gpu).as_strided((2, 3, Lq, 128), (3 * 128, 128, stride, 1)).copy_(qd)
+    o, _, lse = pkg.fwd_jvp(q.to(gpu).contiguous(), kd, vd)
+    got = pkg.ops.bwd(qd, kd, vd, o, lse, dd)
+    same = pkg.ops.bwd(qd.contiguous(), kd, vd, o, lse, dd.contiguous())
+    for name, a, b, ref in zip(("dq", "dk", "dv"), got, same, oracle.grads_closed_form(q, k, v, dout)):
+        assert torch.equal(a, b), name
+        check(oracle, name, a, ref)
+
+
 def test_bwd_through_autograd_function(pkg, oracle, gpu):
     """`attention(q, k, v, tq, tk, tv, causal, sm_scale)[0].backward(dout)` like the reference's procedure."""
     q, k, v, tq, tk, tv = oracle.make_inputs((1, 2, 300, 64), (1, 2, 300, 64), seed=3, primal_std=0.5)
