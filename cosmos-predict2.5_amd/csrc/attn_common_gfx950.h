@@ -20,6 +20,8 @@ __device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 // A value that exists once per 32-lane half of a wavefront, made visible to both halves: afterwards, in every lane l,
 // `lo` is what lane l % 32 held and `hi` what lane 32 + l % 32 held (one v_permlane32_swap, no LDS round trip).  The
 // instruction is written out: given one value for both of its operands, the compiler's builtin treats its two results as
@@ -81,7 +83,7 @@ __device__ __host__ constexpr float max_slack_of(bool with_tangents) {
 // fragment index travels in the instruction's immediate offset, which is added to both addresses.
 struct LoadJob {
     __amdgpu_buffer_rsrc_t rsrc;
-    int lane_off;            // 16 * lane
+    int lane_off, k_lane_off;   // 16 * lane; for K parts 16 * the lane whose unit this one copies
     int k_src, v_src;        // byte offsets of this wavefront's runs in the packed buffer
     char *k_dst, *v_dst;     // LDS destinations of the runs
 };

@@ -17,6 +17,7 @@
 //     every 32 keys, so the softmax row reductions are in-lane plus ONE exchange with lane^32, and the
 //     fp32 S^T registers, once converted to 16-bit, ARE the B operand of O^T = V^T P^T -- no LDS or
 //     cross-lane shuffle between the two GEMM stages.
+//     (At head dim 128 the large forward-only workgroups and the stream with all tangents work in 16 x 16 x 32 products: attn_mfma16_gfx950.h.)
 //   * K, V (and dK, dV) are re-tiled ONCE per call by `pack_kv_kernel` into "LDS images": for every
 //     32-key tile, the exact byte order in which the MFMA A-operand fragments are consumed
 //     (1 KB per fragment = 64 lanes x 16 B, V already transposed and key-permuted to match the
@@ -194,7 +195,7 @@ template <typename C>
 __device__ __forceinline__ void issue_group(const LoadJob& j) {
     static_assert(C::KP_LOADS <= 4 && C::VP_LOADS <= 4, "a part has at most 16 fragments");
     issue_part<C::VP_LOADS>(j.rsrc, j.v_dst, j.lane_off, j.v_src);
-    issue_part<C::KP_LOADS>(j.rsrc, j.k_dst, j.lane_off, j.k_src);
+    issue_part<C::KP_LOADS>(j.rsrc, j.k_dst, j.k_lane_off, j.k_src);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -213,6 +214,7 @@ struct ScoreWave {
     // 8 (e/4) + 4 (lane/32) + e%4 of the tile) -- the accumulator registers of the score MFMAs themselves.
     struct Scores { f32x16 s, ds; };
 
+    static constexpr int N = 1, NQ = NC;    // (queries of a lane, chunks of channels: see ScoreWave16)
     V8 qf[NC], tqf[NC];
     float m_run, l_run, r_run;
     float scale_log2, sm_scale;
@@ -233,6 +235,18 @@ struct ScoreWave {
         for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x.s[e]);
         return mx;
     }
+
+    // what attn_qstream_kernel calls, of this and of ScoreWave16
+    __device__ __forceinline__ void start() { m_run = -INFINITY; l_run = r_run = 0.f; }
+    __device__ __forceinline__ static float both(float x) {
+        float lo, hi;
+        both_halves(x, lo, hi);
+        return lo + hi;
+    }
+    __device__ __forceinline__ float l_total() const { return both(l_run); }
+    __device__ __forceinline__ float r_total() const { return both(r_run); }
+    __device__ __forceinline__ void mask(Scores& x, int key0, int kv_len) const { mask_scores(x, key0 + 4 * (lane >> 5), kv_len, false, 0); }
+    __device__ __forceinline__ float fold_max(const Scores& x) { return update_max(lane_max(x)); }
 
     // Rare path (last tile of a ragged / padded key range, causal diagonal): masked keys (>= kv_len, or above the
     // diagonal when causal) get score -inf, hence p = 0 and H = 0.
@@ -358,6 +372,23 @@ struct OutputWave {
     f32x16 acc[NDB], acct[NDB];
     int lane;
 
+    // what attn_qstream_kernel calls, of this and of OutputWave16: channels 8 N g + 4 (lane / (32 / N)) .. + 3 of query n
+    static constexpr int N = 1;
+    __device__ __forceinline__ static f32x4 four(const f32x16* a, int g) {
+        const f32x16& b = a[g >> 2];
+        const int e = 4 * (g & 3);
+        return f32x4{b[e], b[e + 1], b[e + 2], b[e + 3]};
+    }
+    __device__ __forceinline__ f32x4 acc4(int g, int) const { return four(acc, g); }
+    __device__ __forceinline__ f32x4 acct4(int g, int) const { return four(acct, g); }
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int i = 0; i < NDB; ++i) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) { acc[i][e] = 0.f; if (JVP) acct[i][e] = 0.f; }
+        }
+    }
+
     __device__ __forceinline__ V8 lds_frag(const char* base, int frag) const {
         return *reinterpret_cast<const V8*>(base + frag * kFragBytes + lane * 16);
     }
@@ -460,6 +491,8 @@ struct OutputWave {
     }
 };
 
+#include "attn_mfma16_gfx950.h"
+
 template <typename T, int DQK, int DV, int MODE, bool RAW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kAttnThreads, kAttnThreads), amdgpu_waves_per_eu(2, 2)))
 attn_fwd_jvp_kernel(const AttnParams p) {
@@ -521,7 +554,7 @@ attn_fwd_jvp_kernel(const AttnParams p) {
     // tk / tv: tiles whose K part / V part the group copies; ku / vu: sweep positions that pick the ring slots
     auto make_job = [&](int tk, int ku, int tv, int vu) {
         LoadJob jb;
-        jb.rsrc = kv_rsrc; jb.lane_off = lane * 16;
+        jb.rsrc = kv_rsrc; jb.lane_off = jb.k_lane_off = lane * 16;
         jb.k_src = tk * TILE_BYTES + k_run; jb.k_dst = kring + (ku % kRingK) * KP_BYTES + k_run;
         jb.v_src = tv * TILE_BYTES + KP_BYTES + v_run; jb.v_dst = vring + (vu % kRingV) * VP_BYTES + v_run;
         return jb;
@@ -765,11 +798,12 @@ template <typename T, int DQK, int DV, int MODE>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kAttnThreads, kAttnThreads), amdgpu_waves_per_eu(2, 2)))
 attn_qstream_kernel(const AttnParams p) {
     typedef AttnCfg<DQK, DV, MODE> C;
-    typedef ScoreWave<T, DQK, DV, MODE> SW;
-    typedef OutputWave<T, DQK, DV, MODE> OW;
+    constexpr bool M16 = DQK == 128 && DV == 128 && MODE == MODE_JVP_FULL;        // measured both ways: attn_mfma16_gfx950.h
+    typedef std::conditional_t<M16, ScoreWave16<T, MODE>, ScoreWave<T, DQK, DV, MODE>> SW;
+    typedef std::conditional_t<M16, OutputWave16<T, MODE>, OutputWave<T, DQK, DV, MODE>> OW;
+    constexpr int N = SW::N, NQ = SW::NQ, QR = 32 / N;      // a lane's queries are QR n + lane % QR
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
-    constexpr int NC = C::NC, NDB = C::NDB;
     constexpr bool JVP = C::JVP;
     constexpr int KP_BYTES = C::KP_BYTES, VP_BYTES = C::VP_BYTES, TILE_BYTES = C::TILE_BYTES;
     typedef StreamStores<DV, MODE> ST;
@@ -791,6 +825,7 @@ attn_qstream_kernel(const AttnParams p) {
     const bool score_role = wave < 4;
     const int qw = wave & 3;
     const int j = lane & 31, hh = lane >> 5;
+    const int jq = lane % QR, pq = lane / QR;
 
     // Which (query block, head) pairs this workgroup serves.  All pairs, in the order (batch, head, query block), form one
     // line of work; a pair of batch row b weighs 2 n_b + kStreamBlockCost half steps (n_b key tiles per block, plus what
@@ -857,7 +892,7 @@ attn_qstream_kernel(const AttnParams p) {
     const int k_run = ((qw * C::KP_LOADS) % C::KP_FR) * kFragBytes, v_run = ((qw * C::VP_LOADS) % C::VP_FR) * kFragBytes;
     auto make_job = [&](int tk, int ku, int tv, int vu) {
         LoadJob jb;
-        jb.rsrc = kv_rsrc; jb.lane_off = lane * 16;
+        jb.rsrc = kv_rsrc; jb.lane_off = lane * 16; jb.k_lane_off = (M16 ? k_fill_lane(lane) : lane) * 16;
         jb.k_src = tk * TILE_BYTES + k_run; jb.k_dst = kring + (ku % kRingK) * KP_BYTES + k_run;
         jb.v_src = tv * TILE_BYTES + KP_BYTES + v_run; jb.v_dst = vring + (vu % kRingV) * VP_BYTES + v_run;
         return jb;
@@ -866,7 +901,7 @@ attn_qstream_kernel(const AttnParams p) {
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
             const LoadJob jb = make_job(tile_at(u), u, 0, 0);
-            issue_part<C::KP_LOADS>(jb.rsrc, jb.k_dst, jb.lane_off, jb.k_src);
+            issue_part<C::KP_LOADS>(jb.rsrc, jb.k_dst, jb.k_lane_off, jb.k_src);
         }
         issue_group<C>(make_job(tile_at(3), 3, tile_at(0), 0));
     }
@@ -882,28 +917,28 @@ attn_qstream_kernel(const AttnParams p) {
         w.lane = lane;
         w.scale_log2 = p.scale_log2;
         w.sm_scale = p.sm_scale;
-        // Q (and dQ) fragments of a query block: B operand of S^T = K Q^T; lane holds Q[row][16 c + 8 hh .. +7] (rows past
+        // Q (and dQ) fragments of a query block: B operand of S^T = K Q^T; lane holds Q[row][16 N c + 8 pq .. +7] (rows past
         // Lq read the last row instead: their results are never stored).  Addresses are a wavefront-uniform base (scalar
         // registers) plus a 32-bit lane offset (the launch code sends only tensors here whose heads span less than 2 GiB):
         // no 64-bit per-lane pointers live across the steps.
         const char* const q_head = reinterpret_cast<const char*>(p.q) + ((int64_t)b * p.q_sb + (int64_t)h * p.q_sh) * 2;
         const char* const tq_head = reinterpret_cast<const char*>(JVP ? p.tq : p.q) + ((int64_t)b * p.q_sb + (int64_t)h * p.q_sh) * 2;
-        auto q_off = [&](int qt) {
-            int row = qt * kBlockM + qw * 32 + j;
+        auto row_off = [&](int qt, int r) {        // byte offset of row r of this wavefront's 32
+            int row = qt * kBlockM + qw * 32 + r;
             row = row < p.Lq ? row : p.Lq - 1;
-            return ((unsigned)row * (unsigned)p.q_sl + 8u * hh) * 2u;
+            return (unsigned)row * (unsigned)p.q_sl * 2u;
         };
-        {
-            const unsigned off = q_off(qt0);
+        auto q_off = [&](int qt, int n) { return row_off(qt, QR * n + jq) + 16u * pq; };
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                w.qf[c] = *reinterpret_cast<const V8*>(q_head + off + 32 * c);
-                if (JVP) w.tqf[c] = *reinterpret_cast<const V8*>(tq_head + off + 32 * c);
+        for (int n = 0; n < N; ++n) {
+            const unsigned off = q_off(qt0, n);
+#pragma unroll
+            for (int c = 0; c < NQ; ++c) {
+                w.qf[n * NQ + c] = *reinterpret_cast<const V8*>(q_head + off + 32 * N * c);
+                if (JVP) w.tqf[n * NQ + c] = *reinterpret_cast<const V8*>(tq_head + off + 32 * N * c);
             }
         }
-        w.m_run = -INFINITY;
-        w.l_run = 0.f;
-        w.r_run = 0.f;
+        w.start();
         // The next block's rows replace the current ones in place.  With tangents on k and v: step n-2 of a block computes
         // the block's last scores, and right after the MFMAs of d chunk c it fetches chunk c of the next block into the
         // same registers; step n-1 (the next block's first scores) then waits chunk by chunk.  That leaves a load one step
@@ -974,8 +1009,8 @@ attn_qstream_kernel(const AttnParams p) {
         asm volatile("" ::: "memory");
         float alpha = 1.0f;
         auto fold = [&](typename SW::Scores& x, int t) {
-            if (need_mask(t)) SW::mask_scores(x, t * kBlockN + 4 * hh, kv_len, false, 0);
-            alpha = w.update_max(SW::lane_max(x));
+            if (need_mask(t)) w.mask(x, t * kBlockN, kv_len);
+            alpha = w.fold_max(x);
         };
         w.scores_plain(sc0, kring);
         fold(sc0, tile_at(0));
@@ -999,26 +1034,34 @@ attn_qstream_kernel(const AttnParams p) {
             const unsigned ph_out = lds0 + ph_base + (f & 1) * 4 * C::PH_BYTES, alpha_out = lds0 + alpha_base + (f & 1) * 4 * 256;
             const char* const kpart = kring + ((f + 1) % kRingK) * KP_BYTES;
             if (KIND == 0 && more && s_in == 0) {
-                const unsigned off = q_off(qt0 + qi + 1) - 16u * hh + (Q_LINES > 1 ? 128u * hh : 0u);
+                const unsigned off = row_off(qt0 + qi + 1, j) + (Q_LINES > 1 ? 128u * hh : 0u);
                 warm_q = *reinterpret_cast<const int*>(q_head + off);
                 if (JVP) warm_tq = *reinterpret_cast<const int*>(tq_head + off);
             }
             if (KIND == 2 && TRICKLE && more) {
-                // the next block's rows, from the pair's LDS region: 16-byte piece k = 2 c + hh of row j sits at position
-                // k ^ (j mod CPR) of the row
-                const char* const src = smem + xp_base + j * ST::ROW_BYTES;
+                // the next block's rows, from the pair's LDS region: 16-byte piece k of row r sits at position k ^ (r mod CPR) of the row
 #pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    const unsigned pos = (unsigned)((2 * c + hh) ^ (j & (ST::CPR - 1))) << 4;
-                    w.qf[c] = *reinterpret_cast<const V8*>(src + pos);
-                    if (JVP) w.tqf[c] = *reinterpret_cast<const V8*>(src + 32 * ST::ROW_BYTES + pos);
+                for (int n = 0; n < N; ++n) {
+                    const int r = QR * n + jq;
+                    const char* const src = smem + xp_base + r * ST::ROW_BYTES;
+#pragma unroll
+                    for (int c = 0; c < NQ; ++c) {
+                        const unsigned pos = (unsigned)((2 * N * c + pq) ^ (r & (ST::CPR - 1))) << 4;
+                        w.qf[n * NQ + c] = *reinterpret_cast<const V8*>(src + pos);
+                        if (JVP) w.tqf[n * NQ + c] = *reinterpret_cast<const V8*>(src + 32 * ST::ROW_BYTES + pos);
+                    }
                 }
             }
             if (KIND == 1 && !TRICKLE && more) {
-                const unsigned off = q_off(qt0 + qi + 1);
+                unsigned off[N];
+#pragma unroll
+                for (int n = 0; n < N; ++n) off[n] = q_off(qt0 + qi + 1, n);
                 w.step(cur, nxt, kpart, ph_out, alpha_out, alpha, [&](int c) {
-                    w.qf[c] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(q_head + off + 32 * c));
-                    if (JVP) w.tqf[c] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(tq_head + off + 32 * c));
+#pragma unroll
+                    for (int n = 0; n < N; ++n) {
+                        w.qf[n * NQ + c] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(q_head + off[n] + 32 * N * c));
+                        if (JVP) w.tqf[n * NQ + c] = __builtin_nontemporal_load(reinterpret_cast<const V8*>(tq_head + off[n] + 32 * N * c));
+                    }
                 });
             } else {
                 w.step(cur, nxt, kpart, ph_out, alpha_out, alpha);
@@ -1030,10 +1073,7 @@ attn_qstream_kernel(const AttnParams p) {
             }
             if (KIND == 2) {
                 // statistics of the finished block: 1 / l and r / l to the output wavefront, LSE = (m + log2 l) ln 2
-                float l_lo, l_hi, r_lo, r_hi;
-                both_halves(w.l_run, l_lo, l_hi);
-                both_halves(w.r_run, r_lo, r_hi);
-                const float l_tot = l_lo + l_hi, r_tot = r_lo + r_hi;
+                const float l_tot = w.l_total(), r_tot = w.r_total();
                 const float inv_l = 1.0f / l_tot;
                 const float r_over_l = r_tot * inv_l;
                 const unsigned sa = lds0 + stat_base + (qi & 1) * 2 * 4 * 256 + 4 * lane;
@@ -1042,7 +1082,7 @@ attn_qstream_kernel(const AttnParams p) {
                 const int row = (qt0 + qi) * kBlockM + qw * 32 + j;
                 if (row < p.Lq && p.lse && hh == 0)
                     p.lse[(int64_t)bh * p.Lq + row] = (w.m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
-                w.m_run = -INFINITY; w.l_run = 0.f; w.r_run = 0.f;
+                w.start();
             }
             if (f + 1 < n_flat) fold(nxt, t_v);
             if (KIND == 2) alpha = 0.0f;         // the next block's first tile: see above
@@ -1076,14 +1116,7 @@ attn_qstream_kernel(const AttnParams p) {
     } else {
         OW w;
         w.lane = lane;
-        auto zero_acc = [&]() {
-#pragma unroll
-            for (int i = 0; i < NDB; ++i) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) { w.acc[i][e] = 0.f; if (JVP) w.acct[i][e] = 0.f; }
-            }
-        };
-        zero_acc();
+        w.clear();
         // TRICKLE: the next block's Q (and dQ) rows of this pair go to the pair's LDS region during the score wavefront's
         // step n-2, as direct-to-LDS loads of 1 KB each that cover whole rows (RPS rows per load, SPT loads per tensor):
         // lane l fills 16-byte position l % CPR of row l / CPR with piece (l % CPR) ^ (row mod CPR) of that row, the
@@ -1137,56 +1170,58 @@ attn_qstream_kernel(const AttnParams p) {
                        smem + alpha_base + ((f - 1) & 1) * 4 * 256);
                 if (++s_in == n) {
                     // O = acc / l ; dO = (T - (r / l) acc) / l   (statistics published by the barrier at the top of this step)
-                    const char* st = smem + stat_base + (qi & 1) * 2 * 4 * 256 + 4 * lane;
-                    const float inv_l = *reinterpret_cast<const float*>(st);
-                    const float r_over_l = *reinterpret_cast<const float*>(st + 1024);
+                    const char* st = smem + stat_base + (qi & 1) * 2 * 4 * 256 + 4 * jq;
+                    float inv_l[N], r_over_l[N];
+#pragma unroll
+                    for (int n = 0; n < N; ++n) {
+                        inv_l[n] = *reinterpret_cast<const float*>(st + 4 * QR * n);
+                        r_over_l[n] = *reinterpret_cast<const float*>(st + 1024 + 4 * QR * n);
+                    }
                     const int row0 = (qt0 + qi) * kBlockM + qw * 32;
+                    auto four = [&](int g, int n) {        // channels 8 N g + 4 pq .. + 3 of query n
+                        const f32x4 a = w.acc4(g, n);
+                        V4 ov;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) ov[r] = (T)(a[r] * inv_l[n]);
+                        return ov;
+                    };
+                    auto four_t = [&](int g, int n) {
+                        const f32x4 a = w.acc4(g, n), at = w.acct4(g, n);
+                        V4 tov;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) tov[r] = (T)((at[r] - r_over_l[n] * a[r]) * inv_l[n]);
+                        return tov;
+                    };
+                    constexpr int NG = DV / (8 * N);
                     if constexpr (TRICKLE) {
-                        // accumulator lane (j, hh) holds channels 32 db + 8 g + 4 hh .. +3 of row j: 8 bytes of 16-byte chunk
-                        // 4 db + g, which goes to chunk position (4 db + g) ^ (j mod CPR) of row j of the region
-                        // (the row address is made opaque here so that the chunk addresses are computed on the spot, one XOR
+                        // 8 bytes of 16-byte chunk N g + pq / 2 of row QR n + jq, which goes to chunk position (N g + pq / 2) ^ (jq mod CPR) of that row of
+                        // the region  (the row address is made opaque here so that the chunk addresses are computed on the spot, one XOR
                         // each, instead of being kept in registers across the whole stream)
-                        unsigned xw = lds0 + xp_base + j * ST::ROW_BYTES + 8 * hh + ((j & (ST::CPR - 1)) << 4);
+                        unsigned xw = lds0 + xp_base + jq * ST::ROW_BYTES + 8 * (pq & 1) + ((unsigned)((pq >> 1) ^ (jq & (ST::CPR - 1))) << 4);
                         asm volatile("" : "+v"(xw));
 #pragma unroll
-                        for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-                            for (int g = 0; g < 4; ++g) {
-                                if (32 * db + 8 * g < DV) {
-                                    const unsigned a = xw ^ ((4 * db + g) << 4);
-                                    V4 ov, tov;
-#pragma unroll
-                                    for (int r = 0; r < 4; ++r) {
-                                        ov[r] = (T)(w.acc[db][4 * g + r] * inv_l);
-                                        if (JVP) tov[r] = (T)((w.acct[db][4 * g + r] - r_over_l * w.acc[db][4 * g + r]) * inv_l);
-                                    }
-                                    asm volatile("ds_write_b64 %0, %1" ::"v"(a), "v"(ov) : "memory");
-                                    if (JVP) asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(tov), "n"(32 * ST::ROW_BYTES) : "memory");
-                                }
+                        for (int g = 0; g < NG; ++g) {
+                            const unsigned a = xw ^ ((N * g) << 4);
+                            asm volatile("ds_write_b64 %0, %1" ::"v"(a), "v"(four(g, 0)) : "memory");
+                            if (JVP) asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(four_t(g, 0)), "n"(32 * ST::ROW_BYTES) : "memory");
+                            if constexpr (N > 1) {
+                                asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(four(g, 1)), "n"(QR * ST::ROW_BYTES) : "memory");
+                                if (JVP) asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(a), "v"(four_t(g, 1)), "n"((32 + QR) * ST::ROW_BYTES) : "memory");
                             }
                         }
                         __builtin_amdgcn_s_waitcnt(0xC07F);   // the region is complete before the next barrier publishes it
                     } else if (row0 < p.Lq) {           // wavefront-uniform: every wavefront that stores issues all N_STORES stores
-                        const int row = row0 + j;
-                        const int64_t off = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl;
-                        T* op = reinterpret_cast<T*>(p.o) + off;
-                        T* top = reinterpret_cast<T*>(p.to) + off;
-                        if (row < p.Lq) {
 #pragma unroll
-                            for (int db = 0; db < NDB; ++db) {
+                        for (int n = 0; n < N; ++n) {
+                            const int row = row0 + QR * n + jq;
+                            const int64_t off = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl + 4 * pq;
+                            T* op = reinterpret_cast<T*>(p.o) + off;
+                            T* top = reinterpret_cast<T*>(p.to) + off;
+                            if (row < p.Lq) {
 #pragma unroll
-                                for (int g = 0; g < 4; ++g) {
-                                    const int d = 32 * db + 8 * g + 4 * hh;   // registers 4g..4g+3 are 4 consecutive d
-                                    if (32 * db + 8 * g < DV) {
-                                        V4 ov, tov;
-#pragma unroll
-                                        for (int r = 0; r < 4; ++r) {
-                                            ov[r] = (T)(w.acc[db][4 * g + r] * inv_l);
-                                            if (JVP) tov[r] = (T)((w.acct[db][4 * g + r] - r_over_l * w.acc[db][4 * g + r]) * inv_l);
-                                        }
-                                        asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(op + d), "v"(ov) : "memory");
-                                        if (JVP) asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(top + d), "v"(tov) : "memory");
-                                    }
+                                for (int g = 0; g < NG; ++g) {
+                                    asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(op + 8 * N * g), "v"(four(g, n)) : "memory");
+                                    if (JVP) asm volatile("global_store_dwordx2 %0, %1, off" ::"v"(top + 8 * N * g), "v"(four_t(g, n)) : "memory");
                                 }
                             }
                         }
@@ -1215,9 +1250,8 @@ attn_qstream_kernel(const AttnParams p) {
 // the matrix unit) and some 125 such turns, 64 of them in 16 exponentials; in long calls the part's power limit on top (80 % MFMA duty
 // at 1.53 GHz, 37440 positions; 66 % at 1.76 GHz before).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
 // formed where it did not move (kMaxTileSum).  Measured, us, before either / with the softmax between the MFMAs / with both: 16 heads,
-// d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120.
-// Not faster: v_mfma_f32_16x16x32 (less energy, but twice the MFMA instructions to issue: 37440 9450, 3520 142), operand fetches three
-// groups ahead, the fills spread over the step.
+// d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120; with 384 rows a workgroup in
+// 16 x 16 x 32 products another 5 % of the long ones (SymWave16).  Not faster: operand fetches three groups ahead, the fills spread over the step.
 //
 // A workgroup is RG groups of 32 query rows x KG groups of keys: of every KG tiles of 32 keys a wavefront takes one, and the KG partial
 // results of a row group (accumulator, running max, row sum) are merged through LDS at the end.  Large calls take 12 x 1; 8 x 1 and 4 x 2
@@ -1250,6 +1284,8 @@ struct SymWave {
     static constexpr int NB = 2 * NDB;      // P.V MFMA groups of a tile, (c, db) at index c * NDB + db
     static constexpr int PD = COSMOS_ATTN_PREFETCH_GROUPS;
 
+    static constexpr int N = 1, NQ = NC;    // (queries of a lane, chunks of channels: see SymWave16)
+    typedef f32x16 Scores;
     V8 qf[NC];
     f32x16 acc[NDB];
     float m_run, l_run, scale_log2;
@@ -1283,6 +1319,33 @@ struct SymWave {
     __device__ __forceinline__ V8 lds_frag(const char* base, int frag) const {
         return *reinterpret_cast<const V8*>(base + frag * kFragBytes + lane * 16);
     }
+    // what attn_fwd_sym_kernel calls, of this and of SymWave16
+    __device__ __forceinline__ void start(int l) {
+        lane = l;
+        m_run = -INFINITY;
+        l_run = l_tile = 0.f;
+#pragma unroll
+        for (int i = 0; i < NDB; ++i) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
+        }
+        if constexpr (RAW) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { vt_off[i] = raw_vt_offset(i, l); k_off[i] = raw_k_offset(i, l); }
+        }
+    }
+    __device__ __forceinline__ f32x4 acc4(int g, int) const {
+        const f32x16& b = acc[g >> 2];
+        const int e = 4 * (g & 3);
+        return f32x4{b[e], b[e + 1], b[e + 2], b[e + 3]};
+    }
+    __device__ __forceinline__ float l_total() const { return l_run + __shfl_xor(l_run, 32); }
+    __device__ __forceinline__ float m_total() const { return m_run; }
+    __device__ __forceinline__ static void of_rows(float x, float* one) { one[0] = x; }
+    __device__ __forceinline__ void mask(f32x16& x, int key0, int kv_len, bool causal, int row0) const {
+        mask_scores(x, key0 + 4 * (lane >> 5), kv_len, causal, row0 + (lane & 31));
+    }
+    __device__ __forceinline__ void first_max(const f32x16& x) { raise_max(x); }
     // this lane's scores of a tile: its query column x 16 of the 32 keys (element e is key 8 (e/4) + 4 (lane/32) + e%4)
     __device__ __forceinline__ static float lane_max(const f32x16& s) {
         float mx = s[0];
@@ -1402,11 +1465,14 @@ template <typename T, int DQK, int DV, int RG, int KG, bool RAW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * RG * KG, 64 * RG * KG), amdgpu_waves_per_eu(RG * KG / 4, RG * KG / 4)))
 attn_fwd_sym_kernel(const AttnParams p) {
     typedef SymCfg<DQK, DV, RG, KG> C;
-    typedef SymWave<T, DQK, DV, RAW> W;
+    constexpr bool M16 = RG == 12 && DQK == 128 && DV == 128;                  // measured both ways: attn_mfma16_gfx950.h
+    typedef std::conditional_t<M16, SymWave16<T>, SymWave<T, DQK, DV, RAW>> W;
+    constexpr int N = W::N, NQ = W::NQ, QR = 32 / N;        // a lane's queries are QR n + lane % QR
+    static_assert(!M16 || KG == 1, "the merge of key groups is SymWave's");
     static_assert(!RAW || (DQK == 128 && DV == 128), "rows of 256 bytes");
     typedef typename VecOf<T>::v8 V8;
     typedef typename VecOf<T>::v4 V4;
-    constexpr int NC = C::NC, NDB = C::NDB, BLOCK_M = 32 * RG;
+    constexpr int NDB = C::NDB, BLOCK_M = 32 * RG;
     constexpr int TILE_BYTES = C::TILE_BYTES, KS_BYTES = C::KS_BYTES, VS_BYTES = C::VS_BYTES, TPS = C::TPS, RING = C::RING;
     // K(s), V(s): the K parts / V parts of the TPS packed tiles at sweep position s ("step tile" t = tiles TPS t .. TPS t + TPS - 1).
     // KG = 1: a wavefront does the two tiles of a step one after the other; KG = 2: one of them.  Step s reads K(s), K(s+1), V(s) and
@@ -1424,9 +1490,8 @@ attn_fwd_sym_kernel(const AttnParams p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rg = wave % RG, kg = wave / RG;
-    const int j = lane & 31, hh = lane >> 5;
+    auto here = [&]() { return M16 ? lane_again() : lane; };
     const int row0 = qt * BLOCK_M + rg * 32;        // first query row of this wavefront
-    const int row = row0 + j;                       // this lane's query row (lanes l and l^32 share it)
 
     int kv_len = p.Lkv;
     if (p.key_lens) { const int kl = p.key_lens[b]; kv_len = kl < kv_len ? (kl < 0 ? 0 : kl) : kv_len; }
@@ -1458,14 +1523,14 @@ attn_fwd_sym_kernel(const AttnParams p) {
             raw_k.template k<C::K_LOADS>(kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, (t * TPS + kf0 / C::K_FR) * kBlockN, kf0 % C::K_FR, lane);
             return;
         }
-        if (wave < C::FW) issue_part<C::K_LOADS>(kv_rsrc, kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + k_src_run);
+        if (wave < C::FW) issue_part<C::K_LOADS>(kv_rsrc, kring + (u % RING) * KS_BYTES + kf0 * kFragBytes, (M16 ? k_fill_lane(here()) : lane) * 16, t * TPS * TILE_BYTES + k_src_run);
     };
     auto fill_v = [&](int t, int u) {
         if constexpr (RAW) {
             raw_v.template v<C::V_LOADS>(vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, (t * TPS + vf0 / C::VT_FR) * kBlockN + 4 * (vf0 % C::VT_FR), lane);
             return;
         }
-        if (wave < C::FW) issue_part<C::V_LOADS>(kv_rsrc, vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, lane * 16, t * TPS * TILE_BYTES + v_src_run);
+        if (wave < C::FW) issue_part<C::V_LOADS>(kv_rsrc, vring + (u % RING) * VS_BYTES + vf0 * kFragBytes, here() * 16, t * TPS * TILE_BYTES + v_src_run);
     };
     constexpr int PRE = RING - 1;
 #pragma unroll
@@ -1475,43 +1540,33 @@ attn_fwd_sym_kernel(const AttnParams p) {
     }
 
     W w;
-    w.lane = lane;
-    w.scale_log2 = p.scale_log2;
-    if constexpr (RAW) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { w.vt_off[i] = raw_vt_offset(i, lane); w.k_off[i] = raw_k_offset(i, lane); }
-    }
-    {
-        const int64_t off = (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)row * p.q_sl + 8 * hh;
-        const T* qp = reinterpret_cast<const T*>(p.q) + off;
+    for (int n = 0; n < N; ++n) {
+        const int row = row0 + QR * n + lane % QR;
+        const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)row * p.q_sl + 8 * (lane / QR);
         const bool live = row < p.Lq;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            V8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-            w.qf[c] = live ? *reinterpret_cast<const V8*>(qp + 16 * c) : z;
+        for (int c = 0; c < NQ; ++c) {
+            const V8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+            w.qf[n * NQ + c] = live ? *reinterpret_cast<const V8*>(qp + 16 * N * c) : z;
         }
     }
-#pragma unroll
-    for (int i = 0; i < NDB; ++i) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) w.acc[i][e] = 0.f;
-    }
+    w.start(lane);
+    w.scale_log2 = p.scale_log2;
     // (a key group's tiles may all be masked for a while, or throughout: its max starts at a number, so that exp2(-inf - max) is 0)
-    w.m_run = KG == 1 ? -INFINITY : -3.0e38f;
-    w.l_run = 0.f;
+    if constexpr (KG > 1) w.m_run = -3.0e38f;
 
     const bool causal = p.causal != 0;
     auto need_mask = [&](int t) { return (t * kBlockN + kBlockN > kv_len) || (causal && (t * kBlockN + kBlockN - 1 > row0)); };
-    auto mask = [&](f32x16& x, int t) { if (need_mask(t)) W::mask_scores(x, t * kBlockN + 4 * hh, kv_len, causal, row); };
-    f32x16 sc0, sc1;   // scores of the current / next tile, swapping roles every tile
+    auto mask = [&](typename W::Scores& x, int t) { if (need_mask(t)) w.mask(x, t * kBlockN, kv_len, causal, row0); };
+    typename W::Scores sc0, sc1;   // scores of the current / next tile, swapping roles every tile
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): Q and this wavefront's share of the first fills are here
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     w.scores_plain(sc0, kring + kg * C::KP_BYTES);
-    w.l_tile = 0.f;
     if (n_steps > 0) {
         mask(sc0, TPS * tile_at(0) + kg);
-        w.raise_max(sc0);
+        w.first_max(sc0);
         w.softmax_elems(sc0, 0, 8);
     }
     // past the last position there is no next tile: whatever scores are formed for it are masked, so that they add nothing
@@ -1531,7 +1586,7 @@ attn_fwd_sym_kernel(const AttnParams p) {
         }
     } else {
         int g_nxt = tile_at(1), g_fill = tile_at(RING - 1), slot = 0;
-        auto body = [&](int s, f32x16& x, f32x16& xn) {
+        auto body = [&](int s, typename W::Scores& x, typename W::Scores& xn) {
             __builtin_amdgcn_s_waitcnt(WAIT_FILLS);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
@@ -1551,14 +1606,16 @@ attn_fwd_sym_kernel(const AttnParams p) {
     __builtin_amdgcn_s_waitcnt(0x0F70);   // drain the (unused) trailing fills before the LDS is released or reused
 
     // ---- epilogue: O = acc / l ; LSE = (m + log2 l) ln 2 ----
-    float l_tot = w.l_run + __shfl_xor(w.l_run, 32);
+    // (by rows: of query lane % 32)
+    const int at = here(), j = at & 31, hh = at >> 5;
+    float l_tot = w.l_total(), m_all = w.m_total();
     if constexpr (KG > 1) {
         // merge the key groups: the wavefront of key group db % KG finishes 32-channel block db; the others hand it theirs
         __syncthreads();
-        float2* const stat = reinterpret_cast<float2*>(smem + C::STAT_OFF) + lane;
+        float2* const stat = reinterpret_cast<float2*>(smem + C::STAT_OFF) + at;
         auto block_at = [&](int src, int db) {   // slot of key group src's block db
             const int i = (src - db % KG + KG) % KG - 1;
-            return reinterpret_cast<float4*>(smem + ((i * RG + rg) * NDB + db) * C::BLK_BYTES) + lane;
+            return reinterpret_cast<float4*>(smem + ((i * RG + rg) * NDB + db) * C::BLK_BYTES) + at;
         };
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
@@ -1567,9 +1624,9 @@ attn_fwd_sym_kernel(const AttnParams p) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) dst[64 * g] = make_float4(w.acc[db][4 * g], w.acc[db][4 * g + 1], w.acc[db][4 * g + 2], w.acc[db][4 * g + 3]);
         }
-        stat[64 * wave] = make_float2(w.m_run, l_tot);
+        stat[64 * wave] = make_float2(m_all, l_tot);
         __syncthreads();
-        float wgt[KG], m_all = w.m_run;
+        float wgt[KG];
         float2 st[KG];
 #pragma unroll
         for (int k = 0; k < KG; ++k) { st[k] = stat[64 * (k * RG + rg)]; m_all = fmaxf(m_all, st[k].x); }
@@ -1577,7 +1634,6 @@ attn_fwd_sym_kernel(const AttnParams p) {
 #pragma unroll
         for (int k = 0; k < KG; ++k) { wgt[k] = __builtin_amdgcn_exp2f(st[k].x - m_all); l_tot += st[k].y * wgt[k]; }
         const float own = __builtin_amdgcn_exp2f(w.m_run - m_all);
-        w.m_run = m_all;
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
             if (db % KG != kg) continue;
@@ -1599,40 +1655,40 @@ attn_fwd_sym_kernel(const AttnParams p) {
         // a key range only: leave acc, m, l as they are for attn_combine_kernel (rows past Lq are written too and
         // never combined)
         const int64_t slot = (int64_t)(pair - p.n_full) * p.splits + split;
-        const int wrow = rg * 32 + j;
-        float* pa = p.part_acc + (slot * BLOCK_M + wrow) * DV;
+        if (kg == 0 && hh == 0) p.part_stat[slot * BLOCK_M + rg * 32 + j] = make_float4(m_all, l_tot, 0.f, 0.f);
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-            if (KG > 1 && db % KG != kg) continue;
+        for (int n = 0; n < N; ++n) {
+            float* pa = p.part_acc + (slot * BLOCK_M + rg * 32 + QR * n + at % QR) * DV;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * db + 8 * g + 4 * hh;
-                if (d < DV)
-                    *reinterpret_cast<float4*>(pa + d) = make_float4(w.acc[db][4 * g], w.acc[db][4 * g + 1], w.acc[db][4 * g + 2], w.acc[db][4 * g + 3]);
+            for (int g = 0; g < 4 * NDB / N; ++g) {
+                if (KG > 1 && (g >> 2) % KG != kg) continue;
+                const int d = 8 * N * g + 4 * (at / QR);
+                if (d < DV) *reinterpret_cast<f32x4*>(pa + d) = w.acc4(g, n);
             }
         }
-        if (kg == 0 && hh == 0) p.part_stat[slot * BLOCK_M + wrow] = make_float4(w.m_run, l_tot, 0.f, 0.f);
         return;
     }
-    const float inv_l = 1.0f / l_tot;
-    if (row < p.Lq) {
+    float inv_l[N];
+    W::of_rows(1.0f / l_tot, inv_l);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const int row = row0 + QR * n + at % QR;
+        if (row >= p.Lq) continue;
         T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl;
 #pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-            if (KG > 1 && db % KG != kg) continue;
+        for (int g = 0; g < 4 * NDB / N; ++g) {
+            if (KG > 1 && (g >> 2) % KG != kg) continue;
+            const int d = 8 * N * g + 4 * (at / QR);          // four consecutive channels
+            if (d < DV) {
+                const f32x4 a = w.acc4(g, n);
+                V4 ov;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * db + 8 * g + 4 * hh;   // registers 4g..4g+3 are 4 consecutive d
-                if (d < DV) {
-                    V4 ov;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) ov[r] = (T)(w.acc[db][4 * g + r] * inv_l);
-                    *reinterpret_cast<V4*>(op + d) = ov;
-                }
+                for (int r = 0; r < 4; ++r) ov[r] = (T)(a[r] * inv_l[n]);
+                *reinterpret_cast<V4*>(op + d) = ov;
             }
         }
-        if (p.lse && kg == 0 && hh == 0) p.lse[(int64_t)bh * p.Lq + row] = (w.m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
     }
+    if (row0 + j < p.Lq && p.lse && kg == 0 && hh == 0) p.lse[(int64_t)bh * p.Lq + row0 + j] = (m_all + __builtin_log2f(l_tot)) * 0.6931471805599453f;
 }
 
 // Merge the key-range partial results of one query row:  M = max m_i,  w_i = 2^(m_i - M),  L = sum l_i w_i,

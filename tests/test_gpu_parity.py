@@ -412,6 +412,21 @@ def test_streaming_kernels_random_shapes(pkg, oracle, gpu, stream_override, chun
                  seed=9000 + 100 * chunk + it)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("edge", [15, 16, 17, 24, 31])
+def test_halves_of_sixteen_queries_and_eight_keys(pkg, oracle, gpu, stream_override, forward_override, edge, dtype):
+    """The kernels that work in 16 x 16 products (forward only with 384 rows a workgroup, streams with all tangents; head dim 128): queries that end inside a half of 16 and
+    keys inside a run of eight, in the last and in the only tile, with and without a causal diagonal through them."""
+    stream_override(chunk=1)
+    forward_override(384)
+    for Lq, Lkv in [(edge, edge + 1), (384 + edge, 32 + edge - 7)]:
+        run_case(pkg, oracle, gpu, (1, 2, Lq, 128), (1, 2, Lkv, 128), seed=edge, dtype=dtype, tangents="none")
+    run_case(pkg, oracle, gpu, (1, 2, 64 + edge, 128), causal=True, seed=edge, dtype=dtype, tangents="none")
+    stream_override(chunk=2)
+    run_case(pkg, oracle, gpu, (1, 2, 256 + edge, 128), (1, 2, 32 + edge - 7, 128), seed=edge, dtype=dtype, tangents="full")
+    run_case(pkg, oracle, gpu, (2, 2, 256 + edge, 128), (2, 2, 100, 128), key_lens=[edge, 64 + edge], seed=edge, dtype=dtype, tangents="full")
+
+
 @pytest.mark.parametrize("tangents,Lq,Lkv", [("q", 2120, 1024), ("none", 6500, 1024)])
 def test_packed_run_is_compared_with_the_uncut_kernel(pkg, oracle, gpu, stream_override, tangents, Lq, Lkv):
     """The two-stage run never cuts key ranges: it streams where streaming beats the uncut kernel (by 16 % at both sizes), also where
