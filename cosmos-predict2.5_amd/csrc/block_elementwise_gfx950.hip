@@ -522,7 +522,9 @@ __global__ void __launch_bounds__(kThreads) gated_residual_bwd_kernel(const Gate
 // them is reading the weights once (12 MB at 2B: 2 us) and the launches: one launch per layer for all three MLPs, instead of five
 // to eight library launches for each.  A wavefront forms a 16 x 16 tile (outputs x rows) on v_mfma_f32_16x16x32, its operands read
 // straight from memory, 16 bytes a lane (both operands with the same k order, so that order is free).  The first layer has few
-// outputs and a long k: eight wavefronts share a tile's k and add their parts in LDS, else 48 wavefronts would read all weights.
+// outputs and a long k: sixteen wavefronts share a tile's k and add their parts in LDS, else 48 wavefronts would read all weights.  All loads of a
+// wavefront are in flight before the first product, with no branch that differs between lanes among them: with eight wavefronts and one load after the other (a branch
+// around a missing row's) the layers took 14.4 and 6.8 us inside a network on one image, now 8.5 and 6.0, of which silu, formed by each workgroup for itself, is some 3.
 // Measured per block (2048 channels, in a replayed graph): one row 46 -> 16 us, 24 rows 72 -> 15, 5 rows with tangents 219 -> 14;
 // outside a graph the launches count too: a 28-block network on one image 24.0 -> 20.4 ms.
 struct ModulationParams {
@@ -550,35 +552,51 @@ template <> struct Half8<false> {
     }
 };
 
-constexpr int kModSplit = 8;       // wavefronts that share a first-layer tile
+constexpr int kModSplit = 16;      // wavefronts that share a first-layer tile
+constexpr int kModLoads = 4;       // k steps of a wavefront whose loads are in flight together, first layer (twice as many: second)
 // grid (3 hidden / 16, ceil(rows_all / 16)), 64 kModSplit threads
 template <bool BF16>
 __global__ void __launch_bounds__(64 * kModSplit) modulation_hidden_kernel(const ModulationParams p) {
     typedef typename Half8<BF16>::v4f v4f;
     __shared__ float4 part[kModSplit][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tiles = p.hidden / 16, mod = blockIdx.x / tiles, n0 = (blockIdx.x % tiles) * 16;
     const int row = blockIdx.y * 16 + (lane & 15);
-    const bool live = row < p.rows_all, tangent = row >= p.rows;
+    const bool live = row < p.rows_all, tangent = row >= p.rows, moves = p.rows_all > p.rows && p.temb;
     const uint16_t* w = (mod == 0 ? p.w1[0] : mod == 1 ? p.w1[1] : p.w1[2]) + (int64_t)(n0 + (lane & 15)) * p.K;
-    const uint16_t* e = p.emb + (int64_t)(tangent ? row - p.rows : row) * p.K;
-    const uint16_t* te = tangent && p.temb ? p.temb + (int64_t)(row - p.rows) * p.K : nullptr;
+    // (a row that is not there reads row 0 and forms a column that nobody reads)
+    const int64_t at = live ? (int64_t)(tangent ? row - p.rows : row) * p.K : 0;
+    const uint16_t *e = p.emb + at, *te = moves ? p.temb + at : nullptr;
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 32 * wave + 8 * (lane >> 4); k < p.K; k += 32 * kModSplit) {
-        const uint4 a = *reinterpret_cast<const uint4*>(w + k);
-        uint4 b = make_uint4(0u, 0u, 0u, 0u);
-        if (live && (!tangent || te)) {
-            float f[8], t[8];
-            unpack8<BF16>(*reinterpret_cast<const uint4*>(e + k), f);
-            if (tangent) unpack8<BF16>(*reinterpret_cast<const uint4*>(te + k), t);
+    for (int k0 = 32 * wave; k0 < p.K; k0 += 32 * kModSplit * kModLoads) {
+        uint4 a[kModLoads], x[kModLoads], tx[kModLoads];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float sig = 1.0f / (1.0f + __expf(-f[i]));
-                f[i] = tangent ? t[i] * (sig * (1.0f + f[i] * (1.0f - sig))) : f[i] * sig;
+        for (int i = 0; i < kModLoads; ++i) {
+            a[i] = x[i] = tx[i] = make_uint4(0u, 0u, 0u, 0u);
+            if (k0 + 32 * kModSplit * i < p.K) {       // (K is a multiple of 32: the same in all lanes)
+                const int k = k0 + 32 * kModSplit * i + 8 * (lane >> 4);
+                a[i] = *reinterpret_cast<const uint4*>(w + k);
+                x[i] = *reinterpret_cast<const uint4*>(e + k);
+                if (moves) tx[i] = *reinterpret_cast<const uint4*>(te + k);
             }
-            b = pack8<BF16>(f);
         }
-        acc = Half8<BF16>::mfma(a, b, acc);
+#pragma unroll
+        for (int i = 0; i < kModLoads; ++i) {
+            float f[8], sig[8];
+            unpack8<BF16>(x[i], f);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sig[j] = 1.0f / (1.0f + __expf(-f[j]));
+            if (p.rows_all > p.rows) {
+                float t[8];
+                unpack8<BF16>(tx[i], t);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) f[j] = tangent ? t[j] * (sig[j] * (1.0f + f[j] * (1.0f - sig[j]))) : f[j] * sig[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) f[j] *= sig[j];
+            }
+            acc = Half8<BF16>::mfma(a[i], pack8<BF16>(f), acc);
+        }
     }
     part[wave][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
     __syncthreads();
@@ -601,13 +619,21 @@ __global__ void __launch_bounds__(kThreads) modulation_out_kernel(const Modulati
     const int n0 = (tile % tiles) * 16, row = blockIdx.y * 16 + (lane & 15);
     const bool live = row < p.rows_all, tangent = row >= p.rows;
     const uint16_t* w = (mod == 0 ? p.w2[0] : mod == 1 ? p.w2[1] : p.w2[2]) + (int64_t)(n0 + (lane & 15)) * p.hidden;
-    const uint16_t* h = p.h + ((int64_t)mod * p.rows_all + row) * p.hidden;
+    const uint16_t* h = p.h + ((int64_t)mod * p.rows_all + (live ? row : 0)) * p.hidden;
     v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int k = 8 * (lane >> 4); k < p.hidden; k += 32) {
-        const uint4 a = *reinterpret_cast<const uint4*>(w + k);
-        const uint4 b = live ? *reinterpret_cast<const uint4*>(h + k) : make_uint4(0u, 0u, 0u, 0u);
-        acc = Half8<BF16>::mfma(a, b, acc);
+    for (int k0 = 0; k0 < p.hidden; k0 += 64 * kModLoads) {
+        uint4 a[2 * kModLoads], b[2 * kModLoads];
+#pragma unroll
+        for (int i = 0; i < 2 * kModLoads; ++i) {
+            a[i] = b[i] = make_uint4(0u, 0u, 0u, 0u);
+            if (k0 + 32 * i < p.hidden) {
+                const int k = k0 + 32 * i + 8 * (lane >> 4);
+                a[i] = *reinterpret_cast<const uint4*>(w + k);
+                b[i] = *reinterpret_cast<const uint4*>(h + k);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * kModLoads; ++i) acc = Half8<BF16>::mfma(a[i], b[i], acc);
     }
     if (!live) return;
     const int n = n0 + 4 * (lane >> 4), r = tangent ? row - p.rows : row;      // D is a multiple of 16: a tile is in one vector
