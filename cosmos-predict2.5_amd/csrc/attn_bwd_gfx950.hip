@@ -117,8 +117,9 @@ __global__ void __launch_bounds__(kPackThreads) bwd_stats_kernel(const StatsPara
 // ---------------------------------------------------------------------------------------------- stream re-tiling
 // Order of the 16-byte units (row r, chunk C of 8 channels) of a stream part of attn_dkdv_quad_kernel in LDS: read with ds_read_b128
 // (lane = row) and with transposing reads (ds_read_b64_tr_b16) without bank conflicts, and filled four whole rows a load (attn_bwd_quad_gfx950.h).
+__host__ __device__ constexpr int quad_swizzle(int r4) { return (r4 & 1) * 2 + (r4 >> 1 & 1); }
 __host__ __device__ constexpr int quad_unit_slot(int r, int C) {
-    return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ ((r >> 2) & 3));
+    return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ quad_swizzle(r >> 2));
 }
 
 struct PackSrc { const uint16_t* ptr; int64_t sb, sh, sl; };
@@ -181,7 +182,7 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
     }
 }
 
-// What attn_dkdv_quad_kernel streams beside Q and dO (head dim 128): per tile of 32 queries 32 values LSE log2 e, then 32 row sums dout . o.  With COPY also
+// What attn_dkdv_quad_kernel streams beside Q and dO (head dim 128): per tile of 32 queries 32 values LSE log2 e, then 32 negated row sums dout . o.  With COPY also
 // rows of q and dout, one behind the other, for a call whose own rows the kernel does not read.  HBM-bound; eight threads per row, two 16-byte units of each tensor
 // per thread, rows read whole.  grid (n_tiles, B*H).
 constexpr int kQuadStatBytes = 2 * kRows * (int)sizeof(float);
@@ -228,11 +229,10 @@ __global__ void __launch_bounds__(kPackThreads) quad_stats_kernel(const QuadStat
     acc += __shfl_xor(acc, 1); acc += __shfl_xor(acc, 2); acc += __shfl_xor(acc, 4);
     if (part == 0) {
         if (live && p.stats) p.stats[(int64_t)bh * p.L + row] = make_float2(lse, acc);
-        // 32 LSE values, then 32 D values, each half wavefront's 16 streamed rows together
+        // 32 LSE values, then 32 D values, negated: they start the sums of dP
         float* st = reinterpret_cast<float*>(p.tile_stats + ((size_t)bh * p.n_tiles + t) * kQuadStatBytes);
-        const int idx = 16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3);
-        st[idx] = lse;
-        st[32 + idx] = acc;
+        st[r] = lse;
+        st[32 + r] = -acc;
     }
 }
 
@@ -801,6 +801,7 @@ __global__ void __launch_bounds__(256) bwd_combine_kernel(const BwdParams p, int
 // One workgroup fills a compute unit (144 KB of ring), so where the queries give more blocks than units each workgroup walks several, the next block's
 // first loads in flight while the last steps and the stores of the one before run: at 512 keys (16 steps a block) of 16 heads x 37440 queries 192 -> 171 us
 // (4.5 TB/s), at 37440 keys the same time.  Causal blocks have unequal lengths, which a fixed share would not balance: one workgroup each.
+// (v_mfma_f32_16x16x32 here: odd lane groups have to exchange what they read; 37440 x 512 2 % less of a backward, 24640 x 24640 0.6 % more, so not here.)
 constexpr int kDsLoadPolicy = 2;     // cache policy bits of the dS loads: non-temporal (each tile is read once; 4 % faster than plain loads)
 constexpr int kDsRing = 6;            // steps of dS / K^T in flight per workgroup
 constexpr int kDqWaves = 8;           // query tiles per workgroup
@@ -886,12 +887,12 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
     }
     // transposing read: byte offset, inside a dS tile, of the 8 bytes this lane passes for key chunk 0, read 0
     //   group g = lane / 16: queries 16 (g % 2) .. + 15, key half g / 2;  lane i of the group passes row r = i:
-    //   queries 16 (g%2) + 4 (r%4) .. + 3 of key 4 (g/2) + r/4  (+ 16 c + 8 t).  In the tile the 16-byte unit (query half c' = g%2,
-    //   key, lane half hh' = r%2 of the wavefront that formed it) sits at slot 16 (key / 4) + 8 c' + 4 hh' + key % 4, and the lane
-    //   wants its second 8 bytes when (r%4)/2: the 32 lanes of a pass touch 256 consecutive bytes, every bank once.
+    //   queries 16 (g%2) + 4 (r%4) .. + 3 of key 4 (g/2) + r/4  (+ 16 c + 8 t).  In the tile the 16-byte unit (key, lane group g' of
+    //   the wavefront that formed it: queries 4 g' .. + 3 and 16 + 4 g' .. + 3) sits at slot 16 (key / 4) + 4 g' + key % 4, and the lane
+    //   wants its second 8 bytes when g%2: the 32 lanes of a pass touch 256 consecutive bytes, every bank once.
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;   // LDS address of smem[0]
     const int g16 = lane >> 4, r16 = lane & 15;
-    const unsigned tr_off = (unsigned)(256 * (g16 >> 1) + 128 * (g16 & 1) + 64 * (r16 & 1) + 16 * (r16 >> 2) + 8 * ((r16 & 3) >> 1));
+    const unsigned tr_off = (unsigned)(256 * (g16 >> 1) + 64 * (r16 & 3) + 16 * (r16 >> 2) + 8 * (g16 & 1));
 
     int r_slot = 0;
     auto step = [&](int s, int qt, bool live_tile) {

@@ -17,9 +17,6 @@
 // eight keys 0, 2, 1, 3; as the image has them the two runs of a half would lie in the same banks).
 // Statistics of a row exist as the pair a lane uses (queries i, 16 + i) and, for what is done once per row, "by rows": of query lane % 32.
 
-__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
 __device__ __forceinline__ int lane_key(int lane) { return 16 * (lane >> 5) + 4 * ((lane >> 4) & 1); }      // = tile_key(4 (lane / 16)): 16 (i / 8) + 4 ((i / 4) % 2) + i % 4
 __device__ __forceinline__ int k_fill_lane(int lane) { return (lane & ~24) | ((lane & 8) << 1) | ((lane & 16) >> 1); }
 // where this lane reads V^T fragment n (channels 16 n .. + 15, the tile's 32 keys), from the V^T section's start: 2048 (n / 2) + 256 (n % 2) behind this;

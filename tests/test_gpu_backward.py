@@ -132,6 +132,14 @@ def test_bwd_several_query_blocks_per_workgroup(pkg, oracle, gpu, Lkv):
     run_bwd(pkg, oracle, gpu, (5, 13, 1070, 128), (5, 13, Lkv, 128), seed=Lkv)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Lq, Lkv, causal", [(15, 17, False), (16, 16, True), (17, 113, False), (48, 81, False), (113, 113, True), (145, 63, False)])
+def test_bwd_at_the_edges_of_16(pkg, oracle, gpu, Lq, Lkv, causal, dtype):
+    """The dK/dV kernel's results come in 16 queries x 16 keys: both on either side of a multiple, a query half and a key group without a row, the diagonal in each
+    (same tolerances)."""
+    run_bwd(pkg, oracle, gpu, (2, 3, Lq, 128), (2, 3, Lkv, 128), causal=causal, seed=Lq, dtype=dtype)
+
+
 @pytest.mark.parametrize("Lq", [1, 32, 45, 300])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("which", ["q", "dout", "far"])
