@@ -16,6 +16,12 @@ from torch.autograd import forward_ad
 from . import ops
 
 
+# Fewer rows than these are the library's in every layer (cosmos_attn_gemm_preferred): the layer's own product, and the first of its backward pass.  Asked first, as the
+# checks and the descriptor cost a layer some 10 us on the host, which a call of few rows waits for.
+FEWEST_ROWS = 1024
+FEWEST_ROWS_BACKWARD = 256
+
+
 def bare(m: nn.Module) -> bool:
     """Is calling m the same as computing its forward?"""
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__
@@ -79,13 +85,16 @@ class _LinearFn(torch.autograd.Function):
 
 def linear(layers: Sequence[nn.Module], x: torch.Tensor) -> list:
     """``[m(x) for m in layers]``: up to three layers without bias."""
+    rows = x.shape[:-1].numel()
+    recording = torch.is_grad_enabled()
+    if rows < (FEWEST_ROWS_BACKWARD if recording else FEWEST_ROWS):
+        return [m(x) for m in layers]
     ws = _weights(layers, x)
     if ws is None:
         return [m(x) for m in layers]
-    rows = x.numel() // x.shape[-1]
-    with torch.no_grad():
-        made = ops.gemm("xwt", [x.view(rows, -1)] * len(ws), ws, if_preferred=True, lead=x.shape[:-1])
-    if torch.is_grad_enabled() and (x.requires_grad or any(w.requires_grad for w in ws)):
-        # (the products of the backward pass are chosen there; below 256 rows they are the library's like these)
-        return list(_LinearFn.apply(made, x, *ws)) if made is not None or rows >= 256 else [m(x) for m in layers]
+    made = None
+    if rows >= FEWEST_ROWS:
+        made = ops.gemm("xwt", [x.detach().view(rows, -1)] * len(ws), ws, if_preferred=True, lead=x.shape[:-1])
+    if recording and (x.requires_grad or any(w.requires_grad for w in ws)):
+        return list(_LinearFn.apply(made, x, *ws))
     return made if made is not None else [m(x) for m in layers]

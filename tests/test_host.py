@@ -705,3 +705,22 @@ def test_dense16_copies_what_starts_off_16_bytes(pkg, first):
     assert got.is_contiguous() and got.data_ptr() % 16 == 0 and torch.equal(got, t)
     assert (got is t) == (first % 8 == 0)
     assert torch.equal(pkg.ops._dense16(t.t()), t.t()) and pkg.ops._dense16(t.t()).is_contiguous()
+
+
+@pytest.mark.parametrize("cols, depth", [(64, 64), (2048, 2048), (8192, 2048), (2048, 8192), (20480, 5120)])
+@pytest.mark.parametrize("count", [1, 2, 3])
+def test_rows_below_which_no_layer_asks_are_below_the_rule(pkg, cols, depth, count):
+    """linear.linear does not ask cosmos_attn_gemm_preferred below these rows; its answer there is no."""
+    from sys import modules
+    L, lin = pkg._lib, modules[pkg.__name__ + ".linear"]
+    D = L.GemmDesc()
+    D.abi_version, D.dtype, D.count = L.ABI_VERSION, L.DTYPE_BF16, count
+    for i in range(3):
+        D.a[i] = D.b[i] = D.c[i] = 16
+    for order, rows, c, d in ((L.GEMM_XWT, lin.FEWEST_ROWS - 1, cols, depth), (L.GEMM_XW, lin.FEWEST_ROWS_BACKWARD - 1, depth, cols),
+                              (L.GEMM_XTX, cols, depth, lin.FEWEST_ROWS_BACKWARD - 1)):
+        D.order, D.flags, D.rows, D.cols, D.depth = order, (L.GEMM_SUM if order == L.GEMM_XW else 0), rows, c, d
+        D.lda, D.ldb, D.ldc = max(rows + -rows % 8 if order == L.GEMM_XTX else d, 256), max(d if order == L.GEMM_XWT else c, 256), c
+        assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == 0
+    D.order, D.flags, D.rows, D.cols, D.depth, D.lda, D.ldb, D.ldc = L.GEMM_XWT, 0, lin.FEWEST_ROWS, 2048, 2048, 2048, 2048, 2048
+    assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == 1
