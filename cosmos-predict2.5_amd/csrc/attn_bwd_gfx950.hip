@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(kPackThreads) bwd_stats_kernel(const StatsPara
 // ---------------------------------------------------------------------------------------------- stream re-tiling
 // Order of the 16-byte units (row r, chunk C of 8 channels) of a stream part of attn_dkdv_quad_kernel in LDS: read with ds_read_b128
 // (lane = row) and with transposing reads (ds_read_b64_tr_b16) without bank conflicts, and filled four whole rows a load (attn_bwd_quad_gfx950.h).
-__host__ __device__ constexpr int quad_swizzle(int r4) { return (r4 & 1) * 2 + (r4 >> 1 & 1); }
+__host__ __device__ constexpr int quad_swizzle(int r4) { return ((r4 ^ r4 >> 1) & 1) * 2 + (r4 >> 1 & 1); }
 __host__ __device__ constexpr int quad_unit_slot(int r, int C) {
     return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ quad_swizzle(r >> 2));
 }

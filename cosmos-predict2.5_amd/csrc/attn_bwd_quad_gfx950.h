@@ -32,8 +32,9 @@
 // lane) and get them from the SAME units with the transposing read ds_read_b64_tr_b16 (within 16 lanes, lane i passes the address
 // of 8 bytes -- row i of a 16 x 4 matrix M of 16-bit values -- and receives M[i/4 + 4k][i%4], k = 0..3): no second, transposed copy
 // of the tile in memory, in the fills or in LDS.  The unit (r, C) lies at
-//     slot(r, C) = 64 (r/4) + 16 (C/4) + 4 (r%4) + (C%4 XOR quad_swizzle(r/4)), the swizzle 0, 2, 1, 3 for r/4 = 0 .. 3:
-// the 16 lanes of a ds_read_b128 pass (16 consecutive rows, one C) and the 32 lanes of a transposing pass (two runs of 4 rows x 2 chunks, both
+//     slot(r, C) = 64 (r/4) + 16 (C/4) + 4 (r%4) + (C%4 XOR quad_swizzle(r/4)), the swizzle 0, 2, 3, 1 for r/4 = 0 .. 3:
+// the lanes that a ds_read_b128 serves together (0 .. 3, 12 .. 15 and 20 .. 27, or the rest of 32: rows of two chunks; with the swizzle 0, 2, 1, 3, right for 16 consecutive lanes,
+// SQ_LDS_BANK_CONFLICT was 7 % of the cycles, the time the same within 0.3 %, now it is 0) and the 32 lanes of a transposing pass (two runs of 4 rows x 2 chunks, both
 // 8-byte halves of each unit) touch 256 consecutive-bank bytes each, and a direct-to-LDS load of 64 units is four whole rows, so
 // that the fills read Q and dO rows where they are (or in the copy that is made of rows which they cannot address).
 // LDS: rings of the two stream parts (Q 7 deep: fetched three steps before S1 uses it, kept until O2 has used it three steps
