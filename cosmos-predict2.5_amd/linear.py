@@ -28,20 +28,27 @@ def bare(m: nn.Module) -> bool:
                 or nn.modules.module._has_any_global_hook())
 
 
+def _memory_says_all(*tensors: torch.Tensor) -> bool:
+    """Is nothing lost by reading the tensors' memory: no tangent (dual levels), no level of a function transform or of batched gradients (their tensors have
+    no storage of their own, ``is_grads_batched``'s older ones with no other mark), no subclass?"""
+    return forward_ad._current_level < 0 and all(
+        type(t) in (torch.Tensor, nn.Parameter) and torch._C._has_storage(t) and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+
+
 def _weights(layers: Sequence[nn.Module], x: torch.Tensor) -> Optional[list]:
     """The layers' weights, if their products with x may be formed by ``ops.gemm``."""
     if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or type(x) is not torch.Tensor or x.numel() == 0:
         return None
-    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0:
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing():
         return None
-    if torch._C._functorch.is_functorch_wrapped_tensor(x) or not ops._is_dense16(x):
+    if not _memory_says_all(x) or not ops._is_dense16(x):
         return None
     ws = []
     for m in layers:
         if type(m) is not nn.Linear or m.bias is not None or not bare(m):
             return None
         w = m.weight
-        if type(w) is not nn.Parameter or torch._C._functorch.is_functorch_wrapped_tensor(w) or w.dtype != x.dtype or w.device != x.device or w.shape != layers[0].weight.shape or not ops._is_dense16(w):
+        if type(w) is not nn.Parameter or not _memory_says_all(w) or w.dtype != x.dtype or w.device != x.device or w.shape != layers[0].weight.shape or not ops._is_dense16(w):
             return None
         ws.append(w)
     if ws[0].shape[1] != x.shape[-1]:
@@ -65,7 +72,8 @@ class _LinearFn(torch.autograd.Function):
         x2 = x.reshape(-1, x.shape[-1])
         g2 = {i: dy[i].reshape(-1, dy[i].shape[-1]) for i in given}
         dx, dw = None, [None] * len(w)
-        own = not torch.is_grad_enabled()        # (create_graph: the gradients are differentiated again)
+        # (create_graph: the gradients are differentiated again)
+        own = not torch.is_grad_enabled() and _memory_says_all(x, *w, *(dy[i] for i in given))
         if own:
             g2 = {i: ops._dense16(g) for i, g in g2.items()}
         if ctx.needs_input_grad[1] and given:

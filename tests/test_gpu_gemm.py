@@ -114,6 +114,25 @@ def test_layer_gradients_of_a_part_and_twice(pkg):
     assert _rel(ddx, 2 * x.detach().double() @ h @ h) < 4 * 2e-3
 
 
+def test_layer_gradients_of_dual_cotangents(pkg):
+    """A graph recorded outside of any dual level, its gradients then dual: their tangents come through where the own products are preferred.  (Batched
+    cotangents: on the CPU, test_host.py.)"""
+    from sys import modules
+    from torch.autograd import forward_ad as fwad
+    linear = modules[pkg.__name__ + ".linear"].linear
+    layers = _layers(3, 512, 512, torch.bfloat16)
+    rn = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    x, dy, tdy = rn(1560, 512).requires_grad_(True), [rn(1560, 512) for _ in layers], [rn(1560, 512) for _ in layers]
+    ys, wrt = linear(layers, x), [x] + [m.weight for m in layers]
+    assert pkg.ops.gemm("xw", dy, [m.weight.detach() for m in layers], total=True, if_preferred=True) is not None
+    plain = [torch.autograd.grad(ys, wrt, d, retain_graph=True) for d in (dy, tdy)]
+    with fwad.dual_level():
+        got = [fwad.unpack_dual(t) for t in torch.autograd.grad(ys, wrt, [fwad.make_dual(d, t) for d, t in zip(dy, tdy)])]
+    for i, pair in enumerate(got):        # (the gradients are linear in the cotangent)
+        for part, want in zip(pair, (plain[0][i], plain[1][i])):
+            assert part is not None and _rel(part, want.double()) < 4 * 2e-3       # (up to three roundings on one side, one on the other)
+
+
 @pytest.mark.parametrize("how", ["hook", "subclass", "bias", "autocast", "float", "strided", "jvp", "vmap"])
 def test_layers_with_a_meaning_of_their_own_go_through_the_module(pkg, how):
     from sys import modules

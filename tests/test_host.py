@@ -724,3 +724,47 @@ def test_rows_below_which_no_layer_asks_are_below_the_rule(pkg, cols, depth, cou
         assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == 0
     D.order, D.flags, D.rows, D.cols, D.depth, D.lda, D.ldb, D.ldc = L.GEMM_XWT, 0, lin.FEWEST_ROWS, 2048, 2048, 2048, 2048, 2048
     assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == 1
+
+
+def _by_address(t):
+    """What a launch would read of t: its memory, and nothing else that belongs to it."""
+    assert t.stride(1) == 1
+    n = (t.shape[0] - 1) * t.stride(0) + t.shape[1]
+    return torch.frombuffer(bytearray(ctypes.string_at(t.data_ptr(), n * t.element_size())), dtype=t.dtype).as_strided(t.shape, t.stride())
+
+
+@pytest.fixture
+def gemm_by_address(pkg, monkeypatch):
+    """ops.gemm on the CPU, on what it would find at its operands' addresses; always preferred."""
+    def gemm(order, a, b, total=False, shape=0, if_preferred=False, lead=None):
+        out = [(_by_address(x).t() if order == "xtx" else _by_address(x)) @ (_by_address(y).t() if order == "xwt" else _by_address(y)) for x, y in zip(a, b)]
+        return sum(out) if total else out
+    monkeypatch.setattr(pkg.ops, "gemm", gemm)
+
+
+def _layer_inputs(n=2, rows=6, depth=8, cols=16):
+    g = torch.Generator().manual_seed(5)
+    rn = lambda *s: torch.randn(*s, generator=g).bfloat16()
+    return rn(rows, depth).requires_grad_(True), [torch.nn.Parameter(rn(cols, depth)) for _ in range(n)], [rn(rows, cols) for _ in range(n)], [rn(rows, cols) for _ in range(n)]
+
+
+@pytest.mark.parametrize("cotangent", ["dual", "batched"])
+def test_layer_gradients_of_cotangents_that_are_more_than_memory(pkg, gemm_by_address, cotangent):
+    """A gradient that is a dual tensor keeps its tangent, one that is a batch is taken whole: as in nn.Linear's backward pass."""
+    from sys import modules
+    from torch.autograd import forward_ad as fwad
+    linear_fn = modules[pkg.__name__ + ".linear"]._LinearFn
+    x, w, dy, tdy = _layer_inputs()
+    ys, wants = linear_fn.apply(None, x, *w), [torch.nn.functional.linear(x, v) for v in w]
+    if cotangent == "dual":
+        with fwad.dual_level():
+            def grads(out):
+                g = torch.autograd.grad(out, [x, *w], [fwad.make_dual(d, t) for d, t in zip(dy, tdy)])
+                return [part for t in g for part in fwad.unpack_dual(t)]
+            got, want = grads(ys), grads(wants)
+    else:
+        batch = [torch.stack([d, t]) for d, t in zip(dy, tdy)]
+        got, want = (torch.autograd.grad(out, [x, *w], batch, is_grads_batched=True) for out in (ys, wants))
+    for a, b in zip(got, want):
+        assert a is not None and a.shape == b.shape
+        assert (a.double() - b.double()).norm() <= 3 * 2e-3 * b.double().norm()      # (dx: the products' order and their roundings, three at most)
