@@ -2,7 +2,7 @@
 :349-358) on the package's own matrix products where those are faster, several layers of one input in a launch; ``nn.Linear`` itself elsewhere.
 
 The parameters stay where they are.  Whatever gives calling the module a meaning of its own (hooks, another class, a parametrization, autocast, function
-transforms, forward-mode AD, compilation, tensor subclasses) goes through the module.
+transforms, forward-mode AD, compilation, tensor subclasses, modes that watch operators) goes through the module.
 """
 from __future__ import annotations
 
@@ -12,6 +12,8 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import ops
 
@@ -35,11 +37,19 @@ def _memory_says_all(*tensors: torch.Tensor) -> bool:
         type(t) in (torch.Tensor, nn.Parameter) and torch._C._has_storage(t) and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
 
 
+def _watched() -> bool:
+    """Does a mode see the operators that are called (a FLOP counter, selective checkpointing, a user's own)?  Products launched by address pass it by.  (A default
+    device is a mode as well, of factory functions.)"""
+    if torch._C._len_torch_dispatch_stack():
+        return True
+    return bool(torch._C._len_torch_function_stack()) and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())
+
+
 def _weights(layers: Sequence[nn.Module], x: torch.Tensor) -> Optional[list]:
     """The layers' weights, if their products with x may be formed by ``ops.gemm``."""
     if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or type(x) is not torch.Tensor or x.numel() == 0:
         return None
-    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing():
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing() or _watched():
         return None
     if not _memory_says_all(x) or not ops._is_dense16(x):
         return None
@@ -73,7 +83,7 @@ class _LinearFn(torch.autograd.Function):
         g2 = {i: dy[i].reshape(-1, dy[i].shape[-1]) for i in given}
         dx, dw = None, [None] * len(w)
         # (create_graph: the gradients are differentiated again)
-        own = not torch.is_grad_enabled() and _memory_says_all(x, *w, *(dy[i] for i in given))
+        own = not torch.is_grad_enabled() and not _watched() and _memory_says_all(x, *w, *(dy[i] for i in given))
         if own:
             g2 = {i: ops._dense16(g) for i, g in g2.items()}
         if ctx.needs_input_grad[1] and given:

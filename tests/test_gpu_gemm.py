@@ -133,7 +133,7 @@ def test_layer_gradients_of_dual_cotangents(pkg):
             assert part is not None and _rel(part, want.double()) < 4 * 2e-3       # (up to three roundings on one side, one on the other)
 
 
-@pytest.mark.parametrize("how", ["hook", "subclass", "bias", "autocast", "float", "strided", "jvp", "vmap"])
+@pytest.mark.parametrize("how", ["hook", "subclass", "bias", "autocast", "float", "strided", "jvp", "vmap", "flops", "function mode"])
 def test_layers_with_a_meaning_of_their_own_go_through_the_module(pkg, how):
     from sys import modules
     lin = modules[pkg.__name__ + ".linear"]
@@ -159,6 +159,18 @@ def test_layers_with_a_meaning_of_their_own_go_through_the_module(pkg, how):
         elif how == "vmap":
             t = x.view(2, 1024, 512)
             got, want = (torch.func.vmap(lambda t: lin.linear([m], t)[0])(t),), (torch.func.vmap(m)(t),)
+        elif how == "flops":
+            from torch.utils.flop_counter import FlopCounterMode
+            with FlopCounterMode(display=False) as counter:
+                got, want = (lin.linear([m], x)[0],), (m(x),)
+            assert counter.get_total_flops() == 2 * 2 * 2048 * 512 * 512
+        elif how == "function mode":
+            class Doubled(torch.overrides.TorchFunctionMode):
+                def __torch_function__(self, fn, types, args=(), kwargs=None):
+                    y = fn(*args, **(kwargs or {}))
+                    return 2 * y if fn is torch.nn.functional.linear else y
+            with Doubled():
+                got, want = (lin.linear([m], x)[0],), (m(x),)
         else:
             with torch.autocast("cuda", dtype=torch.float16, enabled=how == "autocast"):
                 got, want = (lin.linear([m], x)[0],), (m(x),)

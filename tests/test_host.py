@@ -736,9 +736,12 @@ def _by_address(t):
 @pytest.fixture
 def gemm_by_address(pkg, monkeypatch):
     """ops.gemm on the CPU, on what it would find at its operands' addresses; always preferred."""
+    from torch.utils._python_dispatch import _disable_current_modes
+
     def gemm(order, a, b, total=False, shape=0, if_preferred=False, lead=None):
-        out = [(_by_address(x).t() if order == "xtx" else _by_address(x)) @ (_by_address(y).t() if order == "xwt" else _by_address(y)) for x, y in zip(a, b)]
-        return sum(out) if total else out
+        with _disable_current_modes():         # (no mode sees a launch)
+            out = [(_by_address(x).t() if order == "xtx" else _by_address(x)) @ (_by_address(y).t() if order == "xwt" else _by_address(y)) for x, y in zip(a, b)]
+            return sum(out) if total else out
     monkeypatch.setattr(pkg.ops, "gemm", gemm)
 
 
@@ -768,3 +771,14 @@ def test_layer_gradients_of_cotangents_that_are_more_than_memory(pkg, gemm_by_ad
     for a, b in zip(got, want):
         assert a is not None and a.shape == b.shape
         assert (a.double() - b.double()).norm() <= 3 * 2e-3 * b.double().norm()      # (dx: the products' order and their roundings, three at most)
+
+
+def test_layer_gradients_are_seen_by_a_mode_that_watches_operators(pkg, gemm_by_address):
+    from sys import modules
+    from torch.utils.flop_counter import FlopCounterMode
+    linear_fn = modules[pkg.__name__ + ".linear"]._LinearFn
+    x, w, dy, _ = _layer_inputs()
+    ys = linear_fn.apply(None, x, *w)
+    with FlopCounterMode(display=False) as counter:
+        torch.autograd.grad(ys, [x, *w], dy)
+    assert counter.get_total_flops() == 2 * 2 * 2 * 6 * 8 * 16        # per layer dx and dw
