@@ -71,7 +71,9 @@ class _LinearFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, made, x, *w):
-        ctx.save_for_backward(x, *w)
+        # as nn.Linear: x for the weights' gradients, the weights for x's; what no gradient asks for may be freed or written over
+        ctx.save_for_backward(x if any(ctx.needs_input_grad[2:]) else None, *(w if ctx.needs_input_grad[1] else ()))
+        ctx.x_shape = x.shape
         ctx.set_materialize_grads(False)
         return tuple(made if made is not None else [F.linear(x, v) for v in w])
 
@@ -79,11 +81,10 @@ class _LinearFn(torch.autograd.Function):
     def backward(ctx, *dy):
         x, *w = ctx.saved_tensors
         given = [i for i, g in enumerate(dy) if g is not None]
-        x2 = x.reshape(-1, x.shape[-1])
         g2 = {i: dy[i].reshape(-1, dy[i].shape[-1]) for i in given}
-        dx, dw = None, [None] * len(w)
+        dx, dw = None, [None] * len(dy)
         # (create_graph: the gradients are differentiated again)
-        own = not torch.is_grad_enabled() and not _watched() and _memory_says_all(x, *w, *(dy[i] for i in given))
+        own = not torch.is_grad_enabled() and not _watched() and _memory_says_all(*w, *(t for t in (x, *(dy[i] for i in given)) if t is not None))
         if own:
             g2 = {i: ops._dense16(g) for i, g in g2.items()}
         if ctx.needs_input_grad[1] and given:
@@ -92,9 +93,10 @@ class _LinearFn(torch.autograd.Function):
             if dx is None:
                 for g, v in zip(gs, ws):
                     dx = g @ v if dx is None else dx + g @ v
-            dx = dx.reshape(x.shape)
+            dx = dx.reshape(ctx.x_shape)
         wanted = [i for i in given if ctx.needs_input_grad[2 + i]]
         if wanted:
+            x2 = x.reshape(-1, x.shape[-1])
             made = ops.gemm("xtx", [g2[i] for i in wanted], [x2] * len(wanted), if_preferred=True) if own else None
             for k, i in enumerate(wanted):
                 dw[i] = made[k] if made is not None else g2[i].t() @ x2

@@ -782,3 +782,23 @@ def test_layer_gradients_are_seen_by_a_mode_that_watches_operators(pkg, gemm_by_
     with FlopCounterMode(display=False) as counter:
         torch.autograd.grad(ys, [x, *w], dy)
     assert counter.get_total_flops() == 2 * 2 * 2 * 6 * 8 * 16        # per layer dx and dw
+
+
+@pytest.mark.parametrize("frozen", ["weights", "input"])
+def test_layer_keeps_only_what_its_gradients_need(pkg, gemm_by_address, frozen):
+    """Frozen weights need no x, a frozen x no weights: written over between the passes, or freed, they change nothing (as for nn.Linear)."""
+    from sys import modules
+    linear_fn = modules[pkg.__name__ + ".linear"]._LinearFn
+    x, w, dy, _ = _layer_inputs()
+    for t in (w if frozen == "weights" else [x]):
+        t.requires_grad_(False)
+    saved = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or t, lambda t: t):
+        ys = linear_fn.apply(None, x, *w)
+    assert sum(t.numel() for t in saved) == (sum(v.numel() for v in w) if frozen == "weights" else x.numel())
+    wrt = [x] if frozen == "weights" else w
+    want = torch.autograd.grad(ys, wrt, dy, retain_graph=True)
+    with torch.no_grad():
+        for t in ([x] if frozen == "weights" else w):
+            t.zero_()
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(ys, wrt, dy), want))
