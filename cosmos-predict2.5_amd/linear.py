@@ -85,8 +85,8 @@ class _LinearFn(torch.autograd.Function):
         dx, dw = None, [None] * len(dy)
         # (create_graph: the gradients are differentiated again)
         own = not torch.is_grad_enabled() and not _watched() and _memory_says_all(*w, *(t for t in (x, *(dy[i] for i in given)) if t is not None))
-        if own:
-            g2 = {i: ops._dense16(g) for i, g in g2.items()}
+        if own:          # (hooks on saved tensors may bring them back in another layout)
+            g2, w = {i: ops._dense16(g) for i, g in g2.items()}, [ops._dense16(v) for v in w]
         if ctx.needs_input_grad[1] and given:
             gs, ws = [g2[i] for i in given], [w[i] for i in given]
             dx = ops.gemm("xw", gs, ws, total=True, if_preferred=True) if own else None
@@ -97,6 +97,8 @@ class _LinearFn(torch.autograd.Function):
         wanted = [i for i in given if ctx.needs_input_grad[2 + i]]
         if wanted:
             x2 = x.reshape(-1, x.shape[-1])
+            if own:
+                x2 = ops._dense16(x2)
             made = ops.gemm("xtx", [g2[i] for i in wanted], [x2] * len(wanted), if_preferred=True) if own else None
             for k, i in enumerate(wanted):
                 dw[i] = made[k] if made is not None else g2[i].t() @ x2

@@ -713,8 +713,12 @@ def gemm(order: str, a, b, total: bool = False, shape: int = 0, if_preferred: bo
     for group, like in ((a, a[0]), (b, b[0])):
         for t in group:
             if t.dim() != 2 or t.shape != like.shape or t.stride() != like.stride() or t.stride(1) != 1:
+                if if_preferred:
+                    return None
                 raise ValueError("the matrices of a launch need one shape and one line stride, with elements of a line side by side")
             if t.dtype != a[0].dtype or t.device != a[0].device:
+                if if_preferred:
+                    return None
                 raise ValueError("the matrices of a launch need one type and device")
     D = _gemm_desc(order, a, b, total, shape)
     depth = b[0].shape[1] if order == "xwt" else b[0].shape[0]

@@ -802,3 +802,24 @@ def test_layer_keeps_only_what_its_gradients_need(pkg, gemm_by_address, frozen):
         for t in ([x] if frozen == "weights" else w):
             t.zero_()
     assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(ys, wrt, dy), want))
+
+
+def test_layer_gradients_of_saved_tensors_that_come_back_in_another_layout(pkg, gemm_by_address):
+    from sys import modules
+    linear_fn = modules[pkg.__name__ + ".linear"]._LinearFn
+    x, w, dy, _ = _layer_inputs()
+    want = torch.autograd.grad(linear_fn.apply(None, x, *w), [x, *w], dy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().t().contiguous(), lambda t: t.t()):
+        ys = linear_fn.apply(None, x, *w)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(ys, [x, *w], dy), want))
+
+
+def test_products_that_are_only_asked_for_if_preferred_are_not_refused(pkg, monkeypatch):
+    """A column of rows is contiguous with any stride between its single elements: None, for the caller's own product, and no error."""
+    monkeypatch.setattr(pkg.ops, "_check_elementwise", lambda x: None)      # (nothing is launched: CPU tensors do)
+    x, w = torch.zeros(1, 2048, dtype=torch.bfloat16).t(), torch.zeros(64, 1, dtype=torch.bfloat16)
+    assert x.is_contiguous() and x.stride(1) != 1
+    for order, a, b in (("xwt", [x], [w]), ("xtx", [x], [x.float()]), ("xtx", [x, x[:1024]], [x, x])):
+        assert pkg.ops.gemm(order, a, b, if_preferred=True) is None
+        with pytest.raises(ValueError):
+            pkg.ops.gemm(order, a, b)
