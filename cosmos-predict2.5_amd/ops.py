@@ -163,17 +163,18 @@ def fwd_jvp(
 # struct cosmos_attn_desc in one go: the fields one by one take 2.5 us, a tenth of a small call
 _ATTN_DESC = struct.Struct("@9if6Q9q2Q3q2Q")
 assert _ATTN_DESC.size == ctypes.sizeof(_lib.AttnDesc)
-_IN_PLACE_ROWS = 6144      # (no call of more is taken; the library decides below)
+_ONE_DESCRIPTOR_ROWS = 6144      # (of a longer call nobody sees the host's share)
 
 
-def forward_in_place(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, sm_scale: Optional[float]) -> Optional[torch.Tensor]:
-    """Forward-only attention of ``[B, S, H, 128]`` tensors where the library reads k and v where they are (a small call: 9 us on the host through here, 20
-    through ``fwd_jvp``); None where the call is another one, whatever is wrong or special about it."""
+def forward_short(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, sm_scale: Optional[float]) -> Optional[torch.Tensor]:
+    """Forward-only attention of ``[B, S, H, 128]`` tensors, up to some thousand queries, with the least work on the host: one packed descriptor, given to the call
+    that reads k and v where they are, and where the library does not do that, to the one that re-tiles them.  None where the call is another one, whatever is
+    wrong or special about it.  A pass of few queries, us, here / through ``fwd_jvp``: in place 12 / 27, re-tiled 17 / 27."""
     if q.dim() != 4 or k.dim() != 4 or not q.is_cuda:
         return None
     B, S, H, D = q.shape
     Lkv = k.shape[1]
-    if D != 128 or S > _IN_PLACE_ROWS or k.shape != (B, Lkv, H, D) or v.shape != (B, Lkv, H, D):
+    if D != 128 or S > _ONE_DESCRIPTOR_ROWS or k.shape != (B, Lkv, H, D) or v.shape != (B, Lkv, H, D):
         return None
     code, device = _DTYPES.get(q.dtype), q.device
     if code is None or k.dtype != q.dtype or v.dtype != q.dtype or k.device != device or v.device != device or (causal and S != Lkv) or min(B, S, H, Lkv) < 1:
@@ -187,10 +188,13 @@ def forward_in_place(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: 
     o = torch.empty((B, S, H, D), device=device, dtype=q.dtype)
     desc = _ATTN_DESC.pack(_lib.ABI_VERSION, code, B, H, S, Lkv, D, D, 1 if causal else 0, D ** -0.5 if sm_scale is None else sm_scale,
                            pq, pk, pv, 0, 0, 0, qb, qh, ql, kb, kh, kl, vb, vh, vl, o.data_ptr(), 0, S * H * D, D, H * D, 0, 0)
-    run = _lib.load_library().cosmos_attn_fwd_in_place
-    status = _on_device(device, lambda stream: run(desc, stream))
+    lib = _lib.load_library()
+    status = _on_device(device, lambda stream: lib.cosmos_attn_fwd_in_place(desc, stream))
     if status == _lib.ST_WORKSPACE:
-        return None
+        same = _lib.AttnDesc.from_buffer_copy(desc)
+        ws_bytes = lib.cosmos_attn_workspace_bytes(same)
+        workspace = torch.empty(ws_bytes, device=device, dtype=torch.uint8)
+        status = _on_device(device, lambda stream: lib.cosmos_attn_fwd_jvp(same, workspace.data_ptr(), ws_bytes, stream))
     _lib.raise_for_status(status)
     return o
 
