@@ -19,7 +19,7 @@
 //     at 8192^3, these 1.53 / 1.55 / 1.53).  The 16-byte chunks of a row are stored XOR-swizzled (the load's lanes pick their source): no bank conflicts.
 //   * Persistent workgroups: the loads run over tile boundaries, so that only a workgroup's first tile waits for memory.  An XCD serves a
 //     contiguous run of tiles, 8 rows of tiles high, so that its L2 holds the panels that its compute units share.
-// Measured, us, library -> this, bf16 (rows x cols x depth): 37440 x 2048 x 2048 y 287 -> 225, dx 290 -> 230, dw (2048 x 2048 x 37440) 325 -> 331;
+// Measured, us, library -> this, bf16 (rows x cols x depth): 37440 x 2048 x 2048 y 287 -> 225, dx 290 -> 230;
 // 37440 x 8192 x 2048 931 -> 874, 1127 -> 912, 1042 -> 827; 10920 x 2048 x 2048 78 -> 76, 87 -> 78, 121 -> 84; 3520 x 2048 x 2048 34 -> 30, 36 -> 31.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -442,15 +442,6 @@ int choose_shape(const cosmos_attn_gemm_desc* d, double* cost) {
     return best;
 }
 
-// Where these kernels are the faster ones and where the library's (cosmos_attn_gemm_preferred).  Both measured at 256 .. 70400 rows, 2048 and 5120 wide layers and 4 times
-// that, us, library / this:
-//   dw: this one everywhere (0.50 .. 0.86 of the library's time), but for few tiles over a long contraction, where a workgroup reads
-//     on its own what others have long left (2048 x 2048: 24640 rows 355 / 192, 37440 rows 329 / 369).
-//   dx: from an estimated 1.02 PFLOP/s on (3520 x 20480 x 5120 995 / 710, 10920 x 5120 x 5120 463 / 423; below: 3520 x 5120 x 5120 167 / 178), and small ones, where
-//     the library is furthest from it (3520 x 2048 x 2048 33 / 29).  The sum of three is compared with the library's three and their additions (3520 rows 119 / 72).
-//   y: the library spreads a last round of tiles over the chip; that is better for wide layers on few rows (7040 x 2048 x 8192 157 / 165, 1560 x 20480 x 5120 267 / 297), worse
-//     from some 8000 rows on (17600 x 2048 x 8192 595 / 485, 37440 x 2048 x 2048 285 / 235; 0.94 of its time on average, 1.07 at most at 10920 x 2048 x 8192) and for small layers
-//     (3520 x 2048 x 2048 31 / 29).  Three in a launch are compared with three of the library's (3520 rows 97 / 79, 10920 237 / 226, 37440 881 / 691).
 template <typename T, int SHAPE, bool ACOL, bool BCOL>
 int launch(GemmParams& p, int products, hipStream_t stream) {
     constexpr Shape s = kShapes[SHAPE];
@@ -517,20 +508,53 @@ int check(const cosmos_attn_gemm_desc* d) {
     }
     return COSMOS_ATTN_OK;
 }
+// Where these kernels are the faster ones and where the library's.  Both sides measured on two cards at 256 .. 90 000 rows (ragged ones and whole frames), layers 512 to 5120 wide
+// and MLPs of four times that, 1700 sizes for one product, 1000 for several; below: this one's share of the library's time, mean (worst).  The kernels' own time follows cost_of within
+// 10 %.  The library's does not follow from the sizes: its choice of tiles is 7 % faster than this one where they fill the chip and up to twice as slow just past a whole round (9360 x 2048 x 8192
+// 506 us, 10920 279), and changes from one number of rows to the next.  What is common to the widths is how many rounds its largest tiles take:
+//   y, one product.  A half filled to just full round, the second half of a second one and a fourth one are the library's (1.08 (1.29), 1.02 (1.14), 1.00 (1.10)); third and fifth ones this
+//     one's (0.88 (1.15), 0.94 (1.12)), and for short contractions also the first half of a first round and of a second (0.76 (1.03), 0.92 (1.11); deep ones 1.01 (1.56), 1.00 (1.26)).  From
+//     five rounds on 0.97 (1.09) up to 5120 deep, 1.01 (1.12) deeper.  In all 0.90 (1.15) where it is chosen; "every 8192 rows and more, small layers from 1024 on" was 0.95 (1.56).
+//   dx, one product: from an estimated 1.02 PFLOP/s on, and small ones, where the library is furthest from it; but for the second half of a first round (1.00 (1.17)) and deep
+//     contractions just past one (0.95 (1.20)).  0.87 (1.08) where it is chosen.
+//   dw: this one, whatever the number of rounds, where a product has three quarters of one (0.74 (0.87)).  Fewer tiles leave the chip to few workgroups, each with the whole contraction, which
+//     the library splits if it is long: from a quarter round on up to 8192 deep (0.84 (0.97); 1.01 (1.16) above), an eighth to a quarter (2048 x 2048) up to 27 000 (0.64 (0.91); 1.08 (1.36)
+//     above), below that up to 4096 (0.68 (1.06); 0.99 (1.14) up to 16 000, 1.8 from 60 000 on).  Two in a launch are filled twice as well (limits 16 384, none, 32 768: 0.66 (0.99)), three
+//     always well enough (0.57 (0.85)).
+//   Several products of y, or dx summed, are compared with as many of the library's and their additions, at a rate and a launch that these take at best: 0.81 (1.10), 0.67 (0.96).
+//     (Of y, 12 us a launch: the 52 measured sizes that 8 us would leave to the library are 0.86 (1.08), the 38 that 12 leaves 0.93 (1.18).)
+// On a third card, at other rows and at widths of 1536, 2560 (MLP) and 4096 that no line was drawn by: y 0.92 (1.10) where chosen and 1.03 where not, dx 0.87 (1.06), dw 0.71 (0.98).
+bool preferred(const cosmos_attn_gemm_desc* d) {
+    double us = 0.0;
+    choose_shape(d, &us);
+    const double one = 2.0 * d->rows * d->cols * d->depth, rate = one * d->count / us;     // operations, per microsecond
+    const double rounds = (double)(ceil_div(d->rows, 256) * ceil_div(d->cols, 256)) / kNumCUs;      // of one product
+    const int64_t depth = d->depth;
+    if (d->order == COSMOS_GEMM_XTX) {
+        if (depth < 256) return false;
+        const bool two = d->count == 2;
+        if (d->count == 3 || rounds > 0.75) return true;
+        if (rounds > 0.25) return depth <= (two ? 16384 : 8192);
+        if (rounds > 0.125) return two || depth <= 27000;
+        return depth <= (two ? 32768 : 4096);
+    }
+    if (d->rows < 1024) return false;
+    if (d->order == COSMOS_GEMM_XW) {
+        if (d->count > 1) return us <= d->count * (one / 1.25e9 + 10.0);
+        if ((rounds > 0.5 && rounds <= 0.75) || (rounds > 1.0 && rounds <= 1.2 && depth > 2048)) return false;
+        return rate >= 1.02e9 || (one <= 6e10 && rate >= 0.55e9);
+    }
+    if (d->count > 1) return us <= d->count * (one / 1.35e9 + 12.0);
+    if (rounds <= 0.5 || (rounds > 1.0 && rounds <= 1.5)) return depth <= 2048;
+    if (rounds <= 2.0 || (rounds > 3.0 && rounds <= 4.0)) return false;
+    return rounds <= 5.0 || depth <= 5120;
+}
 }  // namespace
 
 extern "C" {
 
 COSMOS_ATTN_API int cosmos_attn_gemm_preferred(const cosmos_attn_gemm_desc* d) {
-    if (check(d) != COSMOS_ATTN_OK) return 0;
-    double us = 0.0;
-    const int shape = choose_shape(d, &us);
-    const double one = 2.0 * d->rows * d->cols * d->depth, rate = one * d->count / us;     // operations, per microsecond
-    if (d->order == COSMOS_GEMM_XTX) return d->depth >= 256 && !(shape == 3 && d->depth > 32768);
-    if (d->rows < 1024) return 0;
-    if (d->order == COSMOS_GEMM_XW) return d->count > 1 ? us <= d->count * (one / 1.25e9 + 10.0) : rate >= 1.02e9 || (one <= 6e10 && rate >= 0.55e9);
-    if (d->count > 1) return us <= d->count * (one / 1.35e9 + 12.0);
-    return d->rows >= 8192 || (int64_t)d->cols * d->depth <= (int64_t)1 << 22;
+    return check(d) == COSMOS_ATTN_OK && preferred(d) ? 1 : 0;
 }
 
 COSMOS_ATTN_API int cosmos_attn_gemm(const cosmos_attn_gemm_desc* d, void* stream_handle) {

@@ -726,6 +726,37 @@ def test_rows_below_which_no_layer_asks_are_below_the_rule(pkg, cols, depth, cou
     assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == 1
 
 
+@pytest.mark.parametrize("order, rows, cols, depth, own", [
+    # y: the library's time here, us, and this one's, measured
+    ("xwt", 10920, 2048, 8192, False),      # 279 / 305
+    ("xwt", 12480, 2048, 8192, False),      # 289 / 328
+    ("xwt", 4680, 2048, 2048, False),       # 35 / 41
+    ("xwt", 28160, 2048, 2048, False),      # 170 / 186
+    ("xwt", 1024, 1024, 4096, False),       # 19 / 29
+    ("xwt", 37440, 2048, 2048, True),       # 285 / 233
+    ("xwt", 17600, 2048, 8192, True),       # 594 / 485
+    ("xwt", 10920, 8192, 2048, True),       # 305 / 263
+    ("xwt", 3520, 2048, 2048, True),        # 29 / 27
+    ("xw", 9360, 2048, 8192, False),        # 258 / 296
+    ("xw", 4680, 2048, 8192, False),        # 130 / 142
+    ("xw", 37440, 2048, 2048, True),        # 290 / 230
+    ("xtx", 512, 512, 30000, False),        # 119 / 186
+    ("xtx", 2048, 1024, 30000, False),      # 223 / 287
+    ("xtx", 2048, 2048, 28160, False),      # 235 / 282
+    ("xtx", 3072, 3072, 30000, False),      # 554 / 592
+    ("xtx", 2048, 2048, 10920, True),       # 121 / 84
+    ("xtx", 8192, 2048, 84480, True),
+])
+def test_products_are_preferred_where_they_are_the_faster_ones(pkg, order, rows, cols, depth, own):
+    L = pkg._lib
+    D = L.GemmDesc()
+    D.abi_version, D.dtype, D.count, D.order = L.ABI_VERSION, L.DTYPE_BF16, 1, pkg.ops.GEMM_ORDERS[order]
+    D.a[0] = D.b[0] = D.c[0] = 16
+    D.rows, D.cols, D.depth, D.ldc = rows, cols, depth, cols
+    D.lda, D.ldb = rows if order == "xtx" else depth, depth if order == "xwt" else cols
+    assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == own
+
+
 def _by_address(t):
     """What a launch would read of t: its memory, and nothing else that belongs to it."""
     assert t.stride(1) == 1
