@@ -276,8 +276,8 @@ EXPORTS = {
     "cosmos_gated_residual_bwd": (ctypes.c_int, [ctypes.POINTER(GatedResidualBwdDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "cosmos_ln_modulation_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(ModulationDesc)]),
     "cosmos_ln_modulation": (ctypes.c_int, [ctypes.POINTER(ModulationDesc), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
-    "cosmos_attn_gemm": (ctypes.c_int, [ctypes.POINTER(GemmDesc), ctypes.c_void_p]),
-    "cosmos_attn_gemm_preferred": (ctypes.c_int, [ctypes.POINTER(GemmDesc)]),
+    "cosmos_attn_gemm": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p]),               # (a descriptor, also as packed bytes)
+    "cosmos_attn_gemm_preferred": (ctypes.c_int, [ctypes.c_void_p]),                      # (as well)
     "cosmos_gelu": (ctypes.c_int, [ctypes.POINTER(GeluDesc), ctypes.c_void_p]),
 }
 

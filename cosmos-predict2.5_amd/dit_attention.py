@@ -28,7 +28,7 @@ from torch import nn
 from . import ops
 from .attention import results_are_kept
 from .attn_op import HipAttnOp
-from .linear import linear
+from .linear import linear, linear_one
 
 
 class HeadRMSNormWeight(nn.Module):
@@ -193,7 +193,7 @@ class Attention(nn.Module):
         if context is None:
             q, k, v = linear([self.q_proj, self.k_proj, self.v_proj], x)
         else:
-            (q,), (k, v) = linear([self.q_proj], x), linear([self.k_proj, self.v_proj], context)
+            q, (k, v) = linear_one(self.q_proj, x), linear([self.k_proj, self.v_proj], context)
         q, k, v = self._heads(q), self._heads(k), self._heads(self.v_norm(v))
         q, _ = self._norm_rope(q, self.q_norm, rope_emb)
         k, _ = self._norm_rope(k, self.k_norm, rope_emb)
@@ -201,15 +201,15 @@ class Attention(nn.Module):
 
     def compute_attention(self, q, k, v, video_size=None):
         result = self.attn_op(q, k, v, video_size=video_size)   # [B, S, H*D]
-        return self.output_dropout(linear([self.output_proj], result)[0])
+        return self.output_dropout(linear_one(self.output_proj, result))
 
     def forward(self, x, context: Optional[torch.Tensor] = None, rope_emb: Optional[torch.Tensor] = None, video_size=None):
         """x: ``[B, Mq, K]`` (or ``[B, T, H, W, K]``); context: ``[B, Mk, Kc]`` or None for self-attention; rope_emb: the
         angles ``[Mq, 1, 1, D]`` (self-attention only).  Returns ``[B, Mq, K]`` in the shape of x."""
         if self._context_is_fixed(x, context):
-            q, _ = self._norm_rope(self._heads(linear([self.q_proj], x)[0]), self.q_norm, rope_emb)
+            q, _ = self._norm_rope(self._heads(linear_one(self.q_proj, x)), self.q_norm, rope_emb)
             packed = self._packed_context("context", context, self.k_proj, self.k_norm, self.v_proj)
-            out = self.output_dropout(linear([self.output_proj], self.attn_op.forward_packed(q, packed))[0])
+            out = self.output_dropout(linear_one(self.output_proj, self.attn_op.forward_packed(q, packed)))
             return out.reshape(*x.shape[:-1], out.shape[-1])
         q, k, v = self.compute_qkv(x, context, rope_emb=rope_emb)
         out = self.compute_attention(q, k, v, video_size=video_size)
@@ -279,16 +279,16 @@ class I2VCrossAttention(Attention):
     def compute_attention(self, q, k, v, k_img, v_img):
         result = self.attn_op(q, k, v)
         result_img = self.attn_op(q, k_img, v_img)
-        return self.output_dropout(linear([self.output_proj], result + result_img)[0])
+        return self.output_dropout(linear_one(self.output_proj, result + result_img))
 
     def forward(self, x, context=None, rope_emb=None, video_size=None):
         del video_size
         if x.is_cuda and not torch.is_grad_enabled() and not results_are_kept():
             text_context, img_context = context
-            q, _ = self._norm_rope(self._heads(linear([self.q_proj], x)[0]), self.q_norm, rope_emb)
+            q, _ = self._norm_rope(self._heads(linear_one(self.q_proj, x)), self.q_norm, rope_emb)
             result = self.attn_op.forward_packed(q, self._packed_context("text", text_context, self.k_proj, self.k_norm, self.v_proj))
             result_img = self.attn_op.forward_packed(q, self._packed_context("image", img_context, self.k_img, self.k_img_norm, self.v_img))
-            out = self.output_dropout(linear([self.output_proj], result + result_img)[0])
+            out = self.output_dropout(linear_one(self.output_proj, result + result_img))
             return out.reshape(*x.shape[:-1], out.shape[-1])
         q, k, v, k_img, v_img = self.compute_qkv(x, context, rope_emb)
         out = self.compute_attention(q, k, v, k_img, v_img)

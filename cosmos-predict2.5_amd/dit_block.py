@@ -25,7 +25,7 @@ from torch import nn
 
 from . import ops
 from .dit_attention import Attention, I2VCrossAttention
-from .linear import bare, linear
+from .linear import bare, linear_one
 
 
 def _per_row(m, like):
@@ -181,20 +181,20 @@ class GPT2FeedForward(nn.Module):
         torch.nn.init.trunc_normal_(self.layer2.weight, std=std, a=-3 * std, b=3 * std)
 
     def forward(self, x: torch.Tensor):
-        (h,) = linear([self.layer1], x)
+        h = linear_one(self.layer1, x)
         if h.is_cuda and h.numel() % 8 == 0 and h.dtype in (torch.bfloat16, torch.float16):
             if torch.is_grad_enabled() and h.requires_grad:
-                return linear([self.layer2], _GeluFn.apply(h))[0]
-            return linear([self.layer2], ops.gelu(h, inplace=True)[0])[0]      # inference: one fused pass, in place
+                return linear_one(self.layer2, _GeluFn.apply(h))
+            return linear_one(self.layer2, ops.gelu(h, inplace=True)[0])      # inference: one fused pass, in place
         return self.layer2(self.activation(h))
 
     @torch.no_grad()
     def forward_jvp(self, x: torch.Tensor, tx: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         b = x.shape[0]
         both = ops.as_stacked(x, tx)
-        (h,) = linear([self.layer1], both if both is not None else torch.cat([x, tx], dim=0))
+        h = linear_one(self.layer1, both if both is not None else torch.cat([x, tx], dim=0))
         ops.gelu(h[:b], h[b:], inplace=True)       # a = gelu(h), ta = th gelu'(h), in place on the stacked buffer
-        (y,) = linear([self.layer2], h)
+        y = linear_one(self.layer2, h)
         return y[:b], y[b:]
 
 

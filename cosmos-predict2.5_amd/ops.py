@@ -8,6 +8,7 @@ stream, never synchronises, and allocates outputs with ``torch.empty`` like the 
 from __future__ import annotations
 
 import ctypes
+import functools
 import struct
 from typing import Optional, Tuple
 
@@ -694,16 +695,35 @@ def modulation(emb, lora, w1, w2, temb=None, tlora=None, tangent: bool = False):
 GEMM_ORDERS = {"xwt": _lib.GEMM_XWT, "xw": _lib.GEMM_XW, "xtx": _lib.GEMM_XTX}
 
 
-def _gemm_desc(order: str, a, b, total: bool, shape: int) -> "_lib.GemmDesc":
-    D = _lib.GemmDesc()
-    D.abi_version, D.dtype, D.order = _lib.ABI_VERSION, _DTYPES[a[0].dtype], GEMM_ORDERS[order]
-    D.flags, D.count, D.shape = (_lib.GEMM_SUM if total else 0), len(a), shape
-    D.rows, D.depth = a[0].shape if order != "xtx" else a[0].shape[::-1]
-    D.cols = b[0].shape[1] if order != "xwt" else b[0].shape[0]
-    D.lda, D.ldb, D.ldc = a[0].stride(0), b[0].stride(0), D.cols
-    for i in range(len(a)):
-        D.a[i], D.b[i] = a[i].data_ptr(), b[i].data_ptr()
-    return D
+# struct cosmos_attn_gemm_desc in one go, as _ATTN_DESC
+_GEMM_DESC = struct.Struct("@10i3q9Q")
+assert _GEMM_DESC.size == ctypes.sizeof(_lib.GemmDesc)
+
+
+def _pack_gemm(order: str, dtype: int, rows: int, cols: int, depth: int, lda: int, ldb: int, a, b, c, total: bool, shape: int = 0) -> bytes:
+    three = lambda p: (*p, 0, 0)[:3]
+    return _GEMM_DESC.pack(_lib.ABI_VERSION, dtype, GEMM_ORDERS[order], _lib.GEMM_SUM if total else 0, len(a), shape, rows, cols, depth, 0,
+                           lda, ldb, cols, *three(a), *three(b), *three(c))
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_preferred(order: str, rows: int, cols: int, depth: int, lda: int, ldb: int, count: int = 1, total: bool = False) -> bool:
+    """Does the library take ``count`` such products, and faster than the vendor's library does?  Follows from the sizes alone."""
+    if max(rows, cols, depth) >= 1 << 31:
+        return False
+    at = (16,) * count
+    return bool(_lib.load_library().cosmos_attn_gemm_preferred(_pack_gemm(order, _lib.DTYPE_BF16, rows, cols, depth, lda, ldb, at, at, at, total)))
+
+
+def launch_gemm(order: str, rows: int, cols: int, depth: int, lda: int, ldb: int, a, b, total: bool = False, shape: int = 0, lead=None):
+    """:func:`gemm` of operands that are known to be right: of tensors of any dimensions only the address is taken."""
+    like = a[0]
+    outs = [torch.empty((*(lead or (rows,)), cols), device=like.device, dtype=like.dtype) for _ in range(1 if total else len(a))]
+    at = lambda ts: [t.data_ptr() for t in ts]
+    D = _pack_gemm(order, _DTYPES[like.dtype], rows, cols, depth, lda, ldb, at(a), at(b), at(outs), total, shape)
+    run = _lib.load_library().cosmos_attn_gemm
+    _lib.raise_for_status(_on_device(like.device, lambda stream: run(D, stream)))
+    return outs[0] if total else outs
 
 
 def gemm(order: str, a, b, total: bool = False, shape: int = 0, if_preferred: bool = False, lead=None):
@@ -724,21 +744,14 @@ def gemm(order: str, a, b, total: bool = False, shape: int = 0, if_preferred: bo
                 if if_preferred:
                     return None
                 raise ValueError("the matrices of a launch need one type and device")
-    D = _gemm_desc(order, a, b, total, shape)
-    depth = b[0].shape[1] if order == "xwt" else b[0].shape[0]
-    if D.depth != depth:
+    rows, depth = a[0].shape if order != "xtx" else a[0].shape[::-1]
+    cols, same = b[0].shape[::-1] if order != "xwt" else b[0].shape
+    if depth != same:
         raise ValueError("the matrices' contractions differ")
-    n = 1 if total else len(a)
-    if if_preferred:
-        for i in range(n):
-            D.c[i] = 16            # (the outputs are allocated only where they are written)
-        if not _lib.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)):
-            return None
-    outs = [torch.empty((*(lead or (D.rows,)), D.cols), device=a[0].device, dtype=a[0].dtype) for _ in range(n)]
-    for i, o in enumerate(outs):
-        D.c[i] = o.data_ptr()
-    _launch("cosmos_attn_gemm", D, a[0].device)
-    return outs[0] if total else outs
+    lda, ldb = a[0].stride(0), b[0].stride(0)
+    if if_preferred and (any(t.data_ptr() % 16 for t in (*a, *b)) or not gemm_preferred(order, rows, cols, depth, lda, ldb, len(a), total)):
+        return None
+    return launch_gemm(order, rows, cols, depth, lda, ldb, a, b, total, shape, lead)
 
 
 def gelu(h, th=None, inplace: bool = False):

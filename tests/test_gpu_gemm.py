@@ -178,6 +178,24 @@ def test_layers_with_a_meaning_of_their_own_go_through_the_module(pkg, how):
     assert how != "hook" or len(calls) == 2
 
 
+@pytest.mark.parametrize("how", ["one frame", "one row", "slice"])
+def test_layers_of_dense_inputs_with_strides_of_their_own(pkg, how):
+    """Dense is what is_contiguous calls so: a dimension of one has any stride."""
+    from sys import modules
+    lin = modules[pkg.__name__ + ".linear"]
+    (m,) = _layers(1, 512, 512, torch.bfloat16)
+    x = torch.randn(1, 2048, 512, device="cuda").bfloat16()
+    x = {"one frame": x.transpose(0, 1), "one row": x.view(2048, 1, 512).as_strided((2048, 1, 512), (512, 8, 1)), "slice": x[:, 8:1600]}[how]
+    assert x.is_contiguous() and lin._own(x.shape[:-1].numel(), 512, 512, 1, False)[0]
+    with torch.no_grad():
+        got = lin.linear([m], x)[0]
+    assert got.shape == x.shape and _rel(got, x.double() @ m.weight.double().t()) < 2e-3
+    x = x.clone(memory_format=torch.preserve_format).requires_grad_(True)
+    dx, dw = torch.autograd.grad(lin.linear_one(m, x), [x, m.weight], got)
+    g, w = got.double().reshape(-1, 512), m.weight.detach().double()
+    assert _rel(dx.reshape(-1, 512), g @ w) < 2e-3 and _rel(dw, g.t() @ x.detach().double().reshape(-1, 512)) < 2e-3
+
+
 def test_products_replayed_from_a_graph(pkg):
     ops = pkg.ops
     a, b = torch.randn(1560, 512, device="cuda").bfloat16(), torch.randn(768, 512, device="cuda").bfloat16()

@@ -757,23 +757,26 @@ def test_products_are_preferred_where_they_are_the_faster_ones(pkg, order, rows,
     assert L.load_library().cosmos_attn_gemm_preferred(ctypes.byref(D)) == own
 
 
-def _by_address(t):
+def _by_address(t, lines, width, ld):
     """What a launch would read of t: its memory, and nothing else that belongs to it."""
-    assert t.stride(1) == 1
-    n = (t.shape[0] - 1) * t.stride(0) + t.shape[1]
-    return torch.frombuffer(bytearray(ctypes.string_at(t.data_ptr(), n * t.element_size())), dtype=t.dtype).as_strided(t.shape, t.stride())
+    n = (lines - 1) * ld + width
+    return torch.frombuffer(bytearray(ctypes.string_at(t.data_ptr(), n * t.element_size())), dtype=t.dtype).as_strided((lines, width), (ld, 1))
 
 
 @pytest.fixture
 def gemm_by_address(pkg, monkeypatch):
-    """ops.gemm on the CPU, on what it would find at its operands' addresses; always preferred."""
+    """The layers' own products on the CPU, formed of what a launch would find at its operands' addresses; always preferred."""
     from torch.utils._python_dispatch import _disable_current_modes
 
-    def gemm(order, a, b, total=False, shape=0, if_preferred=False, lead=None):
+    def launch(order, rows, cols, depth, lda, ldb, a, b, total=False, shape=0, lead=None):
         with _disable_current_modes():         # (no mode sees a launch)
-            out = [(_by_address(x).t() if order == "xtx" else _by_address(x)) @ (_by_address(y).t() if order == "xwt" else _by_address(y)) for x, y in zip(a, b)]
-            return sum(out) if total else out
-    monkeypatch.setattr(pkg.ops, "gemm", gemm)
+            a = [_by_address(x, *((depth, rows) if order == "xtx" else (rows, depth)), lda) for x in a]
+            b = [_by_address(y, *((cols, depth) if order == "xwt" else (depth, cols)), ldb) for y in b]
+            out = [(x.t() if order == "xtx" else x) @ (y.t() if order == "xwt" else y) for x, y in zip(a, b)]
+            out = [y.reshape(*(lead or (rows,)), cols) for y in ([sum(out)] if total else out)]
+            return out[0] if total else out
+    monkeypatch.setattr(pkg.ops, "launch_gemm", launch)
+    monkeypatch.setattr(pkg.ops, "gemm_preferred", lambda *a, **kw: True)
 
 
 def _layer_inputs(n=2, rows=6, depth=8, cols=16):
