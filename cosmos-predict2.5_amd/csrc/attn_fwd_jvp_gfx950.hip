@@ -2148,8 +2148,10 @@ bool reads_in_place(const cosmos_attn_desc* d, const SplitPlan& sp) {
     const int mode = mode_of(d);
     if (d->d_qk != 128 || d->d_v != 128 || mode == MODE_JVP_Q || d->Lq > kInPlaceRows[mode == MODE_FWD ? 0 : 1]) return false;
     if ((mode == MODE_FWD && sp.shape == 0) || stream_groups_of(d, sp)) return false;
-    for (const int64_t stride : {d->k_stride[2], d->v_stride[2]})       // 32-bit buffer offsets, also of the rows behind the last one
-        if (stride < 0 || stride >= (int64_t)1 << 30 || (d->Lkv + 4 * kBlockN) * stride * 2 >= (int64_t)1 << 31) return false;
+    // 32-bit buffer offsets, also of the rows behind the last one, which have to lie past the buffer: of rows that overlap (an expanded tensor's) they would read as numbers,
+    // and 0 times what is there is not 0 where that is infinite
+    for (const int64_t stride : {d->k_stride[2], d->v_stride[2]})
+        if (stride < 128 || stride >= (int64_t)1 << 30 || (d->Lkv + 4 * kBlockN) * stride * 2 >= (int64_t)1 << 31) return false;
     return true;
 }
 // `room`: bytes behind the re-tiled K/V image that key-range partial results may take.  cosmos_attn_run only reads its workspace, so

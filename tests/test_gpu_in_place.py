@@ -102,3 +102,15 @@ def test_attention_is_the_general_call(pkg, monkeypatch, B, S, H, Lkv, causal, s
         pkg.attention_forward(q, k[:, :-1], v, dtype=dtype)
     with torch.no_grad(), pytest.raises((RuntimeError, NotImplementedError)):
         pkg.attention_forward(q.cpu(), k.cpu(), v.cpu(), dtype=dtype)
+
+
+@pytest.mark.parametrize("how", ["expanded", "dense"])
+def test_infinite_values_stay_what_they_are(pkg, how):
+    """A value that is infinite in every row gives infinity and not NaN, also where rows behind the last one are formed (40 keys of a step of 64)."""
+    q = torch.randn(1, 70, 2, 128, device="cuda").bfloat16()
+    k, v = (torch.randn(1, 1, 2, 128, device="cuda").bfloat16() for _ in range(2))
+    v[..., 5] = float("inf")
+    k, v = (x.expand(1, 40, 2, 128) if how == "expanded" else x.repeat(1, 40, 1, 1) for x in (k, v))
+    with torch.no_grad():
+        o = pkg.attention_forward(q, k, v, dtype=torch.bfloat16)
+    assert torch.isposinf(o[..., 5]).all() and torch.isfinite(o[..., :5]).all() and torch.isfinite(o[..., 6:]).all()

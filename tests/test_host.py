@@ -857,3 +857,14 @@ def test_products_that_are_only_asked_for_if_preferred_are_not_refused(pkg, monk
         assert pkg.ops.gemm(order, a, b, if_preferred=True) is None
         with pytest.raises(ValueError):
             pkg.ops.gemm(order, a, b)
+
+
+@pytest.mark.parametrize("stride, status", [(0, "ST_WORKSPACE"), (64, "ST_WORKSPACE"), (120, "ST_WORKSPACE"), (128, None)])
+def test_overlapping_rows_are_not_read_in_place(pkg, stride, status):
+    L = pkg._lib
+    desc = lambda s: pkg.ops._ATTN_DESC.pack(L.ABI_VERSION, L.DTYPE_BF16, 1, 2, 70, 40, 128, 128, 0, 0.1, 16, 16, 16, 0, 0, 0,
+                                             70 * 256, 128, 256, 40 * 256, 40 * 128, 128, 40 * 256, 40 * 128, s, 16, 0, 70 * 256, 128, 256, 0, 0)
+    if status is not None:
+        assert L.load_library().cosmos_attn_fwd_in_place(desc(stride), None) == getattr(L, status)
+    elif not torch.cuda.is_available():      # (accepted: nothing of these sizes is refused before the device is looked at)
+        assert L.load_library().cosmos_attn_fwd_in_place(desc(stride), None) not in (L.ST_WORKSPACE, 0)
