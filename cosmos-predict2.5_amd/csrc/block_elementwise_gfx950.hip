@@ -586,14 +586,14 @@ __global__ void __launch_bounds__(64 * kModSplit) modulation_hidden_kernel(const
             unpack8<BF16>(x[i], f);
 #pragma unroll
             for (int j = 0; j < 8; ++j) sig[j] = 1.0f / (1.0f + __expf(-f[j]));
-            if (p.rows_all > p.rows) {
+            if (moves) {
                 float t[8];
                 unpack8<BF16>(tx[i], t);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) f[j] = tangent ? t[j] * (sig[j] * (1.0f + f[j] * (1.0f - sig[j]))) : f[j] * sig[j];
-            } else {
+            } else {         // (emb does not move: its tangent's activations are zeros, whatever its values)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) f[j] *= sig[j];
+                for (int j = 0; j < 8; ++j) f[j] = tangent ? 0.f : f[j] * sig[j];
             }
             acc = Half8<BF16>::mfma(a[i], pack8<BF16>(f), acc);
         }

@@ -185,7 +185,7 @@ def test_reverse_mode_without_eps(pkg, gpu, rows, rpg, D):
 @pytest.mark.parametrize("rows,K,hidden,D", [(1, 32, 32, 16), (3, 2048, 256, 2048), (8, 256, 64, 48), (16, 288, 32, 80), (17, 5120, 256, 128), (40, 96, 96, 32)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_modulation(pkg, gpu, rows, K, hidden, D, dtype):
-    """One row to several tiles of 16, k shorter than the eight wavefronts that share it and with a remainder, vectors that end
+    """One row to several tiles of 16, k shorter than the sixteen wavefronts that share it and with a remainder, vectors that end
     inside a workgroup; in 64 bits with the two intermediate roundings that the library's layers have as well."""
     g = torch.Generator().manual_seed(rows + K)
     emb, temb = rnd(g, dtype, rows, K), rnd(g, dtype, rows, K, std=0.3)
@@ -209,6 +209,17 @@ def test_modulation(pkg, gpu, rows, K, hidden, D, dtype):
         check("out", out, want, dtype, flip)
         twant = torch.stack([cut(layers(tact if te is not None else 0 * tact, i) + (0 if tl is None else tl.double())) for i in range(3)])
         check("tout", tout, twant, dtype, flip)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), -3.0e38])
+def test_modulation_of_an_embedding_that_does_not_move(pkg, gpu, value):
+    """Its tangent is the added vectors' own, whatever the embedding's values are: no 0 times infinity."""
+    rn = lambda *s: torch.randn(*s, device=gpu).bfloat16()
+    emb, lora, tlora = rn(3, 64), rn(3, 48), rn(3, 48)
+    w1, w2 = [rn(32, 64) for _ in range(3)], [rn(48, 32) for _ in range(3)]
+    emb[1, 5] = value
+    _, tout = pkg.ops.modulation(emb, lora, w1, w2, tlora=tlora, tangent=True)
+    assert torch.equal(tout, tlora.reshape(3, 3, 16).transpose(0, 1).expand(3, 3, 3, 16))
 
 
 @pytest.mark.parametrize("rows,K,hidden,D", [(1, 32, 32, 16), (24, 256, 64, 48), (40, 96, 96, 32)])
