@@ -30,7 +30,7 @@ def _matrix(g, rows, cols, dtype, ld=None):
     (1, 8, 64, 1, False),            # smaller than any tile, one step
     (264, 520, 128, 3, False),       # a tile and a few rows and columns more; two steps
     (257, 136, 448, 2, True),        # products summed: steps of one after the other
-    (2304, 256, 192, 1, False),      # a full group of rows of tiles and one more; more tiles than one XCD's share
+    (2304, 256, 192, 1, False),      # a full group of rows of tiles and one more
 ])
 def test_products(pkg, order, shape, dtype, rows, cols, depth, count, total):
     ops = pkg.ops
@@ -47,6 +47,30 @@ def test_products(pkg, order, shape, dtype, rows, cols, depth, count, total):
     want = [x @ (y.double().t() if order == "xwt" else y.double()) for x, y in zip(left, b)]
     for y, w in zip([got] if total else got, [sum(want)] if total else want):
         assert torch.isfinite(y).all() and _rel(y, w) < REL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape, rows, cols", [(1, 4360, 4360), (2, 4360, 4360), (3, 4360, 4360), (4, 4360, 4360), (4, 264, 33032)])
+@pytest.mark.parametrize("order", ["xwt", "xw", "xtx"])
+def test_products_of_more_tiles_than_workgroups(pkg, order, shape, rows, cols, dtype):
+    """Workgroups that walk several tiles: their loads, waits (which count the stores of the tile before) and accumulators over a tile's end.  256 workgroups, of 128 x 128 tiles
+    512; 324, 630, 630, 1225 and 777 tiles.  Steps per tile: one (every step a tile's first), two and five, in one product, three products and sums of two and three."""
+    ops = pkg.ops
+    g = torch.Generator(device="cuda").manual_seed(shape)
+    wide = {1: (256, 256), 2: (256, 128), 3: (128, 256), 4: (128, 128)}[shape]
+    assert -(-rows // wide[0]) * -(-cols // wide[1]) > (512 if shape == 4 else 256)
+    for depth, count, total in ((64, 1, False), (64, 3, True), (128, 2, True), (320, 1, False), (128, 3, False)):
+        depth += 5 if order == "xtx" and depth > 64 else 0
+        a_shape, b_shape = (depth, rows) if order == "xtx" else (rows, depth), (cols, depth) if order == "xwt" else (depth, cols)
+        a, b = [_matrix(g, *a_shape, dtype) for _ in range(count)], [_matrix(g, *b_shape, dtype, b_shape[1] + -b_shape[1] % 8) for _ in range(count)]
+        got = ops.gemm(order, a, b, total=total, shape=shape)
+        want = [(x.double().t() if order == "xtx" else x.double()) @ (y.double().t() if order == "xwt" else y.double()) for x, y in zip(a, b)]
+        for y, w in zip([got] if total else got, [sum(want)] if total else want):
+            assert torch.isfinite(y).all() and _rel(y, w) < REL[dtype]
+            # (a tile that is wrong as a whole would be a few thousandths of all: every block of rows and of columns by itself as well)
+            d = (y.double() - w).pow(2)
+            for dim in (0, 1):
+                assert (d.sum(dim) <= (4 * REL[dtype]) ** 2 * w.pow(2).sum(dim)).all()
 
 
 def test_refused_matrices(pkg):
