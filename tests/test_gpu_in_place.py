@@ -1,5 +1,7 @@
 """Attention calls that read K and V where they are (head dim 128, few query rows): the same bits as the same kernels on the re-tiled image (without
 tangents), and parity with the oracle (with all tangents), where what lies behind the last row is not a number."""
+import ctypes
+
 import pytest
 import torch
 
@@ -16,32 +18,59 @@ def _rows(g, B, L, H, dtype, scale, layout):
     return view
 
 
-# keys: one, a tile's edge, a step's edge, ragged; 128-row workgroups of two key groups (few rows) and 256-row ones
+# keys: one, a tile's edge, a step's edge, ragged; the same workgroup shape (128 rows and two key groups, 256 rows) on both sides, no cut, no stream
+@pytest.mark.parametrize("dtype, layout", [(torch.bfloat16, "blhd"), (torch.float16, "bhld")])
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("B, H, Lq, Lkv, causal, lens", [
+    (1, 2, 1, 1, False, None), (2, 3, 129, 32, False, None), (1, 2, 300, 33, False, None), (1, 16, 255, 255, False, None), (2, 16, 520, 520, True, None),
+    (1, 40, 1000, 1000, False, None), (1, 40, 1100, 65, False, None), (2, 16, 513, 700, False, (1, 411)),
+])
+def test_forward_gives_the_bits_of_the_re_tiled_image(pkg, stream_override, forward_override, rows, B, H, Lq, Lkv, causal, lens, dtype, layout):
+    ops = pkg.ops
+    stream_override(chunk=1)
+    forward_override(rows, 1)
+    g = torch.Generator(device="cuda").manual_seed(Lq + Lkv)
+    q = _rows(g, B, Lq, H, dtype, 1.0, layout)
+    k, v = _rows(g, B, Lkv, H, dtype, 2.0, layout), _rows(g, B, Lkv, H, dtype, 1.0, layout)
+    lens = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda")
+    lib, packed = pkg._lib.load_library(), ops.pack_kv(k, v)
+    results = []
+    for in_place in (True, False):
+        o, lse = torch.full((B, H, Lq, 128), float("nan"), device="cuda", dtype=dtype), torch.full((B, H, Lq), float("nan"), device="cuda")
+        d = ops._packed_desc(B, H, Lq, Lkv, 128, 128, dtype, 128 ** -0.5)
+        d.causal, d.q, d.k, d.v, d.o, d.lse = int(causal), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr()
+        d.key_lens = None if lens is None else lens.data_ptr()
+        d.q_stride, d.k_stride, d.v_stride, d.o_stride = (ops._strides3(t) for t in (q, k, v, o))
+        stream = torch.cuda.current_stream().cuda_stream
+        assert (lib.cosmos_attn_fwd_in_place(ctypes.byref(d), stream) if in_place
+                else lib.cosmos_attn_run(ctypes.byref(d), packed.image.data_ptr(), packed.image.numel(), stream)) == 0
+        results.append((o, lse))
+    (o, lse), (want, want_lse) = results
+    assert torch.isfinite(o).all() and torch.isfinite(lse).all()
+    assert torch.equal(lse, want_lse) and torch.equal(o, want)
+
+
 @pytest.mark.parametrize("dtype, layout", [(torch.bfloat16, "blhd"), (torch.float16, "bhld")])
 @pytest.mark.parametrize("B, H, Lq, Lkv, causal, lens", [
     (1, 2, 1, 1, False, None), (2, 3, 129, 32, False, None), (1, 2, 300, 33, False, None), (1, 16, 255, 255, False, None), (2, 16, 520, 520, True, None),
     (1, 40, 1000, 1000, False, None), (1, 40, 1100, 65, False, None), (2, 16, 513, 700, False, (1, 411)),
 ])
-def test_forward_gives_the_bits_of_the_re_tiled_image(pkg, B, H, Lq, Lkv, causal, lens, dtype, layout):
+def test_forward_by_the_library_s_choice(pkg, B, H, Lq, Lkv, causal, lens, dtype, layout):
+    """Whichever kernels the two ways take: parity in 64 bits."""
     ops = pkg.ops
     g = torch.Generator(device="cuda").manual_seed(Lq + Lkv)
     q = _rows(g, B, Lq, H, dtype, 1.0, layout)
     k, v = _rows(g, B, Lkv, H, dtype, 2.0, layout), _rows(g, B, Lkv, H, dtype, 1.0, layout)
     lens = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda")
     o, _, lse = ops.fwd_jvp(q, k, v, causal=causal, key_lens=lens)
-    assert torch.isfinite(o).all() and torch.isfinite(lse).all()
+    s = (q.double() @ k.double().transpose(-1, -2)) * 128 ** -0.5
     if causal:
-        s = (q.double() @ k.double().transpose(-1, -2)) * 128 ** -0.5
         s.masked_fill_(torch.ones(Lq, Lkv, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
-        want = s.softmax(-1) @ v.double()
-        assert (o.double() - want).norm() / want.norm() < (5e-3 if dtype == torch.bfloat16 else 5e-3 / 8)      # limit of the parity tests; fp16 rounds 8 times finer
-        return
-    want, _, want_lse = ops.run_packed(q, ops.pack_kv(k, v), key_lens=lens)
-    # (a two-stage run may stream its query blocks or take 384-row workgroups: the same sums in another order then)
-    if torch.equal(lse, want_lse):
-        assert torch.equal(o, want)
-    else:
-        assert (lse - want_lse).abs().max() < 1e-4 and (o.double() - want.double()).norm() / want.double().norm() < (5e-3 if dtype == torch.bfloat16 else 5e-3 / 8)
+    if lens is not None:
+        s.masked_fill_(torch.arange(Lkv, device="cuda")[None, None, None] >= lens[:, None, None, None], float("-inf"))
+    want = s.softmax(-1) @ v.double()
+    # limits of the parity tests; fp16 rounds 8 times finer
+    assert (o.double() - want).norm() / want.norm() < (5e-3 if dtype == torch.bfloat16 else 5e-3 / 8) and (lse - s.logsumexp(-1)).abs().max() < 2e-3
 
 
 @pytest.mark.parametrize("dtype, layout", [(torch.bfloat16, "blhd"), (torch.float16, "bhld")])
