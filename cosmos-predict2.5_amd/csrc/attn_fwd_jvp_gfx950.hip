@@ -1251,7 +1251,7 @@ attn_qstream_kernel(const AttnParams p) {
 // at 1.53 GHz, 37440 positions; 66 % at 1.76 GHz before).  Hence the softmax is written between the MFMAs of both stages of a tile and kept there (tile_step), and the max is not
 // formed where it did not move (kMaxTileSum).  Measured, us, before either / with the softmax between the MFMAs / with both: 16 heads,
 // d = 128, 37440 positions 9558 / 9300 / 8937, 24640 4190 / 4060 / 3860, 3520 (384 rows a workgroup) 132 / 125 / 120; with 384 rows a workgroup in
-// 16 x 16 x 32 products another 5 % of the long ones (SymWave16).  Not faster: operand fetches three groups ahead, the fills spread over the step.
+// 16 x 16 x 32 products another 1 to 3 % of the long ones (SymWave16).  Not faster: operand fetches three groups ahead, the fills spread over the step.
 //
 // A workgroup is RG groups of 32 query rows x KG groups of keys: of every KG tiles of 32 keys a wavefront takes one, and the KG partial
 // results of a row group (accumulator, running max, row sum) are merged through LDS at the end.  Large calls take 12 x 1; 8 x 1 and 4 x 2
@@ -1744,15 +1744,14 @@ typedef void (*attn_kernel_t)(const AttnParams);
 
 // Workgroups of attn_fwd_sym_kernel, groups of 32 query rows x groups of keys, and what they cost at head dims 16, 32, 64, 128 (StepCost):
 // the least estimate is taken (plan_split).  Fits to 255 .. 13000 positions and 600 .. 37440 x 512 .. 2048, B*H = 16 and 40, S = 1 .. 16, each
-// shape with each S measured.  us, 12 x 1 / 8 x 1 / 4 x 2, uncut, d = 128, with the re-tiling: 16 heads 255 positions 18.8 / 17.5 / 14.9,
-// 700 34.8 / 30.1 / 25.3, 1560 61 / 50 / 40, 3520 120 / 110 / 124, 5000 205 / 267 / 245; 40 heads 1000 49 / 41 / 56, 1560 75 / 98 / 100.
-// (Three key groups are no faster than two.)
-// The smaller shapes are chosen from only where a call fits into one round of them.  There the choice takes 1.003 times the best shape's time
-// on average and 1.08 at most (64 calls of those ranges at random, each shape uncut and with its own cut).  Past one round 12 x 1 is taken, whose
-// thin last round is cut: over 59 calls 1.012 on average, but 1.14 at most, since a last round of 64 .. 128 pairs is where two rounds of 8 x 1 can be
-// shorter (us, 12 x 1 cut / 8 x 1: 16 heads 7410 x 883 at head dim 32 43 / 38, 8120 x 1024 at 64 63 / 55, 2 x 16 heads 3520 225 / 215; the other way
-// 40 heads 3520 272 / 309, 16 heads 9452 at 64 409 / 488).  Where no keys are cut (two-stage runs, masks) such a call loses more: 16 heads 7040
-// 485 / 392, 2 x 16 heads 3520 262 / 215.  Causal calls are priced as if every workgroup walked all keys.
+// shape with each S measured, with the re-tiling and with 12 x 1 in 32 x 32 x 16 products.  (Three key groups are no faster than two.)
+// At head dim 128 the kernels have moved since: 12 x 1 is in 16 x 16 x 32 products, 8 x 1 and 4 x 2 read K and V in place up to 6144 rows (kInPlaceRows).  As they are, us, 12 x 1
+// (with the re-tiling) / 8 x 1 / 4 x 2, uncut: 16 heads 255 positions 21.1 / 15.4 / 12.1, 700 38.8 / 25.0 / 18.3, 1560 66.6 / 45.4 / 33.2, 3520 134.7 / 111.3 / 126.8, 5000 214 / 280 / 257;
+// 40 heads 1000 53.3 / 35.3 / 50.2, 1560 80.2 / 96.3 / 96.7.  The smaller shapes are chosen from only where a call fits into one round of them; there the choice among the three
+// takes 1.013 times the best one's time on average and 1.25 at most (40 heads 656 positions 27.4 / 21.9: priced for a re-tiling that is not done; 27 calls at random).  Past one round 12 x 1 is
+// taken, whose thin last round is cut: 1.010 on average, 1.05 at most (37 calls), since a last round of 64 .. 128 pairs is where two rounds of 8 x 1 can be shorter (us, 12 x 1 cut / 8 x 1: 16 heads
+// 7410 x 883 at head dim 32 43 / 38, 8120 x 1024 at 64 63 / 55, 2 x 16 heads 3520 234 / 222; the other way 40 heads 3520 291 / 321, 16 heads 9452 at 64 409 / 488).  Where no keys are cut
+// (two-stage runs, masks) such a call loses more: 16 heads 7040 519 / 420, 2 x 16 heads 3520 282 / 222.  Causal calls are priced as if every workgroup walked all keys.
 struct SymShape { int rg, kg; double step_us[4], alone[4], range_us[4]; };
 constexpr SymShape kSymShapes[] = {
     {12, 1, {1.09, 1.12, 1.55, 2.42}, {1.0, 1.0, 0.86, 0.72}, {5.5, 5.8, 7.8, 12.7}},
@@ -1943,15 +1942,18 @@ size_t planned_partial_bytes(const cosmos_attn_desc* d) {
 // block_us + tile_us per key tile each and start_us once, comes out faster than the other kernels' rounds: a finished block costs it
 // little, a key tile costs it more than the forward-only kernel (which has three wavefronts per SIMD).  Measured (us, stream / other kernel,
 // 16 heads): tangent on q 3520 x 512 keys 45 / 62, 7040 x 512 78 / 109, 37440 x 2048
-// 1162 / 1294; forward only, with the re-tiling, 3520 x 512 29 / 31, 37440 x 512 206 / 220, x 1024 382 / 344, x 2048 738 / 591; at head dim 64
+// 1148 / 1294; forward only, with the re-tiling, 3520 x 512 30 / 31, 37440 x 512 209 / 220, x 1024 382 / 330, x 2048 738 / 555; at head dim 64
 // 8010 x 361 34 / 37, 6880 x 145 20 / 27, 6868 x 958 70 / 56; below that the forward-only kernel is the faster one (head dim 32: 1560 x 512 15 / 13,
 // 3520 x 512 23 / 16, 40 heads 1560 x 512 32 / 20).
 // The constants are fits at each head dim to 600 .. 37440 x 64 .. 2048, B*H = 16 and 40, both ways measured: with a tangent the way chosen takes
 // 1.0000 to 1.008 times the better one's time on average, 1.12 at most; forward only 1.00 on average, 1.04 at most (68 calls, with all three
-// workgroup shapes on the other side).  The two-stage run never cuts key ranges (no room), so that its
+// workgroup shapes on the other side) -- both sides with the re-tiling, as in two-stage runs.  A one-call form of up to some 1500 rows at head dim 128 does without it on the other side, which
+// is not priced: the stream it takes is 1.25 times the time of the better shape in place on average, 1.38 at most (16 heads 1560 positions 41 / 33, 1039 31 / 24, 80 heads 665 45 / 33; 15 calls).
+// The two-stage run never cuts key ranges (no room), so that its
 // other way is the uncut one: 16 heads, us, stream / uncut: tangent on q 2120 x 1024 60 / 71, 2200 x 2048 111 / 121 (one call, which cuts, with its
-// re-tiling: 67, 101); forward only 6500 x 1024 80 / 88, 6800 x 1536 115 / 119 (one call 83, 110).  With all tangents the
-// two are within a tenth of each other either way; there the stream starts at four blocks per unit (37440 x 512 527 / 596).
+// re-tiling: 67, 101); forward only 6500 x 1024 80 / 88, 6800 x 1536 115 / 119 (one call 83, 110).  With all tangents the stream
+// starts at four blocks per unit, a line from before its 16 x 16 x 32 products, when the two were within a tenth of each other: from there on it takes 0.82 of the other's time now (0.63 .. 0.96;
+// 37440 x 512 509 / 632), but 0.86 (0.75 .. 0.97) from one and a half blocks on already, 1.04 (0.99 .. 1.16) at one and a bit and 1.13 below (46 calls of 70 .. 1856 keys).
 // Padded keys (key_lens, which the host does not read) are priced at their full length, so that a call at a tie may take the way that is slower on
 // its shorter rows: head dim 64, 700 x 700, 40 heads, stream / 4 x 2 (taken) 22.2 / 22.0, with half of the keys valid 15.7 / 17.9; 2 x 16 heads
 // 1000 x 1000 27.5 / 24.2 and 18.5 / 19.6.  (At head dims 16, 32 and 128 the way taken is no slower at any share of valid keys measured.)

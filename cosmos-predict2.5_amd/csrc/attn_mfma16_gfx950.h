@@ -4,8 +4,9 @@
 //
 // Why, and where.  A product is issued in half the cycles, two of them in the place of one v_mfma_f32_32x32x16: the VALU work between them comes in smaller
 // pieces, and accumulators are read and written half as often.  It pays where three wavefronts share a SIMD or steps are long, and costs the issue of the second
-// product (4 cycles in 32) where that is what bounds.  Measured, us, 32x32x16 / 16x16x32, 16 heads: forward only, 384 rows a workgroup, 37440 positions 8840 / 8410,
-// 17600 2015 / 1925, 8800 553 / 529; stream with all tangents, 512 keys, 37440 queries 508 / 474, 17600 245 / 228, 8800 138 / 132, 3520 66.7 / 66.6.  Not here, as it was no faster:
+// product (4 cycles in 32) where that is what bounds.  Measured in turn on one card, us, 32x32x16 / 16x16x32, 16 heads: forward only, 384 rows a workgroup,
+// 37440 positions 8832 / 8699 (two runs of one side differ by 1.2 %), 24640 3864 / 3795, 17600 2002 / 1945, 8800 543 / 528, 40 heads 9360 1491 / 1476; stream with all tangents, 512 keys, 37440
+// queries 519 / 486, 17600 247 / 231, 8800 139 / 132, 3520 66.7 / 66.6.  Not here, as it was no faster:
 // the stream forward only (37440 213 / 222, 8800 61 / 63) and with a tangent on q (338 / 366), attn_fwd_jvp_kernel (37440 25950 / 25750, 17600 5830 / 5820, 704, K and V
 // in place, 32.5 / 34.5), forward only with 128 and 256 rows a workgroup (1560 40.2 / 42.1), head dims below 128 (fewer products to a softmax).
 //

@@ -104,8 +104,8 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
 COSMOS_ATTN_API int cosmos_attn_set_forward_override(int query_rows, int key_ranges);
 
 /*
- * Bytes of device workspace the call needs (K, V and their tangents re-tiled into the
- * kernel's LDS image).  0 on invalid descriptors.  The host allocates it however it likes
+ * Bytes of device workspace the call is to be given: K, V and their tangents re-tiled into the kernel's LDS image, and partial
+ * results where keys are cut.  (Asked for also of calls that then read K and V in place and leave the image's part untouched.)  0 on invalid descriptors.  The host allocates it however it likes
  * (the Python host uses torch's caching allocator) and may reuse it across calls on one stream.
  * No counterpart in the reference (Triton reads K/V in place).
  */
@@ -128,7 +128,8 @@ COSMOS_ATTN_API int cosmos_attn_launch_plan(const cosmos_attn_desc *desc, size_t
  * Forward only when all tangent pointers are NULL.
  * Replaces `_attention.forward` -> `_attn_fwd[grid](...)`  (JVP:436-502, JVP:176-378) and, forward only,
  * the SDPA / FA3 call of `attention()` (ATT:119-127, ATT:170-178).
- * Launches the re-tiling kernel and the attention kernel on `stream`; returns a status code.
+ * Launches the attention kernel on `stream`, in front of it the re-tiling kernel (but for short calls at head dim 128, which read
+ * K and V where they are), behind it a merging one where keys are cut; returns a status code.
  */
 COSMOS_ATTN_API int cosmos_attn_fwd_jvp(const cosmos_attn_desc *desc, void *workspace, size_t workspace_bytes, void *stream);
 
@@ -192,7 +193,8 @@ typedef struct cosmos_attn_bwd_desc {
     int64_t dq_stride[3], dk_stride[3], dv_stride[3];
 } cosmos_attn_bwd_desc;
 
-/* Bytes of device workspace `cosmos_attn_bwd` needs (per-row statistics and the re-tiled query and key streams). */
+/* Bytes of device workspace `cosmos_attn_bwd` is to be given (per-row statistics, the re-tiled query and key streams, kept dS, partial results).  At head dim 128 the
+ * query stream's part is room for a copy of q and dout, made only of rows that cannot be read where they are. */
 COSMOS_ATTN_API size_t cosmos_attn_bwd_workspace_bytes(const cosmos_attn_bwd_desc *desc);
 
 /* dq, dk, dv from dout.  Asynchronous on `stream`, no atomics (bitwise reproducible); returns a status code. */
