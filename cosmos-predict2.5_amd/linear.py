@@ -103,7 +103,8 @@ class _LinearFn(torch.autograd.Function):
         # (grad mode: the gradients are differentiated again.  Hooks on saved tensors may bring them back as something else, or in another layout)
         saved = ([x2] if wanted else []) + (w if of_x else [])
         like = g2[given[0]]
-        own = not torch.is_grad_enabled() and not _watched() and _memory_says_all(*saved, *(dy[i] for i in given)) and all(t.dtype == like.dtype and t.device == like.device for t in saved)
+        as_saved = (not wanted or x.shape == ctx.x_shape) and all(t.dtype == like.dtype and t.device == like.device for t in saved) and (not of_x or all(v.shape == (cols, depth) for v in w))
+        own = as_saved and not torch.is_grad_enabled() and not _watched() and _memory_says_all(*saved, *(dy[i] for i in given))
         rows = like.shape[0]
         if own:
             g2 = {i: ops._dense16(g) for i, g in g2.items()}

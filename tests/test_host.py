@@ -848,6 +848,19 @@ def test_layer_gradients_of_saved_tensors_that_come_back_in_another_layout(pkg, 
     assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(ys, [x, *w], dy), want))
 
 
+@pytest.mark.parametrize("what", ["rows", "columns", "dtype"])
+def test_layer_gradients_of_saved_tensors_that_come_back_as_others_are_torch_s_errors(pkg, gemm_by_address, what):
+    """Nothing is launched with the sizes of tensors that are not there."""
+    from sys import modules
+    linear_fn = modules[pkg.__name__ + ".linear"]._LinearFn
+    x, w, dy, _ = _layer_inputs()
+    other = {"rows": lambda t: t[:-1], "columns": lambda t: t[:, :-1], "dtype": lambda t: t.float()}[what]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach(), other):
+        ys = linear_fn.apply(None, x, *w)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(ys, [x, *w], dy)
+
+
 def test_products_that_are_only_asked_for_if_preferred_are_not_refused(pkg, monkeypatch):
     """A column of rows is contiguous with any stride between its single elements: None, for the caller's own product, and no error."""
     monkeypatch.setattr(pkg.ops, "_check_elementwise", lambda x: None)      # (nothing is launched: CPU tensors do)
