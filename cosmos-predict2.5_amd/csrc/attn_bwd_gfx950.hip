@@ -15,7 +15,7 @@
 //       scores  Sq = Q k^T,  dPq = dO v^T  (rows = streamed queries, columns = own keys),
 //       U = P, W = dS as 16-bit B operands,   dV^T += dO^T U,   dK^T += Q^T W.
 //     LSE and D vary along the streamed rows; they travel with the stream as one extra fragment per tile.
-//     Head dim 128: attn_dkdv_quad_kernel (four roles per 64 keys, attn_bwd_quad_gfx950.h), which can also keep every dS tile
+//     Head dim 128: attn_dkdv_kernel (wavefronts that do all of it for their keys, attn_bwd_dkdv_gfx950.h), which can also keep every dS tile
 //     in memory; other head dims: attn_bwd_kernel<T, D, KIND_DKDV> (score wavefront + output wavefront per 32 keys).
 //   * dQ from kept dS (head dim 128, when the workspace budget allows): attn_dq_from_ds_kernel streams the 16-bit dS tiles
 //     back once, dQ^T += K^T W with W = dS^T -- five matrix products per call in all, as the reference counts them.
@@ -115,11 +115,11 @@ __global__ void __launch_bounds__(kPackThreads) bwd_stats_kernel(const StatsPara
 }
 
 // ---------------------------------------------------------------------------------------------- stream re-tiling
-// Order of the 16-byte units (row r, chunk C of 8 channels) of a stream part of attn_dkdv_quad_kernel in LDS: read with ds_read_b128
-// (lane = row) and with transposing reads (ds_read_b64_tr_b16) without bank conflicts, and filled four whole rows a load (attn_bwd_quad_gfx950.h).
-__host__ __device__ constexpr int quad_swizzle(int r4) { return ((r4 ^ r4 >> 1) & 1) * 2 + (r4 >> 1 & 1); }
-__host__ __device__ constexpr int quad_unit_slot(int r, int C) {
-    return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ quad_swizzle(r >> 2));
+// Order of the 16-byte units (row r, chunk C of 8 channels) of a stream part of attn_dkdv_kernel in LDS: read with ds_read_b128
+// (lane = row) and with transposing reads (ds_read_b64_tr_b16) without bank conflicts, and filled four whole rows a load (attn_bwd_dkdv_gfx950.h).
+__host__ __device__ constexpr int part_swizzle(int r4) { return ((r4 ^ r4 >> 1) & 1) * 2 + (r4 >> 1 & 1); }
+__host__ __device__ constexpr int part_unit_slot(int r, int C) {
+    return 64 * (r >> 2) + 16 * (C >> 2) + 4 * (r & 3) + ((C & 3) ^ part_swizzle(r >> 2));
 }
 
 struct PackSrc { const uint16_t* ptr; int64_t sb, sh, sl; };
@@ -182,20 +182,20 @@ __global__ void __launch_bounds__(kPackThreads) pack_stream_kernel(const PackBwd
     }
 }
 
-// What attn_dkdv_quad_kernel streams beside Q and dO (head dim 128): per tile of 32 queries 32 values LSE log2 e, then 32 negated row sums dout . o.  With COPY also
+// What attn_dkdv_kernel streams beside Q and dO (head dim 128): per tile of 32 queries 32 values LSE log2 e, then 32 negated row sums dout . o.  With COPY also
 // rows of q and dout, one behind the other, for a call whose own rows the kernel does not read.  HBM-bound; eight threads per row, two 16-byte units of each tensor
 // per thread, rows read whole.  grid (n_tiles, B*H).
-constexpr int kQuadStatBytes = 2 * kRows * (int)sizeof(float);
-struct QuadStatsParams {
+constexpr int kTileStatBytes = 2 * kRows * (int)sizeof(float);
+struct TileStatsParams {
     PackSrc q, g, o;             // q, dout, o
     const float* lse;            // [B,H,L]
     float2* stats;               // [B*H][L] : (LSE log2 e, D); null: nobody reads it
-    char* tile_stats;            // [B*H][n_tiles][kQuadStatBytes]
+    char* tile_stats;            // [B*H][n_tiles][kTileStatBytes]
     uint4 *q_rows, *g_rows;      // COPY: [B*H][32 n_tiles][16 units]
     int H, L, n_tiles;
 };
 template <bool BF16, bool COPY>
-__global__ void __launch_bounds__(kPackThreads) quad_stats_kernel(const QuadStatsParams p) {
+__global__ void __launch_bounds__(kPackThreads) tile_stats_kernel(const TileStatsParams p) {
     static_assert(kPackThreads == 8 * kRows, "eight threads per row of a tile");
     const int bh = blockIdx.y, b = bh / p.H, h = bh % p.H, t = blockIdx.x;
     const int r = threadIdx.x >> 3, part = threadIdx.x & 7, row = t * kRows + r;
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(kPackThreads) quad_stats_kernel(const QuadStat
     if (part == 0) {
         if (live && p.stats) p.stats[(int64_t)bh * p.L + row] = make_float2(lse, acc);
         // 32 LSE values, then 32 D values, negated: they start the sums of dP
-        float* st = reinterpret_cast<float*>(p.tile_stats + ((size_t)bh * p.n_tiles + t) * kQuadStatBytes);
+        float* st = reinterpret_cast<float*>(p.tile_stats + ((size_t)bh * p.n_tiles + t) * kTileStatBytes);
         st[r] = lse;
         st[32 + r] = -acc;
     }
@@ -251,21 +251,21 @@ __global__ void __launch_bounds__(kPackThreads) pack_kt_kernel(const PackSrc k, 
 }
 
 // ---------------------------------------------------------------------------------------------- main kernels
-struct QuadRows { const char* ptr; int64_t sb, sh; int row; };   // bytes between batches, heads, rows
+struct StreamRows { const char* ptr; int64_t sb, sh; int row; };   // bytes between batches, heads, rows
 struct BwdParams {
     const void *st1, *st2;             // stationary operands: rows of (q, dout) for dQ, of (k, v) for dK/dV
     int64_t s1_sb, s1_sh, s1_sl, s2_sb, s2_sh, s2_sl;
     void *out1, *out2;                 // dq | dv, dk
     int64_t o1_sb, o1_sh, o1_sl, o2_sb, o2_sh, o2_sl;
     const float2* stats;               // [B*H][Lq]
-    const char* stream;                // packed stream tiles [B*H][n_tiles][tile bytes]; attn_dkdv_quad_kernel: their statistics alone
-    QuadRows rows_q, rows_do;          // attn_dkdv_quad_kernel: Q and dO
+    const char* stream;                // packed stream tiles [B*H][n_tiles][tile bytes]; attn_dkdv_kernel: their statistics alone
+    StreamRows rows_q, rows_do;          // attn_dkdv_kernel: Q and dO
     int H, L_stat, L_stream, n_tiles, causal;
     float sm_scale, scale_log2;
     // 1-D grid: workgroups [0, n_full) each own a (block of 128 stationary rows, head) pair; the remaining n_rem pairs
     // are cut into `splits` ranges of the stream, one workgroup each, which leave fp32 partial sums for bwd_combine_kernel
-    int n_blk, n_full, n_rem, splits;
-    float* part;                       // [(pair - n_full) * splits + split][kBlock][D] (dQ) or [..][kBlock][2][D] (dV, dK)
+    int n_blk, n_full, n_rem, splits, block;      // block: stationary rows of a workgroup
+    float* part;                       // [(pair - n_full) * splits + split][block][D] (dQ) or [..][block][2][D] (dV, dK)
     // A launch serves the heads [bh0, bh0 + pairs / n_blk) of the call (one group of heads at a time when dS is kept).
     int bh0;
     // dK/dV kernel that keeps dS: every 32 x 32 tile of dS = P * (dP - D) it forms is also written, as the two 1 KB operand
@@ -622,7 +622,7 @@ attn_bwd_kernel(const BwdParams p) {
     }
 }
 
-#include "attn_bwd_quad_gfx950.h"
+#include "attn_bwd_dkdv_gfx950.h"
 
 // ---------------------------------------------------------------------------------------------- head dim 256
 // At d = 256 the stationary rows of a wavefront are 128 registers and its accumulators up to 256, and a stream tile is
@@ -759,15 +759,15 @@ __global__ void __launch_bounds__(256) bwd_combine_kernel(const BwdParams p, int
     const int tpr = D / 4;
     const int64_t r = (int64_t)blockIdx.x * (256 / tpr) + threadIdx.x / tpr;
     const int c = (threadIdx.x % tpr) * 4;
-    const int pair_i = (int)(r / kBlock), wrow = (int)(r % kBlock);
+    const int pair_i = (int)(r / p.block), wrow = (int)(r % p.block);
     const int pair = p.n_full + pair_i;
     const int blk = pair % p.n_blk, bh = p.bh0 + pair / p.n_blk, b = bh / p.H, h = bh % p.H;
-    const int row = blk * kBlock + wrow;
+    const int row = blk * p.block + wrow;
     if (pair_i >= p.n_rem || row >= p.L_stat) return;
     const int W = DKDV ? 2 * D : D;
     float4 a1 = make_float4(0.f, 0.f, 0.f, 0.f), a2 = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int i = 0; i < p.splits; ++i) {
-        const float* pa = p.part + (((int64_t)pair_i * p.splits + i) * kBlock + wrow) * W + c;
+        const float* pa = p.part + (((int64_t)pair_i * p.splits + i) * p.block + wrow) * W + c;
         const float4 x = *reinterpret_cast<const float4*>(pa);
         a1.x += x.x; a1.y += x.y; a1.z += x.z; a1.w += x.w;
         if (DKDV) {
@@ -815,6 +815,7 @@ struct DqFromDsParams {
     void* dq;
     int64_t o_sb, o_sh, o_sl;
     int H, Lq, Lkv, n_q_tiles, n_k_tiles, n_blk, bh0, heads, causal;      // heads: of this launch, from bh0 on
+    int block_tiles;                   // key tiles of a workgroup of the dK/dV kernel
     float sm_scale;
 };
 
@@ -912,7 +913,7 @@ attn_dq_from_ds_kernel(const DqFromDsParams p) {
         wf[0] = __builtin_shufflevector(__builtin_bit_cast(V4, t00), __builtin_bit_cast(V4, t01), 0, 1, 2, 3, 4, 5, 6, 7);
         wf[1] = __builtin_shufflevector(__builtin_bit_cast(V4, t10), __builtin_bit_cast(V4, t11), 0, 1, 2, 3, 4, 5, 6, 7);
         // dead operands become zeros: tiles the (causal) dK/dV kernel never formed, keys past the end of the last tile
-        const bool unformed = p.causal && (s / 4) * 4 > qt;
+        const bool unformed = p.causal && (s / p.block_tiles) * p.block_tiles > qt;
         if (unformed || !live_tile || s * kRows + kRows > p.Lkv) {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
@@ -978,26 +979,34 @@ typedef void (*dq_from_ds_kernel_t)(const DqFromDsParams);
 
 // Keeping dS pays where the two products it saves are large next to the 4 bytes per score element it moves: head dim 128.
 inline bool spill_head_dim(int d) { return d == 128; }
-// head dim 128: the four-role dK/dV kernel, with or without keeping dS (the other head dims: attn_bwd_kernel<T, D, KIND_DKDV>)
-template <typename T>
-bwd_kernel_t pick_dkdv_quad(int d, bool keep_ds) {
-    if (d != 128) return nullptr;
-    return keep_ds ? attn_dkdv_quad_kernel<T, 128, true> : attn_dkdv_quad_kernel<T, 128, false>;
+// head dim 128: attn_dkdv_kernel, with or without keeping dS (the other head dims: attn_bwd_kernel<T, D, KIND_DKDV>)
+template <typename T, int NG>
+bwd_kernel_t pick_dkdv_groups(bool keep_ds, bool causal) {
+    return keep_ds ? (causal ? attn_dkdv_kernel<T, NG, true, true> : attn_dkdv_kernel<T, NG, true, false>)
+                   : (causal ? attn_dkdv_kernel<T, NG, false, true> : attn_dkdv_kernel<T, NG, false, false>);
 }
-inline size_t dkdv_lds_bytes(int d, size_t two_role) { return d == 128 ? (size_t)QuadCfg<128>::LDS_BYTES : two_role; }
+template <typename T>
+bwd_kernel_t pick_dkdv(int groups, bool keep_ds, bool causal) {
+    return groups == 2 ? pick_dkdv_groups<T, 2>(keep_ds, causal) : groups == 3 ? pick_dkdv_groups<T, 3>(keep_ds, causal) : pick_dkdv_groups<T, 4>(keep_ds, causal);
+}
 template <typename T>
 dq_from_ds_kernel_t pick_dq_from_ds(int d) { return d == 128 ? attn_dq_from_ds_kernel<T, 128> : nullptr; }
 
 template <typename T, int KIND>
+bwd_kernel_t pick_bwd_128() {          // (dK, dV: pick_dkdv)
+    if constexpr (KIND == KIND_DQ) return attn_bwd_kernel<T, 128, KIND_DQ>;
+    return nullptr;
+}
+template <typename T, int KIND>
 bwd_kernel_t pick_bwd(int d) {
 #ifdef COSMOS_ATTN_ONLY_D128   // development builds: instantiate the d=128 kernels only
-    return d == 128 ? attn_bwd_kernel<T, 128, KIND> : nullptr;
+    return d == 128 ? pick_bwd_128<T, KIND>() : nullptr;
 #endif
     switch (d) {
         case 16: return attn_bwd_kernel<T, 16, KIND>;
         case 32: return attn_bwd_kernel<T, 32, KIND>;
         case 64: return attn_bwd_kernel<T, 64, KIND>;
-        case 128: return attn_bwd_kernel<T, 128, KIND>;
+        case 128: return pick_bwd_128<T, KIND>();
         default: return nullptr;
     }
 }
@@ -1009,8 +1018,8 @@ struct BwdGeom {
     size_t stats_bytes, q_img_bytes, k_img_bytes;
     explicit BwdGeom(const cosmos_attn_bwd_desc* d) {
         nc = d->d / 16; ndb = (d->d + 31) / 32;
-        quad = d->d == 128;   // attn_dkdv_quad_kernel: one copy of the query stream ([Q | dO | statistics])
-        q_tile_bytes = (size_t)(quad ? 2 * nc + 1 : 2 * nc + 4 * ndb + 1) * kFragBytes;
+        rows = d->d == 128;   // attn_dkdv_kernel: one copy of the query stream ([Q | dO | statistics])
+        q_tile_bytes = (size_t)(rows ? 2 * nc + 1 : 2 * nc + 4 * ndb + 1) * kFragBytes;
         k_tile_bytes = (size_t)(2 * nc + 2 * ndb) * kFragBytes;
         lds_dkdv = (size_t)kRingS * 2 * nc * kFragBytes + (size_t)kRingO * 4 * ndb * kFragBytes + 2 * 4 * 4 * kFragBytes + kRingStats * kFragBytes;
         lds_dq = (size_t)kRingS * 2 * nc * kFragBytes + (size_t)kRingO * 2 * ndb * kFragBytes + 2 * 4 * 2 * kFragBytes;
@@ -1020,17 +1029,30 @@ struct BwdGeom {
         q_img_bytes = bh * n_q_tiles * q_tile_bytes;
         k_img_bytes = bh * n_k_tiles * k_tile_bytes;
         if (d->d == 256) {   // attn_bwd_wide_kernel: blocks of 32 stationary rows, never cut
-            dkdv = Plan{(d->Lkv + kRows - 1) / kRows, (d->Lkv + kRows - 1) / kRows * (int)bh, (d->Lkv + kRows - 1) / kRows * (int)bh, 0, 1};
-            dq = Plan{(d->Lq + kRows - 1) / kRows, (d->Lq + kRows - 1) / kRows * (int)bh, (d->Lq + kRows - 1) / kRows * (int)bh, 0, 1};
+            dkdv = Plan{(d->Lkv + kRows - 1) / kRows, (d->Lkv + kRows - 1) / kRows * (int)bh, (d->Lkv + kRows - 1) / kRows * (int)bh, 0, 1, kRows};
+            dq = Plan{(d->Lq + kRows - 1) / kRows, (d->Lq + kRows - 1) / kRows * (int)bh, (d->Lq + kRows - 1) / kRows * (int)bh, 0, 1, kRows};
             part_bytes = 0;
             return;
         }
-        const int n_kblk = (d->Lkv + kBlock - 1) / kBlock;
+        int block = kBlock;
+        const int64_t budget = d->max_ds_mib < 0 ? 0 : (int64_t)(d->max_ds_mib > 0 ? d->max_ds_mib : kDefaultDsMiB) << 20;
+        if (rows) {      // keys of a workgroup of attn_dkdv_kernel: the least estimate for all heads at once
+            double least = 0.0;
+            bool least_fits = false;
+            for (int i = 2; i <= 4; ++i) {
+                const int blocks = (d->Lkv + 64 * i - 1) / (64 * i);
+                const bool fits = (int64_t)n_q_tiles * blocks * 2 * i * 2 * kFragBytes <= budget;      // a head's dS (padded keys are in it)
+                const double us = plan(blocks, (int)bh, n_q_tiles, d->causal != 0, d->d, true, 64 * i, dkdv_cost(i)).us;
+                if (i == 2 || (fits && !least_fits) || (fits == least_fits && us < least)) { least = us; least_fits = fits; groups = i; }
+            }
+            block = 64 * groups;
+        }
+        const StepCost cost = rows ? dkdv_cost(groups) : recompute_cost(d->d);
+        const int n_kblk = (d->Lkv + block - 1) / block;
         // Keep dS?  Its tiles for one head take n_q_tiles * n_kt_pad * 2 KB; heads are served in groups that fit the budget
         // (desc->max_ds_mib: 0 = kDefaultDsMiB, > 0 = that many MiB, < 0 = never keep dS).
-        n_kt_pad = 4 * n_kblk;
+        n_kt_pad = block / kRows * n_kblk;
         ds_head_bytes = (size_t)n_q_tiles * n_kt_pad * 2 * kFragBytes;
-        const int64_t budget = d->max_ds_mib < 0 ? 0 : (int64_t)(d->max_ds_mib > 0 ? d->max_ds_mib : kDefaultDsMiB) << 20;
         if (spill_head_dim(d->d) && (int64_t)ds_head_bytes <= budget && (int64_t)n_kt_pad * 2 * kFragBytes < ((int64_t)1 << 31)) {
             spill = true;
             const int64_t fit = budget / (int64_t)ds_head_bytes;
@@ -1039,31 +1061,39 @@ struct BwdGeom {
             k_tile_bytes = (size_t)(2 * ndb) * kFragBytes;            // the key stream holds K^T alone
             k_img_bytes = bh * n_k_tiles * k_tile_bytes;
         }
-        dkdv = plan(n_kblk, spill ? group : (int)bh, n_q_tiles, d->causal != 0, d->d, true);
-        dq = plan((d->Lq + kBlock - 1) / kBlock, (int)bh, n_k_tiles, d->causal != 0, d->d, false);
-        size_t p1 = (size_t)dkdv.n_rem * dkdv.splits * kBlock * 2 * d->d * sizeof(float);
+        dkdv = plan(n_kblk, spill ? group : (int)bh, n_q_tiles, d->causal != 0, d->d, true, block, cost);
+        dq = plan((d->Lq + kBlock - 1) / kBlock, (int)bh, n_k_tiles, d->causal != 0, d->d, false, kBlock, recompute_cost(d->d));
+        size_t p1 = (size_t)dkdv.n_rem * dkdv.splits * block * 2 * d->d * sizeof(float);
         if (spill && bh % group) {   // the last, smaller group has a plan of its own
-            const Plan last = plan(n_kblk, (int)(bh % group), n_q_tiles, d->causal != 0, d->d, true);
-            const size_t p3 = (size_t)last.n_rem * last.splits * kBlock * 2 * d->d * sizeof(float);
+            const Plan last = plan(n_kblk, (int)(bh % group), n_q_tiles, d->causal != 0, d->d, true, block, cost);
+            const size_t p3 = (size_t)last.n_rem * last.splits * block * 2 * d->d * sizeof(float);
             p1 = p1 > p3 ? p1 : p3;
         }
         const size_t p2 = spill ? 0 : (size_t)dq.n_rem * dq.splits * kBlock * d->d * sizeof(float);
         part_bytes = ((p1 > p2 ? p1 : p2) + 1023) / 1024 * 1024;     // the two kernels run one after the other
     }
     static constexpr int kDefaultDsMiB = 32 * 1024;
-    bool quad = false;
+    bool rows = false;
+    int groups = 0;                     // of 16 keys of a wavefront of attn_dkdv_kernel
     bool spill = false;
     int group = 0, n_kt_pad = 0;        // heads per group; key tiles per query tile in the dS buffer
     size_t ds_head_bytes = 0, ds_bytes = 0;
     // How the (block of stationary rows, head) pairs of a kernel are dealt out (see choose_splits): the pairs of a partly
     // filled last round of workgroups are cut along the stream and bwd_combine_kernel adds the ranges up.
-    struct Plan { int n_blk, n_pairs, n_full, n_rem, splits; };
-    static Plan plan(int n_blk, int bh, int n_stream_tiles, bool causal, int d, bool dkdv) {
+    struct Plan { int n_blk, n_pairs, n_full, n_rem, splits, block; double us = 0.0; };      // us: estimated time
+    // A barrier step (32 stream rows) in full rounds and in a few workgroups, and what a workgroup costs besides: see StepCost.  attn_dkdv_kernel, by groups of 16 keys of a
+    // wavefront: more keys are less LDS traffic and, per key, fewer instructions; fewer keys are more workgroups and less padding.  Fits to 24 sizes of 255 .. 84480 queries
+    // x 64 .. 10920 keys, B*H = 16 .. 80, with 2, 3 and 4 groups and S = 1 .. 16 measured: the choice takes 1.001 times the best one's time on average, 1.02 at most
+    // (us of a backward pass, 4 / 3 / 2 groups: 16 heads 37440 x 512 515 / 575 / 547, 37440 x 300 460 / 422 / 459, 1560 x 1560 113 / 111 / 100, 10920 x 10920 2410 / 2460 / 2630).
+    static StepCost dkdv_cost(int groups) { return groups == 4 ? StepCost{1.78, 8.0, 0.64} : groups == 3 ? StepCost{1.42, 8.0, 0.65} : StepCost{1.04, 8.0, 0.69}; }
+    static StepCost recompute_cost(int d) { return StepCost{1.08 * (0.3 + 0.7 * d / 128.0), 8.0}; }
+    static Plan plan(int n_blk, int bh, int n_stream_tiles, bool causal, int d, bool dkdv, int block, StepCost cost) {
         Plan s;
-        s.n_blk = n_blk; s.n_pairs = n_blk * bh; s.n_full = s.n_pairs; s.n_rem = 0; s.splits = 1;
+        s.block = block; s.n_blk = n_blk; s.n_pairs = n_blk * bh; s.n_full = s.n_pairs; s.n_rem = 0; s.splits = 1;
         const int rem = s.n_pairs % kNumCUs;
-        const double part = 0.3 + 0.7 * d / 128.0;
-        const int splits = causal ? 1 : choose_splits(rem, n_stream_tiles, StepCost{1.08 * part, 8.0}, (double)kBlock * (dkdv ? 2 : 1) * d * sizeof(float));
+        const double full_us = rounds_cost(s.n_pairs - rem, n_stream_tiles, cost), slot_bytes = (double)block * (dkdv ? 2 : 1) * d * sizeof(float);
+        const int splits = causal ? 1 : choose_splits(rem, n_stream_tiles, cost, slot_bytes);
+        s.us = full_us + split_cost(rem, n_stream_tiles, splits, cost, slot_bytes);
         if (splits < 2) return s;
         s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = splits;
         return s;
@@ -1091,10 +1121,10 @@ int validate_bwd(const cosmos_attn_bwd_desc* d) {
     return COSMOS_ATTN_OK;
 }
 
-// Does attn_dkdv_quad_kernel read Q and dO where they are?  It addresses a head's rows with 31-bit offsets, and rows past the end have to lie past the buffer.  Where
+// Does attn_dkdv_kernel read Q and dO where they are?  It addresses a head's rows with 31-bit offsets, and rows past the end have to lie past the buffer.  Where
 // it can it does: a row's 256 bytes are whole cache lines wherever they lie, and a copy is two more passes over both.  Backward, us, copied / in place (bf16, rows 4 KB
 // apart): 16 heads x 37440 queries x 512 keys 654 / 578, 84480 x 300 1200 / 985, 3520 x 512 86 / 80, 1560 x 1560 107 / 104, 17600 x 17600 6983 / 6958.
-bool quad_in_place(const cosmos_attn_bwd_desc* d) {
+bool rows_in_place(const cosmos_attn_bwd_desc* d) {
     const int64_t n = (int64_t)(d->Lq + kRows - 1) / kRows * kRows;
     auto addressed = [&](const int64_t* s) { return s[2] >= d->d && s[2] * 2 <= ((int64_t)1 << 31) / n - 1; };
     return addressed(d->q_stride) && addressed(d->dout_stride);
@@ -1122,8 +1152,8 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
     const bool bf16 = d->dtype == COSMOS_ATTN_BF16;
     const bool wide = d->d == 256;
     bwd_kernel_t k_dkdv = bf16 ? pick_bwd<__bf16, KIND_DKDV>(d->d) : pick_bwd<_Float16, KIND_DKDV>(d->d);
-    if (bwd_kernel_t quad = bf16 ? pick_dkdv_quad<__bf16>(d->d, false) : pick_dkdv_quad<_Float16>(d->d, false)) k_dkdv = quad;
-    const size_t lds_dkdv = dkdv_lds_bytes(d->d, g.lds_dkdv);
+    if (g.rows) k_dkdv = bf16 ? pick_dkdv<__bf16>(g.groups, g.spill, d->causal != 0) : pick_dkdv<_Float16>(g.groups, g.spill, d->causal != 0);
+    const size_t lds_dkdv = g.rows ? (size_t)kDkdvLdsBytes : g.lds_dkdv;
     bwd_kernel_t k_dq = bf16 ? pick_bwd<__bf16, KIND_DQ>(d->d) : pick_bwd<_Float16, KIND_DQ>(d->d);
     if (!wide && (!k_dkdv || !k_dq)) return COSMOS_ATTN_UNSUPPORTED;
     char* ws = (char*)workspace;
@@ -1134,7 +1164,7 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
     char* ds = (char*)part + g.part_bytes;
     const int BH = d->B * d->H;
     auto launch = [&](bwd_kernel_t fn, size_t lds, const BwdGeom::Plan& pl, BwdParams& bp, bool is_dkdv) {
-        bp.n_blk = pl.n_blk; bp.n_full = pl.n_full; bp.n_rem = pl.n_rem; bp.splits = pl.splits; bp.part = part;
+        bp.n_blk = pl.n_blk; bp.n_full = pl.n_full; bp.n_rem = pl.n_rem; bp.splits = pl.splits; bp.block = pl.block; bp.part = part;
         if (wide) {
             auto wfn = is_dkdv ? (bf16 ? attn_bwd_wide_kernel<__bf16, KIND_DKDV> : attn_bwd_wide_kernel<_Float16, KIND_DKDV>)
                                : (bf16 ? attn_bwd_wide_kernel<__bf16, KIND_DQ> : attn_bwd_wide_kernel<_Float16, KIND_DQ>);
@@ -1142,10 +1172,10 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
             return true;
         }
         if (!allow_lds((const void*)fn, lds)) return false;
-        hipLaunchKernelGGL(fn, dim3((unsigned)(pl.n_full + pl.n_rem * pl.splits)), dim3(kBwdThreads), lds, stream, bp);
+        hipLaunchKernelGGL(fn, dim3((unsigned)(pl.n_full + pl.n_rem * pl.splits)), dim3(is_dkdv && g.rows ? kDkdvThreads : kBwdThreads), lds, stream, bp);
         if (pl.splits > 1) {
             const int rows_per_block = 256 / (d->d / 4);
-            const dim3 cgrid((unsigned)(((int64_t)pl.n_rem * kBlock + rows_per_block - 1) / rows_per_block));
+            const dim3 cgrid((unsigned)(((int64_t)pl.n_rem * pl.block + rows_per_block - 1) / rows_per_block));
             auto cfn = is_dkdv ? (bf16 ? bwd_combine_kernel<__bf16, true> : bwd_combine_kernel<_Float16, true>)
                                : (bf16 ? bwd_combine_kernel<__bf16, false> : bwd_combine_kernel<_Float16, false>);
             hipLaunchKernelGGL(cfn, cgrid, dim3(256), 0, stream, bp, d->d);
@@ -1154,18 +1184,18 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
     };
 
     BwdParams bp{};
-    if (g.quad) {   // query stream of attn_dkdv_quad_kernel: Q and dO where they are, statistics
-        const bool copy = !quad_in_place(d);
+    if (g.rows) {   // query stream of attn_dkdv_kernel: Q and dO where they are, statistics
+        const bool copy = !rows_in_place(d);
         const size_t rows_bytes = (size_t)BH * g.n_q_tiles * kRows * 256;
-        QuadStatsParams pp;
+        TileStatsParams pp;
         pp.q = src_of(d->q, d->q_stride); pp.g = src_of(d->dout, d->dout_stride); pp.o = src_of(d->o, d->o_stride);
         pp.q_rows = (uint4*)q_img; pp.g_rows = (uint4*)(q_img + rows_bytes); pp.tile_stats = q_img + 2 * rows_bytes;
         pp.lse = d->lse; pp.stats = g.spill ? nullptr : stats; pp.H = d->H; pp.L = d->Lq; pp.n_tiles = g.n_q_tiles;
-        auto fn = bf16 ? (copy ? quad_stats_kernel<true, true> : quad_stats_kernel<true, false>) : (copy ? quad_stats_kernel<false, true> : quad_stats_kernel<false, false>);
+        auto fn = bf16 ? (copy ? tile_stats_kernel<true, true> : tile_stats_kernel<true, false>) : (copy ? tile_stats_kernel<false, true> : tile_stats_kernel<false, false>);
         hipLaunchKernelGGL(fn, dim3(g.n_q_tiles, BH), dim3(kPackThreads), 0, stream, pp);
         auto rows = [&](const void* ptr, const int64_t* s, const uint4* copied) {
             const int64_t head = (int64_t)g.n_q_tiles * kRows * 256;
-            return copy ? QuadRows{(const char*)copied, d->H * head, head, 256} : QuadRows{(const char*)ptr, 2 * s[0], 2 * s[1], (int)(2 * s[2])};
+            return copy ? StreamRows{(const char*)copied, d->H * head, head, 256} : StreamRows{(const char*)ptr, 2 * s[0], 2 * s[1], (int)(2 * s[2])};
         };
         bp.rows_q = rows(d->q, d->q_stride, pp.q_rows); bp.rows_do = rows(d->dout, d->dout_stride, pp.g_rows);
         q_img = pp.tile_stats;
@@ -1216,9 +1246,8 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
     };
     if (g.spill) {
         // dS kept: per group of heads, the dK/dV kernel (which writes the group's dS tiles), then the pass that turns them into dQ
-        bwd_kernel_t k_spill = bf16 ? pick_dkdv_quad<__bf16>(d->d, true) : pick_dkdv_quad<_Float16>(d->d, true);
         dq_from_ds_kernel_t k_ds = bf16 ? pick_dq_from_ds<__bf16>(d->d) : pick_dq_from_ds<_Float16>(d->d);
-        if (!k_spill || !k_ds) return COSMOS_ATTN_UNSUPPORTED;
+        if (!k_ds) return COSMOS_ATTN_UNSUPPORTED;
         const size_t lds_ds = (size_t)kDsRing * (kDqWaves * 2 * kFragBytes + 2 * g.ndb * kFragBytes);
         if (!allow_lds((const void*)k_ds, lds_ds)) return COSMOS_ATTN_LAUNCH_FAILED;
         set_dkdv();
@@ -1227,12 +1256,12 @@ COSMOS_ATTN_API int cosmos_attn_bwd(const cosmos_attn_bwd_desc* d, void* workspa
         qp.ds = ds; qp.ds_head_bytes = (int64_t)g.ds_head_bytes; qp.n_kt_pad = g.n_kt_pad; qp.kt_img = k_img;
         qp.dq = d->dq; qp.o_sb = d->dq_stride[0]; qp.o_sh = d->dq_stride[1]; qp.o_sl = d->dq_stride[2];
         qp.H = d->H; qp.Lq = d->Lq; qp.Lkv = d->Lkv; qp.n_q_tiles = g.n_q_tiles; qp.n_k_tiles = g.n_k_tiles;
-        qp.n_blk = (g.n_q_tiles + kDqWaves - 1) / kDqWaves; qp.causal = d->causal; qp.sm_scale = d->sm_scale;
+        qp.n_blk = (g.n_q_tiles + kDqWaves - 1) / kDqWaves; qp.causal = d->causal; qp.block_tiles = g.dkdv.block / kRows; qp.sm_scale = d->sm_scale;
         for (int bh0 = 0; bh0 < BH; bh0 += g.group) {
             const int heads = BH - bh0 < g.group ? BH - bh0 : g.group;
-            const BwdGeom::Plan pl = heads == g.group ? g.dkdv : BwdGeom::plan(g.dkdv.n_blk, heads, g.n_q_tiles, d->causal != 0, d->d, true);
+            const BwdGeom::Plan pl = heads == g.group ? g.dkdv : BwdGeom::plan(g.dkdv.n_blk, heads, g.n_q_tiles, d->causal != 0, d->d, true, g.dkdv.block, BwdGeom::dkdv_cost(g.groups));
             bp.bh0 = bh0;
-            if (!launch(k_spill, lds_dkdv, pl, bp, true)) return COSMOS_ATTN_LAUNCH_FAILED;
+            if (!launch(k_dkdv, lds_dkdv, pl, bp, true)) return COSMOS_ATTN_LAUNCH_FAILED;
             qp.bh0 = bh0; qp.heads = heads;
             const int items = qp.n_blk * heads, grid = !d->causal && items > kNumCUs ? kNumCUs : items;
             hipLaunchKernelGGL(k_ds, dim3((unsigned)grid), dim3(kDqThreads), lds_ds, stream, qp);

@@ -10,6 +10,11 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
+// f(Int<0>{}) ... f(Int<N - 1>{})
+template <int I> struct Int { static constexpr int value = I; };
+template <typename F, int... I> __device__ __forceinline__ void for_each_of(F&& f, std::integer_sequence<int, I...>) { (f(Int<I>{}), ...); }
+template <int N, typename F> __device__ __forceinline__ void for_each(F&& f) { for_each_of(f, std::make_integer_sequence<int, N>{}); }
+
 template <typename T> struct VecOf;
 template <> struct VecOf<__bf16> { typedef bf16x8 v8; typedef bf16x4 v4; };
 template <> struct VecOf<_Float16> { typedef f16x8 v8; typedef f16x4 v4; };

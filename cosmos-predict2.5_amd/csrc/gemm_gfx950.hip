@@ -37,10 +37,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-template <int I> struct Int { static constexpr int value = I; };
-template <typename F, int... I> __device__ __forceinline__ void for_each_of(F&& f, std::integer_sequence<int, I...>) { (f(Int<I>{}), ...); }
-template <int N, typename F> __device__ __forceinline__ void for_each(F&& f) { for_each_of(f, std::make_integer_sequence<int, N>{}); }
-
 constexpr int kStep = 64;            // contraction indexes per step
 constexpr int kTileGroup = 8;        // rows of tiles that are served together
 constexpr int kMostProducts = 3;

@@ -140,6 +140,30 @@ def test_bwd_at_the_edges_of_16(pkg, oracle, gpu, Lq, Lkv, causal, dtype):
     run_bwd(pkg, oracle, gpu, (2, 3, Lq, 128), (2, 3, Lkv, 128), causal=causal, seed=Lq, dtype=dtype)
 
 
+@pytest.mark.parametrize("Lkv", [4097, 6144, 6145, 8191])
+@pytest.mark.parametrize("Lq", [1, 33, 230])
+def test_bwd_workgroups_of_192_and_256_keys(pkg, oracle, gpu, Lkv, Lq):
+    """Workgroups of 192 keys (8 heads, up to 6144 keys) and of 256 (more): one query tile, two, and more than the seven that LDS holds; last workgroups that are
+    filled, that hold one key, and that lack one (same tolerances)."""
+    run_bwd(pkg, oracle, gpu, (1, 8, Lq, 128), (1, 8, Lkv, 128), seed=Lq + Lkv, dtype=torch.float16 if Lq == 33 else torch.bfloat16)
+
+
+@pytest.mark.parametrize("shape, keys, causal", [((2, 40, 700, 128), 700, True), ((1, 64, 760, 128), 760, True), ((1, 16, 20000, 128), 510, False), ((1, 16, 8000, 128), 192, False)])
+@pytest.mark.parametrize("max_ds_mib", [None, -1])
+def test_bwd_heads_of_larger_calls(pkg, oracle, gpu, shape, keys, causal, max_ds_mib):
+    """Workgroups of 256, 192, 256 and 192 keys: the diagonal through them, and queries cut into ranges; dS kept and not.  The first, the last and one other head against the
+    oracle (heads are independent; same tolerances)."""
+    q, k, v, _, _, _ = oracle.make_inputs(shape, (*shape[:2], keys, 128), seed=9)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(10)).to(torch.bfloat16)
+    qd, kd, vd, dd = (x.to(gpu) for x in (q, k, v, dout))
+    o, _, lse = pkg.attention_with_lse(qd, kd, vd, causal=causal)
+    got = pkg.ops.bwd(qd, kd, vd, o, lse, dd, causal=causal, max_ds_mib=max_ds_mib)
+    for h in (0, 7, shape[1] - 1):
+        one = lambda x: x[-1:, h:h + 1]
+        for name, a, ref in zip(("dq", "dk", "dv"), got, oracle.grads_closed_form(one(q), one(k), one(v), one(dout), causal=causal)):
+            check(oracle, f"head {h} {name}", one(a), ref)
+
+
 @pytest.mark.parametrize("Lq", [1, 32, 45, 300])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("which", ["q", "dout", "far"])
