@@ -340,8 +340,9 @@ attn_dkdv_kernel(const BwdParams p) {
         int s = 0;
 #pragma clang loop unroll(disable)
         do step(); while (++s < n);
-        // what is left of the last tile: its dS, dK
+        // what is left of the last tile: its dS, dK.  (What was read ahead is not used, but its registers are not anybody's before it is here.)
         wait_lds<0>();
+        for_each<3>([&](auto i) { group_landed(i); });
         for_each<DS_OPS - ds_before(SLOTS)>([&](auto i) { ds_op(Int<ds_before(SLOTS) + decltype(i)::value>{}); });
         if constexpr (SPILL) for_each<NG>([&](auto i) { store_ds(i); });
         SCHED_FENCE();
