@@ -152,7 +152,7 @@ struct AttnParams {
     float sm_scale, scale_log2;
     // 1-D grid: workgroups [0, n_full) each own a (query block, head) pair; the remaining n_rem pairs are cut into
     // `splits` key ranges, one workgroup each, which leave unnormalised partial results for attn_combine_kernel.
-    // slot = (pair - n_full) * splits + split; block_m = query rows per workgroup (128; forward only 128, 256 or 384)
+    // slot = (pair - n_full) * splits + split; block_m = query rows per workgroup (128; forward only 128, 256 or 384; attn_jvp_rows_kernel 192)
     int n_qt, n_full, n_rem, splits;
     // attn_qstream_kernel: BH = batch * heads (the kernel deals the (query block, head) pairs out over its workgroups itself)
     int BH, q_chunk;
@@ -492,6 +492,7 @@ struct OutputWave {
 };
 
 #include "attn_mfma16_gfx950.h"
+#include "attn_jvp_rows_gfx950.h"
 
 template <typename T, int DQK, int DV, int MODE, bool RAW>
 __global__ void __attribute__((amdgpu_flat_work_group_size(kAttnThreads, kAttnThreads), amdgpu_waves_per_eu(2, 2)))
@@ -1761,12 +1762,13 @@ constexpr SymShape kSymShapes[] = {
 constexpr int kSymStepTiles = 2;      // tiles of 32 keys per barrier step (SymCfg::TPS)
 constexpr int kNumSymShapes = sizeof(kSymShapes) / sizeof(kSymShapes[0]);
 
-struct Kernel { attn_kernel_t fn; int lds_bytes; };
+constexpr int kRowsShape = 1, kRowsGroups = 3;        // with tangents: shape 1 is attn_jvp_rows_kernel
+struct Kernel { attn_kernel_t fn; int lds_bytes, threads = kAttnThreads; };
 template <typename T, int DQK, int DV, int SHAPE, bool RAW = false>
 Kernel pick_sym() {
     typedef SymCfg<DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg> C;
     static_assert(C::TPS == kSymStepTiles, "plans count steps of that many tiles");
-    return {attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg, RAW>, C::LDS_BYTES};
+    return {attn_fwd_sym_kernel<T, DQK, DV, kSymShapes[SHAPE].rg, kSymShapes[SHAPE].kg, RAW>, C::LDS_BYTES, 64 * C::NW};
 }
 template <typename T, int DQK, int DV>
 Kernel pick_mode(int mode, int shape) {
@@ -1777,8 +1779,12 @@ Kernel pick_mode(int mode, int shape) {
                 case 1: return pick_sym<T, DQK, DV, 1>();
                 default: return pick_sym<T, DQK, DV, 2>();
             }
-        case MODE_JVP_Q: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q, false>, AttnCfg<DQK, DV, MODE_JVP_Q>::LDS_BYTES};
-        default: return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL, false>, AttnCfg<DQK, DV, MODE_JVP_FULL>::LDS_BYTES};
+        case MODE_JVP_Q:
+            if constexpr (__is_same(T, __bf16) && DQK == 128 && DV == 128) { if (shape == kRowsShape) return {attn_jvp_rows_kernel<T, MODE_JVP_Q, kRowsGroups>, RowsCfg<MODE_JVP_Q, kRowsGroups>::LDS_BYTES, kRowsThreads}; }
+            return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_Q, false>, AttnCfg<DQK, DV, MODE_JVP_Q>::LDS_BYTES};
+        default:
+            if constexpr (__is_same(T, __bf16) && DQK == 128 && DV == 128) { if (shape == kRowsShape) return {attn_jvp_rows_kernel<T, MODE_JVP_FULL, kRowsGroups>, RowsCfg<MODE_JVP_FULL, kRowsGroups>::LDS_BYTES, kRowsThreads}; }
+            return {attn_fwd_jvp_kernel<T, DQK, DV, MODE_JVP_FULL, false>, AttnCfg<DQK, DV, MODE_JVP_FULL>::LDS_BYTES};
     }
 }
 // the kernels that read K and V where they are
@@ -1861,6 +1867,11 @@ struct SplitPlan { int shape, block_m, n_qt, n_pairs, n_full, n_rem, splits; dou
 constexpr double kStepUs[2][4] = {{0.54, 0.56, 0.68, 0.86}, {0.54, 0.60, 0.82, 1.21}};   // MODE_JVP_Q, MODE_JVP_FULL
 constexpr double kStepAlone[4] = {0.9, 0.9, 0.9, 0.7};
 constexpr double kPairUs[4] = {5.0, 5.0, 5.0, 13.0};          // what a workgroup that is a whole pair costs besides its steps
+// bf16 at head dim 128: attn_jvp_rows_kernel's workgroups of 192 rows, whole pairs and cut ones, where they are the cheaper plan: from about one round of them on.  Fits to 255 .. 10000
+// positions and 1560 .. 37440 x 100 .. 2048, B*H = 16, 40 and 80, S = 1 .. 11 of both kernels measured; of all plans the one taken is 1.01 (tangent on q 1.005) times the best one's time
+// on average.  us, attn_fwd_jvp_kernel / this, 16 heads, all tangents (tangent on q): 1560 72 / 93 (60 / 73), 2500 167 / 155 (131 / 112), 3520 299 / 284 (225 / 208), 7040 1071 / 953 (790 / 687),
+// 10000 2060 / 1880 (1560 / 1350), 33000 20040 / 17770 (15060 / 12710).
+constexpr StepCost kRowsWhole[2] = {{1.13, 15.5, 0.95}, {1.70, 14.5, 0.85}}, kRowsCut[2] = {{1.13, 12.0, 0.95}, {1.70, 8.2, 0.85}};      // MODE_JVP_Q, MODE_JVP_FULL
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // partial results of the split pairs: fp32 accumulators (O, and T with tangents), then the row statistics
 size_t partial_acc_bytes(const cosmos_attn_desc* d, const SplitPlan& s) {
@@ -1876,8 +1887,8 @@ constexpr size_t kNoLimit = ~(size_t)0;
 bool may_cut(const cosmos_attn_desc* d, int n_steps) {
     return n_steps >= 2 * kMinStepsPerSplit && !d->causal && !d->key_lens && !is_wide(d);
 }
-// cosmos_attn_set_forward_override() (tuning and tests), 0 = the library's own choice: rows of a forward-only workgroup, key ranges
-std::atomic<int> g_sym_rows{0}, g_sym_ranges{0};
+// cosmos_attn_set_forward_override() (tuning and tests), 0 = the library's own choice: rows of a forward-only workgroup, key ranges; attn_jvp_rows_kernel wherever it is built
+std::atomic<int> g_sym_rows{0}, g_sym_ranges{0}, g_tangent_rows{0};
 // The best cut for workgroups of block_m rows and n_steps barrier steps: `whole` is what a pair that is not cut costs, `cut` one of
 // which S ranges may be made.
 SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int block_m, int n_steps, StepCost whole, StepCost cut) {
@@ -1895,7 +1906,8 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     const SplitPlan uncut = s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
     while (s.splits > 1 && partial_bytes(d, s) > room) --s.splits;
-    const int asked = mode_of(d) == MODE_FWD ? g_sym_ranges.load(std::memory_order_relaxed) : 0;
+    const bool steered = mode_of(d) == MODE_FWD || g_tangent_rows.load(std::memory_order_relaxed);
+    const int asked = steered ? g_sym_ranges.load(std::memory_order_relaxed) : 0;
     if (asked > 0) s.splits = rem == 0 ? 1 : std::min({asked, s.splits, n_steps / kMinStepsPerSplit});
     else s.splits = choose_splits(rem, n_steps, cut, slot_bytes, s.splits);
     if (s.splits < 2) return uncut;
@@ -1915,7 +1927,14 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
     if (mode != MODE_FWD || is_wide(d)) {                          // a barrier step is 32 keys
         const int m = mode == MODE_JVP_Q ? 0 : 1;
         const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
-        return plan_shape(d, room, 0, kBlockM, n_tiles, StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+        const SplitPlan s = plan_shape(d, room, 0, kBlockM, n_tiles, StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+        // (output rows that overlap hold what is stored last: such a call keeps the kernel, and with it the order)
+        // (without room for partial results, as in the two-stage run, below seven eighths of a round: the workgroups that it always had there, to the bit, though these are the faster ones
+        // from some three quarters on: 16 heads 2120 x 1024, tangent on q, 54.5 us for 60 of attn_qstream_kernel)
+        if (d->dtype != COSMOS_ATTN_BF16 || d->d_qk != 128 || d->d_v != 128 || d->o_stride[2] < d->d_v) return s;
+        const SplitPlan r = plan_shape(d, room, kRowsShape, 64 * kRowsGroups, n_tiles, kRowsWhole[m], kRowsCut[m]);
+        if (g_tangent_rows.load(std::memory_order_relaxed)) return r;
+        return r.us < s.us && (room || 8 * r.n_pairs >= 7 * kNumCUs) ? r : s;
     }
     const int rows = g_sym_rows.load(std::memory_order_relaxed);
     SplitPlan best;
@@ -2049,10 +2068,12 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
 }
 
 COSMOS_ATTN_API int cosmos_attn_set_forward_override(int query_rows, int key_ranges) {
-    bool known = query_rows == 0;
+    const bool tangents = query_rows == 64 * kRowsGroups;
+    bool known = query_rows == 0 || tangents;
     for (const SymShape& w : kSymShapes) known = known || query_rows == 32 * w.rg;
     if (!known || key_ranges < 0) return COSMOS_ATTN_BAD_ARG;
-    g_sym_rows.store(query_rows, std::memory_order_relaxed);
+    g_sym_rows.store(tangents ? 0 : query_rows, std::memory_order_relaxed);
+    g_tangent_rows.store(tangents ? query_rows : 0, std::memory_order_relaxed);
     g_sym_ranges.store(key_ranges, std::memory_order_relaxed);
     return COSMOS_ATTN_OK;
 }
@@ -2149,7 +2170,7 @@ constexpr int kInPlaceRows[2] = {6144, 3072};       // forward only, all tangent
 bool reads_in_place(const cosmos_attn_desc* d, const SplitPlan& sp) {
     const int mode = mode_of(d);
     if (d->d_qk != 128 || d->d_v != 128 || mode == MODE_JVP_Q || d->Lq > kInPlaceRows[mode == MODE_FWD ? 0 : 1]) return false;
-    if ((mode == MODE_FWD && sp.shape == 0) || stream_groups_of(d, sp)) return false;
+    if (sp.shape == (mode == MODE_FWD ? 0 : kRowsShape) || stream_groups_of(d, sp)) return false;
     // 32-bit buffer offsets, also of the rows behind the last one, which have to lie past the buffer: of rows that overlap (an expanded tensor's) they would read as numbers,
     // and 0 times what is there is not 0 where that is infinite
     for (const int64_t stride : {d->k_stride[2], d->v_stride[2]})
@@ -2213,7 +2234,7 @@ int run_impl(const cosmos_attn_desc* d, void* workspace, size_t workspace_bytes,
         ap.part_stat = (float4*)((char*)workspace + image_bytes + partial_acc_bytes(d, sp));
     }
     const int64_t blocks = (int64_t)sp.n_full + (int64_t)sp.n_rem * sp.splits;
-    hipLaunchKernelGGL(kernel.fn, dim3((unsigned)blocks), dim3(mode == MODE_FWD ? 64 * kSymShapes[sp.shape].rg * kSymShapes[sp.shape].kg : kAttnThreads), kernel.lds_bytes, (hipStream_t)stream, ap);
+    hipLaunchKernelGGL(kernel.fn, dim3((unsigned)blocks), dim3(kernel.threads), kernel.lds_bytes, (hipStream_t)stream, ap);
     if (hipGetLastError() != hipSuccess) return COSMOS_ATTN_LAUNCH_FAILED;
     if (sp.splits > 1) {
         const int rows_per_block = 256 / (d->d_v / 4);

@@ -99,7 +99,8 @@ COSMOS_ATTN_API void cosmos_attn_set_stream_override(int blocks_per_workgroup, i
  * Tuning and test hook, process-wide, like the one above, for the kernel that calls without tangents run where they are not streamed: workgroups of
  * query_rows rows (128, 256 or 384; 0: the library's choice), and key_ranges for the pairs of a partly filled last round (1: never cut;
  * n > 1: n, where the call may be cut at all, or as many as its length and the workspace allow; 0: the library's choice).  (0, 0) restores
- * the default.  It steers sizes and launches alike: set it before the workspace is asked for.  A status code.
+ * the default.  192 rows: calls with tangents in bf16 at head dim 128 run their kernel of that many rows whatever their size, with key_ranges as
+ * above, and calls without tangents the library's choice.  It steers sizes and launches alike: set it before the workspace is asked for.  A status code.
  */
 COSMOS_ATTN_API int cosmos_attn_set_forward_override(int query_rows, int key_ranges);
 

@@ -262,6 +262,87 @@ def test_forward_only_scores_that_move_the_max(pkg, oracle, gpu, stream_override
     assert oracle.error_metrics(lse.cpu(), lse_ref)[0] <= LSE_ABS * 4      # (log-sum-exp of 60: 4 bits fewer behind the point)
 
 
+ROWS_KERNEL = 192      # rows of a workgroup of the kernel that bf16 calls with tangents take from about a round of workgroups on
+
+
+@pytest.mark.parametrize("tangents", ["q", "full"])
+@pytest.mark.parametrize("Lq, Lkv", [(1, 31), (15, 40), (47, 32), (48, 33), (49, 64), (191, 65), (192, 96), (193, 129), (400, 160), (577, 300), (33, 513)])
+def test_tangent_rows_kernel_ragged(pkg, oracle, gpu, stream_override, forward_override, Lq, Lkv, tangents):
+    """Rows on either side of 16, of a wavefront's 48 and of a workgroup; one tile of keys and two, on either side of the rings' 4 and 5 and many more; same tolerances."""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL)
+    run_case(pkg, oracle, gpu, (2, 3, Lq, 128), (2, 3, Lkv, 128), seed=Lq + Lkv, tangents=tangents)
+
+
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_masks(pkg, oracle, gpu, stream_override, forward_override, tangents):
+    """(A row of one key has no tangent from q alone: what is left is rounding, which no relative bound holds for.)"""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL)
+    for lens in ([64, 512], [7, 33], [300, 31], [3, 65], [97, 511]):
+        run_case(pkg, oracle, gpu, (2, 2, 450, 128), (2, 2, 512, 128), key_lens=lens, seed=sum(lens), tangents=tangents)
+    for L in (17, 33, 128, 193, 200, 515, 1000):
+        run_case(pkg, oracle, gpu, (1, 2, L, 128), causal=True, seed=L, tangents=tangents)
+
+
+@pytest.mark.parametrize("ranges", [1, 3])
+@pytest.mark.parametrize("order", ["rising", "falling", "spike"])
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_scores_that_move_the_max(pkg, oracle, gpu, stream_override, forward_override, order, ranges, tangents):
+    """As test_forward_only_scores_that_move_the_max: everything formed so far is scaled, the rounded operands of the tile before among it.  The tangents
+    are differences of sums that the scores' range makes large: theirs is the error of the other kernel, which forms the same ones."""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL, ranges)
+    Lkv = 777
+    q, k, v, tq, tk, tv = oracle.make_inputs((1, 2, 300, 128), (1, 2, Lkv, 128), seed=Lkv)
+    top = {"rising": torch.linspace(-60, 60, Lkv), "falling": torch.linspace(60, -60, Lkv),
+           "spike": torch.where(torch.arange(Lkv) == Lkv - 3, 60.0, 0.0)}[order]
+    q = (0.1 * q.float() + 1.0).to(torch.bfloat16)
+    k = (0.1 * k.float() + (top * 128 ** -0.5).view(1, 1, Lkv, 1)).to(torch.bfloat16)
+    if tangents == "q":
+        tk = tv = None
+    dev = lambda x: None if x is None else x.to(gpu)
+    o, to, lse = pkg.fwd_jvp(*(dev(x) for x in (q, k, v, tq, tk, tv)))
+    forward_override(0)
+    to_other = pkg.fwd_jvp(*(dev(x) for x in (q, k, v, tq, tk, tv)))[1]
+    o_ref, to_ref, lse_ref = oracle.closed_form(q, k, v, tq, tk, tv)
+    check(oracle, "o", o, o_ref)
+    other = oracle.error_metrics(to_other.float().cpu(), to_ref)
+    check(oracle, "to", to, to_ref, max_abs=max(MAX_ABS, 1.5 * other[0]), rel_l2=max(REL_L2, 1.1 * other[1]))
+    assert oracle.error_metrics(lse.cpu(), lse_ref)[0] <= LSE_ABS * 4
+
+
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_ranges_layouts_and_choice(pkg, oracle, gpu, stream_override, forward_override, tangents):
+    """Key ranges; [B, S, H, D] storage; bit for bit the same twice; the library's own choice of it at one round of workgroups (dense rows; fp16 and overlapping output rows: not)."""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL, 4)
+    a = run_case(pkg, oracle, gpu, (1, 3, 500, 128), (1, 3, 1000, 128), seed=5, tangents=tangents)
+    b = run_case(pkg, oracle, gpu, (1, 3, 500, 128), (1, 3, 1000, 128), seed=5, tangents=tangents)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    forward_override(ROWS_KERNEL)
+    t = lambda x: None if x is None else x.transpose(1, 2).contiguous().to(gpu).transpose(1, 2)
+    q, k, v, tq, tk, tv = oracle.make_inputs((2, 3, 333, 128), (2, 3, 257, 128), seed=6)
+    tk, tv = (None, None) if tangents == "q" else (tk, tv)
+    o, to, _ = pkg.fwd_jvp(*(t(x) for x in (q, k, v, tq, tk, tv)), out_layout="blhd")
+    o_ref, to_ref, _ = oracle.closed_form(q, k, v, tq, tk, tv)
+    check(oracle, "o", o, o_ref)
+    check(oracle, "to", to, to_ref)
+    forward_override(0)
+    L, lib, fake = pkg._lib, pkg._lib.load_library(), 0x7F0000000000
+    for dtype, row, rows in ((L.DTYPE_BF16, 128, 192), (L.DTYPE_FP16, 128, 128), (L.DTYPE_BF16, 64, 128)):
+        D, plan = L.AttnDesc(), L.AttnPlan()
+        D.abi_version, D.dtype, D.B, D.H, D.Lq, D.Lkv, D.d_qk, D.d_v, D.sm_scale = L.ABI_VERSION, dtype, 1, 16, 3000, 3000, 128, 128, 0.1
+        D.q = D.k = D.v = D.o = D.to = D.tq = fake
+        if tangents == "full":
+            D.tk = D.tv = fake
+        dense = (ctypes.c_int64 * 3)(16 * 3000 * 128, 3000 * 128, 128)
+        D.q_stride = D.k_stride = D.v_stride = dense
+        D.o_stride = (ctypes.c_int64 * 3)(16 * 3000 * row, 3000 * row, row)
+        assert lib.cosmos_attn_launch_plan(ctypes.byref(D), ctypes.c_size_t(-1).value, ctypes.byref(plan)) == 0
+        assert plan.query_rows == rows
+
+
 @pytest.mark.parametrize("chunk", range(4))
 def test_random_shapes_all_modes(pkg, oracle, gpu, chunk):
     """40 seeded random cases (10 per chunk): batch, heads, lengths, head dims, dtype and tangent set drawn at random --
