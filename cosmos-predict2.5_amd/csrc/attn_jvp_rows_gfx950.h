@@ -33,17 +33,17 @@ typedef unsigned rows_u32x4 __attribute__((ext_vector_type(4)));
 // (PAUSE: in front of the loop and behind it, where the compiler may copy an operand just before its use; of the wait that this takes it does not know, asm being asm)
 #define ROWS_MFMA(OP)                                                                                                                                 \
     template <bool PAUSE, bool TAN> static __device__ __forceinline__ void first(f32x4& c, rows_u32x4 a, rows_u32x4 b) {                              \
-        if constexpr (PAUSE) asm volatile("s_nop 7\n\t" OP " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));                                            \
+        if constexpr (PAUSE) asm volatile("s_nop 3\n\t" OP " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));                                            \
         else if constexpr (TAN) asm volatile(OP " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "a"(b));                                                        \
         else asm volatile(OP " %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));                                                                           \
     }                                                                                                                                                 \
     template <bool PAUSE, bool TAN> static __device__ __forceinline__ void more(f32x4& c, rows_u32x4 a, rows_u32x4 b) {                               \
-        if constexpr (PAUSE) asm volatile("s_nop 7\n\t" OP " %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));                                            \
+        if constexpr (PAUSE) asm volatile("s_nop 3\n\t" OP " %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));                                            \
         else if constexpr (TAN) asm volatile(OP " %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(b));                                                        \
         else asm volatile(OP " %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));                                                                           \
     }                                                                                                                                                 \
     template <bool PAUSE> static __device__ __forceinline__ void sum(f32x4& c, rows_u32x4 a, rows_u32x4 b) {                                          \
-        if constexpr (PAUSE) asm volatile("s_nop 7\n\t" OP " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));                                            \
+        if constexpr (PAUSE) asm volatile("s_nop 3\n\t" OP " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));                                            \
         else asm volatile(OP " %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));                                                                           \
     }
 template <typename T> struct RowsMfma;
@@ -102,12 +102,6 @@ attn_jvp_rows_kernel(const AttnParams p) {
     const int k_run = wave * C::K_LOADS * kFragBytes, v_run = wave * C::V_LOADS * kFragBytes;
     auto load_k = [&](int t, unsigned slot) __attribute__((always_inline)) { issue_part<C::K_LOADS>(kv_rsrc, smem + C::KRING_OFF + slot + k_run, k_lane, t * TILE_BYTES + k_run); };
     auto load_v = [&](int t, unsigned slot) __attribute__((always_inline)) { issue_part<C::V_LOADS>(kv_rsrc, smem + C::VRING_OFF + slot + v_run, v_lane, t * TILE_BYTES + KP_BYTES + v_run); };
-    // step t forms S of tile t and adds tile t - 1 to the outputs; it loads K of tile t + KRING - 1 and V of tile t + VRING - 2
-#pragma unroll
-    for (int u = 0; u < C::KRING; ++u) load_k(tile_at(u), u * KP_BYTES);
-#pragma unroll
-    for (int u = 0; u < C::VRING - 1; ++u) load_v(tile_at(u), u * VP_BYTES);
-
     // ---- this wavefront's Q and dQ rows as B operands: row 16 j + l16, channels 32 c + 8 g .. + 7
     rows_u32x4 qb[NG][NC], tb[NG][NC];
 #pragma unroll
@@ -123,6 +117,16 @@ attn_jvp_rows_kernel(const AttnParams p) {
             qb[j][c] = live ? *reinterpret_cast<const rows_u32x4*>(qp + 32 * c) : z;
             tb[j][c] = live ? *reinterpret_cast<const rows_u32x4*>(tp + 32 * c) : z;
         }
+    }
+
+    // step t forms S of tile t and adds tile t - 1 to the outputs; it loads K of tile t + KRING - 1 and V of tile t + VRING - 2.  Here in the order in which the first steps wait for them,
+    // behind Q: the first S wants nothing but that and K
+    static_assert(C::KRING == 5 && C::VRING == 4, "the order");
+    load_k(tile_at(0), 0);
+#pragma unroll
+    for (int u = 0; u < C::VRING; ++u) {
+        load_k(tile_at(u + 1), (u + 1) * KP_BYTES);
+        if (u < C::VRING - 1) load_v(tile_at(u), u * VP_BYTES);
     }
 
     // ---- state.  S^T of 16 keys x 16 rows: [16 rows][key half], register r: row 16 j + l16, key lane_key(lane) + 8 m + r of the tile
@@ -375,7 +379,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
         const rows_u32x4 z = {0, 0, 0, 0};
         for_each<C::V_LOADS>([&](auto i) { lds_write<decltype(i)::value * kFragBytes>(at, z); });
     }
-    __builtin_amdgcn_s_waitcnt(0x0070);        // Q, dQ and the first tiles are here
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(3 * C::K_LOADS + 3 * C::V_LOADS) : "memory");       // Q, dQ and K of two tiles are here (the first step reads ahead)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (n > 0) {
