@@ -1983,6 +1983,9 @@ constexpr int kStreamGroupsPerCU = 1;       // one workgroup fills a compute uni
 constexpr double kStreamTileUs[2][4] = {{0.32, 0.32, 0.44, 0.63}, {0.58, 0.62, 0.60, 0.79}};
 constexpr double kStreamBlockUs[2][4] = {{2.5, 2.0, 0.5, 1.0}, {3.5, 2.5, 0.5, 6.0}};
 constexpr double kStreamStartUs[4] = {5.0, 5.0, 5.0, 0.0};
+// attn_jvp_rows_kernel on the other side: its tiles are the cheaper ones, its workgroups the dearer.  us, stream / that, 16 heads: tangent on q 20000 x 1024 318 / 336, x 2048 600 / 573; all
+// tangents 37440 x 512 470 / 491 (2 x 16 heads 930 / 937), 20000 x 1024 451 / 437, x 2048 808 / 772.
+constexpr int kStreamRowsTiles[2] = {48, 24};
 constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
 std::atomic<int> g_stream_groups{0};      // number of workgroups, 0 = the library's own choice
@@ -2001,6 +2004,7 @@ int stream_groups_of(const cosmos_attn_desc* d, const SplitPlan& other) {
     if (pairs < kStreamMinPairs) return 0;
     const int groups = kNumCUs * kStreamGroupsPerCU;
     const int mode = mode_of(d);
+    if (mode != MODE_FWD && other.shape == kRowsShape && n_tiles_of(d) > kStreamRowsTiles[mode == MODE_JVP_Q ? 0 : 1]) return 0;
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
     const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
     const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
