@@ -36,7 +36,7 @@ PEAK_BF16_TFLOPS = 256 * 4096 * 2.4e9 / 1e12
 # with the 1 GiB copy of --copy-calib) whose summary is the named file; the JSON line carries the file name next to the
 # number ("traffic_source").  A workload without a counter run reports null.
 MEASURED_TRAFFIC_BYTES = {
-    "c3": ((2 * 2.633e7 + 710537) * 1024, "profiles/attn_fwd_jvp_kernel_bf16_d128_workload_c3.txt"),
+    "c3": ((2 * 1.5002e7 + 719150) * 1024, "profiles/attn_jvp_rows_kernel_bf16_d128_workload_c3.txt"),
     "nr": ((2 * 359157 + 676527) * 1024, "profiles/norm_rope_kernel_bf16_d128_workload_nr.txt"),
     "c2": ((2 * 1.770e6 + 1.998e5) * 1024, "profiles/attn_fwd_sym_kernel_bf16_d128_workload_c2.txt"),
     "c5": ((2 * 326847 + 603763) * 1024, "profiles/attn_qstream_kernel_bf16_d128_workload_c5.txt"),
@@ -269,7 +269,7 @@ def bench_module(args, pkg, dev, desc_txt, B, H, L, D):
                    "pct_of_bf16_mfma_peak": 100.0 * flops / sec / 1e12 / PEAK_BF16_TFLOPS},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_BF16_TFLOPS, "traffic": None,
-                     "kernel": "whole module call (attn_fwd_jvp_kernel dominates)", "kernel_ms_avg": avg},
+                     "kernel": "whole module call (attn_jvp_rows_kernel dominates)", "kernel_ms_avg": avg},
     }
     print(json.dumps(result), flush=True)
 
@@ -709,7 +709,7 @@ def bench_attention(args, pkg, lib, dev, name, steps, warmup, full=True):
     roofline.update({"frac": roofline["achieved"] / roofline["peak"], "traffic": traffic, "traffic_source": traffic_source,
                      "algorithmic_bytes": alg_bytes,
                      "kernel": "attn_qstream_kernel" if name == "c5" else
-                               ("attn_fwd_sym_kernel" if tangents == "none" and not padded else "attn_fwd_jvp_kernel") + " (+ attn_combine_kernel)",
+                               ("attn_fwd_sym_kernel" if tangents == "none" and not padded else "attn_jvp_rows_kernel") + " (+ attn_combine_kernel)",
                      "kernel_ms_avg": run_avg, "kernel_ms_min": min(run_ms),
                      "kernel_ms_median": sorted(run_ms)[len(run_ms) // 2], "pack_kv_kernel_ms_avg": pack_avg})
     result = {

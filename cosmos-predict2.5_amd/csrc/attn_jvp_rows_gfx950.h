@@ -7,7 +7,7 @@
 //
 // What bounds it: the part's power limit and, next to that, instruction issue.  A wavefront alone on its SIMD hides two other instructions behind a v_mfma_f32_16x16x32 of
 // 16 cycles (measured: with two 18 cycles, three 22, four 26; an exponential counts twice), so a step is written in slots, a product and what is issued beside it, with the elements'
-// work spread by the room that LDS reads, waits and loads leave (fixed(), room(), args_before(), exps_before()).  A step of 144 products takes 3190 cycles at 1.95 GHz.
+// work spread by the room that LDS reads, waits and loads leave (fixed(), room(), args_before(), exps_before()).  A step of 144 products takes 3030 cycles (84480 positions, all tangents: matrix units busy 78 %, 1.93 GHz).
 // 16 heads x 33000 positions, all tangents, attn_fwd_jvp_kernel / this: LDS-active cycles 1085 / 364 million, 34.3 / 35.4 million cycles, 1.69 / 1.95 GHz, 20.36 / 18.18 ms; tangent on q
 // 15.06 / 12.71 ms (further sizes beside kRowsWhole).
 //
