@@ -1921,20 +1921,30 @@ SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {
     const StepCost c{by_head_dim(w.step_us, dim), by_head_dim(w.range_us, dim), by_head_dim(w.alone, dim)};
     return plan_shape(d, room, shape, 32 * w.rg, sym_steps(d), c, c);
 }
-SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
-    const int mode = mode_of(d), n_tiles = n_tiles_of(d);
+// with tangents, and head dim 256: 128 rows a workgroup (score and output wavefronts), a barrier step is 32 keys
+SplitPlan plan_roles(const cosmos_attn_desc* d, size_t room) {
+    const int m = mode_of(d) == MODE_JVP_Q ? 0 : 1;
     const double dim = 0.5 * (d->d_qk + d->d_v);
-    if (mode != MODE_FWD || is_wide(d)) {                          // a barrier step is 32 keys
+    const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
+    return plan_shape(d, room, 0, kBlockM, n_tiles_of(d), StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+}
+bool in_place_whole(const cosmos_attn_desc* d);
+SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
+    const int mode = mode_of(d);
+    if (mode != MODE_FWD || is_wide(d)) {
         const int m = mode == MODE_JVP_Q ? 0 : 1;
-        const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
-        const SplitPlan s = plan_shape(d, room, 0, kBlockM, n_tiles, StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+        const SplitPlan s = plan_roles(d, room);
         // (output rows that overlap hold what is stored last: such a call keeps the kernel, and with it the order)
-        // (without room for partial results, as in the two-stage run, below seven eighths of a round: the workgroups that it always had there, to the bit, though these are the faster ones
-        // from some three quarters on: 16 heads 2120 x 1024, tangent on q, 54.5 us for 60 of attn_qstream_kernel)
         if (d->dtype != COSMOS_ATTN_BF16 || d->d_qk != 128 || d->d_v != 128 || d->o_stride[2] < d->d_v) return s;
-        const SplitPlan r = plan_shape(d, room, kRowsShape, 64 * kRowsGroups, n_tiles, kRowsWhole[m], kRowsCut[m]);
+        const SplitPlan r = plan_shape(d, room, kRowsShape, 64 * kRowsGroups, n_tiles_of(d), kRowsWhole[m], kRowsCut[m]);
         if (g_tangent_rows.load(std::memory_order_relaxed)) return r;
-        return r.us < s.us && (room || 8 * r.n_pairs >= 7 * kNumCUs) ? r : s;
+        // Whole pairs are dealt out alike whether there is room for partial results or not, so that the two-stage run, which has none, and the in-place call take the kernel that the
+        // one-call form takes wherever that does not cut: from seven eighths of a round of them on.  (Below, the estimate for a round that is not full is the less sure one: 16 heads,
+        // tangent on q, 2120 x 1024 54.5 us for 60 of attn_qstream_kernel, but 8 heads x 4213 causal 146 for 132, all tangents 16 x 2197 causal 113 for 101.)
+        if (r.us >= s.us || (r.splits < 2 && 8 * r.n_pairs < 7 * kNumCUs)) return s;
+        // A call that can be read in place, whole pairs of 128 rows, is: the estimates are of calls that are re-tiled.  us, in place / 192 rows: 16 heads 368 21.6 / 32.6, 500 26.0 / 36.5, 8 heads
+        // 345 20.3 / 30.1, 80 heads 459 55.3 / 51.5, 2411 670 / 654.
+        return in_place_whole(d) ? s : r;
     }
     const int rows = g_sym_rows.load(std::memory_order_relaxed);
     SplitPlan best;
@@ -2004,7 +2014,8 @@ int stream_groups_of(const cosmos_attn_desc* d, const SplitPlan& other) {
     if (pairs < kStreamMinPairs) return 0;
     const int groups = kNumCUs * kStreamGroupsPerCU;
     const int mode = mode_of(d);
-    if (mode != MODE_FWD && other.shape == kRowsShape && n_tiles_of(d) > kStreamRowsTiles[mode == MODE_JVP_Q ? 0 : 1]) return 0;
+    // (`other` without room for partial results may be this kernel where with room it is a cut of 128 rows, which then streams: so does the two-stage run)
+    if (mode != MODE_FWD && other.shape == kRowsShape && n_tiles_of(d) > kStreamRowsTiles[mode == MODE_JVP_Q ? 0 : 1] && plan_split(d, kNoLimit).shape == kRowsShape) return 0;
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
     const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
     const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
@@ -2180,6 +2191,12 @@ bool reads_in_place(const cosmos_attn_desc* d, const SplitPlan& sp) {
     for (const int64_t stride : {d->k_stride[2], d->v_stride[2]})
         if (stride < 128 || stride >= (int64_t)1 << 30 || (d->Lkv + 4 * kBlockN) * stride * 2 >= (int64_t)1 << 31) return false;
     return true;
+}
+// with tangents: 128 rows a workgroup, given all the room there could be, are not cut and read K and V where they are
+bool in_place_whole(const cosmos_attn_desc* d) {
+    if (mode_of(d) != MODE_JVP_FULL || d->Lq > kInPlaceRows[1]) return false;
+    const SplitPlan s = plan_roles(d, kNoLimit);
+    return s.splits < 2 && reads_in_place(d, s);
 }
 // `room`: bytes behind the re-tiled K/V image that key-range partial results may take.  cosmos_attn_run only reads its workspace, so
 // that several runs may share one image: 0, never split.  one_call: K and V are re-tiled here, or read where they are.

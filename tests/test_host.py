@@ -2,7 +2,9 @@
 validation returns the documented status codes (validation happens before anything touches the device), and the
 Python operators raise the same exception types as the reference for the same misuse."""
 import ctypes
+import math
 import os
+import random
 import re
 
 import pytest
@@ -167,6 +169,43 @@ def test_workspace_holds_the_plan_that_runs_and_no_more(pkg, d, tangents):
                 uncut = plan_of(pkg, D, packed)
                 assert uncut == "streamed" or uncut[3:] == (0, 1), (H, Lq, Lkv)
     assert shapes == ({(128, 1)} if tangents else {(128, 2), (256, 1), (384, 1)})
+
+
+def dense_desc(pkg, H, Lq, Lkv, tangents, **over):
+    """bf16 at head dim 128, rows one behind the other; tangents None, "q" or "full"."""
+    t = {None: (None, None), "q": (0x7F0000000000, None), "full": (0x7F0000000000, 0x7F0000000000)}[tangents]
+    rows = lambda L: (ctypes.c_int64 * 3)(H * L * 128, L * 128, 128)
+    return good_desc(pkg, H=H, Lq=Lq, Lkv=Lkv, d_v=128, tq=t[0], to=t[0], tk=t[1], tv=t[1], q_stride=rows(Lq), o_stride=rows(Lq), k_stride=rows(Lkv), v_stride=rows(Lkv), **over)
+
+
+@pytest.mark.parametrize("tangents", [None, "q", "full"])
+def test_forms_of_a_call_that_is_not_cut_take_the_same_kernel(pkg, tangents):
+    """What runs without room for partial results (the two-stage run, the in-place call) is what the one-call form runs wherever that cuts no keys: the same results, bit for bit.
+    Drawn sizes, and sizes where they parted."""
+    lib, rng = pkg._lib.load_library(), random.Random(3)
+    log = lambda lo, hi: int(math.exp(rng.uniform(math.log(lo), math.log(hi))))
+    calls = [(40, 1741, 1741, None), (80, 807, 1623, None), (20, 1845, 1855, None), (16, 2197, 2197, "causal"), (8, 4277, 303, "lens")]
+    while len(calls) < 6000:
+        Lq, how = log(100, 12000), rng.choice([None, None, "causal", "lens"])
+        calls.append((rng.choice([1, 2, 8, 12, 16, 20, 24, 32, 40, 64, 80]), Lq, Lq if how == "causal" or rng.random() < 0.5 else log(20, 5000), how))
+    uncut = 0
+    for H, Lq, Lkv, how in calls:
+        D = dense_desc(pkg, H, Lq, Lkv, tangents, causal=int(how == "causal"), key_lens=0x7F0000000000 if how == "lens" else None)
+        plan = plan_of(pkg, D)
+        if plan != "streamed" and plan[4] > 1:
+            continue
+        uncut += 1
+        assert plan_of(pkg, D, lib.cosmos_attn_packed_bytes(ctypes.byref(D))) == plan, (H, Lq, Lkv, how)
+    assert uncut > 2000
+
+
+@pytest.mark.parametrize("H, Lq, Lkv, how", [(16, 2197, 2197, "causal"), (16, 3000, 3000, "causal"), (64, 2196, 2196, "lens"), (40, 1129, 4403, "lens"), (80, 2411, 2411, None), (8, 345, 345, None)])
+def test_calls_with_all_tangents_that_are_read_in_place(pkg, H, Lq, Lkv, how):
+    if torch.cuda.is_available():
+        pytest.skip("an accepted call would be launched")
+    D = dense_desc(pkg, H, Lq, Lkv, "full", causal=int(how == "causal"), key_lens=0x7F0000000000 if how == "lens" else None)
+    assert pkg._lib.load_library().cosmos_attn_fwd_in_place(ctypes.byref(D), None) not in (pkg._lib.ST_WORKSPACE, 0)
+    assert plan_of(pkg, D)[0] == 128
 
 
 def test_forward_override_steers_plan_and_workspace(pkg, forward_override, forward_plan):
