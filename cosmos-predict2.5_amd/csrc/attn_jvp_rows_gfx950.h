@@ -85,11 +85,12 @@ attn_jvp_rows_kernel(const AttnParams p) {
     int n_tiles_all = (kv_len + kBlockN - 1) / kBlockN;
     if (p.causal) { const int lim = (qt * C::ROWS + C::ROWS + kBlockN - 1) / kBlockN; n_tiles_all = n_tiles_all < lim ? n_tiles_all : lim; }
     const int u_lo = partial ? (int)((int64_t)split * n_tiles_all / p.splits) : 0;
-    // (two at least: a second tile that is not there is masked)
+    // (two at least: a second tile that is not there is masked, and zeros.  A loop that may be left at once takes the compiler copies and scratch inside of it)
+    static_assert(kMinStepsPerSplit >= 2, "a range of one tile");
     const int n = partial ? (int)((int64_t)(split + 1) * n_tiles_all / p.splits) - u_lo : n_tiles_all == 1 ? 2 : n_tiles_all;
 
     const __amdgpu_buffer_rsrc_t kv_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char*>(p.kv) + (size_t)bh * p.n_tiles * TILE_BYTES, 0, p.n_tiles * TILE_BYTES, 0x00020000);
+        const_cast<char*>(p.kv) + (size_t)bh * p.n_tiles * TILE_BYTES, 0, n_tiles_all * TILE_BYTES, 0x00020000);
     // sweep order: see attn_fwd_jvp_kernel
     const int n_sweep = n_tiles_all > 1 ? n_tiles_all : 2;
     const int shift = p.causal || n_tiles_all < 2 ? 0 : (((pair >> 3) & 31) * COSMOS_ATTN_SWEEP_STAGGER) % n_sweep;
@@ -100,8 +101,9 @@ attn_jvp_rows_kernel(const AttnParams p) {
     // ---- loads: this wavefront's quarter of a K part or a V part
     const int k_lane = k_fill_lane(lane) * 16, v_lane = lane * 16;
     const int k_run = wave * C::K_LOADS * kFragBytes, v_run = wave * C::V_LOADS * kFragBytes;
-    auto load_k = [&](int t, unsigned slot) __attribute__((always_inline)) { issue_part<C::K_LOADS>(kv_rsrc, smem + C::KRING_OFF + slot + k_run, k_lane, t * TILE_BYTES + k_run); };
-    auto load_v = [&](int t, unsigned slot) __attribute__((always_inline)) { issue_part<C::V_LOADS>(kv_rsrc, smem + C::VRING_OFF + slot + v_run, v_lane, t * TILE_BYTES + KP_BYTES + v_run); };
+    // (`checked`: bytes of the tile's place in the lanes' offset, which the buffer's bounds hold for; the scalar offset's are nobody's to rely on)
+    auto load_k = [&](int t, unsigned slot, int checked = 0) __attribute__((always_inline)) { issue_part<C::K_LOADS>(kv_rsrc, smem + C::KRING_OFF + slot + k_run, k_lane + checked, t * TILE_BYTES + k_run); };
+    auto load_v = [&](int t, unsigned slot, int checked = 0) __attribute__((always_inline)) { issue_part<C::V_LOADS>(kv_rsrc, smem + C::VRING_OFF + slot + v_run, v_lane + checked, t * TILE_BYTES + KP_BYTES + v_run); };
     // ---- this wavefront's Q and dQ rows as B operands: row 16 j + l16, channels 32 c + 8 g .. + 7
     rows_u32x4 qb[NG][NC], tb[NG][NC];
 #pragma unroll
@@ -122,11 +124,11 @@ attn_jvp_rows_kernel(const AttnParams p) {
     // step t forms S of tile t and adds tile t - 1 to the outputs; it loads K of tile t + KRING - 1 and V of tile t + VRING - 2.  Here in the order in which the first steps wait for them,
     // behind Q: the first S wants nothing but that and K
     static_assert(C::KRING == 5 && C::VRING == 4, "the order");
-    load_k(tile_at(0), 0);
+    load_k(0, 0, tile_at(0) * TILE_BYTES);
 #pragma unroll
     for (int u = 0; u < C::VRING; ++u) {
-        load_k(tile_at(u + 1), (u + 1) * KP_BYTES);
-        if (u < C::VRING - 1) load_v(tile_at(u), u * VP_BYTES);
+        load_k(0, (u + 1) * KP_BYTES, tile_at(u + 1) * TILE_BYTES);
+        if (u < C::VRING - 1) load_v(0, u * VP_BYTES, tile_at(u) * TILE_BYTES);
     }
 
     // ---- state.  S^T of 16 keys x 16 rows: [16 rows][key half], register r: row 16 j + l16, key lane_key(lane) + 8 m + r of the tile
@@ -311,7 +313,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
         return 10 * (done / 12) + (rest < 2 ? 0 : rest < 4 ? 1 : rest - 2);
     };
     static_assert(exps_before(15 * PER + NG) >= EXP_HALF, "the first half is rounded behind its last operand's last use");
-    int t_kload = tile_at(C::KRING), t_vload = tile_at(C::VRING - 1);
+    int t_kload = n_tiles_all < 2 ? 0 : tile_at(C::KRING), t_vload = n_tiles_all < 2 ? 0 : tile_at(C::VRING - 1);      // (one tile: one step, whose loads nobody reads)
     auto elements = [&](auto qi) __attribute__((always_inline)) {
         constexpr int Q = decltype(qi)::value;                                  // (of the step's own tile; the next step's slots follow)
         for_each<args_before(Q + 1) - args_before(Q)>([&](auto i) { arg_op(Int<args_before(Q) + decltype(i)::value>{}); });

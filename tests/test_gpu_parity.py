@@ -285,6 +285,38 @@ def test_tangent_rows_kernel_masks(pkg, oracle, gpu, stream_override, forward_ov
         run_case(pkg, oracle, gpu, (1, 2, L, 128), causal=True, seed=L, tangents=tangents)
 
 
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_reads_one_tile_of_keys(pkg, oracle, gpu, stream_override, forward_override, tangents):
+    """Up to 32 keys: neither the padded keys of further tiles nor what lies behind the re-tiled keys enter the results, whatever is there."""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL)
+    lib, lens = pkg._lib.load_library(), [1, 7, 31, 32]
+    x = oracle.make_inputs((4, 2, 230, 128), (4, 2, 100, 128), seed=4)
+    q, k, v, tq, tk, tv = (None if tangents == "q" and i > 3 else t.to(gpu) for i, t in enumerate(x))
+    results = []
+    for there in (0.0, float("nan"), float("inf")):
+        for t in (k, v, tk, tv):
+            if t is not None:
+                t[:, :, 32:] = there
+        results.append(pkg.fwd_jvp(q, k, v, tq, tk, tv, key_lens=torch.tensor(lens, dtype=torch.int32, device=gpu)))
+        assert all(torch.isfinite(t).all() and torch.equal(t, want) for t, want in zip(results[-1], results[0]))
+    for n in lens:      # (one batch row, its own tensors)
+        kk, vv, tkk, tvv = (None if t is None else t[:1, :, :n].contiguous() for t in (k, v, tk, tv))
+        want = pkg.fwd_jvp(q[:1], kk, vv, tq[:1], tkk, tvv)
+        d = pkg.ops._packed_desc(1, 2, 230, n, 128, 128, torch.bfloat16, 128 ** -0.5)
+        o, to, lse = (torch.empty_like(t) for t in want)
+        d.q, d.k, d.v, d.tq, d.o, d.to, d.lse, d.key_lens = *(t.data_ptr() for t in (q, kk, vv, tq, o, to, lse)), None
+        if tangents == "full":
+            d.tk, d.tv = tkk.data_ptr(), tvv.data_ptr()
+        d.q_stride, d.k_stride, d.v_stride, d.o_stride = (pkg.ops._strides3(t) for t in (q, kk, vv, o))
+        nbytes = lib.cosmos_attn_workspace_bytes(ctypes.byref(d))
+        room = torch.full((nbytes // 2 + 65536,), float("nan"), device=gpu, dtype=torch.bfloat16)
+        plan = pkg._lib.AttnPlan()
+        assert lib.cosmos_attn_launch_plan(ctypes.byref(d), nbytes, ctypes.byref(plan)) == 0 and plan.query_rows == ROWS_KERNEL
+        assert lib.cosmos_attn_fwd_jvp(ctypes.byref(d), room.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+        assert all(torch.equal(a, b) for a, b in zip((o, to, lse), want)) and torch.isfinite(o).all() and torch.isfinite(to).all()
+
+
 @pytest.mark.parametrize("ranges", [1, 3])
 @pytest.mark.parametrize("order", ["rising", "falling", "spike"])
 @pytest.mark.parametrize("tangents", ["q", "full"])
