@@ -147,6 +147,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
     // ---- the step's products, in 16 groups of one operand A of K or V and, with tangents on k and v, one of dK or dV:
     // 0 .. 7: S, key half G / 4, channels 32 (G % 4); 8 .. 15: outputs, channels 16 (G % 8)
     constexpr int PER = (FULL ? 3 : 2) * NG, SLOTS = 16 * PER;
+    constexpr int CHECK = 10 * PER;             // where the max is looked at
     constexpr int AHEAD = FULL ? 1 : 2;         // groups that LDS reads run ahead
     rows_u32x4 fa[AHEAD + 1 == 2 ? 2 : 4], fb[2];
     const unsigned frag_lane = lds0 + frag_offset(lane);
@@ -233,34 +234,50 @@ attn_jvp_rows_kernel(const AttnParams p) {
             }
         }
     };
-    // The max that the exponentials refer to moves to a row's own where an argument of that row is larger than kMaxSlack.  What has been formed already is scaled, the 16-bit operands of the
-    // tile before as well: their second rounding is 2^-kMaxSlack of the row's largest, and less, of what it would be there.
+    // The max that the exponentials refer to moves to a row's own where an argument of that row is larger than kMaxSlack.  The sums formed already are scaled in fp32: at once those that hold
+    // the tile before, the others one step later, when its outputs, of P and H as they were rounded, are among them.
+    constexpr int SUMMED = CHECK / PER - 8;     // groups of channels that hold the tile before when the max is looked at
+    bool late = false;                          // the others are still to be scaled, by
+    float factor[NG];
+#pragma unroll
+    for (int j = 0; j < NG; ++j) factor[j] = 1.f;
     auto row_top = [&](int j) {
         float v = fmaxf(fmaxf(fmaxf(x[j][0][0], x[j][0][1]), fmaxf(x[j][0][2], x[j][0][3])), fmaxf(fmaxf(x[j][1][0], x[j][1][1]), fmaxf(x[j][1][2], x[j][1][3])));
         v = fmaxf(v, __shfl_xor(v, 16));
         return fmaxf(v, __shfl_xor(v, 32));
     };
-    // (through LDS, four results at a time: accumulation registers go there as they are, and a copy that the compiler makes in this branch would have it keep them elsewhere)
+    // (through LDS, in which a wavefront's instructions keep their order: accumulation registers go there as they are, and a copy that the compiler makes in this branch would have it keep
+    // them elsewhere.  Four results are under way.)
     const unsigned spare = lds0 + C::SPARE_OFF + wave * 4 * kFragBytes + 16 * lane;
-    auto scale = [&](f32x4* a, int stride, const float* alpha) __attribute__((always_inline)) {
+    auto scale = [&](auto first, auto end, const float* alpha) __attribute__((always_inline)) {
+        constexpr int F0 = decltype(first)::value, N = decltype(end)::value - F0, COUNT = 2 * N * NG;
         f32x4 v[4];
-        for_each<4>([&](auto i) { lds_write_acc<decltype(i)::value * kFragBytes>(spare, a[decltype(i)::value * stride]); });
-        wait_lds<0>();
-        for_each<4>([&](auto i) { lds_read<decltype(i)::value * kFragBytes>(v[decltype(i)::value], spare); });
-        wait_lds<0>();
-        for_each<4>([&](auto i) {
+        auto result = [&](auto i) __attribute__((always_inline)) -> f32x4& {
+            constexpr int I = decltype(i)::value, f = F0 + I / 2 % N, j = I / (2 * N);
+            if constexpr (I % 2) return act[f][j];
+            else return acc[f][j];
+        };
+        auto fetch = [&](auto i) __attribute__((always_inline)) {
             constexpr int I = decltype(i)::value;
-            landed(v[I]);
+            lds_write_acc<I % 4 * kFragBytes>(spare, result(i));
+            lds_read<I % 4 * kFragBytes>(v[I % 4], spare);
+        };
+        for_each<4>(fetch);
+        for_each<COUNT>([&](auto i) {
+            constexpr int I = decltype(i)::value;
+            // LDS instructions behind the fetch of this one: three more fetches, and what the steps since have written and read back
+            constexpr int fetched = COUNT - 1 - I < 3 ? COUNT - 1 - I : 3, steps = I < 3 ? I : 3;
+            wait_lds<2 * fetched + 2 * steps>();
+            landed(v[I % 4]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[I][r] = *alpha > 0.f ? *alpha * v[I][r] : 0.f;
-            lds_write<I * kFragBytes>(spare, __builtin_bit_cast(rows_u32x4, v[I]));
+            for (int r = 0; r < 4; ++r) v[I % 4][r] = alpha[I / (2 * N)] > 0.f ? alpha[I / (2 * N)] * v[I % 4][r] : 0.f;
+            lds_write<I % 4 * kFragBytes>(spare, __builtin_bit_cast(rows_u32x4, v[I % 4]));
+            lds_read_acc<I % 4 * kFragBytes>(result(i), spare);
+            if constexpr (I + 4 < COUNT) fetch(Int<I + 4>{});
         });
         wait_lds<0>();
-        for_each<4>([&](auto i) { lds_read_acc<decltype(i)::value * kFragBytes>(a[decltype(i)::value * stride], spare); });
-        wait_lds<0>();
     };
-    auto raise = [&]() {
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");       // (products are asm: their results are in the registers now)
+    auto raise = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NG; ++j) {
             const float top_j = row_top(j), by = top_j > max_slack_of<T>(true) ? top_j : 0.f, alpha = __builtin_amdgcn_exp2f(-by);
@@ -269,22 +286,9 @@ attn_jvp_rows_kernel(const AttnParams p) {
             r_run[j] *= alpha;
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[j][e >> 2][e & 3] -= by;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const unsigned pi = pw[j][i], hi = hw[j][i];      // (a bit cast takes no element of a vector)
-                V2 a = __builtin_bit_cast(V2, pi), c = __builtin_bit_cast(V2, hi);
-                a = V2{(T)((float)a[0] * alpha), (T)((float)a[1] * alpha)};
-                c = V2{(T)((float)c[0] * alpha), (T)((float)c[1] * alpha)};
-                pw[j][i] = __builtin_bit_cast(unsigned, a);
-                hw[j][i] = __builtin_bit_cast(unsigned, c);
-            }
-#pragma unroll
-            for (int f = 0; f < NF; f += 4) {
-                scale(&acc[f][j], NG, &alpha);
-                scale(&act[f][j], NG, &alpha);
-            }
+            factor[j] = alpha;
         }
-        asm volatile("s_nop 7" ::: "memory");
+        scale(Int<0>{}, Int<SUMMED>{}, factor);
     };
 
     // ---- what a slot holds beside its product
@@ -301,7 +305,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
     };
     constexpr auto share = [room](int n, int q0, int q1, int q) { return q <= q0 ? 0 : q >= q1 ? n : n * room(q0, q) / room(q0, q1); };
     // arguments: of key half 0 behind its products, in the time of half 1's; of half 1 in the first output groups; then the max is looked at
-    constexpr int ARG_OPS = 3 * 2 * NG, CHECK = 10 * PER;
+    constexpr int ARG_OPS = 3 * 2 * NG;
     constexpr auto args_before = [share](int q) { return share(ARG_OPS, 4 * PER + NG, 8 * PER, q) + share(ARG_OPS, 8 * PER + NG, CHECK, q); };
     // P and H: of half 0 up to the last output group, of half 1 into the next step's S of half 0
     constexpr int EXP_HALF = 10 * 2 * NG, E0 = CHECK + 1, E1 = SLOTS + 4 * PER - NG;
@@ -364,7 +368,15 @@ attn_jvp_rows_kernel(const AttnParams p) {
     // Between the arguments of a tile and its exponentials: masks, and a max that has to move.  The loop turns here: what is rare is not inside of its body.
     auto settle = [&](int t) __attribute__((always_inline)) {
         if (need_mask(t)) mask(t);
-        if (__any(top > max_slack_of<T>(true))) raise();
+        const bool move = __any(top > max_slack_of<T>(true));
+        if (late || move) {
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");       // (products are asm: their results are in the registers now)
+            wait_lds<0>();                                            // (and the operands that are read ahead)
+            if (late) scale(Int<SUMMED>{}, Int<NF>{}, factor);
+            if (move) raise();
+            late = move;
+            asm volatile("s_nop 7" ::: "memory");
+        }
         top = -INFINITY;
     };
     // the rest of a step: outputs of the tile before, exponentials of this one
@@ -424,6 +436,10 @@ attn_jvp_rows_kernel(const AttnParams p) {
         for_each<CHECK>([&](auto q) { elements(Int<decltype(q)::value + SLOTS>{}); });
         v_slot = next_v(v_slot);
         SCHED_FENCE();
+        if (late) {
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+            scale(Int<SUMMED>{}, Int<NF>{}, factor);
+        }
         for_each<8>([&](auto gi) { group_now(Int<8 + decltype(gi)::value>{}); });
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products are in their registers

@@ -344,6 +344,31 @@ def test_tangent_rows_kernel_scores_that_move_the_max(pkg, oracle, gpu, stream_o
     assert oracle.error_metrics(lse.cpu(), lse_ref)[0] <= LSE_ABS * 4
 
 
+@pytest.mark.parametrize("behind", [0, 3])
+@pytest.mark.parametrize("moves", [1, 2])
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_rounds_once_where_the_max_moves(pkg, oracle, gpu, stream_override, forward_override, tangents, moves, behind):
+    """Weight in the tile before the one that moves the max, in one tile of four or in the last, once or twice running: P = 2^5 there, exact in 16 bits, v = 1 (and its tangent) and 0 elsewhere,
+    so that o is the one weight over the sum, both fp32, and rounded once: half a unit in the last place, and 2^-10 of one for fp32's own (2^-18: arguments of up to 16, exponentials, sums)."""
+    stream_override(chunk=1)
+    forward_override(ROWS_KERNEL)
+    Lq, Lkv = 150, 32 * (2 + moves + behind)
+    q, k, v = torch.zeros(1, 2, Lq, 128), torch.zeros(1, 2, Lkv, 128), torch.zeros(1, 2, Lkv, 128)
+    q[..., 0], q[..., 1] = 1.0, (0.05 + 2.0 * torch.rand(1, 2, Lq, generator=torch.Generator().manual_seed(moves))).to(torch.bfloat16).float()
+    k[..., 0] = -100.0                              # of no weight
+    k[:, :, 7, 0], k[:, :, 32 + 9, 0] = 0.0, 5.0    # the first max, and the weight that is looked at
+    for i in range(moves):                          # arguments of 6 and something above the max that there is
+        k[:, :, 64 + 32 * i + 20, 0], k[:, :, 64 + 32 * i + 20, 1] = 6.0 * (i + 1), i + 1.0
+    v[:, :, 32 + 9] = 1.0
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    tq, dev, scale = torch.zeros_like(q), lambda x: None if x is None else x.to(gpu), math.log(2.0)
+    o, to, _ = pkg.fwd_jvp(*(dev(x) for x in (q, k, v, tq)), *((None, None) if tangents == "q" else (dev(torch.zeros_like(k)), dev(v))), sm_scale=scale)
+    want = torch.softmax(q.double() @ k.double().transpose(2, 3) * scale, -1) @ v.double()
+    ulp = torch.exp2(torch.floor(torch.log2(want)) - 7)
+    for got in (o,) if tangents == "q" else (o, to):
+        assert ((got.cpu().double() - want).abs() <= (0.5 + 2.0 ** -10) * ulp).all()
+
+
 @pytest.mark.parametrize("tangents", ["q", "full"])
 def test_tangent_rows_kernel_ranges_layouts_and_choice(pkg, oracle, gpu, stream_override, forward_override, tangents):
     """Key ranges; [B, S, H, D] storage; bit for bit the same twice; the library's own choice of it at one round of workgroups (dense rows; fp16 and overlapping output rows: not)."""
