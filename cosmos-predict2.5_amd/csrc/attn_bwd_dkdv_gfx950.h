@@ -221,13 +221,13 @@ attn_dkdv_kernel(const BwdParams p) {
     };
     auto mask = [&](int t) {
         if (row0 + 16 * NG - 1 <= t * kRows) return;
+        // (key <= query, what a lane adds to either on one side: rows of keys, one register each, are not to be had with NG = 4, where dS is kept)
+        const int lane_part = l16 - 4 * g;
 #pragma unroll
         for (int kg = 0; kg < NG; ++kg) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int qrow = t * kRows + 16 * (e >> 2) + 4 * g + (e & 3);
-                x[kg][e >> 2][e & 3] = (row0 + 16 * kg + l16 <= qrow) ? x[kg][e >> 2][e & 3] : -INFINITY;
-            }
+            for (int e = 0; e < 8; ++e)
+                x[kg][e >> 2][e & 3] = lane_part <= t * kRows + 16 * (e >> 2) + (e & 3) - row0 - 16 * kg ? x[kg][e >> 2][e & 3] : -INFINITY;
         }
     };
 
@@ -358,13 +358,14 @@ attn_dkdv_kernel(const BwdParams p) {
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products (written as asm: no hazard checks) are in their registers
     __builtin_amdgcn_s_waitcnt(0x0F70);                     // drain the (unused) trailing loads before the LDS is released
 
-    // ---- epilogue: dV = dV^T, dK = s dK^T
+    // ---- epilogue: dV = dV^T, dK = s dK^T.  (The lane's part is counted anew: kept over the loop it takes registers that NG = 4, causal, dS kept, does not have)
+    const int lane_now = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)), l16_now = lane_now & 15, g_now = lane_now >> 4;
 #pragma unroll
     for (int kg = 0; kg < NG; ++kg) {
-        const int row = row0 + 16 * kg + l16;
+        const int row = row0 + 16 * kg + l16_now;
         if (partial) {   // a range of the stream only: leave the sums for bwd_combine_kernel ([row][dV | dK])
             const int64_t at = ((int64_t)(pair - p.n_full) * p.splits + split) * C::KEYS + row - blk * C::KEYS;
-            float* pa = p.part + at * (2 * D) + 4 * g;
+            float* pa = p.part + at * (2 * D) + 4 * g_now;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
                 asm volatile("" : "+a"(adv[kg][f]), "+a"(adk[kg][f]));
@@ -373,8 +374,8 @@ attn_dkdv_kernel(const BwdParams p) {
                 SCHED_FENCE();
             }
         } else if (row < p.L_stat) {
-            T* dv = reinterpret_cast<T*>(p.out1) + (int64_t)b * p.o1_sb + (int64_t)h * p.o1_sh + (int64_t)row * p.o1_sl + 4 * g;
-            T* dk = reinterpret_cast<T*>(p.out2) + (int64_t)b * p.o2_sb + (int64_t)h * p.o2_sh + (int64_t)row * p.o2_sl + 4 * g;
+            T* dv = reinterpret_cast<T*>(p.out1) + (int64_t)b * p.o1_sb + (int64_t)h * p.o1_sh + (int64_t)row * p.o1_sl + 4 * g_now;
+            T* dk = reinterpret_cast<T*>(p.out2) + (int64_t)b * p.o2_sb + (int64_t)h * p.o2_sh + (int64_t)row * p.o2_sl + 4 * g_now;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
                 asm volatile("" : "+a"(adv[kg][f]), "+a"(adk[kg][f]));

@@ -6,7 +6,9 @@ import math
 import os
 import random
 import re
+import struct
 
+import msgpack
 import pytest
 import torch
 
@@ -225,6 +227,32 @@ def test_forward_override_steers_plan_and_workspace(pkg, forward_override, forwa
         assert forward_plan((1, 3, 300, 128), 520, padded=True) == (rows, groups, pairs, 0, 1)
     forward_override()
     assert forward_plan((1, 3, 300, 128), 520) == default
+
+
+def built_kernels(path):
+    """name -> metadata of every kernel in the library's code objects (ELF images for AMDGPU, machine 224; an ELF note each, in msgpack)."""
+    data, at, kernels = open(path, "rb").read(), 0, {}
+    while (at := data.find(b"\x7fELF", at + 1)) >= 0:
+        if struct.unpack_from("<H", data, at + 18)[0] != 224:
+            continue
+        sections, (count,) = at + struct.unpack_from("<Q", data, at + 40)[0], struct.unpack_from("<H", data, at + 60)
+        for header in range(sections, sections + 64 * count, 64):
+            if struct.unpack_from("<I", data, header + 4)[0] != 7:      # SHT_NOTE
+                continue
+            note = at + struct.unpack_from("<Q", data, header + 24)[0]
+            name_size, size, _ = struct.unpack_from("<III", data, note)
+            body = note + 12 + (name_size + 3) // 4 * 4
+            kernels.update((k[".name"], k) for k in msgpack.unpackb(data[body:body + size], strict_map_key=False)["amdhsa.kernels"])
+    return kernels
+
+
+def test_kernels_of_lone_wavefronts_keep_their_registers(pkg):
+    """One wavefront per SIMD with up to 512 registers: what does not fit waits for memory in front of everything that is under way."""
+    kernels = built_kernels(pkg._lib.LIB_PATH)
+    for name, variants in (("attn_dkdv_kernel", 24), ("attn_jvp_rows_kernel", 2)):
+        found = {k: v for k, v in kernels.items() if name in k}
+        assert len(found) == variants
+        assert not [k for k, v in found.items() if v[".private_segment_fixed_size"] or v[".vgpr_spill_count"] or v[".sgpr_spill_count"]]
 
 
 def good_bwd_desc(pkg, **over):
