@@ -1906,7 +1906,7 @@ SplitPlan plan_shape(const cosmos_attn_desc* d, size_t room, int shape, int bloc
     const SplitPlan uncut = s;
     s.n_rem = rem; s.n_full = s.n_pairs - rem; s.splits = kMaxSplits;
     while (s.splits > 1 && partial_bytes(d, s) > room) --s.splits;
-    const bool steered = mode_of(d) == MODE_FWD || g_tangent_rows.load(std::memory_order_relaxed);
+    const bool tangents = g_tangent_rows.load(std::memory_order_relaxed) != 0, steered = mode_of(d) == MODE_FWD ? !tangents : tangents && shape == kRowsShape;
     const int asked = steered ? g_sym_ranges.load(std::memory_order_relaxed) : 0;
     if (asked > 0) s.splits = rem == 0 ? 1 : std::min({asked, s.splits, n_steps / kMinStepsPerSplit});
     else s.splits = choose_splits(rem, n_steps, cut, slot_bytes, s.splits);

@@ -229,6 +229,16 @@ def test_forward_override_steers_plan_and_workspace(pkg, forward_override, forwa
     assert forward_plan((1, 3, 300, 128), 520) == default
 
 
+@pytest.mark.parametrize("H, Lq, Lkv", [(16, 3520, 3520), (40, 1000, 3000), (3, 300, 520)])
+def test_forward_override_for_tangents_leaves_other_calls_alone(pkg, forward_override, H, Lq, Lkv):
+    other = [dense_desc(pkg, H, Lq, Lkv, None)] + [dense_desc(pkg, H, Lq, Lkv, t, dtype=pkg._lib.DTYPE_FP16) for t in ("q", "full")]
+    want = [plan_of(pkg, D) for D in other]
+    forward_override(192, 3)
+    assert [plan_of(pkg, D) for D in other] == want
+    plan = plan_of(pkg, dense_desc(pkg, H, Lq, Lkv, "full"))
+    assert plan[0] == 192 and plan[4] == 3
+
+
 def built_kernels(path):
     """name -> metadata of every kernel in the library's code objects (ELF images for AMDGPU, machine 224; an ELF note each, in msgpack)."""
     data, at, kernels = open(path, "rb").read(), 0, {}
