@@ -1042,7 +1042,9 @@ struct BwdGeom {
             for (int i = 2; i <= 4; ++i) {
                 const int blocks = (d->Lkv + 64 * i - 1) / (64 * i);
                 const bool fits = (int64_t)n_q_tiles * blocks * 2 * i * 2 * kFragBytes <= budget;      // a head's dS (padded keys are in it)
-                const double us = plan(blocks, (int)bh, n_q_tiles, d->causal != 0, d->d, true, 64 * i, dkdv_cost(i)).us;
+                const double us = d->causal && (int64_t)bh * n_k_tiles <= (kBlock / kRows) * kCausalPairs
+                    ? causal_cost(0, (int64_t)bh * blocks, [&](int64_t at) { return (n_q_tiles - at % blocks * (2 * i)) * dkdv_cost(i).step_us + dkdv_cost(i).range_us; })
+                    : plan(blocks, (int)bh, n_q_tiles, d->causal != 0, d->d, true, 64 * i, dkdv_cost(i)).us;
                 if (i == 2 || (fits && !least_fits) || (fits == least_fits && us < least)) { least = us; least_fits = fits; groups = i; }
             }
             block = 64 * groups;
@@ -1085,6 +1087,8 @@ struct BwdGeom {
     // wavefront: more keys are less LDS traffic and, per key, fewer instructions; fewer keys are more workgroups and less padding.  Fits to 24 sizes of 255 .. 84480 queries
     // x 64 .. 10920 keys, B*H = 16 .. 80, with 2, 3 and 4 groups and S = 1 .. 16 measured: the choice takes 1.001 times the best one's time on average, 1.02 at most
     // (us of a backward pass, 4 / 3 / 2 groups: 16 heads 37440 x 512 515 / 575 / 547, 37440 x 300 460 / 422 / 459, 1560 x 1560 113 / 111 / 100, 10920 x 10920 2410 / 2460 / 2630).
+    // Causal: a head's first block is the longest (causal_cost).  370 sizes of 204 .. 21828 positions, 8 .. 80 heads, all three measured: the choice takes 1.003 times the best one's time on average, and
+    // 1.02 at most that of the kernel of 128 keys before; priced in rounds 1.016 and 1.14.  (us, 4 / 3 / 2 groups, dS kept: 8 heads x 4189 278 / 245 / 219, 12 x 6270 489 / 534 / 484, 40 x 3774 535 / 550 / 622.)
     static StepCost dkdv_cost(int groups) { return groups == 4 ? StepCost{1.78, 8.0, 0.64} : groups == 3 ? StepCost{1.42, 8.0, 0.65} : StepCost{1.04, 8.0, 0.69}; }
     static StepCost recompute_cost(int d) { return StepCost{1.08 * (0.3 + 0.7 * d / 128.0), 8.0}; }
     static Plan plan(int n_blk, int bh, int n_stream_tiles, bool causal, int d, bool dkdv, int block, StepCost cost) {

@@ -230,6 +230,33 @@ inline double rounds_cost(int64_t pairs, double n_steps, StepCost c) {
     const double filled = (double)pairs / (double)(rounds * kNumCUs);
     return (double)rounds * (n_steps * c.step_us * (c.alone + (1.0 - c.alone) * filled * filled) + c.range_us);
 }
+// Causal calls: workgroups of unequal length.  They go out by id, to the 8 dies in turn and inside of a die to its 4 shader engines in turn, and one whose engine has none of its 8 units free holds
+// up the die's others.  So with 32 .. 36 blocks a head an engine gets the long ones of every head, and both sizes of workgroups take a quarter longer there than their work says.  The time of the
+// later of two dies, one of which has workgroup `first`, the longest.  (Up to kCausalPairs workgroups.)
+constexpr int kNumDies = 8, kCausalPairs = 16 * kNumCUs;
+template <typename F> inline double causal_cost(int64_t first, int64_t pairs, F us_of) {
+    constexpr int kEngines = 4, kUnits = kNumCUs / kNumDies / kEngines;
+    double end = 0.0;
+    for (int64_t die = first; die <= first + 2; die += 2) {
+        double free_at[kEngines][kUnits] = {}, now = 0.0;          // heaps: the unit that is free first is [0]
+        int engine = 0;
+        for (int64_t i = die % kNumDies; i < pairs; i += kNumDies, engine = (engine + 1) % kEngines) {
+            double* const unit = free_at[engine];
+            now = unit[0] > now ? unit[0] : now;
+            const double t = now + us_of(i);
+            end = t > end ? t : end;
+            int at = 0;
+            for (int next = 1; next < kUnits; next = 2 * at + 1) {
+                if (next + 1 < kUnits && unit[next + 1] < unit[next]) ++next;
+                if (unit[next] >= t) break;
+                unit[at] = unit[next];
+                at = next;
+            }
+            unit[at] = t;
+        }
+    }
+    return end;
+}
 // a value measured at head dims 16, 32, 64 and 128, and on the line between two of them for calls of unequal head dims
 inline double by_head_dim(const double (&at)[4], double d) {
     const int i = d > 64.0 ? 2 : d > 32.0 ? 1 : 0;
