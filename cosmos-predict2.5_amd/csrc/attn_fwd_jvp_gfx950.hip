@@ -1922,11 +1922,24 @@ SplitPlan plan_sym(const cosmos_attn_desc* d, size_t room, int shape) {
     return plan_shape(d, room, shape, 32 * w.rg, sym_steps(d), c, c);
 }
 // with tangents, and head dim 256: 128 rows a workgroup (score and output wavefronts), a barrier step is 32 keys
-SplitPlan plan_roles(const cosmos_attn_desc* d, size_t room) {
-    const int m = mode_of(d) == MODE_JVP_Q ? 0 : 1;
+StepCost roles_cost(const cosmos_attn_desc* d) {
     const double dim = 0.5 * (d->d_qk + d->d_v);
-    const StepCost cut{by_head_dim(kStepUs[m], dim), 8.0, by_head_dim(kStepAlone, dim)};
-    return plan_shape(d, room, 0, kBlockM, n_tiles_of(d), StepCost{cut.step_us, by_head_dim(kPairUs, dim), cut.alone}, cut);
+    return {by_head_dim(kStepUs[mode_of(d) == MODE_JVP_Q ? 0 : 1], dim), by_head_dim(kPairUs, dim), by_head_dim(kStepAlone, dim)};
+}
+SplitPlan plan_roles(const cosmos_attn_desc* d, size_t room) {
+    const StepCost whole = roles_cost(d);
+    return plan_shape(d, room, 0, kBlockM, n_tiles_of(d), whole, StepCost{whole.step_us, 8.0, whole.alone});
+}
+// Causal: a head's last block is the longest (causal_cost).  300 sizes of 600 .. 16000 positions, 8 .. 80 heads, both kernels measured: the choice takes 1.0035 times the better one's time on average, and
+// 0.973 of the 128-row kernel's, 5 of them more than 1.02 (at most 1.16); priced in rounds 0.994, 33 and 1.33.  (us, 128 / 192 rows: all tangents 12 heads x 6183 415 / 525, 20 x 3328 228 / 249; tangent
+// on q 80 x 6144 1890 / 2050, 80 x 4300 1130 / 810, 40 x 2953 285 / 320.)
+bool rows_cheaper(const cosmos_attn_desc* d, const SplitPlan& rows, const SplitPlan& roles) {
+    if (!d->causal || roles.n_pairs > kCausalPairs) return rows.us < roles.us;
+    auto us = [&](const SplitPlan& s, StepCost c) {
+        const int n_tiles = n_tiles_of(d), per_block = s.block_m / kBlockN;
+        return causal_cost(s.n_pairs - 1, s.n_pairs, [&](int64_t at) { return std::min(n_tiles, (int)(at % s.n_qt + 1) * per_block) * c.step_us + c.range_us; });
+    };
+    return us(rows, kRowsWhole[mode_of(d) == MODE_JVP_Q ? 0 : 1]) < us(roles, roles_cost(d));
 }
 bool in_place_whole(const cosmos_attn_desc* d);
 SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
@@ -1941,7 +1954,7 @@ SplitPlan plan_split(const cosmos_attn_desc* d, size_t room) {
         // Whole pairs are dealt out alike whether there is room for partial results or not, so that the two-stage run, which has none, and the in-place call take the kernel that the
         // one-call form takes wherever that does not cut: from seven eighths of a round of them on.  (Below, the estimate for a round that is not full is the less sure one: 16 heads,
         // tangent on q, 2120 x 1024 54.5 us for 60 of attn_qstream_kernel, but 8 heads x 4213 causal 146 for 132, all tangents 16 x 2197 causal 113 for 101.)
-        if (r.us >= s.us || (r.splits < 2 && 8 * r.n_pairs < 7 * kNumCUs)) return s;
+        if (!rows_cheaper(d, r, s) || (r.splits < 2 && 8 * r.n_pairs < 7 * kNumCUs)) return s;
         // A call that can be read in place, whole pairs of 128 rows, is: the estimates are of calls that are re-tiled.  us, in place / 192 rows: 16 heads 368 21.6 / 32.6, 500 26.0 / 36.5, 8 heads
         // 345 20.3 / 30.1, 80 heads 459 55.3 / 51.5, 2411 670 / 654.
         return in_place_whole(d) ? s : r;
