@@ -2008,6 +2008,8 @@ constexpr double kStreamBlockUs[2][4] = {{2.5, 2.0, 0.5, 1.0}, {3.5, 2.5, 0.5, 6
 constexpr double kStreamStartUs[4] = {5.0, 5.0, 5.0, 0.0};
 // attn_jvp_rows_kernel on the other side: its tiles are the cheaper ones, its workgroups the dearer.  us, stream / that, 16 heads: tangent on q 20000 x 1024 318 / 336, x 2048 600 / 573; all
 // tangents 37440 x 512 470 / 491 (2 x 16 heads 930 / 937), 20000 x 1024 451 / 437, x 2048 808 / 772.
+// Not where keys are padded, of whose number the host does not know: there the line is the one to attn_fwd_jvp_kernel.  us, stream / rows, with all keys valid, a half, a quarter: tangent on q 16 heads 37440 x 1600
+// 896 / 831, 471 / 490, 267 / 342, 40 heads 8000 x 1600 486 / 462, 259 / 282, 152 / 190; all tangents 16 heads 37440 x 1024 798 / 777, 446 / 473, 277 / 321.
 constexpr int kStreamRowsTiles[2] = {48, 24};
 constexpr int kStreamMinPairs = kNumCUs / 2;   // fewer query blocks than that leave most units idle; both ways take some 25 us
 std::atomic<int> g_stream_chunk{0};       // query blocks per workgroup (1 = never stream), 0 = the library's own choice
@@ -2028,11 +2030,12 @@ int stream_groups_of(const cosmos_attn_desc* d, const SplitPlan& other) {
     const int groups = kNumCUs * kStreamGroupsPerCU;
     const int mode = mode_of(d);
     // (`other` without room for partial results may be this kernel where with room it is a cut of 128 rows, which then streams: so does the two-stage run)
-    if (mode != MODE_FWD && other.shape == kRowsShape && n_tiles_of(d) > kStreamRowsTiles[mode == MODE_JVP_Q ? 0 : 1] && plan_split(d, kNoLimit).shape == kRowsShape) return 0;
+    const bool rows = mode != MODE_FWD && other.shape == kRowsShape;
+    if (rows && !d->key_lens && n_tiles_of(d) > kStreamRowsTiles[mode == MODE_JVP_Q ? 0 : 1] && plan_split(d, kNoLimit).shape == kRowsShape) return 0;
     if (mode == MODE_JVP_FULL) return pairs >= 4 * kNumCUs ? groups : 0;
     const double tile_us = by_head_dim(kStreamTileUs[mode], d->d_qk), block_us = by_head_dim(kStreamBlockUs[mode], d->d_qk);
     const double stream_us = by_head_dim(kStreamStartUs, d->d_qk) + (double)((pairs + groups - 1) / groups) * (n_tiles_of(d) * tile_us + block_us);
-    return stream_us <= other.us ? groups : 0;
+    return stream_us <= (rows && d->key_lens ? plan_roles(d, 0).us : other.us) ? groups : 0;
 }
 // LDS of attn_qstream_kernel: the layout of attn_fwd_jvp_kernel (AttnCfg::LDS_BYTES) + the per-block statistics slots
 size_t stream_lds_bytes_of(const cosmos_attn_desc* d) {

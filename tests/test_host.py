@@ -186,6 +186,13 @@ def test_causal_calls_with_tangents_take_the_workgroups_that_end_first(pkg, H, L
     assert plan_of(pkg, dense_desc(pkg, H, L, L, tangents, causal=1))[0] == rows
 
 
+@pytest.mark.parametrize("H, Lq, Lkv, tangents", [(16, 37440, 1600, "q"), (20, 11241, 1910, "q"), (16, 37440, 1024, "full"), (12, 24356, 886, "full")])
+def test_padded_calls_are_streamed(pkg, H, Lq, Lkv, tangents):
+    """A block of the other kernel costs as much beside its keys as sixteen tiles of them, and the host does not know how many are valid."""
+    assert plan_of(pkg, dense_desc(pkg, H, Lq, Lkv, tangents, key_lens=0x7F0000000000)) == "streamed"
+    assert plan_of(pkg, dense_desc(pkg, H, Lq, Lkv, tangents))[0] == 192
+
+
 @pytest.mark.parametrize("tangents", [None, "q", "full"])
 def test_forms_of_a_call_that_is_not_cut_take_the_same_kernel(pkg, tangents):
     """What runs without room for partial results (the two-stage run, the in-place call) is what the one-call form runs wherever that cuts no keys: the same results, bit for bit.
