@@ -157,7 +157,7 @@ struct AttnParams {
     // attn_qstream_kernel: BH = batch * heads (the kernel deals the (query block, head) pairs out over its workgroups itself)
     int BH, q_chunk;
     float* part_acc;           // [slot][block_m][d_v] accumulators; with tangents [slot][block_m][2][d_v] (O, T)
-    float4* part_stat;         // [slot][block_m]: (running max in log2 units, row sum of P, row sum of H, 0)
+    float4* part_stat;         // [slot][block_m]: (running max in log2 units, row sum of P, row sum of H, the row sum of P that outputs are divided by)
 };
 
 extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -662,7 +662,7 @@ attn_fwd_jvp_kernel(const AttnParams p) {
         if (partial) {   // a key range only: leave the statistics for attn_combine_kernel
             if (hh == 0) {
                 const int64_t slot = (int64_t)(pair - p.n_full) * p.splits + split;
-                p.part_stat[slot * kBlockM + qw * 32 + j] = make_float4(w.m_run, l_tot, r_tot, 0.f);
+                p.part_stat[slot * kBlockM + qw * 32 + j] = make_float4(w.m_run, l_tot, r_tot, l_tot);
             }
         } else if (row < p.Lq && p.lse && hh == 0) {
             p.lse[(int64_t)bh * p.Lq + row] = (w.m_run + __builtin_log2f(l_tot)) * 0.6931471805599453f;
@@ -1656,7 +1656,7 @@ attn_fwd_sym_kernel(const AttnParams p) {
         // a key range only: leave acc, m, l as they are for attn_combine_kernel (rows past Lq are written too and
         // never combined)
         const int64_t slot = (int64_t)(pair - p.n_full) * p.splits + split;
-        if (kg == 0 && hh == 0) p.part_stat[slot * BLOCK_M + rg * 32 + j] = make_float4(m_all, l_tot, 0.f, 0.f);
+        if (kg == 0 && hh == 0) p.part_stat[slot * BLOCK_M + rg * 32 + j] = make_float4(m_all, l_tot, 0.f, l_tot);
 #pragma unroll
         for (int n = 0; n < N; ++n) {
             float* pa = p.part_acc + (slot * BLOCK_M + rg * 32 + QR * n + at % QR) * DV;
@@ -1693,8 +1693,8 @@ attn_fwd_sym_kernel(const AttnParams p) {
 }
 
 // Merge the key-range partial results of one query row:  M = max m_i,  w_i = 2^(m_i - M),  L = sum l_i w_i,
-// O = sum acc_i w_i / L,  LSE = (M + log2 L) ln 2; with tangents also T = sum accT_i w_i, R = sum r_i w_i and
-// dO = (T - (R / L) sum acc_i w_i) / L.  One thread per (row, 4 output channels); fixed order over the ranges.
+// O = sum acc_i w_i / D,  D = sum d_i w_i (l_i, or their sum of P as rounded),  LSE = (M + log2 L) ln 2; with tangents also T = sum accT_i w_i, R = sum r_i w_i and
+// dO = (T - (R / D) sum acc_i w_i) / D.  One thread per (row, 4 output channels); fixed order over the ranges.
 template <typename T, bool JVP>
 __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnParams p, int dv, int block_m) {
     typedef typename VecOf<T>::v4 V4;
@@ -1710,7 +1710,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnParams p, i
     const int acc_w = JVP ? 2 * dv : dv;                      // floats per row in part_acc
     float M = -INFINITY;
     for (int i = 0; i < p.splits; ++i) M = fmaxf(M, p.part_stat[(slot0 + i) * block_m + wrow].x);
-    float L = 0.f, R = 0.f;
+    float L = 0.f, R = 0.f, D = 0.f;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f), t = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int i = 0; i < p.splits; ++i) {
         const float4 st = p.part_stat[(slot0 + i) * block_m + wrow];
@@ -1718,6 +1718,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnParams p, i
         const float* pa = p.part_acc + ((slot0 + i) * block_m + wrow) * acc_w + c;
         const float4 a = *reinterpret_cast<const float4*>(pa);
         L += st.y * wgt;
+        D += st.w * wgt;
         o.x += a.x * wgt; o.y += a.y * wgt; o.z += a.z * wgt; o.w += a.w * wgt;
         if (JVP) {
             const float4 at = *reinterpret_cast<const float4*>(pa + dv);
@@ -1725,7 +1726,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnParams p, i
             t.x += at.x * wgt; t.y += at.y * wgt; t.z += at.z * wgt; t.w += at.w * wgt;
         }
     }
-    const float inv_l = 1.0f / L;
+    const float inv_l = 1.0f / D;
     const int64_t off = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl + c;
     V4 ov;
     ov[0] = (T)(o.x * inv_l); ov[1] = (T)(o.y * inv_l); ov[2] = (T)(o.z * inv_l); ov[3] = (T)(o.w * inv_l);

@@ -1,5 +1,5 @@
 // Forward + JVP at head dim 128, bf16, from about a round of workgroups on.  Included inside the anonymous namespace of attn_fwd_jvp_gfx950.hip, behind attn_mfma16_gfx950.h
-// (same image of K and V, same arithmetic and rounding as ScoreWave16 / OutputWave16).
+// (same image of K and V, same arithmetic and rounding as ScoreWave16 / OutputWave16, but for the sums that outputs are divided by).
 //
 // A workgroup of four wavefronts, one per SIMD, owns 64 NG query rows; a wavefront does all of it for its own 16 NG: Q in vector registers and dQ in accumulation registers as B operands, S and dS,
 // the softmax, P and H, which rounded are the B operands of the outputs' products as they lie, O^T and T^T in accumulation registers.  Nothing is handed over through LDS, a K or V
@@ -7,7 +7,7 @@
 //
 // What bounds it: the part's power limit and, next to that, instruction issue.  A wavefront alone on its SIMD hides two other instructions behind a v_mfma_f32_16x16x32 of
 // 16 cycles (measured: with two 18 cycles, three 22, four 26; an exponential counts twice), so a step is written in slots, a product and what is issued beside it, with the elements'
-// work spread by the room that LDS reads, waits and loads leave (fixed(), room(), args_before(), exps_before()).  A step of 144 products takes 3030 cycles (84480 positions, all tangents: matrix units busy 78 %, 1.93 GHz).
+// work spread by the room that LDS reads, waits and loads leave (fixed(), room(), args_before(), exps_before()).  A step is 150 products with all tangents, 102 with one on q alone.
 // 16 heads x 33000 positions, all tangents, attn_fwd_jvp_kernel / this: LDS-active cycles 1085 / 364 million, 34.3 / 35.4 million cycles, 1.69 / 1.95 GHz, 20.36 / 18.18 ms; tangent on q
 // 15.06 / 12.71 ms (further sizes beside kRowsWhole).
 //
@@ -28,6 +28,13 @@ struct RowsCfg {
     static constexpr int K_LOADS = A::KP_FR / 4, V_LOADS = A::VP_FR / 4;      // per wavefront and step
 };
 constexpr int kRowsThreads = 256;
+// How far an argument of the exponentials may lie above the max that they refer to, in powers of two.  Moving the max costs a wavefront some 2 us here, and 192 rows wait for each other: with kMaxSlack, whose
+// 6 keep p in fp16's range, scores of a standard deviation of 4 had it in most steps.  bf16 and fp32 have the range (sums stay below 2^40 times their terms).  What an exact max has is that the
+// largest p, 1, is not rounded; so outputs are divided by sums of p as it is rounded, which a row's largest p has its error in as well: six products a step, for the 24 additions of the sum of H.
+// us, 6 / 40 (attn_fwd_jvp_kernel), 16 heads, scores of standard deviation 4: all tangents 3072 x 2000 256 / 128 (160), 20000 x 2000 1590 / 780 (851), tangent on q 6144 897 / 478 (584), 37440 x 2048 2570 / 1110;
+// 8: 280 / 135 (164), 1760 / 778 (876), 1030 / 480 (591); 1: 128 / 127 (153), 777 / 774 (800), 473 / 478 (559), 20000 4760 / 4840, all tangents 84480 115.0 / 114.9 ms.
+// Error against 64 bits, o (dO of a tangent on q), 1000 keys: 1: 2.359e-3 / 2.353e-3 (2.369 / 2.365); 4: 2.02 / 1.88 (3.97 / 2.75); 8: 1.92 / 1.74 (5.19 / 2.95); attn_fwd_jvp_kernel 2.33 (2.37); 1.83 (3.87); 1.65 (4.72).
+constexpr float kRowsSlack = 40.f;
 
 typedef unsigned rows_u32x4 __attribute__((ext_vector_type(4)));
 // (PAUSE: in front of the loop and behind it, where the compiler may copy an operand just before its use; of the wait that this takes it does not know, asm being asm)
@@ -135,12 +142,16 @@ attn_jvp_rows_kernel(const AttnParams p) {
     f32x4 x[NG][2], y[NG][2];                   // S, then S c - max, then P | dS, then H
     rows_u32x4 pw[NG], hw[NG];                  // P, H rounded: B operands
     f32x4 acc[NF][NG], act[NF][NG];             // O^T, T^T: channels 16 f + 4 g + r of row 16 j + l16
-    float m_run[NG], l_run[NG], r_run[NG];      // running max; this lane's keys' share of the row sums of P and H
+    float m_run[NG], l_run[NG];                 // running max; this lane's keys' share of the row sum of P
+    f32x4 psum[NG], hsum[NG];                   // row sums of P and H as rounded (of row 16 j + l16, in every register): what outputs are divided by has then the same errors as what is divided
+    rows_u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+    landed(ones);                               // (in registers, not formed again in the loop)
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
 #pragma unroll
         for (int f = 0; f < NF; ++f) { acc[f][j] = f32x4{0.f, 0.f, 0.f, 0.f}; act[f][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
-        m_run[j] = l_run[j] = r_run[j] = 0.f;
+        m_run[j] = l_run[j] = 0.f;
+        psum[j] = hsum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         pw[j] = hw[j] = rows_u32x4{0, 0, 0, 0};
     }
 
@@ -187,6 +198,14 @@ attn_jvp_rows_kernel(const AttnParams p) {
         }
     };
 
+    // the sums' products, beside those of a group of outputs
+    constexpr int SUMS_AT = 12;
+    auto sums = [&](auto ki, auto pause) __attribute__((always_inline)) {
+        constexpr int K = decltype(ki)::value;
+        if constexpr (K < NG) M::template more<decltype(pause)::value, false>(hsum[K], ones, hw[K]);
+        else M::template more<decltype(pause)::value, false>(psum[K - NG], ones, pw[K - NG]);
+    };
+
     // ---- the elements' arithmetic, in single instructions, pairs (r even, odd) numbered [key half][16 rows][r / 2]
     constexpr int PAIRS = 4 * NG;
     float top = -INFINITY;                      // of all arguments of the exponentials of this lane
@@ -196,17 +215,14 @@ attn_jvp_rows_kernel(const AttnParams p) {
         if constexpr (K < 2) x[j][m][r + K] = __builtin_fmaf(x[j][m][r + K], p.scale_log2, -m_run[j]);
         else { top = __builtin_fmaxf(__builtin_fmaxf(top, x[j][m][r]), x[j][m][r + 1]); landed(top); }      // (kept here: the compiler would form it at the loop's end)
     };
-    // P and H: per pair two exponentials, two products with the scale, two products, four sums
+    // P and H: per pair two exponentials, two products with the scale, two products, two sums
     auto exp_op = [&](auto oi) __attribute__((always_inline)) {
-        constexpr int O = decltype(oi)::value, P = O / 10, K = O % 10, m = P / (2 * NG), j = P / 2 % NG, r = 2 * (P % 2) + K % 2;
+        constexpr int O = decltype(oi)::value, P = O / 8, K = O % 8, m = P / (2 * NG), j = P / 2 % NG, r = 2 * (P % 2) + K % 2;
         if constexpr (K < 2) x[j][m][r] = __builtin_amdgcn_exp2f(x[j][m][r]);
         else if constexpr (K < 4) y[j][m][r] *= p.sm_scale;
         else if constexpr (K < 6) y[j][m][r] *= x[j][m][r];
-        else if constexpr (K < 8) l_run[j] += x[j][m][r];
-        else r_run[j] += y[j][m][r];
-        // (kept here: the compiler would form the sums at the loop's end)
-        if constexpr (K == 7) landed(l_run[j]);
-        if constexpr (K == 9) landed(r_run[j]);
+        else l_run[j] += x[j][m][r];
+        if constexpr (K == 7) landed(l_run[j]);      // (kept here: the compiler would form the sums at the loop's end)
     };
     // rounding: a pair's word of P or H
     auto round_p = [&](auto pi) __attribute__((always_inline)) {
@@ -234,7 +250,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
             }
         }
     };
-    // The max that the exponentials refer to moves to a row's own where an argument of that row is larger than kMaxSlack.  The sums formed already are scaled in fp32: at once those that hold
+    // The max that the exponentials refer to moves to a row's own where an argument of that row is larger than kRowsSlack.  The sums formed already are scaled in fp32: at once those that hold
     // the tile before, the others one step later, when its outputs, of P and H as they were rounded, are among them.
     constexpr int SUMMED = CHECK / PER - 8;     // groups of channels that hold the tile before when the max is looked at
     bool late = false;                          // the others are still to be scaled, by
@@ -277,13 +293,17 @@ attn_jvp_rows_kernel(const AttnParams p) {
         });
         wait_lds<0>();
     };
+    auto scale_late = [&]() __attribute__((always_inline)) {
+        scale(Int<SUMMED>{}, Int<NF>{}, factor);
+#pragma unroll
+        for (int j = 0; j < NG; ++j) { psum[j] *= factor[j]; hsum[j] *= factor[j]; }
+    };
     auto raise = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NG; ++j) {
-            const float top_j = row_top(j), by = top_j > max_slack_of<T>(true) ? top_j : 0.f, alpha = __builtin_amdgcn_exp2f(-by);
+            const float top_j = row_top(j), by = top_j > kRowsSlack ? top_j : 0.f, alpha = __builtin_amdgcn_exp2f(-by);
             m_run[j] += by;
             l_run[j] *= alpha;
-            r_run[j] *= alpha;
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[j][e >> 2][e & 3] -= by;
             factor[j] = alpha;
@@ -296,7 +316,8 @@ attn_jvp_rows_kernel(const AttnParams p) {
     constexpr auto fixed = [](int q) {
         q %= SLOTS;
         const int G = q / PER, k = q % PER;
-        return (k == 0) + (FULL && k == 1) + (k == PER - 1) + (k == 2 && G == LOAD_AT ? C::K_LOADS : 0) + (k == 2 && G == LOAD_AT + 2 ? C::V_LOADS : 0);
+        // (a slot with two products has room for two instructions more)
+        return (k == 0) + (FULL && k == 1) + (k == PER - 1) + (k == 2 && G == LOAD_AT ? C::K_LOADS : 0) + (k == 2 && G == LOAD_AT + 2 ? C::V_LOADS : 0) - (G == SUMS_AT && k < 2 * NG ? 2 : 0);
     };
     constexpr auto room = [fixed](int q0, int q) {
         int c = 0;
@@ -308,13 +329,13 @@ attn_jvp_rows_kernel(const AttnParams p) {
     constexpr int ARG_OPS = 3 * 2 * NG;
     constexpr auto args_before = [share](int q) { return share(ARG_OPS, 4 * PER + NG, 8 * PER, q) + share(ARG_OPS, 8 * PER + NG, CHECK, q); };
     // P and H: of half 0 up to the last output group, of half 1 into the next step's S of half 0
-    constexpr int EXP_HALF = 10 * 2 * NG, E0 = CHECK + 1, E1 = SLOTS + 4 * PER - NG;
+    constexpr int EXP_HALF = 8 * 2 * NG, E0 = CHECK + 1, E1 = SLOTS + 4 * PER - NG;
     constexpr auto exps_before = [room](int q) {
         if (q <= E0) return 0;
         if (q >= E1) return 2 * EXP_HALF;
-        const int done = 12 * PAIRS * room(E0, q) / room(E0, E1);              // 2 2 1 1 1 1 1 1 1 1 a pair
-        const int rest = done % 12;
-        return 10 * (done / 12) + (rest < 2 ? 0 : rest < 4 ? 1 : rest - 2);
+        const int done = 10 * PAIRS * room(E0, q) / room(E0, E1);              // 2 2 1 1 1 1 1 1 a pair
+        const int rest = done % 10;
+        return 8 * (done / 10) + (rest < 2 ? 0 : rest < 4 ? 1 : rest - 2);
     };
     static_assert(exps_before(15 * PER + NG) >= EXP_HALF, "the first half is rounded behind its last operand's last use");
     int t_kload = n_tiles_all < 2 ? 0 : tile_at(C::KRING), t_vload = n_tiles_all < 2 ? 0 : tile_at(C::VRING - 1);      // (one tile: one step, whose loads nobody reads)
@@ -330,7 +351,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
             constexpr auto pairs_before = [exps_before](int q) {
                 if (q <= SLOTS + NG) return 0;
                 if (q >= SLOTS + 4 * PER - 1) return 2 * NG;
-                const int e = exps_before(q - 1) / 10 - 2 * NG;
+                const int e = exps_before(q - 1) / 8 - 2 * NG;
                 return e < 0 ? 0 : e;
             };
             for_each<pairs_before(Q + 1) - pairs_before(Q)>([&](auto i) {
@@ -346,6 +367,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
         constexpr bool LAST = decltype(last)::value;
         SCHED_FENCE();
         product(Int<G>{}, Int<K>{}, Int<0>{});
+        if constexpr (G == SUMS_AT && K < 2 * NG) sums(Int<K>{}, Int<0>{});
         if constexpr (K == 0) {
             if constexpr (G + AHEAD == 16) k_slot = next_k(k_slot);             // the reads go on to the next K, or V
             if constexpr (G + AHEAD == 8) v_slot = next_v(v_slot);
@@ -368,11 +390,11 @@ attn_jvp_rows_kernel(const AttnParams p) {
     // Between the arguments of a tile and its exponentials: masks, and a max that has to move.  The loop turns here: what is rare is not inside of its body.
     auto settle = [&](int t) __attribute__((always_inline)) {
         if (need_mask(t)) mask(t);
-        const bool move = __any(top > max_slack_of<T>(true));
+        const bool move = __any(top > kRowsSlack);
         if (late || move) {
             asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");       // (products are asm: their results are in the registers now)
             wait_lds<0>();                                            // (and the operands that are read ahead)
-            if (late) scale(Int<SUMMED>{}, Int<NF>{}, factor);
+            if (late) scale_late();
             if (move) raise();
             late = move;
             asm volatile("s_nop 7" ::: "memory");
@@ -438,22 +460,25 @@ attn_jvp_rows_kernel(const AttnParams p) {
         SCHED_FENCE();
         if (late) {
             asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-            scale(Int<SUMMED>{}, Int<NF>{}, factor);
+            scale_late();
         }
         for_each<8>([&](auto gi) { group_now(Int<8 + decltype(gi)::value>{}); });
+        for_each<2 * NG>([&](auto k) { sums(k, Int<1>{}); });
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the last products are in their registers
+#pragma unroll
+    for (int j = 0; j < NG; ++j) { landed(psum[j]); landed(hsum[j]); }      // (all of them: what nobody reads is nobody else's register before)
     __builtin_amdgcn_s_waitcnt(0x0F70);                     // drain the (unused) trailing loads before the LDS is released
 
     // ---- epilogue: O = acc / l ; dO = (T - (r / l) acc) / l ; LSE = (m + log2 l) ln 2
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
         auto total = [](float v) { v += __shfl_xor(v, 16); return v + __shfl_xor(v, 32); };
-        const float l = total(l_run[j]), r = total(r_run[j]);
+        const float l = total(l_run[j]), p_sum = psum[j][0], h_sum = hsum[j][0];
         const int row = row0 + 16 * j + l16;
         if (partial) {   // a key range only: leave accumulators and statistics for attn_combine_kernel
             const int64_t at = ((int64_t)(pair - p.n_full) * p.splits + split) * C::ROWS + wave * 16 * NG + 16 * j + l16;
-            if (g == 0) p.part_stat[at] = make_float4(m_run[j], l, r, 0.f);
+            if (g == 0) p.part_stat[at] = make_float4(m_run[j], l, h_sum, p_sum);
             float* pa = p.part_acc + at * 256 + 4 * g;
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
@@ -463,7 +488,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
                 SCHED_FENCE();
             }
         } else if (row < p.Lq) {
-            const float inv_l = 1.0f / l, r_over_l = r * inv_l;
+            const float inv_l = 1.0f / p_sum, r_over_l = h_sum * inv_l;
             const int64_t off = (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)row * p.o_sl + 4 * g;
             T* op = reinterpret_cast<T*>(p.o) + off;
             T* tp = reinterpret_cast<T*>(p.to) + off;

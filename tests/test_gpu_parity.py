@@ -348,17 +348,17 @@ def test_tangent_rows_kernel_scores_that_move_the_max(pkg, oracle, gpu, stream_o
 @pytest.mark.parametrize("moves", [1, 2])
 @pytest.mark.parametrize("tangents", ["q", "full"])
 def test_tangent_rows_kernel_rounds_once_where_the_max_moves(pkg, oracle, gpu, stream_override, forward_override, tangents, moves, behind):
-    """Weight in the tile before the one that moves the max, in one tile of four or in the last, once or twice running: P = 2^5 there, exact in 16 bits, v = 1 (and its tangent) and 0 elsewhere,
-    so that o is the one weight over the sum, both fp32, and rounded once: half a unit in the last place, and 2^-10 of one for fp32's own (2^-18: arguments of up to 16, exponentials, sums)."""
+    """Weight in the tile before the one that moves the max, in one tile of four or in the last, once or twice running: P = 2^30 there, exact in 16 bits, v = 1 (and its tangent) and 0 elsewhere,
+    so that o is the one weight over the sum, both fp32, and rounded once: half a unit in the last place, and 2^-8 of one for fp32's own (2^-16: arguments of up to 90, exponentials, sums)."""
     stream_override(chunk=1)
     forward_override(ROWS_KERNEL)
     Lq, Lkv = 150, 32 * (2 + moves + behind)
     q, k, v = torch.zeros(1, 2, Lq, 128), torch.zeros(1, 2, Lkv, 128), torch.zeros(1, 2, Lkv, 128)
     q[..., 0], q[..., 1] = 1.0, (0.05 + 2.0 * torch.rand(1, 2, Lq, generator=torch.Generator().manual_seed(moves))).to(torch.bfloat16).float()
     k[..., 0] = -100.0                              # of no weight
-    k[:, :, 7, 0], k[:, :, 32 + 9, 0] = 0.0, 5.0    # the first max, and the weight that is looked at
-    for i in range(moves):                          # arguments of 6 and something above the max that there is
-        k[:, :, 64 + 32 * i + 20, 0], k[:, :, 64 + 32 * i + 20, 1] = 6.0 * (i + 1), i + 1.0
+    k[:, :, 7, 0], k[:, :, 32 + 9, 0] = 0.0, 30.0   # the first max, and the weight that is looked at
+    for i in range(moves):                          # arguments of 41 and something above the max that there is
+        k[:, :, 64 + 32 * i + 20, 0], k[:, :, 64 + 32 * i + 20, 1] = 41.0 * (i + 1), i + 1.0
     v[:, :, 32 + 9] = 1.0
     q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
     tq, dev, scale = torch.zeros_like(q), lambda x: None if x is None else x.to(gpu), math.log(2.0)
@@ -366,7 +366,27 @@ def test_tangent_rows_kernel_rounds_once_where_the_max_moves(pkg, oracle, gpu, s
     want = torch.softmax(q.double() @ k.double().transpose(2, 3) * scale, -1) @ v.double()
     ulp = torch.exp2(torch.floor(torch.log2(want)) - 7)
     for got in (o,) if tangents == "q" else (o, to):
-        assert ((got.cpu().double() - want).abs() <= (0.5 + 2.0 ** -10) * ulp).all()
+        assert ((got.cpu().double() - want).abs() <= (0.5 + 2.0 ** -8) * ulp).all()
+
+
+@pytest.mark.parametrize("ranges", [1, 3])
+@pytest.mark.parametrize("spread", [1.0, 4.0, 8.0])
+@pytest.mark.parametrize("tangents", ["q", "full"])
+def test_tangent_rows_kernel_is_as_exact_on_scores_that_spread(pkg, oracle, gpu, stream_override, forward_override, tangents, spread, ranges):
+    """Scores of that standard deviation, whose largest lie far above the first tile's: the errors are those of the other kernel, whose max follows closer (o: emulated 1.00 to 1.07 times,
+    and 5 % of scatter between two orders of the keys; what is divided by rounded sums cannot be worse for them)."""
+    stream_override(chunk=1)
+    x = list(oracle.make_inputs((1, 4, 600, 128), (1, 4, 1000, 128), seed=int(spread)))
+    x[0], x[1] = ((t.float() * spread ** 0.5).to(torch.bfloat16) for t in x[:2])
+    if tangents == "q":
+        x[4] = x[5] = None
+    want = oracle.closed_form(*x)[:2]
+    errors = []
+    for rows in (0, ROWS_KERNEL):
+        forward_override(rows, ranges if rows else 0)
+        got = pkg.fwd_jvp(*(None if t is None else t.to(gpu) for t in x))[:2]
+        errors.append([oracle.error_metrics(a.float().cpu(), b)[1] for a, b in zip(got, want)])
+    assert errors[1][0] <= 1.12 * errors[0][0] and errors[1][1] <= 1.05 * errors[0][1], errors
 
 
 @pytest.mark.parametrize("tangents", ["q", "full"])
