@@ -32,7 +32,7 @@ constexpr int kRowsThreads = 256;
 // 6 keep p in fp16's range, scores of a standard deviation of 4 had it in most steps.  bf16 and fp32 have the range (sums stay below 2^40 times their terms).  What an exact max has is that the
 // largest p, 1, is not rounded; so outputs are divided by sums of p as it is rounded, which a row's largest p has its error in as well: six products a step, for the 24 additions of the sum of H.
 // us, 6 / 40 (attn_fwd_jvp_kernel), 16 heads, scores of standard deviation 4: all tangents 3072 x 2000 256 / 128 (160), 20000 x 2000 1590 / 780 (851), tangent on q 6144 897 / 478 (584), 37440 x 2048 2570 / 1110;
-// 8: 280 / 135 (164), 1760 / 778 (876), 1030 / 480 (591); 1: 128 / 127 (153), 777 / 774 (800), 473 / 478 (559), 20000 4760 / 4840, all tangents 84480 115.0 / 114.9 ms.
+// 8: 280 / 135 (164), 1760 / 778 (876), 1030 / 480 (591); 1: 128 / 127 (153), 777 / 774 (800), 473 / 476 (559).
 // Error against 64 bits, o (dO of a tangent on q), 1000 keys: 1: 2.359e-3 / 2.353e-3 (2.369 / 2.365); 4: 2.02 / 1.88 (3.97 / 2.75); 8: 1.92 / 1.74 (5.19 / 2.95); attn_fwd_jvp_kernel 2.33 (2.37); 1.83 (3.87); 1.65 (4.72).
 constexpr float kRowsSlack = 40.f;
 
@@ -198,8 +198,10 @@ attn_jvp_rows_kernel(const AttnParams p) {
         }
     };
 
-    // the sums' products, beside those of a group of outputs
-    constexpr int SUMS_AT = 12;
+    // The sums' products, beside those of a group of outputs: the first behind the check (beside the third 0.7 % slower, tangent on q; spread over three groups as well).  All tangents take 0.8 % longer
+    // than with a max that moves at 2^6 and no such sums, tangent on q 0.3 (17600 and 84480 positions, 16 heads, scores of standard deviation 1).
+    constexpr int SUMS_AT = 10;
+    static_assert(SUMS_AT * PER >= CHECK && SUMS_AT < 15, "sums that have the tile before only behind the check, of H before it is formed anew");
     auto sums = [&](auto ki, auto pause) __attribute__((always_inline)) {
         constexpr int K = decltype(ki)::value;
         if constexpr (K < NG) M::template more<decltype(pause)::value, false>(hsum[K], ones, hw[K]);
@@ -316,8 +318,7 @@ attn_jvp_rows_kernel(const AttnParams p) {
     constexpr auto fixed = [](int q) {
         q %= SLOTS;
         const int G = q / PER, k = q % PER;
-        // (a slot with two products has room for two instructions more)
-        return (k == 0) + (FULL && k == 1) + (k == PER - 1) + (k == 2 && G == LOAD_AT ? C::K_LOADS : 0) + (k == 2 && G == LOAD_AT + 2 ? C::V_LOADS : 0) - (G == SUMS_AT && k < 2 * NG ? 2 : 0);
+        return (k == 0) + (FULL && k == 1) + (k == PER - 1) + (k == 2 && G == LOAD_AT ? C::K_LOADS : 0) + (k == 2 && G == LOAD_AT + 2 ? C::V_LOADS : 0);
     };
     constexpr auto room = [fixed](int q0, int q) {
         int c = 0;
