@@ -10,8 +10,8 @@
 // and what is issued beside it.  Measured of a wavefront that has its SIMD to itself, per v_mfma_f32_16x16x32 of 16 cycles: with two other instructions 18 cycles, three 22,
 // four 26 (an exponential counts twice).  A step has 32 NG products and, at NG = 4, 2.3 others to a product, spread evenly (fixed(), room(), exp_before(), ds_before());
 // placed where they are needed first, with all LDS reads of a group in one slot, a step took 3100 cycles instead of 2810.
-// The kernel before this one handed P and dS from wavefronts that formed them to wavefronts that held the accumulators, through LDS, 128 keys a workgroup.  At 16 heads x
-// 24640 queries and keys, dS kept: 17.7 -> 13.1 million cycles, clock 1.84 -> 1.57 GHz, 9.63 -> 8.36 ms; the backward, us, 24640 13 870 -> 12 160, 10920 2750 -> 2465,
+// The kernel before this one handed P and dS from wavefronts that formed them to wavefronts that held the accumulators, through LDS, 128 keys a workgroup.  At 2 heads x
+// 84480 queries and keys, dS kept: 26.2 -> 19.0 million cycles, clock 1.91 -> 1.73 GHz, 13.7 -> 11.0 ms; the backward, us, 16 heads, 24640 13 870 -> 12 160, 10920 2750 -> 2465,
 // 5000 (40 heads) 1578 -> 1398, 3520 330 -> 294, 37440 x 512 571 -> 526, 37440 x 300 468 -> 422.
 //
 // v_mfma_f32_16x16x32: lane (i = lane % 16, g = lane / 16) of an operand has the contraction's elements 8 g .. + 7 of row or column i; of a result column i and rows 4 g .. + 3.

@@ -47,6 +47,7 @@ constexpr int kFragBytes = 1024;   // one MFMA A-operand fragment: 64 lanes x 16
 // reference m, and 16-bit rounding of p is relative, so nothing is lost; what is gained is that the rescaling pass over
 // the accumulators, which otherwise runs in nearly every one of a sweep's first dozens of steps (in every step of a short
 // sweep), runs about once per sweep.
+// (attn_jvp_rows_kernel: kRowsSlack.)
 constexpr float kMaxSlack = 6.0f;
 // attn_fwd_sym_kernel reads whether the max has to move off the row sums instead: a lane's sum of the exponentials of its 16 keys of a tile is
 // at least its largest one, and is formed anyway.  A tile whose lane sums all stay within 2^kMaxSlack is done; otherwise (or if a sum is no

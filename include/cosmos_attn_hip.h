@@ -76,8 +76,9 @@ typedef struct cosmos_attn_desc {
     int64_t o_stride[3];     /* (batch, head, row) element strides of o and to (d stride 1) */
     float *lse;              /* [B,H,Lq] fp32 contiguous: natural-log logsumexp of the scaled scores (JVP:367,376); may be NULL */
 
-    const int32_t *key_lens; /* optional [B] int32 (device): keys >= key_lens[b] are masked out.  No counterpart in the
-                                reference, which never masks (ATT:94-95 ignores k_lens); pinned by the torch oracle. */
+    const int32_t *key_lens; /* optional [B] int32 (device): keys >= key_lens[b] are masked out (their values are read
+                                and have to be finite).  No counterpart in the reference, which never masks
+                                (ATT:94-95 ignores k_lens); pinned by the torch oracle. */
 } cosmos_attn_desc;
 
 /* ABI version of the loaded library. */
